@@ -54,6 +54,20 @@ __device__ __forceinline__ long xcd_tile(long b, long ntiles)
     return (b % kXcds) * m + b / kXcds;
 }
 
+// Work decomposition of the modal operator kernels (modal.hip): strips of W
+// nodes along j, R = W + 1 list columns, blocks of NW waves owning M list
+// entries and TI node layers.  NW = 0: the grid is past the kernel's 32-bit
+// offsets.
+constexpr int kMdMaxWaves = 8;
+struct ModalWork {
+    int NW = 0, W = 0, R = 0, M = 0, TI = 0;
+    int ns = 0, nch = 0, nib = 0;
+    __host__ __device__ long blocks() const { return (long)ns * nch * nib; }
+};
+// el 0: one scale per element, 1: the level-1 element (children: 8 scales)
+ModalWork modal_work(const Grid &g, int bytes, int el, int children);
+bool modal_constants(const double *Ke0, double *C);      // C[8]; false: Ke0 has no isotropic modal form
+
 Tile choose_tile(const Grid &g);   // level-0 node-gather bricks
 Tile stored_tile(const Grid &g);   // stored-matrix operator (at most kStNodes nodes)
 
@@ -69,6 +83,8 @@ struct OpArgsT {
     const T *U;            // input vector
     const T *F;            // right-hand side (defect / Jacobi)
     const T *AD;           // diagonal (Jacobi)
+    const T *RD;           // 1/AD for the modal kernels (null: no Jacobi or prerelaxed mode): one value per
+                           // node where Ke0 has one diagonal value, per DOF for the level-1 operator
     const uint8_t *mask;   // per node: bit d set when DOF 3n+d is fixed
     T *out;                // result vector
     T *out2;               // second result (prerelax+defect writes U and R)
@@ -80,6 +96,9 @@ struct OpArgsT {
     double cx_floor;       // > 0: element scales below it count as 0 (mgcg9 smoother defect)
     int kc;                // Ke0 has the unit-H8 class structure: use kv
     T kv[kKeMaxClasses];   // value of each Ke0 entry class (kKeClass)
+    int modal;             // Ke0 has the isotropic modal form: use mc and mw
+    T mc[8];               // its modal constants
+    ModalWork mw;          // the level's tiling
 };
 using OpArgs = OpArgsT<double>;
 
@@ -130,16 +149,19 @@ __device__ __forceinline__ void batch_shift(OpArgsT<T> &a)
     a.partials = batch_ptr(a.partials, (long)gridDim.x);
     a.ctl = batch_ctl(a.ctl);
 }
+// values of OpArgsT::RD on level l: per node, per DOF on level 1 (which may be
+// the rediscretised one); it follows AD in one allocation
+inline long rd_len(const Grid &g, int l) { return l == 1 ? g.ndof : g.nnod; }
 inline unsigned batch_dim(int nb) { return nb > 1 ? (unsigned)nb : 1u; }
 
 struct Level {
     Grid g;
     Tile t;
-    Tile tmf;                     // tiling of the matrix-free level-1 operator (FP32)
-    Tile tmf64;                   // its FP64 tiling (half the elements per block)
+    ModalWork mw32, mw64;         // tilings of the modal operator (level 1 of REF_C: of its matrix-free operator)
     Tile tg;                      // node-gather tiling of this level (matrix-free levels)
     double *CXl = nullptr;        // element scales of a matrix-free coarse level (mgcg9)
     double *U = nullptr, *F = nullptr, *R = nullptr, *AD = nullptr, *T = nullptr;
+    double *RD = nullptr;         // 1/AD of the levels the modal kernels apply (OpArgsT::RD)
     double *A = nullptr;          // packed element matrices (levels >= 1)
     double *S = nullptr;          // the level's operator as node stencils (stored levels below the coarsest)
     uint8_t *mask = nullptr;      // fixed-DOF node mask
@@ -203,6 +225,8 @@ struct gputo_handle {
     double *Ke = nullptr;         // fine element matrix (row-major, symmetric)
     int ke_classes = 0;           // Ke has the unit-H8 class structure (values in kv)
     double kv[gputo::kKeMaxClasses] = {};
+    int ke_modal = 0;             // and the isotropic modal form (constants in mc)
+    double mc[8] = {};
     double *Aelm = nullptr;       // level-1 Gauss-point matrices, packed [300][8]
     double *CX = nullptr;         // element scales of level 0
     double *Fv = nullptr, *Uv = nullptr, *R = nullptr, *P = nullptr, *Q = nullptr, *Z = nullptr;
@@ -232,9 +256,25 @@ namespace gputo {
 // ---- launch helpers (kernels.hip) ------------------------------------
 template <class T> void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a);
 void launch_op0_uf(hipStream_t s, const OpArgs &a);  // OP_MATVEC_UF
+template <class T> void launch_op0_modal(hipStream_t s, int mode, const OpArgsT<T> &a);
+// whether launch_op0 takes the modal kernel for `mode`, and the blocks
+// (= partial sums per right-hand side) of its launch
+template <class T>
+inline bool op0_is_modal(const OpArgsT<T> &a, int mode)
+{
+    return a.modal && a.mw.NW > 0 && (a.RD || mode == OP_MATVEC || mode == OP_MATVEC_UF || mode == OP_DEFECT);
+}
+template <class T>
+inline int op0_blocks(const OpArgsT<T> &a, int mode)
+{
+    return (int)xcd_launch(op0_is_modal(a, mode) ? a.mw.blocks() : a.t.blocks());
+}
 template <class T> void launch_opA(hipStream_t s, int mode, const OpArgsT<T> &a);
-void launch_diag0(hipStream_t s, const Grid &g, const double *Ke, const double *CX, double *AD);
-void launch_diagA(hipStream_t s, const Grid &g, const double *A, double *AD);
+// AD and, when RD is not null, 1/AD (launch_diag0: of the first DOF of each
+// node; the diagonal entries of an isotropic Ke0 are equal)
+void launch_diag0(hipStream_t s, const Grid &g, const double *Ke, const double *CX, double *AD, double *RD = nullptr);
+void launch_diagA(hipStream_t s, const Grid &g, const double *A, double *AD, double *RD = nullptr);
+void launch_recip(hipStream_t s, const double *AD, double *RD, long n, int stride);  // RD[i] = 1/AD[stride i]
 // S = the operator of the packed element matrices A as node stencils
 void launch_stencil_build(hipStream_t s, const Grid &g, const double *A, double *S);
 constexpr int kStencilEntries = 126;  // the own and 13 forward 3 x 3 blocks per node (the rest by symmetry)

@@ -294,6 +294,7 @@ __global__ __launch_bounds__(kBlock) void k_gather(OpArgsT<T> a)
 template <class T>
 void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a)
 {
+    if (op0_is_modal(a, mode)) return launch_op0_modal<T>(s, mode, a);
     const dim3 grid((unsigned)xcd_launch(a.t.blocks()), 1, batch_dim(a.nb)), block(kBlock);
     if (a.kc) {
         switch (mode) {
@@ -642,6 +643,7 @@ template void launch_op0<double>(hipStream_t, int, const OpArgsT<double> &);
 
 void launch_op0_uf(hipStream_t s, const OpArgs &a)
 {
+    if (op0_is_modal(a, OP_MATVEC_UF)) return launch_op0_modal<double>(s, OP_MATVEC_UF, a);
     const dim3 grid((unsigned)xcd_launch(a.t.blocks()), 1, batch_dim(a.nb)), block(kBlock);
     if (a.kc)
         k_gather<double, OP_MATVEC_UF, true><<<grid, block, 0, s>>>(a);
@@ -658,7 +660,8 @@ template void launch_opA<float>(hipStream_t, int, const OpArgsT<float> &);
 // ---------------------------------------------------------------------------
 template <bool STORED>
 __global__ __launch_bounds__(kBlock) void k_diag(Grid g, const double *__restrict__ Ke, const double *__restrict__ CX,
-                                                const double *__restrict__ A, double *__restrict__ AD)
+                                                const double *__restrict__ A, double *__restrict__ AD,
+                                                double *__restrict__ RD)
 {
     const long nod = (long)blockIdx.x * kBlock + threadIdx.x;
     if (nod >= g.nnod) return;
@@ -682,19 +685,33 @@ __global__ __launch_bounds__(kBlock) void k_diag(Grid g, const double *__restric
                     d[c] += STORED ? A[pidx(m, m) * g.nel + e] : CX[e] * Ke[25 * m];
                 }
             }
-    AD[3 * nod + 0] = d[0];
-    AD[3 * nod + 1] = d[1];
-    AD[3 * nod + 2] = d[2];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        AD[3 * nod + c] = d[c];
+        if (RD && STORED) RD[3 * nod + c] = 1.0 / d[c];
+    }
+    if (RD && !STORED) RD[nod] = 1.0 / d[0];
 }
 
-void launch_diag0(hipStream_t s, const Grid &g, const double *Ke, const double *CX, double *AD)
+void launch_diag0(hipStream_t s, const Grid &g, const double *Ke, const double *CX, double *AD, double *RD)
 {
-    k_diag<false><<<(unsigned)((g.nnod + kBlock - 1) / kBlock), kBlock, 0, s>>>(g, Ke, CX, nullptr, AD);
+    k_diag<false><<<(unsigned)((g.nnod + kBlock - 1) / kBlock), kBlock, 0, s>>>(g, Ke, CX, nullptr, AD, RD);
 }
 
-void launch_diagA(hipStream_t s, const Grid &g, const double *A, double *AD)
+void launch_diagA(hipStream_t s, const Grid &g, const double *A, double *AD, double *RD)
 {
-    k_diag<true><<<(unsigned)((g.nnod + kBlock - 1) / kBlock), kBlock, 0, s>>>(g, nullptr, nullptr, A, AD);
+    k_diag<true><<<(unsigned)((g.nnod + kBlock - 1) / kBlock), kBlock, 0, s>>>(g, nullptr, nullptr, A, AD, RD);
+}
+
+__global__ void k_recip(const double *__restrict__ AD, double *__restrict__ RD, long n, int stride)
+{
+    const long i = (long)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) RD[i] = 1.0 / AD[stride * i];
+}
+
+void launch_recip(hipStream_t s, const double *AD, double *RD, long n, int stride)
+{
+    k_recip<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(AD, RD, n, stride);
 }
 
 // ---------------------------------------------------------------------------

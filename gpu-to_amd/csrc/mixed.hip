@@ -39,7 +39,8 @@ void mixed_create(gputo_handle *h)
         v.U = malloc_dev<float>(m, g.ndof);
         v.F = malloc_dev<float>(m, g.ndof);
         v.R = malloc_dev<float>(m, g.ndof);
-        v.AD = malloc_dev<float>(m, g.ndof);
+        v.AD = malloc_dev<float>(m, g.ndof + rd_len(g, l));
+        v.RD = v.AD + g.ndof;
         v.Tmp = malloc_dev<float>(m, g.ndof);
         if (l > 0) {
             float *A = malloc_dev<float>(m, 300 * g.nel);
@@ -109,13 +110,15 @@ static void mixed_prepare(gputo_handle *h)
     const Grid &g0 = h->L[0].g;
     launch_copy<double, float>(s, h->Ke, m->Ke32, 576, nullptr);
     launch_copy<double, float>(s, h->CX, m->CX32, g0.nel, nullptr);
-    m->H.l1_mf = use_l1_mf(h->prm, h->nl);
+    m->H.l1_mf = use_l1_mf(h->prm, h->nl, h->L[1].mw64);
     m->H.mg9 = preset_of(h->prm).mg9;
     m->H.per = h->prm.periodic != 0;
     if (m->H.mg9 && !h->C.direct) launch_fill<float>(s, m->H.L[h->nl - 1].U, h->L[h->nl - 1].g.ndof, 0.0);
     for (int l = 0; l < h->nl; ++l) {
         const Level &v = h->L[l];
         launch_copy<double, float>(s, v.AD, m->H.L[l].AD, v.g.ndof, nullptr);
+        if (l <= 1 || m->H.mg9)
+            launch_copy<double, float>(s, v.RD, m->H.L[l].RD, l == 0 || m->H.mg9 ? v.g.nnod : v.g.ndof, nullptr);
         if (m->H.mg9) {
             if (l > 0) launch_copy<double, float>(s, v.CXl, m->CXl32[l], v.g.nel, nullptr);
         } else if (l > 0 && !(l == 1 && m->H.l1_mf)) {
@@ -126,7 +129,7 @@ static void mixed_prepare(gputo_handle *h)
                 launch_copy<double, float>(s, v.A, m->A32[l], 300 * v.g.nel, nullptr);
         }
     }
-    m->H.l0 = l0_kind(h->prm, h->prm.precision);
+    m->H.l0 = l0_resolve(h, l0_kind(h->prm, h->prm.precision));
     m->H.l0_ctx = m;
     m->H.learn = h->ln != nullptr;
 }
@@ -238,7 +241,7 @@ int mixed_apply_l0(gputo_handle *h, int kind, const double *u, double *y)
     const Grid &g0 = h->L[0].g;
     launch_copy<double, float>(s, h->Ke, m->Ke32, 576, nullptr);
     launch_copy<double, float>(s, h->CX, m->CX32, g0.nel, nullptr);
-    m->H.l0 = kind;
+    m->H.l0 = l0_resolve(h, kind);
     m->H.l0_ctx = m;
     launch_copy<double, float>(s, u, m->P, g0.ndof, nullptr);
     OpArgsT<float> a = view_args(h, m->H, 0, nullptr);
@@ -269,7 +272,7 @@ int mixed_bench_operator(gputo_handle *h, int kind, int reps, double *avg_ms)
     MixedState *m = h->mx;
     hipStream_t s = h->stream;
     mixed_prepare(h);
-    m->H.l0 = kind;
+    m->H.l0 = l0_resolve(h, kind);
     launch_fill<float>(s, m->P, h->L[0].g.ndof, 1.0);
     OpArgsT<float> a = view_args(h, m->H, 0, nullptr);
     a.U = m->P;

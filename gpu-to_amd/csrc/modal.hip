@@ -1,0 +1,747 @@
+// Matrix-free hex operators in the element's modal basis: the level-0
+// operator of a unit-H8 Ke0 (multAV0c / defect0c, Cantilever/TOP3D125MGCGCUDA/
+// mgcg1.cu:941-997,1208-1264), the same operator on every level of the mgcg9
+// engine, and the rediscretised level-1 operator of the REF_C hierarchy
+// (coarseAe2c applied with defectc, mgcg1.cu:2042-2070,1266-1324) from the
+// child densities.
+//
+// Modal basis.  Along each direction a node pair (u0, u1) becomes the sum
+// u0 + u1 (index 0) and the difference u1 - u0 (index 1); the 8 values of one
+// displacement component become 8 modes m(a, b, c).  The three reflections of
+// the cube leave an isotropic element unchanged, so its matrix couples only
+// modes of equal parity, and the 24 x 24 products shrink to 33 operations:
+//   m(1,0,0) of u, m(0,1,0) of v, m(0,0,1) of w   normal strains (full 3 x 3)
+//   u(0,1,0) + v(1,0,0) and its two rotations      shears (rank one)
+//   v(1,1,0), w(1,0,1) and their two rotations     bending pairs (2 x 2)
+//   u(0,1,1), v(1,0,1), w(1,1,0)                   twist (full 3 x 3)
+//   u(1,1,1), v(1,1,1), w(1,1,1)                   one value each
+// and the three translations to nothing.  Sums and differences are formed
+// once per node pair along j, once per face along k and i.  Per element that
+// is about 190 operations in place of 576 multiply-adds, and the differences
+// are taken between neighbouring nodes first, so a smooth field loses no
+// digits in the products.  The level-1 operator uses the same basis: the
+// displacement gradient at the 2 x 2 x 2 Gauss points is a sum and difference
+// transform of the modes again (a derivative along x does not depend on x).
+//
+// Work of a block.  The nodes of a plane i = const are cut into strips of W
+// nodes along j; the strip's rows follow each other in one list of R = W + 1
+// columns each (column c holds element column and node j0 - 1 + c), and a
+// block owns M consecutive entries of that list and TI node layers.  Entry t
+// of a block is thread column t; element t reaches nodes t, t + 1, t + R and
+// t + R + 1, so the block works on R + 1 entries before its own, too.  It
+// marches along i, one element layer per step:
+//   * each lane loads the node pairs (k, j..j+1) and (k+1, j..j+1) of the next
+//     layer (48 contiguous bytes each in FP64) while it works on this one;
+//   * sums and differences along j, k and i, the modal products, and back:
+//     the i direction meets in the lane's registers;
+//   * along j the neighbour's share comes by a one-lane shift (consecutive
+//     waves overlap by one entry, so no lane lacks its neighbour);
+//   * along k it goes through LDS, R entries further, one barrier per layer
+//     (two buffers).
+// No atomics and one fixed order of every sum: results are bitwise
+// deterministic.  Elements outside the mesh take loads past the buffer's
+// range, which return 0, so nothing of a neighbouring row enters a sum.
+//
+// Measured on MI355X at 192x96x96 (matvecs back to back; before: node-gather,
+// split-BF16 MFMA and Gauss point by Gauss point kernels): FP64 level 0
+// 75 -> 29 us (101 MB of operands, 3.5 TB/s; 87 % of the VALU operations are
+// the transforms and products above), FP32 level 0 66 (node-gather) and 23
+// (MFMA) -> 18.6 us, FP64 level 1 34 -> 12.4 us, FP32 level 1 24 -> 8.8 us;
+// an FP64 Jacobi sweep in the solve 65 -> 37 us, an FP32 one 34 (MFMA) ->
+// 25 us.  At 16x8x8 a launch takes 3.5 us against 8-10 us: 27 x 24 dependent
+// products per node are gone.  Level 0 is bound by memory and by the two
+// waves per SIMD that cover its latency.
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
+
+#include "vcycle.h"
+
+namespace gputo {
+
+namespace {
+
+typedef float f32x2m __attribute__((ext_vector_type(2)));
+typedef float f32x4m __attribute__((ext_vector_type(4)));
+typedef double f64x2m __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t MdBuf;
+
+constexpr int kMdOut = 0x7f000000;  // a byte offset past every buffer (vectors are below it)
+
+__device__ __forceinline__ MdBuf md_buf(const void *p, long bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes, 0x00020000);
+}
+
+__device__ __forceinline__ f64x2m md_ld2d(MdBuf b, int off, int soff)
+{
+    return __builtin_bit_cast(f64x2m, __builtin_amdgcn_raw_buffer_load_b128(b, off, soff, 0));
+}
+__device__ __forceinline__ f32x4m md_ld4f(MdBuf b, int off, int soff)
+{
+    return __builtin_bit_cast(f32x4m, __builtin_amdgcn_raw_buffer_load_b128(b, off, soff, 0));
+}
+__device__ __forceinline__ f32x2m md_ld2f(MdBuf b, int off, int soff)
+{
+    return __builtin_bit_cast(f32x2m, __builtin_amdgcn_raw_buffer_load_b64(b, off, soff, 0));
+}
+template <class T>
+__device__ __forceinline__ T md_ld1(MdBuf b, int off, int soff);
+template <>
+__device__ __forceinline__ double md_ld1<double>(MdBuf b, int off, int soff)
+{
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, off, soff, 0));
+}
+template <>
+__device__ __forceinline__ float md_ld1<float>(MdBuf b, int off, int soff)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(b, off, soff, 0));
+}
+
+// six consecutive values: a node pair along j
+__device__ __forceinline__ void md_ld6(MdBuf b, int off, int soff, double (&v)[6])
+{
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const f64x2m x = md_ld2d(b, off + 16 * q, soff);
+        v[2 * q] = x[0];
+        v[2 * q + 1] = x[1];
+    }
+}
+__device__ __forceinline__ void md_ld6(MdBuf b, int off, int soff, float (&v)[6])
+{
+    const f32x4m x = md_ld4f(b, off, soff);
+    const f32x2m y = md_ld2f(b, off + 16, soff);
+    v[0] = x[0];
+    v[1] = x[1];
+    v[2] = x[2];
+    v[3] = x[3];
+    v[4] = y[0];
+    v[5] = y[1];
+}
+// two consecutive values
+__device__ __forceinline__ void md_ld2(MdBuf b, int off, int soff, double (&v)[2])
+{
+    const f64x2m x = md_ld2d(b, off, soff);
+    v[0] = x[0];
+    v[1] = x[1];
+}
+__device__ __forceinline__ void md_ld2(MdBuf b, int off, int soff, float (&v)[2])
+{
+    const f32x2m x = md_ld2f(b, off, soff);
+    v[0] = x[0];
+    v[1] = x[1];
+}
+// three consecutive values: one node
+__device__ __forceinline__ void md_ld3(MdBuf b, int off, int soff, double (&v)[3])
+{
+    const f64x2m x = md_ld2d(b, off, soff);
+    v[0] = x[0];
+    v[1] = x[1];
+    v[2] = md_ld1<double>(b, off + 16, soff);
+}
+__device__ __forceinline__ void md_ld3(MdBuf b, int off, int soff, float (&v)[3])
+{
+    const f32x2m x = md_ld2f(b, off, soff);
+    v[0] = x[0];
+    v[1] = x[1];
+    v[2] = md_ld1<float>(b, off + 8, soff);
+}
+
+// the value of the lane below (lane 0: 0), a DPP wave shift
+__device__ __forceinline__ float md_below(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double md_below(double v)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)b, 0x138, 0xf, 0xf, true);
+    const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), 0x138, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Values of one node layer at an element column: [component][b][d], b the
+// mode along j, d the mode along k.
+template <class T>
+struct Jk {
+    T v[3][2][2];
+};
+
+template <class T>
+__device__ __forceinline__ void md_jk(const T (&lo)[6], const T (&hi)[6], Jk<T> &o)
+{
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const T s0 = lo[c] + lo[3 + c], d0 = lo[3 + c] - lo[c];
+        const T s1 = hi[c] + hi[3 + c], d1 = hi[3 + c] - hi[c];
+        o.v[c][0][0] = s0 + s1;
+        o.v[c][0][1] = s1 - s0;
+        o.v[c][1][0] = d0 + d1;
+        o.v[c][1][1] = d1 - d0;
+    }
+}
+
+// Modes m[c][a][b][d] (a along i) to modal forces in place, one scale E for
+// the element (C: the 8 modal constants of Ke0, md_constants).
+template <class T>
+__device__ __forceinline__ void md_element(T (&m)[3][2][2][2], const T *C, T E)
+{
+    {
+        const T t = (C[1] * E) * (m[0][1][0][0] + m[1][0][1][0] + m[2][0][0][1]);
+        const T c0 = C[0] * E;
+        m[0][1][0][0] = fma(c0, m[0][1][0][0], t);
+        m[1][0][1][0] = fma(c0, m[1][0][1][0], t);
+        m[2][0][0][1] = fma(c0, m[2][0][0][1], t);
+    }
+    {
+        const T c2 = C[2] * E;
+        m[0][0][1][0] = m[1][1][0][0] = c2 * (m[0][0][1][0] + m[1][1][0][0]);
+        m[1][0][0][1] = m[2][0][1][0] = c2 * (m[1][0][0][1] + m[2][0][1][0]);
+        m[0][0][0][1] = m[2][1][0][0] = c2 * (m[0][0][0][1] + m[2][1][0][0]);
+    }
+    {
+        const T c3 = C[3] * E;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) m[c][1][1][1] *= c3;
+    }
+    {
+        const T c4 = C[4] * E, c5 = C[5] * E;
+        T p, q;
+        p = m[1][1][1][0], q = m[2][1][0][1];
+        m[1][1][1][0] = fma(c4, p, c5 * q);
+        m[2][1][0][1] = fma(c4, q, c5 * p);
+        p = m[0][1][1][0], q = m[2][0][1][1];
+        m[0][1][1][0] = fma(c4, p, c5 * q);
+        m[2][0][1][1] = fma(c4, q, c5 * p);
+        p = m[0][1][0][1], q = m[1][0][1][1];
+        m[0][1][0][1] = fma(c4, p, c5 * q);
+        m[1][0][1][1] = fma(c4, q, c5 * p);
+    }
+    {
+        const T t = (C[7] * E) * (m[0][0][1][1] + m[1][1][0][1] + m[2][1][1][0]);
+        const T c6 = C[6] * E;
+        m[0][0][1][1] = fma(c6, m[0][0][1][1], t);
+        m[1][1][0][1] = fma(c6, m[1][1][0][1], t);
+        m[2][1][1][0] = fma(c6, m[2][1][1][0], t);
+    }
+}
+
+// Sum and difference transform of four values over two directions.
+template <class T>
+__device__ __forceinline__ void md_had4(T (&g)[2][2])
+{
+    const T a = g[0][0] + g[1][0], b = g[0][1] + g[1][1], c = g[0][0] - g[1][0], d = g[0][1] - g[1][1];
+    g[0][0] = a + b;
+    g[0][1] = a - b;
+    g[1][0] = c + d;
+    g[1][1] = c - d;
+}
+
+// The same with one scale per Gauss point (the level-1 operator: the scale
+// of the child at that point), cx[sx][sy][sz], s = 1 the point at +1/sqrt3.
+// C[0] = lam, C[1] = 2 mu, C[2] = mu, each times the 1/64 of the two
+// transforms; C[3] = 1/sqrt3.  A mode of order n enters its derivatives with
+// (1/sqrt3)^(n - 1) and its force collects them with the same weight.
+template <class T>
+__device__ __forceinline__ void md_element_gp(T (&m)[3][2][2][2], const T *C, const T (&cx)[2][2][2])
+{
+    const T g1 = C[3], g2 = C[3] * C[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        m[c][1][1][0] *= g1;
+        m[c][1][0][1] *= g1;
+        m[c][0][1][1] *= g1;
+        m[c][1][1][1] *= g2;
+    }
+    // gradients G[c][x] at (sy, sz), G[c][y] at (sx, sz), G[c][z] at (sx, sy);
+    // index 0 of a transform's result is the point at +1/sqrt3
+    T gx[3][2][2], gy[3][2][2], gz[3][2][2];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                gx[c][p][q] = m[c][1][p][q];
+                gy[c][p][q] = m[c][p][1][q];
+                gz[c][p][q] = m[c][p][q][1];
+            }
+        md_had4(gx[c]);
+        md_had4(gy[c]);
+        md_had4(gz[c]);
+    }
+    // stresses, summed over the direction of the test function's derivative
+    T px[3][2][2], py[3][2][2], pz[3][2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const T e = cx[1 - x][1 - y][1 - z];
+                const T exx = gx[0][y][z], eyy = gy[1][x][z], ezz = gz[2][x][y];
+                const T t = (C[0] * e) * (exx + eyy + ezz);
+                const T c2 = C[1] * e, cm = C[2] * e;
+                const T sxx = fma(c2, exx, t), syy = fma(c2, eyy, t), szz = fma(c2, ezz, t);
+                const T sxy = cm * (gy[0][x][z] + gx[1][y][z]);
+                const T syz = cm * (gz[1][x][y] + gy[2][x][z]);
+                const T szx = cm * (gx[2][y][z] + gz[0][x][y]);
+                const T sx[3] = {sxx, sxy, szx}, sy[3] = {sxy, syy, syz}, sz[3] = {szx, syz, szz};
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    px[c][y][z] = x == 0 ? sx[c] : px[c][y][z] + sx[c];
+                    py[c][x][z] = y == 0 ? sy[c] : py[c][x][z] + sy[c];
+                    pz[c][x][y] = z == 0 ? sz[c] : pz[c][x][y] + sz[c];
+                }
+            }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        md_had4(px[c]);
+        md_had4(py[c]);
+        md_had4(pz[c]);
+        m[c][1][0][0] = px[c][0][0];
+        m[c][0][1][0] = py[c][0][0];
+        m[c][0][0][1] = pz[c][0][0];
+        m[c][1][1][0] = g1 * (px[c][1][0] + py[c][1][0]);
+        m[c][1][0][1] = g1 * (px[c][0][1] + pz[c][1][0]);
+        m[c][0][1][1] = g1 * (py[c][0][1] + pz[c][0][1]);
+        m[c][1][1][1] = g2 * (px[c][1][1] + py[c][1][1] + pz[c][1][1]);
+    }
+}
+
+// Element scales of one element layer at a column: one (level 0) or one per
+// child (level 1).
+template <class T, int EL>
+struct MdScale {
+    T e[EL == 0 ? 1 : 8];
+};
+
+// Waves per SIMD that the registers allow.  A lane holds the modes of the
+// previous layer, of this one and the pending sums (36 values), the next
+// layer's operands (13) and the epilogue's (10): 202-212 registers in FP64
+// and 108-118 in FP32 at level 0; the Gauss points of level 1 add up to 72
+// values, and FP64 takes the whole register file with one wave per SIMD
+// (12.4 us per matvec at 192x96x96; 21.0 us with two waves and 80-230 bytes
+// of scratch per lane).
+template <class T, int EL>
+constexpr int md_min_waves()
+{
+    return sizeof(T) == 8 ? (EL == 0 ? 2 : 1) : (EL == 0 ? 4 : 3);
+}
+
+template <class T, class TU, int MODE, int EL>
+__global__ __launch_bounds__((sizeof(T) == 8 && EL == 1 ? 4 : kMdMaxWaves) * 64) __attribute__((amdgpu_waves_per_eu(md_min_waves<T, EL>())))
+void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
+{
+    constexpr bool PRE = MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT;
+    constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI;
+    constexpr bool MV = MODE == OP_MATVEC || MODE == OP_MATVEC_UF;
+    // the next layer's operands are loaded a layer ahead where the registers
+    // allow it
+    constexpr bool AHEAD = sizeof(T) == 4 ? !PRE : (EL == 0 && !PRE);
+    constexpr int SU = (int)sizeof(TU), S = (int)sizeof(T);
+    batch_shift(a);
+    if (MODE == OP_MATVEC_UF) a.Uf = batch_ptr(a.Uf, a.g.ndof);
+    extern __shared__ double md_lds[];
+    T *ex = reinterpret_cast<T *>(md_lds);  // [2][3][ne]
+    const int ne = 63 * w.NW + 1;
+    const Grid &g = a.g;
+    const unsigned nb = (unsigned)w.blocks();
+    const unsigned tb = (unsigned)xcd_tile(blockIdx.x, nb);
+    if (tb >= nb) {  // padding block of the XCD order
+        if (a.partials && threadIdx.x == 0) a.partials[blockIdx.x] = 0.0;
+        return;
+    }
+    const int ch = (int)(tb % (unsigned)w.nch);
+    const unsigned r1 = tb / (unsigned)w.nch;
+    const int s = (int)(r1 % (unsigned)w.ns), ib = (int)(r1 / (unsigned)w.ns);
+    const int i0 = ib * w.TI, i1 = min(i0 + w.TI, g.nnx);  // owned node layers
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t = wave * 63 + lane;  // the block's entry (a wave's last is the next one's first)
+    // list entry q = ch M - (R + 1) + t -> row k, column c
+    const unsigned qs = (unsigned)(ch * w.M + t + w.R - 1);  // q + 2R >= 0
+    const int kq = (int)(qs / (unsigned)w.R), c = (int)(qs - (unsigned)(kq * w.R));
+    const int k = kq - 2, j = s * w.W - 1 + c;
+    const bool el_ok = k >= 0 && k < g.nz && j >= 0 && j < g.ny;
+    const bool own = lane > 0 && t > w.R && t <= w.R + w.M && c > 0 && k >= 0 && k < g.nnz && j < g.nny;
+    const int plane = g.nny * g.nnz;
+    const int nod0 = k * g.nny + j;  // node in its plane
+    // byte offsets in a plane of the element's two node rows, of its scale(s)
+    // and of the own node
+    const int ulo = el_ok ? 3 * SU * nod0 : kMdOut, uhi = el_ok ? 3 * SU * (nod0 + g.nny) : kMdOut;
+    const int flo = el_ok ? 3 * S * nod0 : kMdOut, fhi = el_ok ? 3 * S * (nod0 + g.nny) : kMdOut;
+    const int eo = el_ok ? (EL == 0 ? S * (k * g.ny + j) : S * (4 * k * g.ny + 2 * j)) : kMdOut;
+    const int oo = own ? 3 * S * nod0 : kMdOut, uo = own ? 3 * SU * nod0 : kMdOut;
+    const long vb = (long)S * g.ndof;
+    const MdBuf BU = PRE ? md_buf(a.F, vb)
+                         : (MODE == OP_MATVEC_UF ? md_buf(a.Uf, (long)SU * g.ndof) : md_buf(a.U, vb));
+    const MdBuf BF = md_buf(a.F, MV ? 0 : vb), BD = md_buf(a.RD, (JAC || PRE) ? (EL == 0 ? vb / 3 : vb) : 0);
+    const MdBuf BE = md_buf(CX, (long)S * (EL == 0 ? 1 : 8) * g.nel), BM = md_buf(a.mask, g.nnod);
+    const int up = 3 * SU * plane, fp = 3 * S * plane;         // bytes of a node layer
+    const int dp = S * plane, dlo = el_ok ? S * nod0 : kMdOut, dhi = el_ok ? S * (nod0 + g.nny) : kMdOut;
+    const int ep = (EL == 0 ? 1 : 4) * S * g.ny * g.nz;        // bytes of a scale layer
+    const T pr = T(a.prerelax), om = T(a.omega);
+
+    struct Raw {
+        TU lo[6], hi[6];
+        T dlo[EL == 0 ? 2 : 6], dhi[EL == 0 ? 2 : 6];  // PRE: 1/AD of the same nodes
+    };
+    auto load = [&](int pl, Raw &x) {
+        md_ld6(BU, PRE ? flo : ulo, pl * (PRE ? fp : up), x.lo);
+        md_ld6(BU, PRE ? fhi : uhi, pl * (PRE ? fp : up), x.hi);
+        if constexpr (PRE && EL == 0) {
+            md_ld2(BD, dlo, pl * dp, x.dlo);
+            md_ld2(BD, dhi, pl * dp, x.dhi);
+        } else if constexpr (PRE) {
+            md_ld6(BD, flo, pl * fp, x.dlo);
+            md_ld6(BD, fhi, pl * fp, x.dhi);
+        }
+    };
+    auto load_e = [&](int ie, MdScale<T, EL> &x) {
+        if (EL == 0) {
+            x.e[0] = md_ld1<T>(BE, eo, ie * ep);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {  // children (is, iz): the pair along j
+                const int off = eo + (q & 1) * 2 * S * g.ny, soff = (2 * ie + (q >> 1)) * ep;
+                if (S == 8) {
+                    const f64x2m v = md_ld2d(BE, off, soff);
+                    x.e[2 * q] = (T)v[0];
+                    x.e[2 * q + 1] = (T)v[1];
+                } else {
+                    const f32x2m v = md_ld2f(BE, off, soff);
+                    x.e[2 * q] = (T)v[0];
+                    x.e[2 * q + 1] = (T)v[1];
+                }
+            }
+        }
+    };
+    auto jk = [&](const Raw &x, Jk<T> &o) {
+        T lo[6], hi[6];
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {
+            lo[q] = PRE ? pr * (T(x.lo[q]) * x.dlo[EL == 0 ? q / 3 : q]) : T(x.lo[q]);
+            hi[q] = PRE ? pr * (T(x.hi[q]) * x.dhi[EL == 0 ? q / 3 : q]) : T(x.hi[q]);
+        }
+        md_jk(lo, hi, o);
+    };
+
+    double part = 0.0;
+    // node layer pl is complete in sum: the k and j directions, the
+    // neighbours' shares and the epilogue
+    struct Epi {
+        T f[3], d[3];
+        TU u[3];
+        unsigned m;
+    };
+    auto load_epi = [&](int pl, Epi &e) {
+        e.m = __builtin_amdgcn_raw_buffer_load_b8(BM, own ? nod0 : kMdOut, pl * plane, 0);
+        if (!MV) md_ld3(BF, oo, pl * fp, e.f);
+        if constexpr (EL == 0) {
+            if (JAC || PRE) e.d[0] = e.d[1] = e.d[2] = md_ld1<T>(BD, own ? S * nod0 : kMdOut, pl * dp);
+        } else {
+            if (JAC || PRE) md_ld3(BD, oo, pl * fp, e.d);
+        }
+        if (!PRE && MODE != OP_DEFECT) md_ld3(BU, uo, pl * up, e.u);
+    };
+    auto finish = [&](int pl, const Jk<T> &sum, const Epi &e) {
+        T y[3];
+        T *buf = ex + (pl & 1) * 3 * ne;
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) {
+            const T l0 = sum.v[cc][0][0] - sum.v[cc][0][1], l1 = sum.v[cc][1][0] - sum.v[cc][1][1];  // row k
+            const T h0 = sum.v[cc][0][0] + sum.v[cc][0][1], h1 = sum.v[cc][1][0] + sum.v[cc][1][1];  // row k + 1
+            y[cc] = (l0 - l1) + md_below(l0 + l1);
+            const T yh = (h0 - h1) + md_below(h0 + h1);
+            if (lane > 0) buf[cc * ne + t] = yh;
+        }
+        __syncthreads();
+        if (!own) return;
+        const long dof = 3 * ((long)pl * plane + nod0);
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) {
+            const T yc = y[cc] + buf[cc * ne + t - w.R];
+            const bool fixed = (e.m >> cc) & 1u;
+            if (MV) {
+                const T v = fixed ? T(0) : yc;
+                a.out[dof + cc] = v;
+                part += (double)e.u[cc] * (double)v;
+            } else if (!JAC) {
+                a.out[dof + cc] = fixed ? T(0) : e.f[cc] - yc;
+                if (PRE) a.out2[dof + cc] = pr * (e.f[cc] * e.d[cc]);
+            } else {
+                // U = (1-w) U + w (R + AD U)/AD = U + w R/AD  (mgcg1.cu:1199-1206)
+                const T u = PRE ? pr * (e.f[cc] * e.d[cc]) : T(e.u[cc]);
+                const T rv = fixed ? T(0) : e.f[cc] - yc;
+                a.out[dof + cc] = fma(om * e.d[cc], rv, u);
+            }
+        }
+    };
+
+    const int lo = max(i0 - 1, 0), hi = min(i1, g.nnx - 1);  // node layers read
+    Raw xa, xb;
+    MdScale<T, EL> ea, eb;
+    load(lo, xa);
+    load(lo + 1, xb);
+    load_e(lo, ea);
+    if (a.ctl && a.ctl[0]) return;  // converged: read with the loads above
+    Jk<T> pa, pb, pend;
+    jk(xa, pa);
+#pragma unroll
+    for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int d = 0; d < 2; ++d) pend.v[cc][b][d] = T(0);
+    // element layer ie = pl - 1 between node layers pl - 1 (modes in prev) and
+    // pl (raw values in x, modes to cur); its loads for the next layer go to
+    // xn, en.  Node layer pl - 1 is complete after it.
+    auto step = [&](int pl, const Jk<T> &prev, Jk<T> &cur, Raw &x, Raw &xn, MdScale<T, EL> &e,
+                    MdScale<T, EL> &en) {
+        const bool emit = pl - 1 >= i0;
+        // loads complete in order for the wait counter: the epilogue's
+        // operands go before the prefetch
+        Epi epi;
+        if (emit && AHEAD) load_epi(pl - 1, epi);
+        if (AHEAD) {
+            if (pl < hi) {
+                load(pl + 1, xn);
+                load_e(pl, en);
+            }
+        } else if (pl > lo + 1) {
+            load(pl, x);
+            load_e(pl - 1, e);
+        }
+        jk(x, cur);
+        T m[3][2][2][2];
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    m[cc][0][b][d] = prev.v[cc][b][d] + cur.v[cc][b][d];
+                    m[cc][1][b][d] = cur.v[cc][b][d] - prev.v[cc][b][d];
+                }
+        if constexpr (EL == 0) {
+            T E = e.e[0];
+            if (a.cx_floor > 0.0 && E < T(a.cx_floor)) E = T(0);  // mgcg9 defect0c skip
+            md_element(m, a.mc, E);
+        } else {
+            const T cx[2][2][2] = {{{e.e[0], e.e[2]}, {e.e[1], e.e[3]}}, {{e.e[4], e.e[6]}, {e.e[5], e.e[7]}}};
+            md_element_gp(m, a.mc, cx);
+        }
+        if (emit && !AHEAD) load_epi(pl - 1, epi);
+        Jk<T> sum;
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    const T r1v = m[cc][1][b][d];
+                    if (b == 0 && d == 0) {  // no force from a translation
+                        sum.v[cc][b][d] = pend.v[cc][b][d] - r1v;
+                        pend.v[cc][b][d] = r1v;
+                    } else {
+                        const T r0v = m[cc][0][b][d];
+                        sum.v[cc][b][d] = pend.v[cc][b][d] + (r0v - r1v);
+                        pend.v[cc][b][d] = r0v + r1v;
+                    }
+                }
+        if (emit) finish(pl - 1, sum, epi);
+    };
+    for (int pl = lo + 1; pl <= hi; pl += 2) {
+        step(pl, pa, pb, xb, AHEAD ? xa : xb, ea, AHEAD ? eb : ea);
+        if (pl + 1 <= hi) step(pl + 1, pb, pa, AHEAD ? xa : xb, xb, AHEAD ? eb : ea, ea);
+    }
+    if (i1 == g.nnx) {  // the last node layer of the mesh ends with what is pending
+        Epi epi;
+        load_epi(g.nnx - 1, epi);
+        finish(g.nnx - 1, pend, epi);
+    }
+    if (MV && a.partials) {
+        // fixed butterfly per wave, then the waves in order
+        __shared__ double ws[kMdMaxWaves];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
+        if (lane == 0) ws[wave] = part;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double v = 0.0;
+            for (int q = 0; q < w.NW; ++q) v += ws[q];
+            a.partials[blockIdx.x] = v;
+        }
+    }
+}
+
+template <class T, int EL>
+void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
+{
+    const ModalWork &w = a.mw;
+    const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb)), block(64 * w.NW);
+    const unsigned lds = 6u * (63u * w.NW + 1u) * sizeof(T);
+    switch (mode) {
+    case OP_MATVEC: k_modal<T, T, OP_MATVEC, EL><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_DEFECT: k_modal<T, T, OP_DEFECT, EL><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_JACOBI: k_modal<T, T, OP_JACOBI, EL><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_PRE_JACOBI: k_modal<T, T, OP_PRE_JACOBI, EL><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_PRE_DEFECT: k_modal<T, T, OP_PRE_DEFECT, EL><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_MATVEC_UF:
+        if constexpr (EL == 0 && std::is_same<T, double>::value)
+            k_modal<double, float, OP_MATVEC_UF, 0><<<grid, block, lds, s>>>(a, w, CX);
+        break;
+    default: break;
+    }
+}
+
+}  // namespace
+
+template <class T>
+void launch_op0_modal(hipStream_t s, int mode, const OpArgsT<T> &a)
+{
+    launch<T, 0>(s, mode, a, a.CX);
+}
+template void launch_op0_modal<double>(hipStream_t, int, const OpArgsT<double> &);
+template void launch_op0_modal<float>(hipStream_t, int, const OpArgsT<float> &);
+
+template <class T>
+void launch_op1_mf(hipStream_t s, int mode, OpArgsT<T> a, const T *CXf, double nu)
+{
+    // Lame constants of D (E = 1), the 1/8 of each transform and the element
+    // of side h = 2: |J| w_g = 1, a derivative is half a node difference
+    const double c1 = 1.0 / ((1 + nu) * (1 - 2 * nu)) / 64.0;
+    a.mc[0] = T(c1 * nu);
+    a.mc[1] = T(c1 * (1 - 2 * nu));
+    a.mc[2] = T(c1 * (1 - 2 * nu) / 2);
+    a.mc[3] = T(1.0 / std::sqrt(3.0));
+    launch<T, 1>(s, mode, a, CXf);
+}
+template void launch_op1_mf<double>(hipStream_t, int, OpArgsT<double>, const double *, double);
+template void launch_op1_mf<float>(hipStream_t, int, OpArgsT<float>, const float *, double);
+
+// sums and differences of the 8 nodal entries x[n * stride] to modes
+// 4a + 2b + d, times 1/8
+static void modal_row(const double *x, int stride, double *m)
+{
+    // node order ie = {0,1,1,0,0,1,1,0}, je = {0,0,1,1,0,0,1,1}, ke = {0,0,0,0,1,1,1,1}
+    static const int node[8] = {0, 4, 3, 7, 1, 5, 2, 6};  // of 4 x + 2 y + z
+    double v[8];
+    for (int q = 0; q < 8; ++q) v[q] = 0.125 * x[node[q] * stride];
+    for (int h = 1; h < 8; h *= 2)
+        for (int q = 0; q < 8; ++q)
+            if (!(q & h)) {
+                const double a = v[q], b = v[q + h];
+                v[q] = a + b;
+                v[q + h] = b - a;
+            }
+    for (int q = 0; q < 8; ++q) m[q] = v[q];
+}
+
+// The 8 modal constants of Ke0; false when its modal matrix is not of the
+// isotropic form above to rounding (1e-14 of its largest entry).
+bool modal_constants(const double *Ke0, double *C)
+{
+    double W[24][24], M[24][24], r8[8];  // M[3q + c][3p + d], mode q = 4a + 2b + d
+    for (int col = 0; col < 24; ++col)
+        for (int c = 0; c < 3; ++c) {
+            modal_row(Ke0 + 24 * c + col, 72, r8);
+            for (int q = 0; q < 8; ++q) W[3 * q + c][col] = r8[q];
+        }
+    for (int row = 0; row < 24; ++row)
+        for (int d = 0; d < 3; ++d) {
+            modal_row(W[row] + d, 3, r8);
+            for (int p = 0; p < 8; ++p) M[row][3 * p + d] = r8[p];
+        }
+    // id of the constant expected at (mode, mode), 0 for none (the 3 x 3
+    // blocks: diagonal = off-diagonal + own)
+    int id[24][24] = {};
+    const int n0[3] = {3 * 4 + 0, 3 * 2 + 1, 3 * 1 + 2};  // u100, v010, w001
+    const int tw[3] = {3 * 3 + 0, 3 * 5 + 1, 3 * 6 + 2};  // u011, v101, w110
+    const int sh[3][2] = {{3 * 2 + 0, 3 * 4 + 1}, {3 * 1 + 1, 3 * 2 + 2}, {3 * 1 + 0, 3 * 4 + 2}};
+    const int bd[3][2] = {{3 * 6 + 1, 3 * 5 + 2}, {3 * 6 + 0, 3 * 3 + 2}, {3 * 5 + 0, 3 * 3 + 1}};
+    for (int p = 0; p < 3; ++p) {
+        for (int q = 0; q < 3; ++q) {
+            id[n0[p]][n0[q]] = p == q ? 1 : 2;
+            id[tw[p]][tw[q]] = p == q ? 7 : 8;
+        }
+        for (int x = 0; x < 2; ++x)
+            for (int y = 0; y < 2; ++y) {
+                id[sh[p][x]][sh[p][y]] = 3;
+                id[bd[p][x]][bd[p][y]] = x == y ? 5 : 6;
+            }
+        id[3 * 7 + p][3 * 7 + p] = 4;
+    }
+    double sum[9] = {}, big = 0.0;
+    int cnt[9] = {};
+    for (int r = 0; r < 24; ++r)
+        for (int c = 0; c < 24; ++c) {
+            big = std::max(big, std::fabs(M[r][c]));
+            sum[id[r][c]] += M[r][c];
+            ++cnt[id[r][c]];
+        }
+    double v[9] = {};
+    for (int q = 1; q < 9; ++q) v[q] = sum[q] / cnt[q];
+    for (int r = 0; r < 24; ++r)
+        for (int c = 0; c < 24; ++c)
+            if (!(std::fabs(M[r][c] - v[id[r][c]]) <= 1e-14 * big)) return false;  // NaN fails too
+    C[0] = v[1] - v[2];
+    C[1] = v[2];
+    C[2] = v[3];
+    C[3] = v[4];
+    C[4] = v[5];
+    C[5] = v[6];
+    C[6] = v[7] - v[8];
+    C[7] = v[8];
+    return true;
+}
+
+// Tiling of grid g for values of `bytes` bytes (el: the level-1 element;
+// children: element scales per element at most).
+// Among waves per block NW, strips along j and the layers TI that fill one,
+// two or three rounds of resident blocks, the smallest modelled time: rounds
+// times the layers a block marches (its first needs the layer before it, and
+// a block takes about two layers' time to start and to end), times the work
+// of a layer, which is bound by the waves that share a SIMD or, when there
+// are few, by one layer's latency.
+ModalWork modal_work(const Grid &g, int bytes, int el, int children)
+{
+    ModalWork best;
+    // 32-bit byte offsets
+    if ((long)bytes * g.ndof >= kMdOut || (long)bytes * children * g.nel >= kMdOut) return best;
+    const int waves = bytes == 8 ? (el ? 1 : 2) : (el ? 3 : 4);  // resident per SIMD (md_min_waves)
+    const double per_wave = el ? 0.9 : 0.38;                     // a wave's layer with its SIMD alone, in us
+    const double latency = 1.2;
+    double cost = 0.0;
+    for (int NW = 1; NW <= (bytes == 8 && el ? 4 : kMdMaxWaves); NW *= 2)
+        for (int ns = 1; ns <= 8; ++ns) {
+            const int W = (g.nny + ns - 1) / ns, R = W + 1;
+            if (ns > 1 && W < 12) break;
+            if (63 * NW - R < 16) continue;
+            const int M = std::min(63 * NW - R, R * g.nnz);
+            const int nsr = (g.nny + W - 1) / W, nch = (R * g.nnz + M - 1) / M;
+            const long per_cu = std::max(1, 4 * waves / NW), slots = 256 * per_cu;
+            for (int round = 1; round <= 3; ++round) {
+                const long fit = std::max(1L, round * slots / ((long)nsr * nch));
+                const int TI = (int)((g.nnx + fit - 1) / fit), nib = (g.nnx + TI - 1) / TI;
+                const long blocks = (long)nsr * nch * nib;
+                const long rounds = (blocks + slots - 1) / slots, on_cu = std::min(per_cu, (blocks + 255) / 256);
+                const double c = rounds * (TI + 3) * std::max(latency, per_wave * (double)(on_cu * NW) / 4.0);
+                if (best.NW == 0 || c < 0.999 * cost) {
+                    cost = c;
+                    best.NW = NW;
+                    best.W = W;
+                    best.R = R;
+                    best.M = M;
+                    best.ns = nsr;
+                    best.nch = nch;
+                    best.TI = TI;
+                    best.nib = nib;
+                }
+            }
+        }
+    return best;
+}
+
+}  // namespace gputo

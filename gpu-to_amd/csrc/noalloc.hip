@@ -96,6 +96,8 @@ extern "C" int gputo_matvec_f64_noalloc(int nelx, int nely, int nelz, const doub
     a.g = g;
     a.t = choose_tile(g);
     a.kc = 1;
+    a.modal = modal_constants(Ke0, a.mc);
+    if (a.modal) a.mw = modal_work(g, 8, 0, 1);
     a.CX = d_CX;
     a.U = d_u;
     a.mask = mask;

@@ -38,6 +38,7 @@ void set_ke(gputo_handle *h, const double *Ke0)
     int ok = 1;
     for (int q = 0; q < 576 && ok; ++q) ok = std::memcmp(&Ke0[q], &h->kv[kKeClass[q]], sizeof(double)) == 0;
     h->ke_classes = ok;
+    h->ke_modal = ok && modal_constants(Ke0, h->mc);
 }
 
 Grid make_grid(int nx, int ny, int nz)
@@ -222,6 +223,7 @@ HierView<double> f64_view(const gputo_handle *h)
         H.L[l].F = v.F;
         H.L[l].R = v.R;
         H.L[l].AD = v.AD;
+        H.L[l].RD = v.RD;
         H.L[l].Tmp = v.T;
         H.L[l].A = v.A;
         H.L[l].S = v.S;
@@ -229,7 +231,7 @@ HierView<double> f64_view(const gputo_handle *h)
     }
     H.Ke = h->Ke;
     H.CX = h->CX;
-    H.l1_mf = use_l1_mf(h->prm, h->nl);
+    H.l1_mf = use_l1_mf(h->prm, h->nl, h->L[1].mw64);
     H.mg9 = preset_of(h->prm).mg9;
     H.per = h->prm.periodic != 0;
     return H;
@@ -328,8 +330,13 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         h->masks_ready = true;
     }
     const bool per = h->prm.periodic != 0;
-    launch_diag0(s, L0.g, h->Ke, h->CX, L0.AD);
-    if (per) launch_per_fold<double>(s, L0.g, L0.AD, 1, nullptr);
+    launch_diag0(s, L0.g, h->Ke, h->CX, L0.AD, per ? nullptr : L0.RD);
+    // RD: per node where the modal kernel applies Ke0 itself, else per DOF
+    auto fold_diag = [&](Level &v, bool node) {
+        launch_per_fold<double>(s, v.g, v.AD, 1, nullptr);
+        launch_recip(s, v.AD, v.RD, node ? v.g.nnod : v.g.ndof, node ? 3 : 1);
+    };
+    if (per) fold_diag(L0, true);
     if (p.mg9) {
         // mgcg9 (initVcycle, mgcg9.cu:342-414): coarse element scales and
         // diagonals from the unit Ke; the coarsest matrix, when factored,
@@ -355,8 +362,8 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         // it, they run while it does
         for (int l = 1; l < h->nl; ++l) {
             Level &v = h->L[l];
-            launch_diag0(s, v.g, h->Ke, v.CXl, v.AD);
-            if (per) launch_per_fold<double>(s, v.g, v.AD, 1, nullptr);
+            launch_diag0(s, v.g, h->Ke, v.CXl, v.AD, per ? nullptr : v.RD);
+            if (per) fold_diag(v, true);
         }
         HIPCHK(hipGetLastError());
         h->hier_ready = true;
@@ -390,8 +397,8 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
     // run on the main stream while it does
     for (int l = 1; l < h->nl; ++l) {
         Level &v = h->L[l];
-        launch_diagA(s, v.g, v.A, v.AD);
-        if (per) launch_per_fold<double>(s, v.g, v.AD, 1, nullptr);
+        launch_diagA(s, v.g, v.A, v.AD, per || l > 1 ? nullptr : v.RD);
+        if (per) fold_diag(v, false);
         if (v.S) launch_stencil_build(s, v.g, v.A, v.S);
     }
     HIPCHK(hipGetLastError());
@@ -488,7 +495,8 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
     Level &L0 = h->L[0];
     const long n = L0.g.ndof;
     const int *ctl = &h->sc->done;
-    const int nmv = (int)xcd_launch(L0.t.blocks());  // partials of the level-0 matvec
+    // partials of the level-0 matvec (FP64, from an FP64 or FP32 direction)
+    const int nmv = op0_blocks(op_args(h, 0), OP_MATVEC);
     const bool per = h->prm.periodic != 0;
     launch_fill(s, U, n, 0.0);
     launch_copy(s, F, h->R, n, nullptr);
@@ -627,7 +635,7 @@ static BatchState &batch_state(gputo_handle *h, int nb)
     b->P = dalloc<double>(h, nb * n);
     b->Q = dalloc<double>(h, nb * n);
     b->Z = dalloc<double>(h, nb * n);
-    const long nmv = xcd_launch(h->L[0].t.blocks());
+    const long nmv = std::max(xcd_launch(h->L[0].t.blocks()), xcd_launch(h->L[0].mw64.blocks()));
     b->partials = dalloc<double>(h, nb * std::max<long>(nmv, 2 * kRedBlocks));
     b->sc = dalloc<CgScalars>(h, nb);
     HIPCHK(hipHostMalloc((void **)&b->sc_host, nb * sizeof(CgScalars), hipHostMallocDefault));
@@ -681,7 +689,7 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
     Level &L0 = h->L[0];
     const long n = L0.g.ndof;
     const int *ctl = &b.sc->done;
-    const int nmv = (int)xcd_launch(L0.t.blocks());
+    const int nmv = op0_blocks(op_args(h, 0), OP_MATVEC);
     const bool per = h->prm.periodic != 0;
     HierView<double> H64 = f64_view(h);
     HierView<float> H32;
@@ -847,13 +855,14 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
             v.tg = choose_tile(v.g);
             maxblocks = std::max<long>(maxblocks, xcd_launch(v.t.blocks()));
             maxblocks = std::max<long>(maxblocks, xcd_launch(v.tg.blocks()));
-            if (l == 1) {
-                v.tmf = l1_tile(v.g);
-                v.tmf64 = l1_tile64(v.g);
-                maxblocks = std::max<long>(maxblocks, std::max(v.tmf.blocks(), v.tmf64.blocks()));
-            }
+            // level 1 of the rediscretised hierarchy takes the level-1 element
+            const int el = l == 1 && !preset_of(h->prm).l1_galerkin && !preset_of(h->prm).mg9;
+            v.mw64 = modal_work(v.g, 8, el, l ? 8 : 1);
+            v.mw32 = modal_work(v.g, 4, el, l ? 8 : 1);
+            maxblocks = std::max<long>(maxblocks, std::max(xcd_launch(v.mw64.blocks()), xcd_launch(v.mw32.blocks())));
             v.R = dalloc<double>(h, v.g.ndof);
-            v.AD = dalloc<double>(h, v.g.ndof);
+            v.AD = dalloc<double>(h, v.g.ndof + rd_len(v.g, l));
+            v.RD = v.AD + v.g.ndof;
             v.T = dalloc<double>(h, v.g.ndof);
             v.mask = dalloc<uint8_t>(h, v.g.nnod);
             v.fixed_d = dalloc<int>(h, v.g.ndof);
@@ -863,7 +872,7 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
                 v.A = dalloc<double>(h, 300 * v.g.nel);
                 v.CXl = dalloc<double>(h, v.g.nel);
                 // node stencils of the stored levels the V-cycle smooths
-                if (l < nl - 1 && !(l == 1 && use_l1_mf(h->prm, nl)))
+                if (l < nl - 1 && !(l == 1 && use_l1_mf(h->prm, nl, v.mw64)))
                     v.S = dalloc<double>(h, (long)kStencilEntries * v.g.nnod);
             }
         }

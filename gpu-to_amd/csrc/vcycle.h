@@ -4,6 +4,8 @@
 // Cantilever/omp/mgcg1.c:283-447).
 #pragma once
 
+#include <type_traits>
+
 #include "gputo_internal.h"
 
 namespace gputo {
@@ -31,12 +33,32 @@ inline Preset preset_of(const gputo_params &prm)
 }
 
 // Level-0 operator implementation of a view.
-// (values match gputo_params.l0_kernel; MFMA flavour = kind - L0_MFMA_F32)
-enum L0Kind { L0_AUTO = 0, L0_GATHER = 1, L0_MFMA_F32 = 2, L0_MFMA_BF16 = 3, L0_MFMA_BF16X3 = 4, L0_MFMA_BF16X1 = 5 };
+// (values match gputo_params.l0_kernel; MFMA flavour = kind - L0_MFMA_F32;
+// L0_MODAL stands for kinds 1 to 4 where Ke0 has the isotropic modal form)
+enum L0Kind {
+    L0_AUTO = 0,
+    L0_GATHER = 1,
+    L0_MFMA_F32 = 2,
+    L0_MFMA_BF16 = 3,
+    L0_MFMA_BF16X3 = 4,
+    L0_MFMA_BF16X1 = 5,
+    L0_MODAL = 6
+};
+
+// The FP32 modal kernel takes the place of the node-gather and of the split-
+// BF16 MFMA kernels whose accuracy it reaches or passes: a matvec takes
+// 18.6 us at 192x96x96, against 23.2 us for the two-part split, 39 us for the
+// three-part one and 66 us for the node-gather.  The one-product flavour
+// keeps its own kernel: its rounding is what that choice asks for.
+inline int l0_resolve(const gputo_handle *h, int kind)
+{
+    return h->ke_modal && h->L[0].mw32.NW > 0 && kind != L0_MFMA_BF16X1 ? L0_MODAL : kind;
+}
 
 template <class T>
 struct LevelView {
     T *U = nullptr, *F = nullptr, *R = nullptr, *AD = nullptr, *Tmp = nullptr;
+    T *RD = nullptr;        // 1/AD of the levels the modal kernels apply (OpArgsT::RD)
     const T *A = nullptr;   // packed element matrices (levels >= 1)
     const T *S = nullptr;   // node stencils of a stored level, or null
     const T *CX = nullptr;  // element scales of a matrix-free level (mgcg9)
@@ -64,16 +86,17 @@ void learn_stage(gputo_handle *h, const HierView<float> &H, int l, const float *
 // level-0 BF16-MFMA operator (mfma.hip); ctx is the MixedState
 void launch_op0_mfma(hipStream_t s, int mode, const OpArgsT<float> &a, const void *ctx, int flavor);
 
-// matrix-free rediscretised level-1 operator (l1op.hip); CXf = level-0 CX
+// matrix-free rediscretised level-1 operator (modal.hip); CXf = level-0 CX
 template <class T>
-void launch_op1_mf(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CXf, const Tile &t, double nu);
-Tile l1_tile(const Grid &g);    // FP32 tiling
-Tile l1_tile64(const Grid &g);  // FP64 tiling
+void launch_op1_mf(hipStream_t s, int mode, OpArgsT<T> a, const T *CXf, double nu);
 constexpr double kL1Nu = 0.3;  // Poisson ratio of the level-1 rediscretisation (mgcg1.c:1539-1584)
 
-// Whether level 1 runs matrix-free under the handle's parameters.
-inline bool use_l1_mf(const gputo_params &prm, int nl)
+// Whether level 1 runs matrix-free under the handle's parameters (mw64: its
+// tiling in the wider type; past the kernel's offsets the stored element
+// matrices are applied).
+inline bool use_l1_mf(const gputo_params &prm, int nl, const ModalWork &mw64)
 {
+    if (mw64.NW == 0) return false;
     if (nl < 3) return false;  // level 1 is the coarsest: its stored matrix feeds the Cholesky
     if (preset_of(prm).mg9) return false;
     const bool rediscretised = !preset_of(prm).l1_galerkin;
@@ -93,6 +116,10 @@ OpArgsT<T> view_args(const gputo_handle *h, const HierView<T> &H, int l, const i
     a.S = H.L[l].S;
     a.mask = h->L[l].mask;
     a.AD = H.L[l].AD;
+    a.RD = H.L[l].RD;
+    a.mw = std::is_same<T, double>::value ? h->L[l].mw64 : h->L[l].mw32;
+    a.modal = h->ke_modal;
+    for (int k = 0; k < 8; ++k) a.mc[k] = (T)h->mc[k];
     a.ctl = ctl;
     a.nb = H.nb;
     const Preset p = preset_of(h->prm);
@@ -114,12 +141,11 @@ void level_op(const gputo_handle *h, const HierView<T> &H, int l, int mode, cons
     if (H.mg9) {
         launch_op0<T>(h->stream, mode, a);  // level scales and the CX floor are in a
     } else if (l == 1 && H.l1_mf) {
-        launch_op1_mf<T>(h->stream, mode, a, H.CX, std::is_same<T, double>::value ? h->L[1].tmf64 : h->L[1].tmf,
-                         kL1Nu);
+        launch_op1_mf<T>(h->stream, mode, a, H.CX, kL1Nu);
     } else if (l > 0) {
         launch_opA<T>(h->stream, mode, a);
     } else if constexpr (std::is_same<T, float>::value) {
-        if (H.l0 >= L0_MFMA_F32)
+        if (H.l0 >= L0_MFMA_F32 && H.l0 != L0_MODAL)
             launch_op0_mfma(h->stream, mode, a, H.l0_ctx, H.l0 - L0_MFMA_F32);
         else
             launch_op0<T>(h->stream, mode, a);

@@ -63,7 +63,8 @@ enum gputo_preset { GPUTO_PRESET_REF_C = 0, GPUTO_PRESET_MATLAB_CFG0 = 1, GPUTO_
  *    with FP32 accumulation, so rounding changes only the iteration count.
  *  GPUTO_PREC_MIXED_BF16: as MIXED_F32 with the V-cycle's fine-level
  *    Ke x u contraction on BF16 MFMA (split-BF16 operands, FP32
- *    accumulation). */
+ *    accumulation); a Ke0 of the isotropic unit-hex form takes the FP32
+ *    modal kernel instead, which is more accurate and faster. */
 enum gputo_precision { GPUTO_PREC_F64 = 0, GPUTO_PREC_MIXED_F32 = 1, GPUTO_PREC_MIXED_BF16 = 2 };
 
 typedef struct gputo_params {
@@ -79,7 +80,9 @@ typedef struct gputo_params {
     int l0_kernel;     /* level-0 operator of the FP32 V-cycle: 0 by precision, 1 FP32
                           node-gather, 2 FP32 MFMA, 3 split-BF16 MFMA (hi+lo),
                           4 split-BF16 MFMA (hi+mid+lo), 5 single-product
-                          BF16 MFMA (smoother-grade accuracy only) */
+                          BF16 MFMA (smoother-grade accuracy only).  For a Ke0 of
+                          the isotropic unit-hex form, 1 to 4 all run the FP32
+                          modal kernel (FP32 accuracy, faster than each) */
     int nswp;          /* GPUTO_PRESET_MGCG9: Jacobi sweeps each way (0: 2, the MEX default) */
     int l1_kernel;     /* level-1 operator in the V-cycle: 0 by preset (matrix-free
                           where level 1 is rediscretised from the child densities,
@@ -177,7 +180,8 @@ int gputo_matvec_f64(gputo_handle *h, const double *Ke0, const double *CX, const
 /* The same product with a reduced-precision level-0 kernel of the
  * mixed-precision solve, FP64 in and out: kernel 1 FP32 node-gather, 2 FP32
  * MFMA, 3 split-BF16 MFMA (hi+lo), 4 split-BF16 MFMA (hi+mid+lo), 5 single
- * BF16 MFMA product bf16(Ke) bf16(u). */
+ * BF16 MFMA product bf16(Ke) bf16(u) (1 to 4: the FP32 modal kernel for an
+ * isotropic unit-hex Ke0, as in the solve). */
 int gputo_matvec_mixed(gputo_handle *h, int kernel, const double *Ke0, const double *CX, const double *u,
                        const double *fixed, int nfd, double *y);
 /* y = K(CX) u with y[fixed] = 0 on device arrays, allocating nothing: the

@@ -1,0 +1,107 @@
+"""The matrix-free operators in the modal basis (csrc/modal.hip) at the edges
+of their tiling, against the oracle's element products (multAV0c / defect0c /
+Jacobc, Cantilever/TOP3D125MGCGCUDA/mgcg1.cu:941-997,1190-1264): one element
+per direction and level, rows longer and shorter than a wave, several strips
+along j, chunks of a plane and layer groups along i, remainders in each.
+
+Tolerances relative to max|y|: FP64 1e-13 (summation order only), FP32 2e-6
+(FP32 rounding of the operands and sums), as the other operator tests.
+"""
+import numpy as np
+import pytest
+
+from conftest import cantilever_case
+
+pytestmark = pytest.mark.gpu
+
+OMEGA, PRERELAX = 0.48, 0.7  # Jacobc, preRelc of the reference smoother
+
+MESHES = [(2, 2, 2, 2), (2, 62, 2, 2), (4, 128, 2, 2), (2, 2, 130, 2), (130, 2, 4, 2), (12, 36, 20, 3), (20, 68, 44, 3),
+          (72, 56, 40, 4), (112, 96, 48, 5)]
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / max(np.abs(b).max(), 1e-300)
+
+
+def references(Ku, u, f, ad, fx):
+    """mode -> reference of gputo_level_apply from the product Ku(u)."""
+    out = {}
+    for mode in range(5):
+        uu = PRERELAX * f / ad if mode in (3, 4) else u
+        y = Ku(uu)
+        r = f - y
+        r[fx] = 0.0
+        if mode == 0:
+            y[fx] = 0.0
+            out[mode] = y
+        elif mode in (1, 4):
+            out[mode] = r
+        else:
+            out[mode] = (1 - OMEGA) * uu + OMEGA * (r + ad * uu) / ad
+    return out
+
+
+@pytest.mark.parametrize("mesh", MESHES)
+def test_modal_operators_vs_oracle(gputo, oracle, mesh):
+    nelx, nely, nelz, nl = mesh
+    print("case", mesh, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=61, kind="smooth")
+    s = gputo.Solver(nelx, nely, nelz, nl, precision=1)
+    s.setup(Ke, CX, fixed)
+    rng = np.random.default_rng(62)
+    for level in range(1 if nl < 3 else 2):
+        if level == 0:
+            ad, fx = oracle.prepad0(Ke, CX, nelx, nely, nelz), (fixed - 1).astype(np.int64)
+
+            def Ku(v):
+                return oracle.matvec0(Ke, CX, v, np.zeros(0), nelx, nely, nelz)
+        else:
+            A, ad, fd = oracle.level_data(Ke, CX, fixed, nelx, nely, nelz, nl, 1)
+            fx = fd.astype(np.int64) - 1
+
+            def Ku(v):
+                return oracle.matvec_el(A, v, np.zeros(0), nelx // 2, nely // 2, nelz // 2)
+        u, f = rng.uniform(-1, 1, ad.size), rng.uniform(-1, 1, ad.size)
+        ref = references(Ku, u, f, ad, fx)
+        for mode in range(5):
+            for fp32, tol in ((False, 1e-13), (True, 2e-6)):
+                y = s.level_apply(level, 1 + level, mode, u, f, fp32=fp32)
+                assert rel(y, ref[mode]) < tol, (level, mode, fp32, rel(y, ref[mode]))
+                assert np.array_equal(y, s.level_apply(level, 1 + level, mode, u, f, fp32=fp32))
+    s.close()
+
+
+@pytest.mark.parametrize("mesh", [(4, 6, 8, 2), (20, 68, 44, 3)])
+def test_modal_keeps_non_finite_values_local(gputo, mesh):
+    """A NaN or infinity at a node reaches the 27 nodes around it and no other
+    (elements outside the mesh are worked on, but read nothing)."""
+    nelx, nely, nelz, nl = mesh
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=63)
+    s = gputo.Solver(nelx, nely, nelz, nl)
+    for i, k, j in ((nelx, nelz, nely), (1, 1, 0), (nelx // 2, nelz, 0), (0, 0, nely)):
+        u = np.zeros((nelx + 1, nelz + 1, nely + 1, 3))
+        u[i, k, j, 1] = np.nan if j else np.inf
+        y = s.matvec(Ke, CX, u.ravel(), fixed).reshape(u.shape)
+        bad = ~np.isfinite(y).all(axis=-1)
+        near = np.zeros_like(bad)
+        near[max(i - 1, 0):i + 2, max(k - 1, 0):k + 2, max(j - 1, 0):j + 2] = True
+        near[0] = False  # the fixed face
+        assert np.array_equal(bad, near)
+        assert not y[~near].any()
+    s.close()
+
+
+@pytest.mark.parametrize("kernel,tol", [(1, 2e-6), (2, 2e-6), (3, 1e-4), (4, 2e-6)])
+def test_other_element_matrices_take_the_general_kernels(gputo, oracle, kernel, tol):
+    """A Ke0 without the isotropic modal form: the node-gather and the MFMA kernels."""
+    nelx, nely, nelz, nl = 40, 20, 12, 3
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=64, kind="smooth")
+    E = np.random.default_rng(65).uniform(-1, 1, (24, 24)) * 1e-3
+    Ke = Ke + (E + E.T)
+    s = gputo.Solver(nelx, nely, nelz, nl, precision=2, l0_kernel=kernel)
+    u = np.random.default_rng(66).uniform(-1, 1, s.ndof)
+    yo = oracle.matvec0(Ke, CX, u, fixed, nelx, nely, nelz)
+    assert rel(s.matvec_mixed(kernel, Ke, CX, u, fixed), yo) < tol
+    assert rel(s.matvec(Ke, CX, u, fixed), yo) < 1e-13
+    s.close()
