@@ -377,7 +377,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     const MdBuf BU = PRE ? md_buf(a.F, vb)
                          : (MODE == OP_MATVEC_UF ? md_buf(a.Uf, (long)SU * g.ndof) : md_buf(a.U, vb));
     const MdBuf BF = md_buf(a.F, MV ? 0 : vb), BD = md_buf(a.RD, (JAC || PRE) ? (EL == 0 ? vb / 3 : vb) : 0);
-    const MdBuf BE = md_buf(CX, (long)S * (EL == 0 ? 1 : 8) * g.nel), BM = md_buf(a.mask, g.nnod);
+    const MdBuf BE = md_buf(CX, (long)S * (EL == 0 ? 1 : 8) * g.nel), BM = md_buf(a.mask, a.mask ? g.nnod : 0);  // no mask: reads 0
     const int up = 3 * SU * plane, fp = 3 * S * plane;         // bytes of a node layer
     const int dp = S * plane, dlo = el_ok ? S * nod0 : kMdOut, dhi = el_ok ? S * (nod0 + g.nny) : kMdOut;
     const int ep = (EL == 0 ? 1 : 4) * S * g.ny * g.nz;        // bytes of a scale layer

@@ -3,11 +3,16 @@
 // gputo_matvec_f64_noalloc is gputo_matvec_f64 (y = K(CX) u, y[fixed] = 0:
 // multAV0c + ZeroBCc, Cantilever/TOP3D125MGCGCUDA/mgcg1.cu:941-997,1326)
 // for callers that cannot call hipMalloc: code under HIP graph capture,
-// serving loops.  The caller passes device inputs and outputs; the only
-// device memory beyond them, the one-byte-per-node fixed-DOF mask the
-// node-gather kernel reads, lives in `scratch`, a static device array of
-// kScratchBytes per GPU, held until the process ends.  Every call on a GPU
-// shares that GPU's array, so calls that overlap on one GPU race.
+// serving loops.  The caller passes device inputs and outputs.
+//
+// An isotropic Ke0 takes the modal kernel without a mask and then zeroes the
+// fixed DOFs of y: two launches and no memory of its own (three launches,
+// with the mask cleared and set first, took 46.6 us per call at 192x96x96
+// against 39.8 us).  Any other Ke0 with
+// the unit-H8 entry structure takes the node-gather kernel, whose one-byte-
+// per-node fixed-DOF mask lives in `scratch`, a static device array of
+// kScratchBytes per GPU, held until the process ends.  Every such call on a
+// GPU shares that GPU's array, so calls that overlap on one GPU race.
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -60,6 +65,15 @@ __global__ void k_mask_set(uint8_t *mask, const int *fixed, int nfd, long ndof)
     atomicOr(reinterpret_cast<unsigned *>(mask + (n & ~3L)), bit);
 }
 
+// y = 0 at the fixed DOFs (those outside [0, ndof) are skipped)
+__global__ void k_zero_fixed(double *y, const int *fixed, int nfd, long ndof)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= nfd) return;
+    const long d = fixed[i];
+    if (d >= 0 && d < ndof) y[d] = 0.0;
+}
+
 }  // namespace
 }  // namespace gputo
 
@@ -85,23 +99,28 @@ extern "C" int gputo_matvec_f64_noalloc(int nelx, int nely, int nelz, const doub
             std::fprintf(stderr, "gputo_matvec_f64_noalloc: Ke0 lacks the unit-H8 entry structure\n");
             return GPUTO_ERR_ARGUMENT;
         }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    a.g = g;
+    a.t = choose_tile(g);
+    a.kc = 1;
+    a.CX = d_CX;
+    a.U = d_u;
+    a.out = d_y;
+    a.modal = modal_constants(Ke0, a.mc);
+    if (a.modal) a.mw = modal_work(g, 8, 0, 1);
+    if (op0_is_modal(a, OP_MATVEC)) {
+        launch_op0<double>(s, OP_MATVEC, a);
+        if (nfd > 0) k_zero_fixed<<<(nfd + 255) / 256, 256, 0, s>>>(d_y, d_fixed, nfd, g.ndof);
+        return hipGetLastError() == hipSuccess ? 0 : GPUTO_ERR_DEVICE;
+    }
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return GPUTO_ERR_DEVICE;
     uint8_t *mask = scratch_ptr(dev);
     if (!mask) return GPUTO_ERR_DEVICE;
-    hipStream_t s = static_cast<hipStream_t>(stream);
     k_mask_clear<<<(unsigned)std::min<long>((nwords + 255) / 256, 1024), 256, 0, s>>>(
         reinterpret_cast<uint32_t *>(mask), nwords);
     if (nfd > 0) k_mask_set<<<(nfd + 255) / 256, 256, 0, s>>>(mask, d_fixed, nfd, g.ndof);
-    a.g = g;
-    a.t = choose_tile(g);
-    a.kc = 1;
-    a.modal = modal_constants(Ke0, a.mc);
-    if (a.modal) a.mw = modal_work(g, 8, 0, 1);
-    a.CX = d_CX;
-    a.U = d_u;
     a.mask = mask;
-    a.out = d_y;
     launch_op0<double>(s, OP_MATVEC, a);
     return hipGetLastError() == hipSuccess ? 0 : GPUTO_ERR_DEVICE;
 }

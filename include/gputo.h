@@ -191,10 +191,11 @@ int gputo_matvec_mixed(gputo_handle *h, int kernel, const double *Ke0, const dou
  * d_CX (nel doubles), d_u and d_y (ndof doubles) and d_fixed (nfd int32,
  * 0-based DOF indices; entries outside [0, ndof) are skipped) are device
  * pointers; Ke0 is a host 24x24 array with the unit-H8 entry structure of
- * the top3D125 Ke0 (GPUTO_ERR_ARGUMENT otherwise).  The node mask lives in
- * a static device buffer of the library, 8 MiB per GPU (meshes up to
- * 8,388,608 nodes; GPUTO_ERR_WORKSPACE beyond), shared by every call on that
- * GPU: calls that overlap on one GPU race.  The work is queued on `stream`
+ * the top3D125 Ke0 (GPUTO_ERR_ARGUMENT otherwise).  Meshes up to 8,388,608
+ * nodes (GPUTO_ERR_WORKSPACE beyond).  A Ke0 that is not isotropic needs a
+ * node mask, which lives in a static device buffer of the library, 8 MiB per
+ * GPU, shared by every such call on that
+ * GPU: those calls race when they overlap on one GPU.  The work is queued on `stream`
  * (a hipStream_t; NULL: the null stream) and not waited for. */
 int gputo_matvec_f64_noalloc(int nelx, int nely, int nelz, const double *Ke0, const double *d_CX, const double *d_u,
                              const int *d_fixed, int nfd, double *d_y, void *stream);
