@@ -84,7 +84,7 @@ struct CorrIO {
     float *e;
 };
 void learn_forward(gputo_handle *h, const int *ctl, const CorrIO *io);  // y = N(x0), activations cached
-void learn_backward(gputo_handle *h);                  // G += d<gy, y>/dtheta
+void learn_backward(gputo_handle *h);                  // G = d<gy, y>/dtheta
 // Extra stage after the level-2 post-smoothing of the FP32 V-cycle:
 // d = F - A U;  e = N(d);  gamma = <d,e>/<e,Ae>;  U += gamma e if gamma > 0.
 // Logs d as a training sample when logging is on.

@@ -358,95 +358,202 @@ __global__ __launch_bounds__(256) void k_conv_fwd_lanes(ConvFwd a)
 }
 
 // gin[ci][q] = sum_co sum_t w[co][ci][t] gz[co][p] over the outputs p that
-// read q through tap t (q = p*s + t - 1), gz = gout * relu'(act).  The
-// block's CT input channels of every output channel's weights are staged
-// in LDS as [co][t][c].
-template <int CT>
-__global__ __launch_bounds__(256) void k_conv_bwd_data(const float *__restrict__ gout, const float *__restrict__ act,
-                                                      int cout, Dims3 dout, const float *__restrict__ w, int cin,
-                                                      Dims3 din, int stride, float *__restrict__ gin)
+// read q through tap t (q = p*s + t - 1); gz is the output gradient already
+// masked by its ReLU.  A 256-thread block owns NP = 256/KS positions and CT
+// input channels; thread (ks, pl) takes position pl and the output channels
+// co = ks, ks + KS, ..., so that a coarse grid (637 positions) still fills
+// the device, and the KS partials of a position are added in ks order.  The
+// block's weights are staged in LDS as [co][t][c].  The sum then takes the
+// skip connection's gradient (add) and the ReLU mask of the layer below
+// (act), so no later pass reads it again.
+//
+// Stride 2: position q is read through taps of its own parity only (one tap
+// per even coordinate, two per odd one: 1 to 8 of 27), so a block takes
+// positions of one parity class.
+//
+// Measured on the 49x25x25 grid's five layers: 458 us with one thread per
+// position over all 27 taps and output channels, 76 us now; bound by the
+// gathers' latency and the staging.
+struct ConvBwd {
+    const float *g;   // masked output gradient [cout][dout]
+    const float *w;
+    int cin, cout;
+    Dims3 din, dout;
+    float *gin;
+    const float *add; // null, or [cin][din] added to the sum
+    const float *act; // null, or [cin][din]: the result is 0 where act <= 0
+    int blk[9];       // stride 2: first block of each parity class
+};
+
+// positions of parity class c (bits 4, 2, 1: odd i, k, j) per axis
+__host__ __device__ __forceinline__ int class_count(int n, int odd) { return odd ? n / 2 : (n + 1) / 2; }
+
+// NT taps with offsets off, weight taps tap and the validity mask
+template <int CT, int KS, int NT>
+__device__ __forceinline__ void bwd_taps(const ConvBwd &a, const float *wl, int ks, const int (&off)[NT],
+                                         const int (&tap)[NT], unsigned valid, float (&acc)[CT])
 {
-    extern __shared__ float wl[];  // [cout*27][CT]
-    const int ci0 = blockIdx.y * CT;
-    stage_lds(wl, cout * 27 * CT, w, [=](int q) {
+    constexpr int GU = NT >= 27 ? 2 : (NT >= 8 ? 4 : 8);  // output channels whose gathers fly together
+    const int nout = (int)a.dout.size();
+    for (int c0 = ks; c0 < a.cout; c0 += GU * KS) {
+        float gv[GU][NT];
+#pragma unroll
+        for (int u = 0; u < GU; ++u) {
+            const int co = c0 + u * KS;
+            const float *g = a.g + (long)(co < a.cout ? co : 0) * nout;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) gv[u][t] = g[off[t]];  // off = 0 outside the grid: masked below
+        }
+#pragma unroll
+        for (int u = 0; u < GU; ++u) {
+            const int co = c0 + u * KS;
+            if (co >= a.cout) break;
+            const float *wc = wl + co * 27 * CT;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const float gz = ((valid >> t) & 1u) ? gv[u][t] : 0.0f;
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[c] = fmaf(wc[tap[t] * CT + c], gz, acc[c]);
+            }
+        }
+    }
+}
+
+template <int CT, int KS, int NI, int NK, int NJ>
+__device__ __forceinline__ void bwd_class(const ConvBwd &a, const float *wl, int ks, int qi, int qk, int qj,
+                                          float (&acc)[CT])
+{
+    // an odd coordinate q is read by outputs (q + 1)/2 (tap 0) and
+    // (q - 1)/2 (tap 2), an even one by q/2 (tap 1)
+    constexpr int NT = NI * NK * NJ;
+    int off[NT], tap[NT];
+    unsigned valid = 0;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int x = n / (NK * NJ), y = (n / NJ) % NK, z = n % NJ;
+        const int ti = NI == 2 ? 2 * x : 1, tk = NK == 2 ? 2 * y : 1, tj = NJ == 2 ? 2 * z : 1;
+        const int pi = (qi + 1 - ti) >> 1, pk = (qk + 1 - tk) >> 1, pj = (qj + 1 - tj) >> 1;
+        const bool ok = pi < a.dout.n0 && pk < a.dout.n1 && pj < a.dout.n2;
+        valid |= (unsigned)ok << n;
+        off[n] = ok ? (pi * a.dout.n1 + pk) * a.dout.n2 + pj : 0;
+        tap[n] = 9 * ti + 3 * tk + tj;
+    }
+    bwd_taps<CT, KS, NT>(a, wl, ks, off, tap, valid, acc);
+}
+
+template <int CT, int KS, int STRIDE>
+__global__ __launch_bounds__(256) void k_conv_bwd_data(ConvBwd a)
+{
+    extern __shared__ float wl[];  // [cout*27][CT], then KS partials [KS][NP][CT]
+    constexpr int NP = 256 / KS;
+    const int ci0 = blockIdx.y * CT, cin = a.cin;
+    stage_lds(wl, a.cout * 27 * CT, a.w, [=](int q) {
         const int c = q % CT, k = q / CT;  // k = co*27 + t
         const int co = k / 27, t = k - 27 * co;
         return (co * cin + ci0 + c) * 27 + t;
     });
     __syncthreads();
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    const int nin = (int)din.size(), nout = (int)dout.size();
-    if (q >= nin) return;
-    int qi, qk, qj;
-    pos3(q, din, qi, qk, qj);
-    int off[27];
-    unsigned valid = 0;
-#pragma unroll
-    for (int t = 0; t < 27; ++t) {
-        const int xi = qi + 1 - t / 9, xk = qk + 1 - (t / 3) % 3, xj = qj + 1 - t % 3;
-        int pi = xi, pk = xk, pj = xj;
-        bool ok = xi >= 0 && xk >= 0 && xj >= 0;
-        if (stride == 2) {
-            ok = ok && !(xi & 1) && !(xk & 1) && !(xj & 1);
-            pi = xi >> 1;
-            pk = xk >> 1;
-            pj = xj >> 1;
-        }
-        ok = ok && pi < dout.n0 && pk < dout.n1 && pj < dout.n2;
-        valid |= (unsigned)ok << t;
-        off[t] = ok ? (pi * dout.n1 + pk) * dout.n2 + pj : 0;
-    }
+    const int pl = threadIdx.x % NP, ks = threadIdx.x / NP;
+    const int nin = (int)a.din.size();
     float acc[CT];
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[c] = 0.0f;
-    for (int co = 0; co < cout; ++co) {
-        const float *g = gout + co * nout;
-        const float *a = act ? act + co * nout : nullptr;
-        const float *wc = wl + co * 27 * CT;
-        float gv[27], av[27];
+    bool live;
+    int q;
+    if constexpr (STRIDE == 1) {
+        q = blockIdx.x * NP + pl;
+        live = q < nin;
+        int qi, qk, qj;
+        pos3(live ? q : 0, a.din, qi, qk, qj);
+        int off[27], tap[27];
+        unsigned valid = 0;
 #pragma unroll
         for (int t = 0; t < 27; ++t) {
-            gv[t] = g[off[t]];  // off = 0 outside the grid: masked below
-            av[t] = a ? a[off[t]] : 1.0f;
+            const int pi = qi + 1 - t / 9, pk = qk + 1 - (t / 3) % 3, pj = qj + 1 - t % 3;
+            const bool ok = pi >= 0 && pk >= 0 && pj >= 0 && pi < a.dout.n0 && pk < a.dout.n1 && pj < a.dout.n2;
+            valid |= (unsigned)ok << t;
+            off[t] = ok ? (pi * a.dout.n1 + pk) * a.dout.n2 + pj : 0;
+            tap[t] = t;
         }
-#pragma unroll
-        for (int t = 0; t < 27; ++t) {
-            const float gz = (((valid >> t) & 1u) && av[t] > 0.0f) ? gv[t] : 0.0f;
-#pragma unroll
-            for (int c = 0; c < CT; ++c) acc[c] = fmaf(wc[t * CT + c], gz, acc[c]);
+        bwd_taps<CT, KS, 27>(a, wl, ks, off, tap, valid, acc);
+    } else {
+        int cls = 0;
+        while (cls < 7 && (int)blockIdx.x >= a.blk[cls + 1]) ++cls;
+        const int oi = cls >> 2, ok = (cls >> 1) & 1, oj = cls & 1;
+        const Dims3 dc = {class_count(a.din.n0, oi), class_count(a.din.n1, ok), class_count(a.din.n2, oj)};
+        const int r = (blockIdx.x - a.blk[cls]) * NP + pl;
+        live = r < (int)dc.size();
+        int i, k, j;
+        pos3(live ? r : 0, dc, i, k, j);
+        const int qi = 2 * i + oi, qk = 2 * k + ok, qj = 2 * j + oj;
+        q = (qi * a.din.n1 + qk) * a.din.n2 + qj;
+        switch (cls) {  // block-uniform
+        case 0: bwd_class<CT, KS, 1, 1, 1>(a, wl, ks, qi, qk, qj, acc); break;
+        case 1: bwd_class<CT, KS, 1, 1, 2>(a, wl, ks, qi, qk, qj, acc); break;
+        case 2: bwd_class<CT, KS, 1, 2, 1>(a, wl, ks, qi, qk, qj, acc); break;
+        case 3: bwd_class<CT, KS, 1, 2, 2>(a, wl, ks, qi, qk, qj, acc); break;
+        case 4: bwd_class<CT, KS, 2, 1, 1>(a, wl, ks, qi, qk, qj, acc); break;
+        case 5: bwd_class<CT, KS, 2, 1, 2>(a, wl, ks, qi, qk, qj, acc); break;
+        case 6: bwd_class<CT, KS, 2, 2, 1>(a, wl, ks, qi, qk, qj, acc); break;
+        default: bwd_class<CT, KS, 2, 2, 2>(a, wl, ks, qi, qk, qj, acc); break;
         }
     }
+    if (KS > 1) {
+        float *part = wl + a.cout * 27 * CT;
 #pragma unroll
-    for (int c = 0; c < CT; ++c) gin[(ci0 + c) * nin + q] = acc[c];
+        for (int c = 0; c < CT; ++c) part[(ks * NP + pl) * CT + c] = acc[c];
+        __syncthreads();
+        if (ks != 0) return;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            float sm = acc[c];
+            for (int k = 1; k < KS; ++k) sm += part[(k * NP + pl) * CT + c];
+            acc[c] = sm;
+        }
+    }
+    if (!live) return;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const long o = (long)(ci0 + c) * nin + q;
+        float r = acc[c];
+        if (a.add) r += a.add[o];
+        if (a.act) r = a.act[o] > 0.0f ? r : 0.0f;
+        a.gin[o] = r;
+    }
 }
 
 // Weight gradient, split over chunks of kWChunk output positions:
 // part[ch][co*cin + ci][t] = sum_{p in chunk ch} gz[co][p] in[ci][p*s + t - 1]
-// and, at t = 27, sum_p gz[co][p].  One block per (co, ci, chunk), fixed-
-// order block reduction; k_conv_bwd_w_sum adds the chunks in order.
-constexpr int kWChunk = 2048;
+// and, at t = 27, sum_p gz[co][p].  One block per (ci, CO output channels,
+// chunk): the 27 inputs gathered at a position serve CO channels.  A lane's
+// 28 CO sums are added over its wave by halving (at each step a lane hands
+// half of its values to its partner and keeps the other half: 126 exchanges
+// for 128 values instead of 6 for each), then over the waves in order.
+// k_conv_bwd_w_sum adds the chunks in order.  Measured on the six layers:
+// 235 us with one block per (co, ci) pair and a tree over the block in LDS,
+// 103 us now.
+constexpr int kWChunk = 1024;
 
-__global__ __launch_bounds__(256) void k_conv_bwd_w(const float *__restrict__ gout, const float *__restrict__ act,
-                                                   Dims3 dout, const float *__restrict__ in, int cin, Dims3 din,
-                                                   int stride, float *__restrict__ part)
+template <int CO>
+__global__ __launch_bounds__(256) void k_conv_bwd_w(const float *__restrict__ gz, Dims3 dout,
+                                                   const float *__restrict__ in, int cin, Dims3 din, int stride,
+                                                   float *__restrict__ part)
 {
-    __shared__ float red[28][257];
-    const int pair = blockIdx.x, co = pair / cin, ci = pair % cin;
+    static_assert(28 * CO <= 128, "sums per lane");
+    __shared__ float red[4][128];
+    const int co0 = (blockIdx.x / cin) * CO, ci = blockIdx.x % cin;
     const int nout = (int)dout.size(), nin = (int)din.size();
-    const float *g = gout + co * nout;
-    const float *a = act ? act + co * nout : nullptr;
-    const float *src = in + ci * nin;
-    float acc[28];
+    const float *src = in + (long)ci * nin;
+    float acc[128];
 #pragma unroll
-    for (int t = 0; t < 28; ++t) acc[t] = 0.0f;
+    for (int t = 0; t < 128; ++t) acc[t] = 0.0f;
     const int p1 = min(nout, (int)(blockIdx.y + 1) * kWChunk);
     for (int p = blockIdx.y * kWChunk + threadIdx.x; p < p1; p += 256) {
-        float gz = g[p];
-        if (a && !(a[p] > 0.0f)) gz = 0.0f;
-        if (gz == 0.0f) continue;
+        float g[CO];
+#pragma unroll
+        for (int c = 0; c < CO; ++c) g[c] = gz[(long)(co0 + c) * nout + p];
         int oi, ok, oj;
         pos3(p, dout, oi, ok, oj);
-        acc[27] += gz;
         float v[27];
 #pragma unroll
         for (int t = 0; t < 27; ++t) {
@@ -456,35 +563,64 @@ __global__ __launch_bounds__(256) void k_conv_bwd_w(const float *__restrict__ go
             v[t] = in_grid ? v[t] : 0.0f;
         }
 #pragma unroll
-        for (int t = 0; t < 27; ++t) acc[t] = fmaf(gz, v[t], acc[t]);
-    }
+        for (int c = 0; c < CO; ++c) {
 #pragma unroll
-    for (int t = 0; t < 28; ++t) red[t][threadIdx.x] = acc[t];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w)
-            for (int t = 0; t < 28; ++t) red[t][threadIdx.x] += red[t][threadIdx.x + w];
-        __syncthreads();
+            for (int t = 0; t < 27; ++t) acc[28 * c + t] = fmaf(g[c], v[t], acc[28 * c + t]);
+            acc[28 * c + 27] += g[c];
+        }
     }
-    if (threadIdx.x < 28) part[((long)blockIdx.y * gridDim.x + pair) * 28 + threadIdx.x] = red[threadIdx.x][0];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // after the step of mask m, lane bit m chose the half it keeps
+#pragma unroll
+    for (int h = 64, m = 32; m > 0; h >>= 1, m >>= 1) {
+        const bool up = lane & m;
+#pragma unroll
+        for (int i = 0; i < h; ++i) {
+            const float keep = up ? acc[i + h] : acc[i], send = up ? acc[i] : acc[i + h];
+            acc[i] = keep + __shfl_xor(send, m, 64);
+        }
+    }
+    // lane bits 32, 16, ... 1 select 64, 32, ... 2: values 2 lane, 2 lane + 1
+    red[wave][2 * lane] = acc[0];
+    red[wave][2 * lane + 1] = acc[1];
+    __syncthreads();
+    const int q = threadIdx.x;
+    if (q < 28 * CO) {
+        const int c = q / 28, t = q - 28 * c;
+        const float sm = (red[0][q] + red[1][q]) + (red[2][q] + red[3][q]);
+        const int npair = (gridDim.x / cin) * CO * cin;
+        part[((long)blockIdx.y * npair + (co0 + c) * cin + ci) * 28 + t] = sm;
+    }
 }
 
-__global__ void k_conv_bwd_w_sum(const float *__restrict__ part, int nch, int npair, int cin, float *__restrict__ gw,
-                                 float *__restrict__ gb)
+// the chunk sums of every layer to its parameter gradients (one launch)
+struct WSum {
+    int first[kNetLayers + 1];  // first thread of each layer
+    int nch[kNetLayers], npair[kNetLayers], cin[kNetLayers];
+    long part[kNetLayers], w_off[kNetLayers], b_off[kNetLayers];
+};
+
+__global__ void k_conv_bwd_w_sum(WSum a, const float *__restrict__ part, float *__restrict__ G)
 {
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= npair * 28) return;
+    int q = blockIdx.x * 256 + threadIdx.x;
+    if (q >= a.first[kNetLayers]) return;
+    int l = 0;
+    while (q >= a.first[l + 1]) ++l;
+    q -= a.first[l];
     const int pair = q / 28, t = q - 28 * pair;
+    const float *p = part + a.part[l] + q;
     float sm = 0.0f;
-    for (int ch = 0; ch < nch; ++ch) sm += part[((long)ch * npair + pair) * 28 + t];
+    for (int ch = 0; ch < a.nch[l]; ++ch) sm += p[(long)ch * a.npair[l] * 28];
     if (t < 27)
-        gw[(long)pair * 27 + t] += sm;
-    else if (pair % cin == 0)
-        gb[pair / cin] += sm;
+        G[a.w_off[l] + (long)pair * 27 + t] = sm;
+    else if (pair % a.cin[l] == 0)
+        G[a.b_off[l] + pair / a.cin[l]] = sm;
 }
 
-// gd[c][pc] = sum over the (up to 8) fine children of pc of gu[c][p]
-__global__ void k_up_bwd(const float *__restrict__ gu, Dims3 df, int C, Dims3 dc, float *__restrict__ gd)
+// gd[c][pc] = sum over the (up to 8) fine children of pc of gu[c][p], 0
+// where act <= 0 (the ReLU mask of the upsampled activation)
+__global__ void k_up_bwd(const float *__restrict__ gu, Dims3 df, int C, Dims3 dc, const float *__restrict__ act,
+                         float *__restrict__ gd)
 {
     const int nc = (int)dc.size(), total = nc * C, nf = (int)df.size();
     for (int q = blockIdx.x * 256 + threadIdx.x; q < total; q += gridDim.x * 256) {
@@ -499,18 +635,8 @@ __global__ void k_up_bwd(const float *__restrict__ gu, Dims3 df, int C, Dims3 dc
                     const int fi = 2 * i + a, fk = 2 * k + b, fj = 2 * j + e;
                     if (fi < df.n0 && fk < df.n1 && fj < df.n2) s += gu[c * nf + (fi * df.n1 + fk) * df.n2 + fj];
                 }
-        gd[q] = s;
+        gd[q] = act[q] > 0.0f ? s : 0.0f;
     }
-}
-
-__global__ void k_add_inplace(float *__restrict__ dst, const float *__restrict__ src, long n)
-{
-    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long)gridDim.x * 256) dst[q] += src[q];
-}
-
-__global__ void k_zero(float *__restrict__ v, long n)
-{
-    for (long q = (long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long)gridDim.x * 256) v[q] = 0.0f;
 }
 
 // ---- the level-2 stage: features, output scaling, loss gradient, step ----
@@ -747,24 +873,58 @@ ConvFwd conv_args(const NetLayer &ly, const float *P, const float *in, Dims3 din
     return a;
 }
 
-// gradients of one layer: weights/bias accumulate into G; gin (if non-null)
-// is overwritten with the input gradient
-void conv_bwd(hipStream_t s, const NetLayer &ly, const float *P, float *G, float *wpart, const float *in, Dims3 din,
-              const float *out, Dims3 dout, const float *gout, float *gin)
+template <int CT, int KS>
+void conv_bwd_data_ks(hipStream_t s, ConvBwd a, int stride)
 {
-    const float *act = ly.relu ? out : nullptr;
-    const int npair = ly.cout * ly.cin, nch = (int)((dout.size() + kWChunk - 1) / kWChunk);
-    k_conv_bwd_w<<<dim3(npair, nch), 256, 0, s>>>(gout, act, dout, in, ly.cin, din, ly.stride, wpart);
-    k_conv_bwd_w_sum<<<(npair * 28 + 255) / 256, 256, 0, s>>>(wpart, nch, npair, ly.cin, G + ly.w_off, G + ly.b_off);
-    if (gin) {
-        const unsigned gx = (unsigned)((din.size() + 255) / 256);
-        if (ly.cin % 4 == 0)
-            k_conv_bwd_data<4><<<dim3(gx, ly.cin / 4), 256, (size_t)ly.cout * 27 * 4 * sizeof(float), s>>>(
-                gout, act, ly.cout, dout, P + ly.w_off, ly.cin, din, ly.stride, gin);
-        else
-            k_conv_bwd_data<1><<<dim3(gx, ly.cin), 256, (size_t)ly.cout * 27 * sizeof(float), s>>>(
-                gout, act, ly.cout, dout, P + ly.w_off, ly.cin, din, ly.stride, gin);
+    constexpr int NP = 256 / KS;
+    const size_t lds = ((size_t)a.cout * 27 * CT + (KS > 1 ? 256 * CT : 0)) * sizeof(float);
+    if (stride == 1) {
+        const dim3 grid((unsigned)((a.din.size() + NP - 1) / NP), (unsigned)(a.cin / CT));
+        k_conv_bwd_data<CT, KS, 1><<<grid, 256, lds, s>>>(a);
+        return;
     }
+    a.blk[0] = 0;
+    for (int c = 0; c < 8; ++c) {
+        const long n = (long)class_count(a.din.n0, c >> 2) * class_count(a.din.n1, (c >> 1) & 1) *
+                       class_count(a.din.n2, c & 1);
+        a.blk[c + 1] = a.blk[c] + (int)((n + NP - 1) / NP);
+    }
+    k_conv_bwd_data<CT, KS, 2><<<dim3((unsigned)a.blk[8], (unsigned)(a.cin / CT)), 256, lds, s>>>(a);
+}
+
+// KS as for the lane kernel of the forward pass: the smallest that gives
+// kLaneBlocks blocks
+void conv_bwd_data(hipStream_t s, const ConvBwd &a, int stride)
+{
+    constexpr int CT = 4;
+    if (a.cin % CT != 0) throw std::runtime_error("conv: input channels not a multiple of 4");
+    int ks = 1;
+    while (ks < 32 && 2 * ks <= a.cout &&
+           ((a.din.size() + 256 / ks - 1) / (256 / ks)) * (a.cin / CT) < kLaneBlocks)
+        ks *= 2;
+    switch (ks) {
+    case 1: conv_bwd_data_ks<CT, 1>(s, a, stride); break;
+    case 2: conv_bwd_data_ks<CT, 2>(s, a, stride); break;
+    case 4: conv_bwd_data_ks<CT, 4>(s, a, stride); break;
+    case 8: conv_bwd_data_ks<CT, 8>(s, a, stride); break;
+    case 16: conv_bwd_data_ks<CT, 16>(s, a, stride); break;
+    default: conv_bwd_data_ks<CT, 32>(s, a, stride); break;
+    }
+}
+
+int w_chunks(const Dims3 &dout) { return (int)((dout.size() + kWChunk - 1) / kWChunk); }
+
+// partial weight gradients of layer l into its part of wpart
+void conv_bwd_w(hipStream_t s, const NetLayer &ly, const float *in, Dims3 din, Dims3 dout, const float *gz,
+                float *wpart)
+{
+    const int nch = w_chunks(dout);
+    if (ly.cout % 4 == 0)
+        k_conv_bwd_w<4><<<dim3(ly.cout / 4 * ly.cin, nch), 256, 0, s>>>(gz, dout, in, ly.cin, din, ly.stride, wpart);
+    else if (ly.cout == 3)
+        k_conv_bwd_w<3><<<dim3(ly.cin, nch), 256, 0, s>>>(gz, dout, in, ly.cin, din, ly.stride, wpart);
+    else
+        throw std::runtime_error("conv: output channels not 3 or a multiple of 4");
 }
 
 }  // namespace
@@ -825,12 +985,11 @@ void learn_create(gputo_handle *h)
     L->count = ldalloc<int>(L, 4);
     L->partials = ldalloc<double>(L, 2 * kRedBlocks);
     {
-        // weight-gradient partials: the largest (cout*cin) x chunks x 28 over the layers
+        // weight-gradient partials: (cout*cin) x chunks x 28 of every layer
         const Dims3 dims[kNetLayers] = {L->d0, L->d1, L->d2, L->d2, L->d1, L->d0};
-        long mx = 1;
-        for (int i = 0; i < kNetLayers; ++i)
-            mx = std::max(mx, (long)L->L[i].cout * L->L[i].cin * 28 * ((dims[i].size() + kWChunk - 1) / kWChunk));
-        L->wpart = ldalloc<float>(L, mx);
+        long n = 0;
+        for (int i = 0; i < kNetLayers; ++i) n += (long)L->L[i].cout * L->L[i].cin * 28 * w_chunks(dims[i]);
+        L->wpart = ldalloc<float>(L, n);
     }
     L->nsamp_max = 64;
     L->samples = ldalloc<float>(L, (size_t)L->nsamp_max * nd);
@@ -908,26 +1067,59 @@ void learn_forward(gputo_handle *h, const int *ctl, const CorrIO *io)
     conv_fwd(s, c6);
 }
 
-// parameter gradients of <gy, y> accumulated into G (forward cache current)
+// parameter gradients of <gy, y> into G (forward cache current).  Every
+// gradient of an activation is stored with the activation's ReLU mask
+// applied.
 void learn_backward(gputo_handle *h)
 {
     LearnState *L = h->ln;
     hipStream_t s = h->stream;
     const Dims3 d0 = L->d0, d1 = L->d1, d2 = L->d2;
-    const float *P = L->P;
-    float *G = L->G;
-    conv_bwd(s, L->L[5], P, G, L->wpart, L->u1, d0, L->y, d0, L->gy, L->gu1);
+    // layer: input, its grid, output grid, masked output gradient
+    const float *in[kNetLayers] = {L->x0, L->e1, L->e2, L->e3, L->u2, L->u1};
+    const Dims3 di[kNetLayers] = {d0, d0, d1, d2, d1, d0}, dd[kNetLayers] = {d0, d1, d2, d2, d1, d0};
+    const float *gz[kNetLayers] = {L->ge1, L->ge2, L->ge3, L->ga2, L->ga1, L->gy};
+    WSum w{};
+    long off = 0;
+    for (int l = 0; l < kNetLayers; ++l) {
+        const NetLayer &ly = L->L[l];
+        w.nch[l] = w_chunks(dd[l]);
+        w.npair[l] = ly.cout * ly.cin;
+        w.cin[l] = ly.cin;
+        w.w_off[l] = ly.w_off;
+        w.b_off[l] = ly.b_off;
+        w.part[l] = off;
+        w.first[l + 1] = w.first[l] + 28 * w.npair[l];
+        off += 28L * w.npair[l] * w.nch[l];
+    }
+    auto layer = [&](int l, float *gin, const float *add, const float *act) {
+        const NetLayer &ly = L->L[l];
+        if (gin) {
+            ConvBwd a{};
+            a.g = gz[l];
+            a.w = L->P + ly.w_off;
+            a.cin = ly.cin;
+            a.cout = ly.cout;
+            a.din = di[l];
+            a.dout = dd[l];
+            a.gin = gin;
+            a.add = add;
+            a.act = act;
+            conv_bwd_data(s, a, ly.stride);
+        }
+        conv_bwd_w(s, ly, in[l], di[l], dd[l], gz[l], L->wpart + w.part[l]);
+    };
+    layer(5, L->gu1, nullptr, nullptr);
     // u1 = up(a1) + e1
-    k_up_bwd<<<grid256(16 * d1.size()), 256, 0, s>>>(L->gu1, d0, 16, d1, L->ga1);
-    conv_bwd(s, L->L[4], P, G, L->wpart, L->u2, d1, L->a1, d1, L->ga1, L->gu2);
+    k_up_bwd<<<grid256(16 * d1.size()), 256, 0, s>>>(L->gu1, d0, 16, d1, L->a1, L->ga1);
+    layer(4, L->gu2, nullptr, nullptr);
     // u2 = up(a2) + e2
-    k_up_bwd<<<grid256(32 * d2.size()), 256, 0, s>>>(L->gu2, d1, 32, d2, L->ga2);
-    conv_bwd(s, L->L[3], P, G, L->wpart, L->e3, d2, L->a2, d2, L->ga2, L->ge3);
-    conv_bwd(s, L->L[2], P, G, L->wpart, L->e2, d1, L->e3, d2, L->ge3, L->ge2);
-    k_add_inplace<<<grid256(32 * d1.size()), 256, 0, s>>>(L->ge2, L->gu2, 32 * d1.size());
-    conv_bwd(s, L->L[1], P, G, L->wpart, L->e1, d0, L->e2, d1, L->ge2, L->ge1);
-    k_add_inplace<<<grid256(16 * d0.size()), 256, 0, s>>>(L->ge1, L->gu1, 16 * d0.size());
-    conv_bwd(s, L->L[0], P, G, L->wpart, L->x0, d0, L->e1, d0, L->ge1, nullptr);
+    k_up_bwd<<<grid256(32 * d2.size()), 256, 0, s>>>(L->gu2, d1, 32, d2, L->a2, L->ga2);
+    layer(3, L->ge3, nullptr, L->e3);
+    layer(2, L->ge2, L->gu2, L->e2);
+    layer(1, L->ge1, L->gu1, L->e1);
+    layer(0, nullptr, nullptr, nullptr);
+    k_conv_bwd_w_sum<<<(w.first[kNetLayers] + 255) / 256, 256, 0, s>>>(w, L->wpart, L->G);
 }
 
 // e = correction for the defect d (features, forward, output scaling)
@@ -1105,7 +1297,6 @@ int learn_train(gputo_handle *h, int steps, double lr, double *loss_first, doubl
     for (int it = 0; it < steps; ++it) {
         const int smp = it % L->nsamp;
         launch_copy<float, float>(s, L->samples + (long)smp * g.ndof, L->d, g.ndof, nullptr);
-        k_zero<<<grid256(L->nparam), 256, 0, s>>>(L->G, L->nparam);
         correction(h, H, l, L->d, nullptr);
         k_scale_features<<<grid256(3 * g.nnod), 256, 0, s>>>(L->x0, g.nnod, L->sc);
         OpArgsT<float> b = view_args(h, H, l, nullptr);
@@ -1247,7 +1438,6 @@ int gputo_learn_grad(gputo_handle *h, const double *x, const double *gy, double 
         to_float(s, x, L->x0, 4 * n0);
         learn_forward(h, nullptr, nullptr);
         to_float(s, gy, L->gy, 3 * n0);
-        k_zero<<<grid256(L->nparam), 256, 0, s>>>(L->G, L->nparam);
         learn_backward(h);
         check_hip(hipGetLastError(), "launch");
         to_double(s, L->G, g, L->nparam);
