@@ -331,12 +331,18 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
     }
     const bool per = h->prm.periodic != 0;
     launch_diag0(s, L0.g, h->Ke, h->CX, L0.AD, per ? nullptr : L0.RD);
-    // RD: per node where the modal kernel applies Ke0 itself, else per DOF
-    auto fold_diag = [&](Level &v, bool node) {
+    // the periodic diagonal and its RD: per node where the modal kernel applies
+    // Ke0 itself (level 0, every level of mgcg9), per DOF on the rediscretised
+    // level 1, none on the levels below (RD has no room for their DOFs)
+    auto fold_diag = [&](int l) {
+        Level &v = h->L[l];
         launch_per_fold<double>(s, v.g, v.AD, 1, nullptr);
-        launch_recip(s, v.AD, v.RD, node ? v.g.nnod : v.g.ndof, node ? 3 : 1);
+        if (l == 0 || p.mg9)
+            launch_recip(s, v.AD, v.RD, v.g.nnod, 3);
+        else if (l == 1)
+            launch_recip(s, v.AD, v.RD, v.g.ndof, 1);
     };
-    if (per) fold_diag(L0, true);
+    if (per) fold_diag(0);
     if (p.mg9) {
         // mgcg9 (initVcycle, mgcg9.cu:342-414): coarse element scales and
         // diagonals from the unit Ke; the coarsest matrix, when factored,
@@ -363,7 +369,7 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         for (int l = 1; l < h->nl; ++l) {
             Level &v = h->L[l];
             launch_diag0(s, v.g, h->Ke, v.CXl, v.AD, per ? nullptr : v.RD);
-            if (per) fold_diag(v, true);
+            if (per) fold_diag(l);
         }
         HIPCHK(hipGetLastError());
         h->hier_ready = true;
@@ -398,7 +404,7 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
     for (int l = 1; l < h->nl; ++l) {
         Level &v = h->L[l];
         launch_diagA(s, v.g, v.A, v.AD, per || l > 1 ? nullptr : v.RD);
-        if (per) fold_diag(v, false);
+        if (per) fold_diag(l);
         if (v.S) launch_stencil_build(s, v.g, v.A, v.S);
     }
     HIPCHK(hipGetLastError());
