@@ -99,6 +99,7 @@ struct OpArgsT {
     int modal;             // Ke0 has the isotropic modal form: use mc and mw
     T mc[8];               // its modal constants
     ModalWork mw;          // the level's tiling
+    int per;               // modal kernels: periodic cell, the result complete on masters and images
 };
 using OpArgs = OpArgsT<double>;
 
@@ -236,6 +237,7 @@ struct gputo_handle {
     int *ctl_zero = nullptr;      // an always-zero control word
     long long bytes = 0;
     bool hier_ready = false;
+    bool per_masks = false;       // periodic cell: on every level an image is fixed where its master is
     bool masks_ready = false;     // level fixed lists and masks match L[0].fixed
     std::vector<void *> allocs;
     struct ToState *to = nullptr;

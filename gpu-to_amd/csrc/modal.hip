@@ -42,6 +42,15 @@
 // deterministic.  Elements outside the mesh take loads past the buffer's
 // range, which return 0, so nothing of a neighbouring row enters a sum.
 //
+// Periodic cells (PER).  An iterate is equal on a master node and its images,
+// a residual lives on the masters and is 0 on the images.  The list's entries
+// before the first column, row and layer hold the last elements of their row
+// instead of none, a block owns masters only, and the epilogue writes the
+// images too: the whole periodic row, its Jacobi update and both node copies
+// come from one launch.  (The operator without the wrap, then a pass that
+// folds the images into the masters, updates and copies back, took 22.9 +
+// 10.4 us per level-0 sweep of six right-hand sides at 48x48x48; 25.8 us now.)
+//
 // Measured on MI355X at 192x96x96 (matvecs back to back; before: node-gather,
 // split-BF16 MFMA and Gauss point by Gauss point kernels): FP64 level 0
 // 75 -> 29 us (101 MB of operands, 3.5 TB/s; 87 % of the VALU operations are
@@ -53,6 +62,7 @@
 // waves per SIMD that cover its latency.
 #include <algorithm>
 #include <cmath>
+#include <stdexcept>
 #include <type_traits>
 
 #include "vcycle.h"
@@ -330,7 +340,7 @@ constexpr int md_min_waves()
     return sizeof(T) == 8 ? (EL == 0 ? 2 : 1) : (EL == 0 ? 4 : 3);
 }
 
-template <class T, class TU, int MODE, int EL>
+template <class T, class TU, int MODE, int EL, bool PER>
 __global__ __launch_bounds__((sizeof(T) == 8 && EL == 1 ? 4 : kMdMaxWaves) * 64) __attribute__((amdgpu_waves_per_eu(md_min_waves<T, EL>())))
 void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
 {
@@ -356,22 +366,31 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     const int ch = (int)(tb % (unsigned)w.nch);
     const unsigned r1 = tb / (unsigned)w.nch;
     const int s = (int)(r1 % (unsigned)w.ns), ib = (int)(r1 / (unsigned)w.ns);
-    const int i0 = ib * w.TI, i1 = min(i0 + w.TI, g.nnx);  // owned node layers
+    // owned node layers (PER: masters only)
+    const int i0 = ib * w.TI, i1 = min(i0 + w.TI, PER ? g.nx : g.nnx);
+    if (PER && i0 >= i1) {
+        if (a.partials && threadIdx.x == 0) a.partials[blockIdx.x] = 0.0;
+        return;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int t = wave * 63 + lane;  // the block's entry (a wave's last is the next one's first)
     // list entry q = ch M - (R + 1) + t -> row k, column c
     const unsigned qs = (unsigned)(ch * w.M + t + w.R - 1);  // q + 2R >= 0
     const int kq = (int)(qs / (unsigned)w.R), c = (int)(qs - (unsigned)(kq * w.R));
     const int k = kq - 2, j = s * w.W - 1 + c;
-    const bool el_ok = k >= 0 && k < g.nz && j >= 0 && j < g.ny;
-    const bool own = lane > 0 && t > w.R && t <= w.R + w.M && c > 0 && k >= 0 && k < g.nnz && j < g.nny;
+    // the entry's element; PER: element -1 is the last one of its row
+    const int ke = PER && k == -1 ? g.nz - 1 : k, je = PER && j == -1 ? g.ny - 1 : j;
+    const bool el_ok = ke >= 0 && ke < g.nz && je >= 0 && je < g.ny;
+    const bool own = lane > 0 && t > w.R && t <= w.R + w.M && c > 0 && k >= 0 && k < (PER ? g.nz : g.nnz) &&
+                     j < (PER ? g.ny : g.nny);
     const int plane = g.nny * g.nnz;
-    const int nod0 = k * g.nny + j;  // node in its plane
+    const int nod0 = k * g.nny + j;    // own node in its plane
+    const int enod = ke * g.nny + je;  // the element's first node
     // byte offsets in a plane of the element's two node rows, of its scale(s)
     // and of the own node
-    const int ulo = el_ok ? 3 * SU * nod0 : kMdOut, uhi = el_ok ? 3 * SU * (nod0 + g.nny) : kMdOut;
-    const int flo = el_ok ? 3 * S * nod0 : kMdOut, fhi = el_ok ? 3 * S * (nod0 + g.nny) : kMdOut;
-    const int eo = el_ok ? (EL == 0 ? S * (k * g.ny + j) : S * (4 * k * g.ny + 2 * j)) : kMdOut;
+    const int ulo = el_ok ? 3 * SU * enod : kMdOut, uhi = el_ok ? 3 * SU * (enod + g.nny) : kMdOut;
+    const int flo = el_ok ? 3 * S * enod : kMdOut, fhi = el_ok ? 3 * S * (enod + g.nny) : kMdOut;
+    const int eo = el_ok ? (EL == 0 ? S * (ke * g.ny + je) : S * (4 * ke * g.ny + 2 * je)) : kMdOut;
     const int oo = own ? 3 * S * nod0 : kMdOut, uo = own ? 3 * SU * nod0 : kMdOut;
     const long vb = (long)S * g.ndof;
     const MdBuf BU = PRE ? md_buf(a.F, vb)
@@ -379,7 +398,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     const MdBuf BF = md_buf(a.F, MV ? 0 : vb), BD = md_buf(a.RD, (JAC || PRE) ? (EL == 0 ? vb / 3 : vb) : 0);
     const MdBuf BE = md_buf(CX, (long)S * (EL == 0 ? 1 : 8) * g.nel), BM = md_buf(a.mask, a.mask ? g.nnod : 0);  // no mask: reads 0
     const int up = 3 * SU * plane, fp = 3 * S * plane;         // bytes of a node layer
-    const int dp = S * plane, dlo = el_ok ? S * nod0 : kMdOut, dhi = el_ok ? S * (nod0 + g.nny) : kMdOut;
+    const int dp = S * plane, dlo = el_ok ? S * enod : kMdOut, dhi = el_ok ? S * (enod + g.nny) : kMdOut;
     const int ep = (EL == 0 ? 1 : 4) * S * g.ny * g.nz;        // bytes of a scale layer
     const T pr = T(a.prerelax), om = T(a.omega);
 
@@ -463,28 +482,42 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
         for (int cc = 0; cc < 3; ++cc) {
             const T yc = y[cc] + buf[cc * ne + t - w.R];
             const bool fixed = (e.m >> cc) & 1u;
+            T v;
             if (MV) {
-                const T v = fixed ? T(0) : yc;
-                a.out[dof + cc] = v;
+                v = fixed ? T(0) : yc;
                 part += (double)e.u[cc] * (double)v;
             } else if (!JAC) {
-                a.out[dof + cc] = fixed ? T(0) : e.f[cc] - yc;
+                v = fixed ? T(0) : e.f[cc] - yc;
                 if (PRE) a.out2[dof + cc] = pr * (e.f[cc] * e.d[cc]);
             } else {
                 // U = (1-w) U + w (R + AD U)/AD = U + w R/AD  (mgcg1.cu:1199-1206)
                 const T u = PRE ? pr * (e.f[cc] * e.d[cc]) : T(e.u[cc]);
                 const T rv = fixed ? T(0) : e.f[cc] - yc;
-                a.out[dof + cc] = fma(om * e.d[cc], rv, u);
+                v = fma(om * e.d[cc], rv, u);
+            }
+            a.out[dof + cc] = v;
+            if (PER) {
+                // the images: an iterate's value, 0 for a residual
+                const bool bi = pl == 0, bk = k == 0, bj = j == 0;
+                if (bi || bk || bj) {
+                    const T im = JAC ? v : T(0);
+                    const long di = 3L * plane * g.nx, dk = 3L * g.nny * g.nz, dj = 3L * g.ny;
+#pragma unroll
+                    for (int q = 1; q < 8; ++q)
+                        if ((!(q & 4) || bi) && (!(q & 2) || bk) && (!(q & 1) || bj))
+                            a.out[dof + cc + (q & 4 ? di : 0) + (q & 2 ? dk : 0) + (q & 1 ? dj : 0)] = im;
+                }
             }
         }
     };
 
-    const int lo = max(i0 - 1, 0), hi = min(i1, g.nnx - 1);  // node layers read
+    // node layers read (PER: layer -1 is layer nx - 1)
+    const int lo = PER ? i0 - 1 : max(i0 - 1, 0), hi = min(i1, g.nnx - 1), first = PER && i0 == 0 ? g.nx - 1 : lo;
     Raw xa, xb;
     MdScale<T, EL> ea, eb;
-    load(lo, xa);
+    load(first, xa);
     load(lo + 1, xb);
-    load_e(lo, ea);
+    load_e(first, ea);
     if (a.ctl && a.ctl[0]) return;  // converged: read with the loads above
     Jk<T> pa, pb, pend;
     jk(xa, pa);
@@ -556,7 +589,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
         step(pl, pa, pb, xb, AHEAD ? xa : xb, ea, AHEAD ? eb : ea);
         if (pl + 1 <= hi) step(pl + 1, pb, pa, AHEAD ? xa : xb, xb, AHEAD ? eb : ea, ea);
     }
-    if (i1 == g.nnx) {  // the last node layer of the mesh ends with what is pending
+    if (!PER && i1 == g.nnx) {  // the last node layer of the mesh ends with what is pending
         Epi epi;
         load_epi(g.nnx - 1, epi);
         finish(g.nnx - 1, pend, epi);
@@ -582,15 +615,24 @@ void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
     const ModalWork &w = a.mw;
     const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb)), block(64 * w.NW);
     const unsigned lds = 6u * (63u * w.NW + 1u) * sizeof(T);
+    if (a.per) {
+        switch (mode) {
+        case OP_MATVEC: k_modal<T, T, OP_MATVEC, EL, true><<<grid, block, lds, s>>>(a, w, CX); break;
+        case OP_DEFECT: k_modal<T, T, OP_DEFECT, EL, true><<<grid, block, lds, s>>>(a, w, CX); break;
+        case OP_JACOBI: k_modal<T, T, OP_JACOBI, EL, true><<<grid, block, lds, s>>>(a, w, CX); break;
+        default: throw std::runtime_error("periodic operator: mode");  // the prerelaxed modes read F on images
+        }
+        return;
+    }
     switch (mode) {
-    case OP_MATVEC: k_modal<T, T, OP_MATVEC, EL><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_DEFECT: k_modal<T, T, OP_DEFECT, EL><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_JACOBI: k_modal<T, T, OP_JACOBI, EL><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_PRE_JACOBI: k_modal<T, T, OP_PRE_JACOBI, EL><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_PRE_DEFECT: k_modal<T, T, OP_PRE_DEFECT, EL><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_MATVEC: k_modal<T, T, OP_MATVEC, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_DEFECT: k_modal<T, T, OP_DEFECT, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_JACOBI: k_modal<T, T, OP_JACOBI, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_PRE_JACOBI: k_modal<T, T, OP_PRE_JACOBI, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_PRE_DEFECT: k_modal<T, T, OP_PRE_DEFECT, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
     case OP_MATVEC_UF:
         if constexpr (EL == 0 && std::is_same<T, double>::value)
-            k_modal<double, float, OP_MATVEC_UF, 0><<<grid, block, lds, s>>>(a, w, CX);
+            k_modal<double, float, OP_MATVEC_UF, 0, false><<<grid, block, lds, s>>>(a, w, CX);
         break;
     default: break;
     }

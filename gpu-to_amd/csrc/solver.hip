@@ -182,6 +182,23 @@ static std::vector<uint8_t> node_mask(const std::vector<int> &fixed, const Grid 
     return m;
 }
 
+// whether every image node of a periodic cell has its master's mask
+static bool images_as_masters(const std::vector<uint8_t> &m, const Grid &g)
+{
+    for (int i = 0; i < g.nnx; ++i)
+        for (int k = 0; k < g.nnz; ++k)
+            for (int j = 0; j < g.nny; ++j) {
+                if (i < g.nx && k < g.nz && j < g.ny) {
+                    j = g.ny - 1;  // to the row's image
+                    continue;
+                }
+                const long p = (long)g.nny * g.nnz * i + (long)g.nny * k + j;
+                const long q = (long)g.nny * g.nnz * (i % g.nx) + (long)g.nny * (k % g.nz) + j % g.ny;
+                if (m[p] != m[q]) return false;
+            }
+    return true;
+}
+
 }  // namespace gputo
 
 using namespace gputo;
@@ -326,6 +343,7 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
                 HIPCHK(hipMemcpyAsync(v.fixed_d, v.fixed.data(), v.fixed.size() * sizeof(int),
                                       hipMemcpyHostToDevice, s));
             HIPCHK(hipStreamSynchronize(s));  // host vectors above are temporaries
+            if (h->prm.periodic) h->per_masks = (l == 0 || h->per_masks) && images_as_masters(m, v.g);
         }
         h->masks_ready = true;
     }
@@ -525,6 +543,7 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
             a.U = h->P;
             a.out = h->Q;
             a.partials = h->partials;
+            a.per = per_fused(h, f64_view(h), 0);
             if (p32) {
                 a.Uf = pk;
                 launch_op0_uf(s, a);
@@ -533,7 +552,7 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
             }
             // p.q over the full grid is the periodic p.Kp before the fold
             // (p is equal on images); the fold completes q for the update
-            if (per) launch_per_fold<double>(s, L0.g, h->Q, 0, ctl);
+            if (per && !a.per) launch_per_fold<double>(s, L0.g, h->Q, 0, ctl);
             if (p32) {
                 launch_cg_alpha_log(s, h->sc, h->partials, nmv, alog + sl);
                 launch_cg_update_r(s, h->R, h->Q, n, h->sc, h->partials, r32, ad32, x0, prx);
@@ -737,8 +756,9 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
             a.partials = b.partials;
             a.ctl = ctl;
             a.nb = nb;
+            a.per = per_fused(h, H64, 0);
             launch_op0(s, OP_MATVEC, a);
-            if (per) launch_per_fold<double>(s, L0.g, b.Q, 0, ctl, nb);
+            if (per && !a.per) launch_per_fold<double>(s, L0.g, b.Q, 0, ctl, nb);
             launch_cg_alpha(s, b.sc, b.partials, nmv, nb);
             launch_cg_update_ur(s, U, b.R, b.P, b.Q, n, b.sc, b.partials, r32, nb);
             launch_cg_check(s, b.sc, b.partials, kRedBlocks, tol, maxit, nb);

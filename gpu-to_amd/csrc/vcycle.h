@@ -154,6 +154,20 @@ void level_op(const gputo_handle *h, const HierView<T> &H, int l, int mode, cons
     }
 }
 
+// Whether level l of a periodic cell runs the modal kernels' periodic form
+// (results complete on masters and images); else the non-periodic operator
+// with the fold and image kernels.
+template <class T>
+bool per_fused(const gputo_handle *h, const HierView<T> &H, int l)
+{
+    if (!H.per || !h->per_masks) return false;
+    const ModalWork &mw = std::is_same<T, double>::value ? h->L[l].mw64 : h->L[l].mw32;
+    if (mw.NW == 0) return false;
+    if (l == 1 && H.l1_mf && !H.mg9) return true;
+    if (!h->ke_modal || (l > 0 && !H.mg9)) return false;
+    return std::is_same<T, double>::value || H.mg9 || H.l0 == L0_GATHER || H.l0 == L0_MODAL;
+}
+
 // Periodic sweeps: each is the non-periodic defect into R, then the
 // Jacobi update of every master from its folded defect, copied to its
 // images; `pre` first sets U = prerelax*F/AD.
@@ -181,8 +195,18 @@ template <class T>
 void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T *U, int n, bool pre, const int *ctl,
               bool in_tmp = false)
 {
-    if (H.per) return sweeps_per(h, H, l, F, U, n, pre, ctl);
+    const bool fused = per_fused(h, H, l);
+    if (H.per && !fused) return sweeps_per(h, H, l, F, U, n, pre, ctl);
     const LevelView<T> &v = H.L[l];
+    if (pre && H.per) {
+        // F is 0 on the images: the prerelaxed iterate is written by its own
+        // pass, where the sweeps from it end in U
+        const Preset p = preset_of(h->prm);
+        in_tmp = n % 2 == 1;
+        launch_per_jacobi<T>(h->stream, h->L[l].g, in_tmp ? v.Tmp : U, v.R, F, v.AD, h->L[l].mask, p.omega, p.prerelax,
+                             1, ctl, H.nb);
+        pre = false;
+    }
     if (pre && l == 0 && n > 0 && !H.mg9 && H.l0 >= L0_MFMA_F32) {
         // MFMA level 0: the prerelaxed iterate is written by an elementwise
         // pass and the first sweep is a plain one (measured at 192x96x96:
@@ -206,6 +230,7 @@ void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T 
         a.U = src;
         a.F = F;
         a.out = dst;
+        a.per = fused;
         level_op(h, H, l, (pre && s == 0) ? OP_PRE_JACOBI : OP_JACOBI, a);
         src = dst;
     }
@@ -271,8 +296,9 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
                 a.U = U;
                 a.F = F;
                 a.out = v.R;
+                a.per = per_fused(h, H, l);
                 level_op(h, H, l, OP_DEFECT, a);
-                if (H.per) launch_per_fold<T>(h->stream, lv.g, v.R, 0, ctl, H.nb);
+                if (H.per && !a.per) launch_per_fold<T>(h->stream, lv.g, v.R, 0, ctl, H.nb);
             }
         } else if (!h->C.direct) {
             // coarsest level too large to factor: 10*npre sweeps from the
@@ -290,7 +316,7 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
         // an odd number of post-sweeps starts from Tmp so the last one
         // writes U without a copy
         const int npost = sweeps_of<T>(h, l, true);
-        const bool to_tmp = !H.per && npost % 2 == 1;
+        const bool to_tmp = (!H.per || per_fused(h, H, l)) && npost % 2 == 1;
         launch_interp_to<T>(h->stream, h->L[l].g, H.L[l + 1].U, U, to_tmp ? H.L[l].Tmp : U, h->L[l].mask,
                             p.zero_after_interp, ctl, H.nb);
         sweeps_t(h, H, l, F, U, npost, false, ctl, to_tmp);

@@ -105,3 +105,24 @@ def test_other_element_matrices_take_the_general_kernels(gputo, oracle, kernel, 
     assert rel(s.matvec_mixed(kernel, Ke, CX, u, fixed), yo) < tol
     assert rel(s.matvec(Ke, CX, u, fixed), yo) < 1e-13
     s.close()
+
+
+@pytest.mark.parametrize("cell", [(4, 4, 4), (8, 136, 4), (4, 24, 68), (68, 4, 20)])
+def test_periodic_form_is_translation_invariant(gputo, cell):
+    """The periodic form of the kernels over cells that need one and several
+    strips, chunks and layer groups: a cell moved by half its size in each
+    direction has the same tensor (1e-8, the CG tolerance), and images hold
+    their masters' values bit for bit."""
+    nx, ny, nz = cell
+    rng = np.random.default_rng(67)
+    x = 0.2 + 0.8 * rng.uniform(size=(nx, nz, ny))
+    Ke = gputo.ke0_h8()
+    s = gputo.Solver(nx, ny, nz, 2, periodic=True)
+    C, _, _, chi = s.homogenize(Ke, x.ravel(), 1e-10, 400, fields=True)
+    C2 = s.homogenize(Ke, np.roll(x, (nx // 2, nz // 2, ny // 2), (0, 1, 2)).ravel(), 1e-10, 400)[0]
+    assert np.abs(C - C2).max() < 1e-8 * np.abs(C).max()
+    u = chi.reshape(6, nx + 1, nz + 1, ny + 1, 3)
+    assert np.array_equal(u[:, 0], u[:, -1])
+    assert np.array_equal(u[:, :, 0], u[:, :, -1])
+    assert np.array_equal(u[:, :, :, 0], u[:, :, :, -1])
+    s.close()
