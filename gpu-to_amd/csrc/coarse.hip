@@ -23,9 +23,13 @@ __device__ constexpr int kKE[8] = {0, 0, 0, 0, 1, 1, 1, 1};
 // Level-1 rediscretisation (coarseAe2c, mgcg1.cu:2042-2070): the packed
 // coarse element matrix is sum_na CX[child(na)] * Aelm[:, na] where Aelm
 // holds the h=2 Gauss-point stiffness matrices and child na = 4 iP + 2 kP
-// + jP.  One thread per coarse element; Aelm is read through the scalar
-// cache (uniform addresses).
+// + jP.  One thread per coarse element and kL1Entries packed entries (so that
+// a small level fills the device, too: 26 us at 128 elements with all 300
+// entries in one thread); Aelm is read through the scalar cache (uniform
+// addresses).
 // ---------------------------------------------------------------------------
+constexpr int kL1Entries = 30;
+
 __global__ __launch_bounds__(256) void k_coarse_l1(Grid gc, const double *__restrict__ Aelm,
                                                   const double *__restrict__ CXf, double *__restrict__ A)
 {
@@ -41,7 +45,8 @@ __global__ __launch_bounds__(256) void k_coarse_l1(Grid gc, const double *__rest
 #pragma unroll
             for (int jP = 0; jP < 2; ++jP)
                 cx[4 * iP + 2 * kP + jP] = CXf[(long)fny * fnz * (2 * i + iP) + (long)fny * (2 * k + kP) + 2 * j + jP];
-    for (int m = 0; m < 300; ++m) {
+    const int m0 = blockIdx.y * kL1Entries;
+    for (int m = m0; m < m0 + kL1Entries; ++m) {
         double s = 0.0;
 #pragma unroll
         for (int na = 0; na < 8; ++na) s += cx[na] * Aelm[8 * m + na];
@@ -51,7 +56,55 @@ __global__ __launch_bounds__(256) void k_coarse_l1(Grid gc, const double *__rest
 
 void launch_coarse_l1(hipStream_t s, const Grid &gc, const double *Aelm, const double *CXf, double *A)
 {
-    k_coarse_l1<<<(unsigned)((gc.nel + 255) / 256), 256, 0, s>>>(gc, Aelm, CXf, A);
+    k_coarse_l1<<<dim3((unsigned)((gc.nel + 255) / 256), 300 / kL1Entries), 256, 0, s>>>(gc, Aelm, CXf, A);
+}
+
+// Diagonal of that operator from the child densities, without its element
+// matrices (AD and 1/AD): sum over a node's 8 elements of sum_na CX[child(na)]
+// Aelm[(m, m), na], in the element order of k_diag.
+__global__ __launch_bounds__(256) void k_diag_l1(Grid g, const double *__restrict__ Aelm,
+                                                const double *__restrict__ CXf, double *__restrict__ AD,
+                                                double *__restrict__ RD)
+{
+    const long nod = (long)blockIdx.x * 256 + threadIdx.x;
+    if (nod >= g.nnod) return;
+    const unsigned nu = (unsigned)nod, q1 = nu / (unsigned)g.nny;
+    const int j = (int)(nu - q1 * (unsigned)g.nny), k = (int)(q1 % (unsigned)g.nnz), i = (int)(q1 / (unsigned)g.nnz);
+    const int fny = 2 * g.ny, fnz = 2 * g.nz;
+    double d[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int ei = 0; ei < 2; ++ei)
+#pragma unroll
+        for (int ek = 0; ek < 2; ++ek)
+#pragma unroll
+            for (int ej = 0; ej < 2; ++ej) {
+                const int ex = i - 1 + ei, ey = j - 1 + ej, ez = k - 1 + ek;
+                if (ex < 0 || ex >= g.nx || ey < 0 || ey >= g.ny || ez < 0 || ez >= g.nz) continue;
+                const int la = lidx2(1 - ei, 1 - ej, 1 - ek);
+                double cx[8];
+#pragma unroll
+                for (int na = 0; na < 8; ++na)
+                    cx[na] = CXf[(long)fny * fnz * (2 * ex + (na >> 2)) + (long)fny * (2 * ez + ((na >> 1) & 1)) + 2 * ey +
+                                 (na & 1)];
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const int m = 3 * la + c;
+                    double s = 0.0;
+#pragma unroll
+                    for (int na = 0; na < 8; ++na) s += cx[na] * Aelm[8 * pidx2(m, m) + na];
+                    d[c] += s;
+                }
+            }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        AD[3 * nod + c] = d[c];
+        if (RD) RD[3 * nod + c] = 1.0 / d[c];
+    }
+}
+
+void launch_diag_l1(hipStream_t s, const Grid &g, const double *Aelm, const double *CXf, double *AD, double *RD)
+{
+    k_diag_l1<<<(unsigned)((g.nnod + 255) / 256), 256, 0, s>>>(g, Aelm, CXf, AD, RD);
 }
 
 // ---------------------------------------------------------------------------
@@ -60,10 +113,12 @@ void launch_coarse_l1(hipStream_t s, const Grid &gc, const double *Aelm, const d
 // the coarse element's 8 nodes onto its 27 fine nodes, so the (a,b) node
 // block of A_c is
 //   sum_ch sum_{p,q} w(a, ch+p) w(b, ch+q) A_ch[p q block],
-// with w(a, x) = prod_axis (1 - |2 a_axis - x_axis| / 2).  One 64-thread
-// block per coarse element stages its 8 children (full 24x24 each) in LDS;
-// thread (a >= b) forms one 3x3 block.  Children come from the packed
-// matrices of the finer level, or are CX*Ke on level 0.
+// with w(a, x) = prod_axis (1 - |2 a_axis - x_axis| / 2).  One block per
+// coarse element stages its 8 children's packed matrices in LDS and forms
+// T_ch = A_ch P_ch (24 x 24 each, sums over q), then the 300 entries of
+// sum_ch P_ch^T T_ch (sums over ch and p).  (36 threads that
+// each ran the triple sum for a 3 x 3 block took 91-95 us a launch, however
+// few the elements; this form 14 us for 54 elements and 24 us for 432.)
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double trilin_w(int a, int x0, int x1, int x2)
 {
@@ -74,60 +129,64 @@ __device__ __forceinline__ double trilin_w(int a, int x0, int x1, int x2)
     return w0 * w1 * w2;
 }
 
-__global__ __launch_bounds__(64) void k_galerkin(Grid gc, const double *__restrict__ Af, const double *__restrict__ Ke,
-                                                const double *__restrict__ CXf, double *__restrict__ Ac)
+constexpr int kGalThreads = 256;
+
+__global__ __launch_bounds__(kGalThreads) void k_galerkin(Grid gc, const double *__restrict__ Af,
+                                                         double *__restrict__ Ac)
 {
-    __shared__ double S[8][576];
+    __shared__ double S[8][300];
+    __shared__ double T[8][24][25];
+    __shared__ double W[8][8][8];  // [child][child node q][coarse node b]
     const long e = blockIdx.x;
     const int j = (int)(e % gc.ny), k = (int)((e / gc.ny) % gc.nz), i = (int)(e / ((long)gc.ny * gc.nz));
-    const int fny = 2 * gc.ny, fnz = 2 * gc.nz;
+    const int fny = 2 * gc.ny, fnz = 2 * gc.nz, tid = threadIdx.x;
     const long nelf = 8 * gc.nel;
-    for (int ch = 0; ch < 8; ++ch) {
-        const int ci = kIE[ch], cj = kJE[ch], ck = kKE[ch];
-        const long eP = (long)fny * fnz * (2 * i + ci) + (long)fny * (2 * k + ck) + 2 * j + cj;
-        const double cx = Af ? 0.0 : CXf[eP];
-        for (int m = threadIdx.x; m < 576; m += 64) {
-            const int r = m / 24, c = m - 24 * r;
-            S[ch][m] = Af ? Af[(long)pidx2(r, c) * nelf + eP] : cx * Ke[m];
-        }
+    constexpr int kIt = (8 * 300 + kGalThreads - 1) / kGalThreads;
+    double v[kIt];
+#pragma unroll
+    for (int u = 0; u < kIt; ++u) {  // child fastest: neighbouring children are neighbouring in memory
+        const int q = tid + u * kGalThreads, ch = q & 7, p = min(q >> 3, 299);
+        const long eP = (long)fny * fnz * (2 * i + (ch >> 2)) + (long)fny * (2 * k + ((ch >> 1) & 1)) + 2 * j + (ch & 1);
+        v[u] = Af[(long)p * nelf + eP];
+    }
+    // children in the order (ci, ck, cj) = bits 4, 2, 1
+#pragma unroll
+    for (int u = 0; u < kIt; ++u) {
+        const int q = tid + u * kGalThreads;
+        if (q < 8 * 300) S[q & 7][q >> 3] = v[u];
+    }
+    for (int q = tid; q < 512; q += kGalThreads) {
+        const int ch = q >> 6, n = (q >> 3) & 7, b = q & 7;
+        W[ch][n][b] = trilin_w(b, (ch >> 2) + kIE[n], (ch & 1) + kJE[n], ((ch >> 1) & 1) + kKE[n]);
     }
     __syncthreads();
-    const int q = threadIdx.x;
-    if (q >= 36) return;
-    int a = 0;
-    while ((a + 1) * (a + 2) / 2 <= q) ++a;
-    const int b = q - a * (a + 1) / 2;
-    double blk[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    for (int ch = 0; ch < 8; ++ch) {
-        const int ci = kIE[ch], cj = kJE[ch], ck = kKE[ch];
+    for (int q = tid; q < 8 * 576; q += kGalThreads) {
+        const int ch = q / 576, r = (q / 24) % 24, n = q % 24, b = n / 3, d = n - 3 * b;
+        double t = 0.0;
+#pragma unroll
         for (int p = 0; p < 8; ++p) {
-            const double wa = trilin_w(a, ci + kIE[p], cj + kJE[p], ck + kKE[p]);
-            if (wa == 0.0) continue;
-            for (int r = 0; r < 8; ++r) {
-                const double wb = trilin_w(b, ci + kIE[r], cj + kJE[r], ck + kKE[r]);
-                if (wb == 0.0) continue;
-                const double w = wa * wb;
-                const double *s = &S[ch][24 * (3 * p) + 3 * r];
-#pragma unroll
-                for (int c = 0; c < 3; ++c)
-#pragma unroll
-                    for (int d = 0; d < 3; ++d) blk[c][d] += w * s[24 * c + d];
-            }
+            const int m = 3 * p + d;
+            t += W[ch][p][b] * S[ch][m <= r ? r * (r + 1) / 2 + m : m * (m + 1) / 2 + r];
         }
+        T[ch][r][n] = t;
     }
+    __syncthreads();
+    for (int q = tid; q < 300; q += kGalThreads) {
+        int m = (int)((sqrtf(8.0f * q + 1.0f) - 1.0f) * 0.5f);
+        m += (m + 1) * (m + 2) / 2 <= q;
+        m -= m * (m + 1) / 2 > q;
+        const int n = q - m * (m + 1) / 2, a = m / 3, c = m - 3 * a;
+        double t = 0.0;
+        for (int ch = 0; ch < 8; ++ch)
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            const int r = 3 * a + c, s = 3 * b + d;
-            if (r >= s) Ac[(long)pidx2(r, s) * gc.nel + e] = blk[c][d];
-        }
+            for (int p = 0; p < 8; ++p) t += W[ch][p][a] * T[ch][3 * p + c][n];
+        Ac[(long)q * gc.nel + e] = t;
+    }
 }
 
-void launch_coarse_galerkin(hipStream_t s, const Grid &gc, const double *Af, const double *Ke, const double *CXf,
-                            double *Ac)
+void launch_coarse_galerkin(hipStream_t s, const Grid &gc, const double *Af, double *Ac)
 {
-    k_galerkin<<<(unsigned)gc.nel, 64, 0, s>>>(gc, Af, Ke, CXf, Ac);
+    k_galerkin<<<(unsigned)gc.nel, kGalThreads, 0, s>>>(gc, Af, Ac);
 }
 
 // ---------------------------------------------------------------------------
@@ -399,43 +458,56 @@ void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, d
 }
 
 // ---------------------------------------------------------------------------
-// Dense coarsest assembly (assembAc, mgcg1.cu:1747-1806): one thread per
-// matrix row gathers the 8 incident element matrices.  The matrix is padded
-// to N = roundup(n, 32) with an identity block so the blocked kernels below
-// work on whole 32x32 tiles.
+// Dense coarsest assembly (assembAc, mgcg1.cu:1747-1806).  The matrix is
+// padded to N = roundup(n, 32) with an identity block so the blocked kernels
+// below work on whole 32x32 tiles.  One block per row writes its columns from
+// `back` tiles before its own tile to the end of that (zeros included: nothing
+// beyond is read), each thread one column: the entry sums the elements that
+// hold both nodes, up to 8.  (One thread per row that added its 192 element
+// entries to zeroed memory one by one took 29-60 us after a fill of the
+// whole matrix; 5-8 us now, and no fill.)
 // ---------------------------------------------------------------------------
 constexpr int NB = 32;
 
-__global__ void k_assemble(Grid g, const double *__restrict__ A, double *__restrict__ AQ, int N)
+__global__ __launch_bounds__(256) void k_assemble(Grid g, const double *__restrict__ A, double *__restrict__ AQ, int N,
+                                                 int back)
 {
-    const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= N) return;
-    if (r >= g.ndof) {
-        AQ[r * N + r] = 1.0;
-        return;
-    }
-    const long nod = r / 3;
-    const int c = (int)(r % 3);
-    const int j = (int)(nod % g.nny), k = (int)((nod / g.nny) % g.nnz), i = (int)(nod / ((long)g.nny * g.nnz));
-    for (int ei = 0; ei < 2; ++ei)
-        for (int ek = 0; ek < 2; ++ek)
-            for (int ej = 0; ej < 2; ++ej) {
-                const int ex = i - 1 + ei, ey = j - 1 + ej, ez = k - 1 + ek;
-                if (ex < 0 || ex >= g.nx || ey < 0 || ey >= g.ny || ez < 0 || ez >= g.nz) continue;
-                const long e = (long)g.ny * g.nz * ex + (long)g.ny * ez + ey;
-                const int la = lidx2(1 - ei, 1 - ej, 1 - ek);
-                for (int lb = 0; lb < 8; ++lb) {
-                    const long nb = (long)g.nny * g.nnz * (ex + kIE[lb]) + (long)g.nny * (ez + kKE[lb]) + (ey + kJE[lb]);
-                    for (int d = 0; d < 3; ++d) AQ[r * N + 3 * nb + d] += A[(long)pidx2(3 * la + c, 3 * lb + d) * g.nel + e];
-                }
+    const int r = blockIdx.x;
+    const int c0 = max(0, r / NB - back) * NB, c1 = (r / NB + 1) * NB;
+    const int nr = r / 3, cr = r - 3 * nr;
+    const int j = nr % g.nny, k = (nr / g.nny) % g.nnz, i = nr / (g.nny * g.nnz);
+    for (int c = c0 + (int)threadIdx.x; c < c1; c += 256) {
+        double v = 0.0;
+        if (r >= g.ndof || c >= g.ndof) {
+            v = r == c ? 1.0 : 0.0;
+        } else {
+            const int nc = c / 3, cc = c - 3 * nc;
+            const int dj = nc % g.nny - j, dk = (nc / g.nny) % g.nnz - k, di = nc / (g.nny * g.nnz) - i;
+            if (abs(di) <= 1 && abs(dk) <= 1 && abs(dj) <= 1) {
+                for (int ei = 0; ei < 2; ++ei)
+                    for (int ek = 0; ek < 2; ++ek)
+                        for (int ej = 0; ej < 2; ++ej) {
+                            const int ex = i - 1 + ei, ey = j - 1 + ej, ez = k - 1 + ek;
+                            const int bx = di + 1 - ei, bz = dk + 1 - ek, by = dj + 1 - ej;
+                            if (ex < 0 || ex >= g.nx || ey < 0 || ey >= g.ny || ez < 0 || ez >= g.nz) continue;
+                            if (bx < 0 || bx > 1 || by < 0 || by > 1 || bz < 0 || bz > 1) continue;
+                            const long e = (long)g.ny * g.nz * ex + (long)g.ny * ez + ey;
+                            const int m = 3 * lidx2(1 - ei, 1 - ej, 1 - ek) + cr, n = 3 * lidx2(bx, by, bz) + cc;
+                            v += A[(long)pidx2(m, n) * g.nel + e];
+                        }
             }
+        }
+        AQ[(long)r * N + c] = v;
+    }
 }
 
-void launch_assemble(hipStream_t s, const Grid &g, const double *A, double *AQ)
+// `bw`: the matrix's lower bandwidth.  The factorisation reads up to nbt =
+// (bw + 2 NB - 2) / NB tiles before a row's own, the corners of the inverse's
+// products up to 2 nbt - 1.
+void launch_assemble(hipStream_t s, const Grid &g, const double *A, double *AQ, int bw)
 {
     const int N = (int)((g.ndof + NB - 1) / NB * NB);
-    launch_fill(s, AQ, (long)N * N, 0.0);
-    k_assemble<<<(N + 255) / 256, 256, 0, s>>>(g, A, AQ, N);
+    k_assemble<<<N, 256, 0, s>>>(g, A, AQ, N, 2 * ((bw + 2 * NB - 2) / NB));
 }
 
 // ---------------------------------------------------------------------------

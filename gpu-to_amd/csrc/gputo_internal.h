@@ -237,6 +237,7 @@ struct gputo_handle {
     int *ctl_zero = nullptr;      // an always-zero control word
     long long bytes = 0;
     bool hier_ready = false;
+    bool l1_built = false;        // level 1's element matrices are those of the current hierarchy
     bool per_masks = false;       // periodic cell: on every level an image is fixed where its master is
     bool masks_ready = false;     // level fixed lists and masks match L[0].fixed
     std::vector<void *> allocs;
@@ -299,25 +300,27 @@ template <class T>  // U = prerelax F / AD
 void launch_prerelax(hipStream_t s, const T *F, const T *AD, T *U, long n, double prerelax, const int *ctl,
                      int nb = 1);
 void launch_coarse_l1(hipStream_t s, const Grid &gc, const double *Aelm, const double *CXf, double *A);
-void launch_coarse_galerkin(hipStream_t s, const Grid &gc, const double *Af, const double *Ke, const double *CXf,
-                            double *Ac);
+// diagonal (and 1/AD) of the rediscretised level 1 from the child densities
+void launch_diag_l1(hipStream_t s, const Grid &g, const double *Aelm, const double *CXf, double *AD, double *RD);
+void launch_coarse_galerkin(hipStream_t s, const Grid &gc, const double *Af, double *Ac);
 void launch_galerkin_table(hipStream_t s, const Grid &gc, int depth, const double *T, const double *CX0, double *A);
 std::vector<std::vector<double>> galerkin_tables(const double *Ke, const double *base1, int maxdepth);
 constexpr int kGtMaxDepth = 4;  // deepest level built from tables (8^4 x 300 doubles = 9.8 MB)
 // A table product costs 300 FMA per level-0 element at every level, spread
-// over nel_l/16 blocks that each stream 8^l table rows; below this many
-// elements the child-by-child Galerkin of the level above (about 1.7e5 FMA
-// per element, one block each) is faster.  Measured at 192x96x96: level 3
-// (3456 elements) takes 260 us from its table and 452 us child by child;
-// level 4 (432 elements) 95 us child by child.
+// over nel_l/32 x 10 waves that each stream 8^l table rows.  Down to level 2
+// (64 rows) it is the cheapest form at any size; deeper levels with fewer
+// elements than this take the child-by-child Galerkin of the level above.
+// Measured at 192x96x96: level 3 (3456 elements) 57 us from its table; level
+// 4 (432 elements, 4096 rows) 24 us child by child.
 constexpr long kGtMinElems = 2048;
+inline bool from_table(int l, long nel) { return l <= kGtMaxDepth && (l <= 2 || nel >= kGtMinElems); }
 void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, double *A, int mirrored);
 // mgcg9 coarse levels: CX_c = 2 mean(children), element matrices CX Ke, and
 // the zeroing of fixed rows/columns of the dense coarsest matrix
 void launch_coarse_cx(hipStream_t s, const Grid &gc, const double *CXf, double *CXc);
 void launch_ke_elements(hipStream_t s, const Grid &g, const double *CX, const double *Ke, double *A);
 void launch_zero_rowcol(hipStream_t s, int N, const int *fixed_d, int nfd, double *AQ);
-void launch_assemble(hipStream_t s, const Grid &g, const double *A, double *AQ);
+void launch_assemble(hipStream_t s, const Grid &g, const double *A, double *AQ, int bw);
 // Factor C.AQ on C.side after the work on s.  lag: when an earlier factor
 // exists, write the new one into the other buffer and let the solves keep
 // the earlier one (coarse_adopt switches at the next setup).
@@ -424,6 +427,9 @@ void launch_homog_rhs(hipStream_t s, const Grid &g, const double *CX, const doub
                       double *F);
 
 int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0);
+// the stored element matrices of level 1 where the V-cycle applies it
+// matrix-free (built on first use after a setup)
+void ensure_level1(gputo_handle *h);
 int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, double *relres, int *nit);
 // nb <= kMaxBatch right-hand sides together (F, U: nb vectors one after another)
 int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double tol, int maxit, double *relres,

@@ -43,9 +43,6 @@ void mixed_create(gputo_handle *h)
         v.RD = v.AD + g.ndof;
         v.Tmp = malloc_dev<float>(m, g.ndof);
         if (l > 0) {
-            float *A = malloc_dev<float>(m, 300 * g.nel);
-            m->A32[l] = A;
-            v.A = A;
             if (h->L[l].S) v.S = m->S32[l] = malloc_dev<float>(m, (long)kStencilEntries * g.nnod);
             v.CX = m->CXl32[l] = malloc_dev<float>(m, g.nel);
         }
@@ -102,33 +99,68 @@ static int l0_kind(const gputo_params &p, int precision)
 }
 
 // FP32 copies of the FP64 hierarchy (operators, diagonals) built by
-// setup_hierarchy.
+// setup_hierarchy: one launch over the list of arrays (a dozen launches of
+// 3-7 us each otherwise).
+struct CastList {
+    static constexpr int kMax = 3 * kMaxLevels + 2;
+    int n = 0;
+    const double *src[kMax];
+    float *dst[kMax];
+    long first[kMax + 1] = {};  // first element of each array in the whole list
+    void add(const double *s, float *d, long len)
+    {
+        src[n] = s;
+        dst[n] = d;
+        first[n + 1] = first[n] + len;
+        ++n;
+    }
+};
+
+__global__ __launch_bounds__(kBlock) void k_cast_list(CastList c)
+{
+    const long stride = (long)gridDim.x * kBlock;
+    int q = 0;
+    for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < c.first[c.n]; i += stride) {
+        while (i >= c.first[q + 1]) ++q;
+        const long o = i - c.first[q];
+        c.dst[q][o] = (float)c.src[q][o];
+    }
+}
+
 static void mixed_prepare(gputo_handle *h)
 {
     MixedState *m = h->mx;
     hipStream_t s = h->stream;
     const Grid &g0 = h->L[0].g;
-    launch_copy<double, float>(s, h->Ke, m->Ke32, 576, nullptr);
-    launch_copy<double, float>(s, h->CX, m->CX32, g0.nel, nullptr);
+    CastList c;
+    c.add(h->Ke, m->Ke32, 576);
+    c.add(h->CX, m->CX32, g0.nel);
     m->H.l1_mf = use_l1_mf(h->prm, h->nl, h->L[1].mw64);
     m->H.mg9 = preset_of(h->prm).mg9;
     m->H.per = h->prm.periodic != 0;
     if (m->H.mg9 && !h->C.direct) launch_fill<float>(s, m->H.L[h->nl - 1].U, h->L[h->nl - 1].g.ndof, 0.0);
     for (int l = 0; l < h->nl; ++l) {
         const Level &v = h->L[l];
-        launch_copy<double, float>(s, v.AD, m->H.L[l].AD, v.g.ndof, nullptr);
+        c.add(v.AD, m->H.L[l].AD, v.g.ndof);
         if (l <= 1 || m->H.mg9)
-            launch_copy<double, float>(s, v.RD, m->H.L[l].RD, l == 0 || m->H.mg9 ? v.g.nnod : v.g.ndof, nullptr);
+            c.add(v.RD, m->H.L[l].RD, l == 0 || m->H.mg9 ? v.g.nnod : v.g.ndof);
         if (m->H.mg9) {
-            if (l > 0) launch_copy<double, float>(s, v.CXl, m->CXl32[l], v.g.nel, nullptr);
-        } else if (l > 0 && !(l == 1 && m->H.l1_mf)) {
-            // the stencil replaces the element matrices where it exists
-            if (m->S32[l])
-                launch_copy<double, float>(s, v.S, m->S32[l], (long)kStencilEntries * v.g.nnod, nullptr);
-            else
-                launch_copy<double, float>(s, v.A, m->A32[l], 300 * v.g.nel, nullptr);
+            if (l > 0) c.add(v.CXl, m->CXl32[l], v.g.nel);
+        } else if (l == 1 ? h->l1_built && l < h->nl - 1 : m->S32[l] != nullptr) {
+            // stored levels are applied as node stencils (the coarsest through
+            // its FP64 factor), level 1 from its element matrices when the
+            // handle was created without a stencil for it
+            if (m->S32[l]) {
+                c.add(v.S, m->S32[l], (long)kStencilEntries * v.g.nnod);
+            } else {
+                if (!m->A32) m->A32 = malloc_dev<float>(m, 300 * v.g.nel);
+                m->H.L[1].A = m->A32;
+                c.add(v.A, m->A32, 300 * v.g.nel);
+            }
         }
     }
+    k_cast_list<<<(unsigned)std::min<long>((c.first[c.n] + kBlock - 1) / kBlock, 4096), kBlock, 0, s>>>(c);
+    check_hip(hipGetLastError(), "launch");
     m->H.l0 = l0_resolve(h, l0_kind(h->prm, h->prm.precision));
     m->H.l0_ctx = m;
     m->H.learn = h->ln != nullptr;
@@ -253,15 +285,13 @@ int mixed_apply_l0(gputo_handle *h, int kind, const double *u, double *y)
     return 0;
 }
 
-// FP32 view of the current hierarchy with every level's stored matrices
-// cast (level-operator checks and benchmarks); vectors X/P/Q are free.
+// FP32 view of the current hierarchy, level 1's stored form included where a
+// caller has built it (ensure_level1); vectors X/P/Q are free.
 HierView<float> mixed_level_view(gputo_handle *h)
 {
     if (!h->mx) mixed_create(h);
     MixedState *m = h->mx;
     mixed_prepare(h);
-    if (m->H.l1_mf && h->nl > 1)
-        launch_copy<double, float>(h->stream, h->L[1].A, m->A32[1], 300 * h->L[1].g.nel, nullptr);
     return m->H;
 }
 

@@ -314,6 +314,20 @@ static void ensure_tables(gputo_handle *h)
     h->gt_ke = ke;
 }
 
+void ensure_level1(gputo_handle *h)
+{
+    Level &v = h->L[1];
+    if (h->l1_built) return;
+    if (!v.A) v.A = dalloc<double>(h, 300 * v.g.nel);
+    if (preset_of(h->prm).l1_galerkin)
+        launch_galerkin_table(h->stream, v.g, 1, h->gt[1], h->CX, v.A);
+    else
+        launch_coarse_l1(h->stream, v.g, h->Aelm, h->CX, v.A);
+    if (v.S && h->nl > 2) launch_stencil_build(h->stream, v.g, v.A, v.S);
+    HIPCHK(hipGetLastError());
+    h->l1_built = true;
+}
+
 // Build the hierarchy for the current Ke, CX (device) and fixed list
 // (initVcycle, mgcg1.cu:326-466).
 static bool coarse_lagged(const gputo_params &p) { return p.coarse_lag >= 1; }
@@ -373,11 +387,12 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         // keeps its iterate from one V-cycle to the next (mgcg9.cu:553-563)
         if (!h->C.direct) launch_fill<double>(s, vc.U, vc.g.ndof, 0.0);
         if (h->C.direct) {
+            if (!vc.A) vc.A = dalloc<double>(h, 300 * vc.g.nel);  // nl = 2
             launch_ke_elements(s, vc.g, vc.CXl, h->Ke, vc.A);
             if (per)
                 launch_assemble_per(s, vc.g, vc.A, h->C.AQ);
             else
-                launch_assemble(s, vc.g, vc.A, h->C.AQ);
+                launch_assemble(s, vc.g, vc.A, h->C.AQ, h->C.bw);
             launch_zero_rowcol(s, (h->C.n + 31) / 32 * 32, vc.fixed_d, (int)vc.fixed.size(), h->C.AQ);
             HIPCHK(hipGetLastError());
             coarse_factor(s, h->C, coarse_lagged(h->prm));
@@ -394,36 +409,52 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         return 0;
     }
     h->C.direct = true;
-    for (int l = 1; l < h->nl; ++l) {
+    // The coarsest matrix first, then its factorisation, which overlaps the
+    // other levels: only the levels it is formed from are built before it.
+    // Level 1 applied matrix-free needs no element matrices at all (531 MB
+    // and 105 us at 192x96x96); ensure_level1 builds them for a caller that
+    // asks for them.
+    h->l1_built = false;
+    const bool l1_mf = use_l1_mf(h->prm, h->nl, h->L[1].mw64);
+    auto build = [&](int l) {
         Level &v = h->L[l];
-        if (l == 1 && !p.l1_galerkin)
-            launch_coarse_l1(s, v.g, h->Aelm, h->CX, v.A);
-        else if (l <= h->gt_max && (v.g.nel >= kGtMinElems || l == 1))
+        if (l == 1)
+            ensure_level1(h);
+        else if (from_table(l, v.g.nel))
             launch_galerkin_table(s, v.g, l, h->gt[l], h->CX, v.A);
         else
-            launch_coarse_galerkin(s, v.g, l == 1 ? nullptr : h->L[l - 1].A, h->Ke, h->CX, v.A);
-        if (l == h->nl - 1) {
-            if (per) {
-                // the wrapped matrix with the fixed rows and columns decoupled
-                launch_assemble_per(s, v.g, v.A, h->C.AQ);
-                launch_zero_rowcol(s, (h->C.n + 31) / 32 * 32, v.fixed_d, (int)v.fixed.size(), h->C.AQ);
-            } else {
-                launch_corrcsa(s, v.g, v.fixed_d, (int)v.fixed.size(), v.A, p.corr_mirrored);
-                launch_assemble(s, v.g, v.A, h->C.AQ);
-            }
+            launch_coarse_galerkin(s, v.g, h->L[l - 1].A, v.A);
+    };
+    int base = h->nl - 1;
+    while (base > 1 && !from_table(base, h->L[base].g.nel)) --base;
+    for (int l = base; l < h->nl; ++l) build(l);
+    {
+        Level &v = h->L[h->nl - 1];
+        if (per) {
+            // the wrapped matrix with the fixed rows and columns decoupled
+            launch_assemble_per(s, v.g, v.A, h->C.AQ);
+            launch_zero_rowcol(s, (h->C.n + 31) / 32 * 32, v.fixed_d, (int)v.fixed.size(), h->C.AQ);
+        } else {
+            launch_corrcsa(s, v.g, v.fixed_d, (int)v.fixed.size(), v.A, p.corr_mirrored);
+            launch_assemble(s, v.g, v.A, h->C.AQ, h->C.bw);
         }
     }
     HIPCHK(hipGetLastError());
     // overlaps the solve (lagged) or the first V-cycle's descent (exact);
     // errors surface in coarse_check / coarse_adopt
     coarse_factor(s, h->C, coarse_lagged(h->prm));
-    // diagonals and node stencils, which the factorisation does not read,
-    // run on the main stream while it does
+    // the other levels, diagonals and node stencils, which the factorisation
+    // does not read, run on the main stream while it does
+    for (int l = 1; l < base; ++l)
+        if (l > 1 || !l1_mf) build(l);
     for (int l = 1; l < h->nl; ++l) {
         Level &v = h->L[l];
-        launch_diagA(s, v.g, v.A, v.AD, per || l > 1 ? nullptr : v.RD);
+        if (l == 1 && l1_mf)
+            launch_diag_l1(s, v.g, h->Aelm, h->CX, v.AD, per ? nullptr : v.RD);
+        else
+            launch_diagA(s, v.g, v.A, v.AD, per || l > 1 ? nullptr : v.RD);
         if (per) fold_diag(l);
-        if (v.S) launch_stencil_build(s, v.g, v.A, v.S);
+        if (v.S && l > 1) launch_stencil_build(s, v.g, v.A, v.S);  // level 1: ensure_level1
     }
     HIPCHK(hipGetLastError());
     h->hier_ready = true;
@@ -895,7 +926,7 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
             if (l > 0) {
                 v.U = dalloc<double>(h, v.g.ndof);
                 v.F = dalloc<double>(h, v.g.ndof);
-                v.A = dalloc<double>(h, 300 * v.g.nel);
+                if (l > 1) v.A = dalloc<double>(h, 300 * v.g.nel);  // level 1: ensure_level1
                 v.CXl = dalloc<double>(h, v.g.nel);
                 // node stencils of the stored levels the V-cycle smooths
                 if (l < nl - 1 && !(l == 1 && use_l1_mf(h->prm, nl, v.mw64)))
@@ -941,7 +972,9 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
         C.flag = dalloc<int>(h, 1);
         std::vector<double> tab = level1_gauss_table(0.3, 2.0);
         HIPCHK(hipMemcpy(h->Aelm, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice));
-        h->gt_max = std::min(nl - 1, kGtMaxDepth);
+        h->gt_max = 0;
+        for (int l = 1; l < nl; ++l)
+            if (from_table(l, h->L[l].g.nel)) h->gt_max = l;
         for (int l = 1; l <= h->gt_max; ++l) h->gt[l] = dalloc<double>(h, (size_t)300 << (3 * l));
         if (h->prm.precision != GPUTO_PREC_F64) mixed_create(h);
         if (h->prm.learned) learn_create(h);
@@ -1209,6 +1242,8 @@ int gputo_level_matrices(gputo_handle *h, int level, double *A, double *ad, doub
         const Level &v = h->L[level];
         hipStream_t s = h->stream;
         if (A && level > 0) {
+            if (level == 1 && !preset_of(h->prm).mg9) ensure_level1(h);
+            if (!v.A) h->L[level].A = dalloc<double>(h, 300 * v.g.nel);  // mgcg9 keeps no element matrices
             std::vector<double> packed(300 * v.g.nel);
             HIPCHK(hipMemcpyAsync(packed.data(), v.A, packed.size() * sizeof(double), hipMemcpyDeviceToHost, s));
             HIPCHK(hipStreamSynchronize(s));
@@ -1359,6 +1394,7 @@ int gputo_level_apply(gputo_handle *h, int level, int op, int mode, int fp32, co
     try {
         hipStream_t s = h->stream;
         const long n = h->L[level].g.ndof;
+        if (level == 1 && op == 1 && !preset_of(h->prm).mg9) ensure_level1(h);
         HIPCHK(hipMemcpyAsync(h->P, u, n * sizeof(double), hipMemcpyHostToDevice, s));
         if (f) HIPCHK(hipMemcpyAsync(h->Z, f, n * sizeof(double), hipMemcpyHostToDevice, s));
         if (fp32) {
@@ -1386,6 +1422,7 @@ int gputo_bench_level(gputo_handle *h, int level, int op, int fp32, int reps, do
     try {
         hipStream_t s = h->stream;
         const long n = h->L[level].g.ndof;
+        if (level == 1 && op == 1 && !preset_of(h->prm).mg9) ensure_level1(h);
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
         HIPCHK(hipEventCreate(&e1));
