@@ -208,6 +208,7 @@ struct BatchState {
     int precision = -1;
     double *R = nullptr, *P = nullptr, *Q = nullptr, *Z = nullptr;
     double *partials = nullptr;  // nb x (the most per-block partials of a launch)
+    double *rr = nullptr;        // nb x (kCgBlocks residual sums), then nb x 2 kCgBlocks dots
     CgScalars *sc = nullptr, *sc_host = nullptr;
     double *v64[kMaxLevels][4] = {};
     float *v32[kMaxLevels][4] = {};
@@ -234,6 +235,8 @@ struct gputo_handle {
     double *partials = nullptr;   // reduction partials
     gputo::CgScalars *sc = nullptr;
     gputo::CgScalars *sc_host = nullptr;  // pinned mirror
+    double *rr = nullptr;         // the PCG's residual sums, then its dots (kCgBlocks + 2 kCgBlocks)
+    unsigned long long *prog = nullptr;   // pinned progress words of the PCG (k_cg_check), one per right-hand side
     int *ctl_zero = nullptr;      // an always-zero control word
     long long bytes = 0;
     bool hier_ready = false;
@@ -340,38 +343,39 @@ template <class T>
 void launch_coarse_solve(hipStream_t s, const Coarse &C, const T *b, T *x, const uint8_t *mask, const int *ctl,
                          int nb = 1);
 
-// PCG scalar steps (single-block kernels reading the reduction partials).
+// Steps of the PCG (cg.hip).  pq: npq per-block sums of p.q; rr, dots: room
+// for kCgBlocks (2 kCgBlocks, flexible beta) sums per right-hand side, apart
+// from pq.
+constexpr int kCgBlocks = 256;  // most blocks of a CG reduction
+constexpr int kCgFuse = 1024;   // most sums that every block of an update reads
+// U = 0, R = F (R32, X0 as launch_cg_update_r) and the first residual norm
+void launch_cg_start(hipStream_t s, const double *F, double *U, double *R, long n, CgScalars *sc, double *rr,
+                     float *R32 = nullptr, const float *AD32 = nullptr, float *X0 = nullptr, double prerelax = 0.0);
+// rho = r.z of the first direction
+template <class TZ>
+void launch_cg_rho(hipStream_t s, const double *r, const TZ *z, long n, CgScalars *sc, double *dots, int nb = 1);
+// the first residual norm from the sums of launch_dot_partial
 void launch_cg_init(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int nb = 1);
-void launch_cg_rho0(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int nb = 1);
-void launch_cg_alpha(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int nb = 1);
-// U += alpha P, R -= alpha Q, partials of R.R; R32 (if not null) gets R in FP32
-template <class T>
-void launch_cg_update_ur(hipStream_t s, T *U, T *R, const T *P, const T *Q, long n, CgScalars *sc, double *partials,
-                         float *R32 = nullptr, int nb = 1);
-void launch_cg_check(hipStream_t s, CgScalars *sc, const double *partials, int nparts, double tol, int maxit,
-                     int nb = 1);
-void launch_cg_beta(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int maxit, int nb = 1);
-template <class T> void launch_cg_update_p(hipStream_t s, T *P, const T *Z, long n, CgScalars *sc, int nb = 1);
-// P = Z + beta P with the FP32 output of the mixed V-cycle (widened exactly)
-void launch_cg_update_p(hipStream_t s, double *P, const float *Z, long n, CgScalars *sc, int nb = 1);
-// the same with P kept in FP32 (Pout = Z + beta Pin, formed in FP64 and
-// rounded once; Pout may be Pin)
-void launch_cg_update_p32(hipStream_t s, float *Pout, const float *Pin, const float *Z, long n, CgScalars *sc);
+// alpha, U += alpha P, R -= alpha Q, sums of R.R; R32 (if not null) gets R in FP32
+void launch_cg_update_ur(hipStream_t s, double *U, double *R, const double *P, const double *Q, long n, CgScalars *sc,
+                         const double *pq, int npq, double *rr, float *R32 = nullptr, int nb = 1);
 // PCG with deferred u: the iterations' alphas are logged (0 once converged)
 // and u += sum alpha_t p_t is applied every kCgLog iterations from the
-// kept FP32 directions
-constexpr int kCgLog = 16;
-void launch_cg_alpha_log(hipStream_t s, CgScalars *sc, const double *partials, int nparts, double *alog);
+// kept FP32 directions.
 // X0 (optional): also writes X0 = prerelax R32 / AD32, the prerelaxed
 // level-0 iterate of the next FP32 V-cycle (mixed_prerelax_target)
-void launch_cg_update_r(hipStream_t s, double *R, const double *Q, long n, CgScalars *sc, double *partials,
-                        float *R32, const float *AD32 = nullptr, float *X0 = nullptr, double prerelax = 0.0);
+constexpr int kCgLog = 16;
+void launch_cg_update_r(hipStream_t s, double *R, const double *Q, long n, CgScalars *sc, const double *pq, int npq,
+                        double *rr, double *alog, float *R32, const float *AD32 = nullptr, float *X0 = nullptr,
+                        double prerelax = 0.0);
 void launch_cg_flush_u(hipStream_t s, double *U, const float *P, long n, const double *alog, int m);
-// flexible beta (partials needs 2*kRedBlocks entries); z FP64, or the
-// mixed V-cycle's FP32 output (products in FP64, the same values)
-template <class TZ>
-void launch_cg_beta_flex(hipStream_t s, const double *r, const TZ *z, const double *q, long n, CgScalars *sc,
-                         double *partials, int maxit, int nb = 1);
+// residual test from the sums of an update over n elements
+void launch_cg_check(hipStream_t s, CgScalars *sc, const double *rr, long n, double tol, unsigned long long *prog,
+                     int nb = 1);
+// dots of z and Pout = z + beta Pin (flex: Polak-Ribiere beta)
+template <class TP, class TZ>
+void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const double *q, TP *Pout, const TP *Pin, long n,
+                         CgScalars *sc, double *dots, bool flex, int maxit, int nb = 1);
 
 void check_hip(hipError_t e, const char *what);  // throws on an error
 #define HIPCHK(x) ::gputo::check_hip((x), #x)

@@ -970,385 +970,4 @@ template void launch_dot_partial<float, float>(hipStream_t, const float *, const
 template void launch_dot_partial<double, float>(hipStream_t, const double *, const float *, long, double *,
                                                 const int *, int);
 
-// Each thread adds p[t], p[t + kBlock], p[t + 2 kBlock], ... in that order;
-// the loads of a chunk are all issued before the first add, so a few
-// thousand partials cost a round trip per chunk, not one per partial.
-__device__ double sum_partials(const double *p, int n)
-{
-    constexpr int kChunk = 16;
-    double s = 0.0;
-    for (int i0 = threadIdx.x; i0 < n; i0 += kChunk * kBlock) {
-        double v[kChunk];
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) v[k] = i0 + k * kBlock < n ? p[i0 + k * kBlock] : 0.0;
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k)
-            if (i0 + k * kBlock < n) s += v[k];
-    }
-    return block_sum(s);
-}
-
-// PCG scalar steps (the scalar arithmetic of mgcg1.cu:235-275, kept on the
-// device so the loop never waits on the host).
-__global__ __launch_bounds__(kBlock) void k_cg_init(CgScalars *sc, const double *p, int n)
-{
-    sc += blockIdx.z;
-    p += (long)blockIdx.z * n;
-    const double ff = sum_partials(p, n);
-    if (threadIdx.x == 0) {
-        sc->res0 = sqrt(ff);
-        sc->done = 0;
-        sc->nit = 0;
-        sc->it = 0;
-        sc->bad = 0;
-        sc->relres = 0.0;
-        if (!(sc->res0 < INFINITY)) {  // NaN or Inf in F
-            sc->bad = 1;
-            sc->done = 1;
-        } else if (sc->res0 == 0.0) {  // F = 0: U = 0 is exact
-            sc->done = 1;
-        }
-    }
-}
-
-// The scalar steps read their CgScalars fields and the partials first and
-// test the converged flag after: one memory round trip, not three.
-__global__ __launch_bounds__(kBlock) void k_cg_rho0(CgScalars *sc, const double *p, int n)
-{
-    sc += blockIdx.z;
-    p += (long)blockIdx.z * n;
-    const double rz = sum_partials(p, n);
-    if (sc->done) return;
-    if (threadIdx.x == 0) {
-        sc->rho = rz;
-        sc->rho_p = rz;
-    }
-}
-
-// alog (optional): the iteration's slot of the alpha log, 0 once converged
-__global__ __launch_bounds__(kBlock) void k_cg_alpha(CgScalars *sc, const double *p, int n, double *alog)
-{
-    sc += blockIdx.z;
-    p += (long)blockIdx.z * n;
-    const double rho_p = sc->rho_p;
-    const double pq = sum_partials(p, n);
-    if (sc->done) {
-        if (alog && threadIdx.x == 0) *alog = 0.0;
-        return;
-    }
-    if (threadIdx.x == 0) {
-        sc->pq = pq;
-        sc->alpha = rho_p / pq;
-        if (alog) *alog = sc->alpha;
-        if (!(fabs(sc->alpha) < INFINITY)) {
-            sc->bad = 1;
-            sc->done = 1;
-            sc->nit = sc->it;
-        }
-    }
-}
-
-template <class T>
-__global__ __launch_bounds__(kBlock) void k_cg_update_ur(T *__restrict__ U, T *__restrict__ R, const T *__restrict__ P,
-                                                        const T *__restrict__ Q, long n, const CgScalars *sc,
-                                                        double *partials, float *__restrict__ R32)
-{
-    sc += blockIdx.z;
-    U = batch_ptr(U, n);
-    R = batch_ptr(R, n);
-    P = batch_ptr(P, n);
-    Q = batch_ptr(Q, n);
-    R32 = batch_ptr(R32, n);
-    partials = batch_ptr(partials, (long)gridDim.x);
-    const T al = (T)sc->alpha;
-    const long stride = (long)kRedBlocks * kBlock;
-    const long i0 = (long)blockIdx.x * kBlock + threadIdx.x;
-    double s = 0.0;
-    // two elements per pass, both loaded before either is stored
-    for (long i = i0; i < n; i += 2 * stride) {
-        const bool two = i + stride < n;
-        const long j = two ? i + stride : i;  // in bounds; unused when !two
-        const T u0 = U[i], p0 = P[i], r0 = R[i], q0 = Q[i];
-        const T u1 = U[j], p1 = P[j], r1 = R[j], q1 = Q[j];
-        if (i == i0 && sc->done) return;  // read with alpha while the loads are in flight
-        const T ra = r0 - al * q0, rb = r1 - al * q1;
-        U[i] = u0 + al * p0;
-        R[i] = ra;
-        if (R32) R32[i] = (float)ra;  // the FP32 V-cycle's right-hand side
-        s += (double)ra * (double)ra;
-        if (two) {
-            U[j] = u1 + al * p1;
-            R[j] = rb;
-            if (R32) R32[j] = (float)rb;
-            s += (double)rb * (double)rb;
-        }
-    }
-    if (sc->done) return;  // every thread tests it before the barrier
-    s = block_sum(s);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
-}
-
-__global__ __launch_bounds__(kBlock) void k_cg_check(CgScalars *sc, const double *p, int n, double tol, int maxit)
-{
-    sc += blockIdx.z;
-    p += (long)blockIdx.z * n;
-    const double res0 = sc->res0;
-    const double rr = sum_partials(p, n);
-    if (sc->done) return;
-    if (threadIdx.x == 0) {
-        sc->rr = rr;
-        sc->relres = sqrt(rr) / res0;
-        if (!(sc->relres < INFINITY)) {
-            sc->bad = 1;
-            sc->done = 1;
-            sc->nit = sc->it;
-        } else if (sc->relres < tol) {
-            sc->done = 1;
-            sc->nit = sc->it;
-        }
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_cg_beta(CgScalars *sc, const double *p, int n, int maxit)
-{
-    sc += blockIdx.z;
-    p += (long)blockIdx.z * n;
-    const double rho_p = sc->rho_p;
-    const double rz = sum_partials(p, n);
-    if (sc->done) return;
-    if (threadIdx.x == 0) {
-        sc->rho = rz;
-        sc->beta = rz / rho_p;
-        sc->rho_p = rz;
-        sc->it += 1;
-        if (sc->it >= maxit) {
-            sc->done = 1;
-            sc->nit = maxit;
-        }
-    }
-}
-
-// Flexible (Polak-Ribiere) beta for a preconditioner that varies between
-// iterations: beta = <z, r - r_old>/rho_old with r - r_old = -alpha q, so
-// beta = -alpha <z,q>/rho_old; rho = <r,z> is kept for the next alpha.
-template <class TZ>
-__global__ __launch_bounds__(kBlock) void k_dot2_partial(const double *__restrict__ r, const TZ *__restrict__ z,
-                                                       const double *__restrict__ q, long n, double *partials,
-                                                       const int *ctl)
-{
-    ctl = batch_ctl(ctl);
-    if (ctl && ctl[0]) return;
-    r = batch_ptr(r, n);
-    z = batch_ptr(z, n);
-    q = batch_ptr(q, n);
-    partials = batch_ptr(partials, 2L * kRedBlocks);
-    double a = 0.0, b = 0.0;
-#pragma unroll 4
-    for (long i = (long)blockIdx.x * kBlock + threadIdx.x; i < n; i += (long)kRedBlocks * kBlock) {
-        const double zi = (double)z[i];  // exact for an FP32 z
-        a += r[i] * zi;
-        b += q[i] * zi;
-    }
-    a = block_sum(a);
-    b = block_sum(b);
-    if (threadIdx.x == 0) {
-        partials[blockIdx.x] = a;
-        partials[kRedBlocks + blockIdx.x] = b;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void k_cg_beta_flex(CgScalars *sc, const double *p, int maxit)
-{
-    sc += blockIdx.z;
-    p += 2L * kRedBlocks * blockIdx.z;
-    const double alpha = sc->alpha, rho_p = sc->rho_p;
-    const double rz = sum_partials(p, kRedBlocks);
-    const double qz = sum_partials(p + kRedBlocks, kRedBlocks);
-    if (sc->done) return;
-    if (threadIdx.x == 0) {
-        sc->rho = rz;
-        sc->beta = -alpha * qz / rho_p;
-        sc->rho_p = rz;
-        sc->it += 1;
-        if (sc->it >= maxit) {
-            sc->done = 1;
-            sc->nit = maxit;
-        }
-    }
-}
-
-template <class TZ>
-void launch_cg_beta_flex(hipStream_t s, const double *r, const TZ *z, const double *q, long n, CgScalars *sc,
-                         double *partials, int maxit, int nb)
-{
-    k_dot2_partial<TZ><<<dim3(kRedBlocks, 1, batch_dim(nb)), kBlock, 0, s>>>(r, z, q, n, partials, &sc->done);
-    k_cg_beta_flex<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, partials, maxit);
-}
-template void launch_cg_beta_flex<double>(hipStream_t, const double *, const double *, const double *, long,
-                                          CgScalars *, double *, int, int);
-template void launch_cg_beta_flex<float>(hipStream_t, const double *, const float *, const double *, long,
-                                         CgScalars *, double *, int, int);
-
-template <class T, class TZ>
-__global__ __launch_bounds__(kBlock) void k_cg_update_p(T *__restrict__ P, const TZ *__restrict__ Z, long n,
-                                                       const CgScalars *sc)
-{
-    sc += blockIdx.z;
-    P = batch_ptr(P, n);
-    Z = batch_ptr(Z, n);
-    const T be = (T)sc->beta;
-    // two elements per pass, as k_prerelax; done is read with beta
-    const long stride = (long)gridDim.x * kBlock, i0 = (long)blockIdx.x * kBlock + threadIdx.x;
-    for (long i = i0; i < n; i += 2 * stride) {
-        const bool two = i + stride < n;
-        const long j = two ? i + stride : i;  // in bounds; unused when !two
-        const T p0 = P[i], p1 = P[j], z0 = (T)Z[i], z1 = (T)Z[j];
-        if (i == i0 && sc->done) return;
-        P[i] = fma(be, p0, z0);
-        if (two) P[j] = fma(be, p1, z1);
-    }
-}
-
-void launch_cg_init(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int nb)
-{
-    k_cg_init<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, partials, nparts);
-}
-void launch_cg_rho0(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int nb)
-{
-    k_cg_rho0<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, partials, nparts);
-}
-void launch_cg_alpha(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int nb)
-{
-    k_cg_alpha<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, partials, nparts, nullptr);
-}
-void launch_cg_alpha_log(hipStream_t s, CgScalars *sc, const double *partials, int nparts, double *alog)
-{
-    k_cg_alpha<<<1, kBlock, 0, s>>>(sc, partials, nparts, alog);
-}
-
-// Residual update of the PCG with deferred u (u += alpha p is applied later
-// from the logged alphas and directions): R -= alpha Q, R32 = R in FP32,
-// partials of R.R, two elements per pass as k_cg_update_ur.  PRE: also the
-// FP32 V-cycle's prerelaxed level-0 iterate X0 = pr R32 / AD32, the
-// expression of k_prerelax on the same FP32 values.
-template <bool PRE>
-__global__ __launch_bounds__(kBlock) void k_cg_update_r(double *__restrict__ R, const double *__restrict__ Q, long n,
-                                                       const CgScalars *sc, double *partials,
-                                                       float *__restrict__ R32, const float *__restrict__ AD32,
-                                                       float *__restrict__ X0, float pr)
-{
-    const double al = sc->alpha;
-    const long stride = (long)kRedBlocks * kBlock;
-    const long i0 = (long)blockIdx.x * kBlock + threadIdx.x;
-    double s = 0.0;
-    for (long i = i0; i < n; i += 2 * stride) {
-        const bool two = i + stride < n;
-        const long j = two ? i + stride : i;  // in bounds; unused when !two
-        const double r0 = R[i], q0 = Q[i], r1 = R[j], q1 = Q[j];
-        float d0 = 0.0f, d1 = 0.0f;
-        if (PRE) {
-            d0 = AD32[i];
-            d1 = AD32[j];
-        }
-        if (i == i0 && sc->done) return;  // read with alpha while the loads are in flight
-        const double ra = r0 - al * q0, rb = r1 - al * q1;
-        const float fa = (float)ra, fb = (float)rb;
-        R[i] = ra;
-        R32[i] = fa;
-        if (PRE) X0[i] = pr * fa / d0;
-        s += ra * ra;
-        if (two) {
-            R[j] = rb;
-            R32[j] = fb;
-            if (PRE) X0[j] = pr * fb / d1;
-            s += rb * rb;
-        }
-    }
-    if (sc->done) return;  // every thread tests it before the barrier
-    s = block_sum(s);
-    if (threadIdx.x == 0) partials[blockIdx.x] = s;
-}
-void launch_cg_update_r(hipStream_t s, double *R, const double *Q, long n, CgScalars *sc, double *partials,
-                        float *R32, const float *AD32, float *X0, double prerelax)
-{
-    if (X0)
-        k_cg_update_r<true><<<kRedBlocks, kBlock, 0, s>>>(R, Q, n, sc, partials, R32, AD32, X0, (float)prerelax);
-    else
-        k_cg_update_r<false><<<kRedBlocks, kBlock, 0, s>>>(R, Q, n, sc, partials, R32, nullptr, nullptr, 0.0f);
-}
-
-// U += alpha_0 P_0 + ... + alpha_{m-1} P_{m-1}, term by term in that order
-// (the same fused multiply-adds as one update per iteration).  Converged
-// iterations logged alpha 0; their directions are finite, so they add 0.
-// One element per thread, its m + 1 loads all in flight together.
-__global__ __launch_bounds__(kBlock) void k_cg_flush_u(double *__restrict__ U, const float *__restrict__ P, long n,
-                                                      const double *__restrict__ alog, int m)
-{
-    const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    float pv[kCgLog];
-#pragma unroll
-    for (int t = 0; t < kCgLog; ++t) pv[t] = t < m ? P[(long)t * n + i] : 0.0f;
-    double u = U[i];
-#pragma unroll
-    for (int t = 0; t < kCgLog; ++t)
-        if (t < m) u = fma(alog[t], (double)pv[t], u);
-    U[i] = u;
-}
-void launch_cg_flush_u(hipStream_t s, double *U, const float *P, long n, const double *alog, int m)
-{
-    if (m > 0) k_cg_flush_u<<<(unsigned)((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(U, P, n, alog, m);
-}
-template <class T>
-void launch_cg_update_ur(hipStream_t s, T *U, T *R, const T *P, const T *Q, long n, CgScalars *sc, double *partials,
-                         float *R32, int nb)
-{
-    k_cg_update_ur<T><<<dim3(kRedBlocks, 1, batch_dim(nb)), kBlock, 0, s>>>(U, R, P, Q, n, sc, partials, R32);
-}
-template void launch_cg_update_ur<double>(hipStream_t, double *, double *, const double *, const double *, long,
-                                          CgScalars *, double *, float *, int);
-template void launch_cg_update_ur<float>(hipStream_t, float *, float *, const float *, const float *, long,
-                                         CgScalars *, double *, float *, int);
-void launch_cg_check(hipStream_t s, CgScalars *sc, const double *partials, int nparts, double tol, int maxit, int nb)
-{
-    k_cg_check<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, partials, nparts, tol, maxit);
-}
-void launch_cg_beta(hipStream_t s, CgScalars *sc, const double *partials, int nparts, int maxit, int nb)
-{
-    k_cg_beta<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, partials, nparts, maxit);
-}
-template <class T>
-void launch_cg_update_p(hipStream_t s, T *P, const T *Z, long n, CgScalars *sc, int nb)
-{
-    k_cg_update_p<T, T><<<dim3(grid_for(n), 1, batch_dim(nb)), kBlock, 0, s>>>(P, Z, n, sc);
-}
-template void launch_cg_update_p<double>(hipStream_t, double *, const double *, long, CgScalars *, int);
-template void launch_cg_update_p<float>(hipStream_t, float *, const float *, long, CgScalars *, int);
-// P = Z + beta P with P kept in FP32: formed in FP64 from the FP32 values,
-// rounded once (two elements per pass, as k_cg_update_p)
-// (Pout = Z + beta Pin; Pout may be Pin)
-__global__ __launch_bounds__(kBlock) void k_cg_update_p32(float *Pout, const float *Pin, const float *__restrict__ Z,
-                                                         long n, const CgScalars *sc)
-{
-    const double be = sc->beta;
-    const long stride = (long)gridDim.x * kBlock, i0 = (long)blockIdx.x * kBlock + threadIdx.x;
-    for (long i = i0; i < n; i += 2 * stride) {
-        const bool two = i + stride < n;
-        const long j = two ? i + stride : i;  // in bounds; unused when !two
-        const float p0 = Pin[i], p1 = Pin[j], z0 = Z[i], z1 = Z[j];
-        if (i == i0 && sc->done) return;
-        Pout[i] = (float)fma(be, (double)p0, (double)z0);
-        if (two) Pout[j] = (float)fma(be, (double)p1, (double)z1);
-    }
-}
-void launch_cg_update_p32(hipStream_t s, float *Pout, const float *Pin, const float *Z, long n, CgScalars *sc)
-{
-    k_cg_update_p32<<<grid_for(n), kBlock, 0, s>>>(Pout, Pin, Z, n, sc);
-}
-
-void launch_cg_update_p(hipStream_t s, double *P, const float *Z, long n, CgScalars *sc, int nb)
-{
-    k_cg_update_p<double, float><<<dim3(grid_for(n), 1, batch_dim(nb)), kBlock, 0, s>>>(P, Z, n, sc);
-}
-
 }  // namespace gputo

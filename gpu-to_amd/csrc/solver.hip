@@ -497,6 +497,32 @@ static void precond(gputo_handle *h, const double *r, double *z, bool r32_ready 
         mixed_vcycle(h, r, z, &h->sc->done, r32_ready, pre0_ready);
 }
 
+// Wait until every right-hand side's progress word shows `seq` tested
+// iterations or convergence; true when all have converged.  rel: the relative
+// residual of the first.  The words come from k_cg_check; a stream that has
+// drained or failed without them ends the wait.
+static bool cg_wait(hipStream_t s, const unsigned long long *prog, int nb, int seq, float *rel)
+{
+    for (long spins = 1;; ++spins) {
+        bool all = true, done = true;
+        for (int q = 0; q < nb; ++q) {
+            const unsigned w = (unsigned)__atomic_load_n(&prog[q], __ATOMIC_RELAXED);
+            done = done && (w & 1u);
+            all = all && ((w & 1u) || (int)(w >> 1) >= seq);
+        }
+        if (all) {
+            if (rel) *rel = __builtin_bit_cast(float, (unsigned)(__atomic_load_n(&prog[0], __ATOMIC_RELAXED) >> 32));
+            return done;
+        }
+        if (spins % 65536 == 0) {
+            const hipError_t e = hipStreamQuery(s);
+            if (e == hipSuccess && spins > 65536L * 64) throw HipError("PCG progress lost");
+            if (e != hipSuccess && e != hipErrorNotReady) check_hip(e, "hipStreamQuery");
+        }
+        __builtin_ia32_pause();
+    }
+}
+
 int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, double *relres, int *nit)
 {
     hipStream_t s = h->stream;
@@ -530,7 +556,9 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
             if (graphs) mixed_graph_drop(h);  // it holds the previous factor
         }
         const bool pre0 = x0 && r32_ready && !z;  // the loop's V-cycles after the residual update
-        if (graphs && r32_ready && !z)
+        // (the first V-cycle, launched from the host, holds the wait for the
+        // coarsest factorisation)
+        if (graphs && vcycles > 0 && r32_ready && !z)
             mixed_vcycle_graph(h, &h->sc->done, pre0);
         else
             precond(h, r, z, r32_ready, pre0);
@@ -553,88 +581,88 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
     // partials of the level-0 matvec (FP64, from an FP64 or FP32 direction)
     const int nmv = op0_blocks(op_args(h, 0), OP_MATVEC);
     const bool per = h->prm.periodic != 0;
-    launch_fill(s, U, n, 0.0);
-    launch_copy(s, F, h->R, n, nullptr);
-    if (per) launch_per_fold<double>(s, L0.g, h->R, 0, nullptr);  // images' share to the masters
-    launch_dot_partial(s, h->R, h->R, n, h->partials, nullptr);
-    launch_cg_init(s, h->sc, h->partials, kRedBlocks);
-    precond_n(h->R, h->P, false);
-    launch_copy(s, h->P, h->Z, n, ctl);
-    if (p32) launch_copy<double, float>(s, h->P, p32, n, ctl);  // exact: z is the V-cycle's FP32 output
-    launch_dot_partial(s, h->R, h->Z, n, h->partials, ctl);
-    launch_cg_rho0(s, h->sc, h->partials, kRedBlocks);
-    const int chunk = 4;
-    int enq = 0;
-    for (;;) {
-        for (int c = 0; c < chunk && enq < maxit; ++c, ++enq) {
-            const int sl = enq % kCgLog;  // ring slot of this iteration's direction
-            float *pk = p32 ? p32 + (long)sl * n : nullptr;
-            OpArgs a = op_args(h, 0);
-            a.cx_floor = 0.0;  // the CG matvec keeps every element (multAV0c, mgcg9.cu:791-848)
-            a.U = h->P;
-            a.out = h->Q;
-            a.partials = h->partials;
-            a.per = per_fused(h, f64_view(h), 0);
-            if (p32) {
-                a.Uf = pk;
-                launch_op0_uf(s, a);
-            } else {
-                launch_op0(s, OP_MATVEC, a);
-            }
-            // p.q over the full grid is the periodic p.Kp before the fold
-            // (p is equal on images); the fold completes q for the update
-            if (per && !a.per) launch_per_fold<double>(s, L0.g, h->Q, 0, ctl);
-            if (p32) {
-                launch_cg_alpha_log(s, h->sc, h->partials, nmv, alog + sl);
-                launch_cg_update_r(s, h->R, h->Q, n, h->sc, h->partials, r32, ad32, x0, prx);
-                if (sl == kCgLog - 1) {  // before slot 0 is overwritten by this iteration's p update
-                    launch_cg_flush_u(s, U, p32, n, alog, kCgLog);
-                    folded = enq + 1;
-                }
-            } else {
-                launch_cg_alpha(s, h->sc, h->partials, nmv);
-                launch_cg_update_ur(s, U, h->R, h->P, h->Q, n, h->sc, h->partials, r32);
-            }
-            launch_cg_check(s, h->sc, h->partials, kRedBlocks, tol, maxit);
-            if (z32) {
-                // the FP32 V-cycle's result feeds the FP64 dots and the P
-                // update directly (widened exactly, so nothing changes but
-                // the traffic of an FP64 copy of z)
-                precond_n(h->R, nullptr, true);
-                if (flex) {
-                    launch_cg_beta_flex<float>(s, h->R, z32, h->Q, n, h->sc, h->partials, maxit);
-                } else {
-                    launch_dot_partial<double, float>(s, h->R, z32, n, h->partials, ctl);
-                    launch_cg_beta(s, h->sc, h->partials, kRedBlocks, maxit);
-                }
-                launch_cg_update_p32(s, p32 + (long)((sl + 1) % kCgLog) * n, pk, z32, n, h->sc);
-                continue;
-            }
-            precond_n(h->R, h->Z, r32 != nullptr);
-            if (flex) {
-                launch_cg_beta_flex<double>(s, h->R, h->Z, h->Q, n, h->sc, h->partials, maxit);
-            } else {
-                launch_dot_partial(s, h->R, h->Z, n, h->partials, ctl);
-                launch_cg_beta(s, h->sc, h->partials, kRedBlocks, maxit);
-            }
-            launch_cg_update_p(s, h->P, h->Z, n, h->sc);
-        }
-        HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(h->sc_host, h->sc, sizeof(CgScalars), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        if (h->sc_host->done || enq >= maxit) {
-            if (p32) {  // the directions since the last pass (converged ones logged alpha 0)
-                launch_cg_flush_u(s, U, p32, n, alog, enq - folded);
-                HIPCHK(hipStreamSynchronize(s));
-            }
-            break;
-        }
-        // the learned stage's fallback watches a trial's progress
-        if (h->ln)
-            learn_poll(h, h->sc_host->it,
-                       std::chrono::duration<double>(std::chrono::steady_clock::now() - t_begin).count(),
-                       h->sc_host->relres);
+    double *rr = h->rr, *dots = h->rr + kCgBlocks;
+    if (per) {
+        launch_fill(s, U, n, 0.0);
+        launch_copy(s, F, h->R, n, nullptr);
+        launch_per_fold<double>(s, L0.g, h->R, 0, nullptr);  // images' share to the masters
+        launch_dot_partial(s, h->R, h->R, n, h->partials, nullptr);
+        launch_cg_init(s, h->sc, h->partials, kRedBlocks);
+    } else {
+        launch_cg_start(s, F, U, h->R, n, h->sc, rr, r32, ad32, x0, prx);
     }
+    if (z32) {  // the first direction is the V-cycle's FP32 output
+        precond_n(h->R, nullptr, true);
+        launch_copy<float, float>(s, z32, p32, n, ctl);
+        launch_cg_rho<float>(s, h->R, z32, n, h->sc, dots);
+    } else {
+        precond_n(h->R, h->P, false);
+        launch_cg_rho<double>(s, h->R, h->P, n, h->sc, dots);
+    }
+    // Iteration k is enqueued in two halves: the matvec, update and residual
+    // test, then the V-cycle and the new direction.  Before the second half the
+    // host waits for the test of iteration k - 1 (a word in pinned memory; the
+    // device is then at the start of that iteration's V-cycle), so the stream
+    // always holds about one iteration of work and never drains, and at
+    // convergence one enqueued iteration skips its work.
+    const OpArgs mv = op_args(h, 0);
+    int enq = 0;
+    h->prog[0] = 0;
+    for (;;) {
+        const int sl = enq % kCgLog;  // ring slot of this iteration's direction
+        float *pk = p32 ? p32 + (long)sl * n : nullptr;
+        if (enq >= maxit) break;
+        OpArgs a = mv;
+        a.cx_floor = 0.0;  // the CG matvec keeps every element (multAV0c, mgcg9.cu:791-848)
+        a.U = h->P;
+        a.out = h->Q;
+        a.partials = h->partials;
+        a.per = per_fused(h, f64_view(h), 0);
+        if (p32) {
+            a.Uf = pk;
+            launch_op0_uf(s, a);
+        } else {
+            launch_op0(s, OP_MATVEC, a);
+        }
+        // p.q over the full grid is the periodic p.Kp before the fold
+        // (p is equal on images); the fold completes q for the update
+        if (per && !a.per) launch_per_fold<double>(s, L0.g, h->Q, 0, ctl);
+        if (p32) {
+            launch_cg_update_r(s, h->R, h->Q, n, h->sc, h->partials, nmv, rr, alog + sl, r32, ad32, x0, prx);
+            if (sl == kCgLog - 1) {  // before slot 0 is overwritten by this iteration's p update
+                launch_cg_flush_u(s, U, p32, n, alog, kCgLog);
+                folded = enq + 1;
+            }
+        } else {
+            launch_cg_update_ur(s, U, h->R, h->P, h->Q, n, h->sc, h->partials, nmv, rr, r32);
+        }
+        launch_cg_check(s, h->sc, rr, n, tol, h->prog);
+        ++enq;
+        HIPCHK(hipGetLastError());
+        if (enq > 1) {
+            float rel = 0.0f;
+            if (cg_wait(s, h->prog, 1, enq - 1, &rel)) break;
+            // the learned stage's fallback watches a trial's progress
+            if (h->ln && (enq - 1) % 4 == 0)
+                learn_poll(h, enq - 1,
+                           std::chrono::duration<double>(std::chrono::steady_clock::now() - t_begin).count(), rel);
+        }
+        if (z32) {
+            // the FP32 V-cycle's result feeds the FP64 dots and the P
+            // update directly (widened exactly, so nothing changes but
+            // the traffic of an FP64 copy of z)
+            precond_n(h->R, nullptr, true);
+            launch_cg_direction<float, float>(s, h->R, z32, h->Q, p32 + (long)((sl + 1) % kCgLog) * n, pk, n, h->sc,
+                                              dots, flex, maxit, 1);
+        } else {
+            precond_n(h->R, h->Z, r32 != nullptr);
+            launch_cg_direction<double, double>(s, h->R, h->Z, h->Q, h->P, h->P, n, h->sc, dots, flex, maxit, 1);
+        }
+    }
+    if (p32) launch_cg_flush_u(s, U, p32, n, alog, enq - folded);  // since the last pass (converged: alpha 0)
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(h->sc_host, h->sc, sizeof(CgScalars), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
     const CgScalars &r = *h->sc_host;
     *relres = r.relres;
     *nit = r.done ? r.nit : maxit;
@@ -693,6 +721,7 @@ static BatchState &batch_state(gputo_handle *h, int nb)
     b->Z = dalloc<double>(h, nb * n);
     const long nmv = std::max(xcd_launch(h->L[0].t.blocks()), xcd_launch(h->L[0].mw64.blocks()));
     b->partials = dalloc<double>(h, nb * std::max<long>(nmv, 2 * kRedBlocks));
+    b->rr = dalloc<double>(h, 3L * nb * kCgBlocks);
     b->sc = dalloc<CgScalars>(h, nb);
     HIPCHK(hipHostMalloc((void **)&b->sc_host, nb * sizeof(CgScalars), hipHostMallocDefault));
     std::memset(b->sc_host, 0, nb * sizeof(CgScalars));
@@ -773,42 +802,32 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
     launch_dot_partial(s, b.R, b.R, n, b.partials, nullptr, nb);
     launch_cg_init(s, b.sc, b.partials, kRedBlocks, nb);
     precond(b.R, b.P, false);
-    launch_copy(s, b.P, b.Z, n, ctl, nb);
-    launch_dot_partial(s, b.R, b.Z, n, b.partials, ctl, nb);
-    launch_cg_rho0(s, b.sc, b.partials, kRedBlocks, nb);
-    const int chunk = 4;
-    int enq = 0;
-    for (;;) {
-        for (int c = 0; c < chunk && enq < maxit; ++c, ++enq) {
-            OpArgs a = op_args(h, 0);
-            a.cx_floor = 0.0;
-            a.U = b.P;
-            a.out = b.Q;
-            a.partials = b.partials;
-            a.ctl = ctl;
-            a.nb = nb;
-            a.per = per_fused(h, H64, 0);
-            launch_op0(s, OP_MATVEC, a);
-            if (per && !a.per) launch_per_fold<double>(s, L0.g, b.Q, 0, ctl, nb);
-            launch_cg_alpha(s, b.sc, b.partials, nmv, nb);
-            launch_cg_update_ur(s, U, b.R, b.P, b.Q, n, b.sc, b.partials, r32, nb);
-            launch_cg_check(s, b.sc, b.partials, kRedBlocks, tol, maxit, nb);
-            precond(b.R, b.Z, r32 != nullptr);
-            if (flex) {
-                launch_cg_beta_flex<double>(s, b.R, b.Z, b.Q, n, b.sc, b.partials, maxit, nb);
-            } else {
-                launch_dot_partial(s, b.R, b.Z, n, b.partials, ctl, nb);
-                launch_cg_beta(s, b.sc, b.partials, kRedBlocks, maxit, nb);
-            }
-            launch_cg_update_p(s, b.P, b.Z, n, b.sc, nb);
-        }
+    double *rr = b.rr, *dots = b.rr + (long)nb * kCgBlocks;
+    launch_cg_rho<double>(s, b.R, b.P, n, b.sc, dots, nb);
+    const OpArgs mv = op_args(h, 0);
+    for (int q = 0; q < nb; ++q) h->prog[q] = 0;
+    for (int enq = 0; enq < maxit;) {  // two halves per iteration, as run_pcg
+        OpArgs a = mv;
+        a.cx_floor = 0.0;
+        a.U = b.P;
+        a.out = b.Q;
+        a.partials = b.partials;
+        a.ctl = ctl;
+        a.nb = nb;
+        a.per = per_fused(h, H64, 0);
+        launch_op0(s, OP_MATVEC, a);
+        if (per && !a.per) launch_per_fold<double>(s, L0.g, b.Q, 0, ctl, nb);
+        launch_cg_update_ur(s, U, b.R, b.P, b.Q, n, b.sc, b.partials, nmv, rr, r32, nb);
+        launch_cg_check(s, b.sc, rr, n, tol, h->prog, nb);
+        ++enq;
         HIPCHK(hipGetLastError());
-        HIPCHK(hipMemcpyAsync(b.sc_host, b.sc, nb * sizeof(CgScalars), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        bool all = true;
-        for (int q = 0; q < nb; ++q) all = all && b.sc_host[q].done;
-        if (all || enq >= maxit) break;
+        if (enq > 1 && cg_wait(s, h->prog, nb, enq - 1, nullptr)) break;
+        precond(b.R, b.Z, r32 != nullptr);
+        launch_cg_direction<double, double>(s, b.R, b.Z, b.Q, b.P, b.P, n, b.sc, dots, flex, maxit, nb);
     }
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(b.sc_host, b.sc, nb * sizeof(CgScalars), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
     if (int frc = coarse_check(h->C)) {  // the solve used a failed factorisation
         h->hier_ready = false;
         coarse_invalidate(h->C);
@@ -945,8 +964,10 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
         h->Q = dalloc<double>(h, g0.ndof);
         h->Z = dalloc<double>(h, g0.ndof);
         h->partials = dalloc<double>(h, maxblocks);
+        h->rr = dalloc<double>(h, 3 * kCgBlocks);
         h->sc = dalloc<CgScalars>(h, 1);
         HIPCHK(hipHostMalloc((void **)&h->sc_host, sizeof(CgScalars), hipHostMallocDefault));
+        HIPCHK(hipHostMalloc((void **)&h->prog, kMaxBatch * sizeof(unsigned long long), hipHostMallocDefault));
         std::memset(h->sc_host, 0, sizeof(CgScalars));
         HIPCHK(hipMemcpy(h->sc, h->sc_host, sizeof(CgScalars), hipMemcpyHostToDevice));
         Coarse &C = h->C;
@@ -997,6 +1018,7 @@ int gputo_destroy(gputo_handle *h)
     if (h->C.side) hipStreamSynchronize(h->C.side);
     for (void *p : h->allocs) hipFree(p);
     if (h->sc_host) hipHostFree(h->sc_host);
+    if (h->prog) (void)hipHostFree(h->prog);
     if (h->bt) {
         if (h->bt->sc_host) hipHostFree(h->bt->sc_host);
         delete h->bt;
