@@ -397,7 +397,7 @@ void launch_ke_elements(hipStream_t s, const Grid &g, const double *CX, const do
     k_ke_elements<<<(unsigned)((300 * g.nel + 255) / 256), 256, 0, s>>>(g, CX, Ke, A);
 }
 
-// CorrCsAQc (:1005-1028): zero the rows and columns of the fixed DOFs of
+// periodic cells, CorrCsAQc (:1005-1028): zero the rows and columns of the fixed DOFs of
 // the dense coarsest matrix (N x N, row-major), then 1e10 on their diagonal
 __global__ void k_zero_rowcol(int N, const int *__restrict__ fixed, int nfd, double *__restrict__ AQ)
 {
@@ -458,32 +458,78 @@ void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, d
 }
 
 // ---------------------------------------------------------------------------
-// Dense coarsest assembly (assembAc, mgcg1.cu:1747-1806).  The matrix is
-// padded to N = roundup(n, 32) with an identity block so the blocked kernels
-// below work on whole 32x32 tiles.  One block per row writes its columns from
-// `back` tiles before its own tile to the end of that (zeros included: nothing
-// beyond is read), each thread one column: the entry sums the elements that
-// hold both nodes, up to 8.  (One thread per row that added its 192 element
-// entries to zeroed memory one by one took 29-60 us after a fill of the
-// whole matrix; 5-8 us now, and no fill.)
+// Order of the factored coarsest matrix.  A band matrix eliminated from one
+// end has no parallelism beyond one column block: its steps are a chain.  The
+// node planes i = const are therefore split at the middle plane a: part 1
+// holds planes 0 .. a-1 in order, part 2 planes nnx-1 .. a+1 in reverse, and
+// the separator, plane a, comes last.  Each part followed by the separator is
+// a band matrix of its own (the parts do not couple), so two workgroups
+// eliminate them at once, the chain is half as long, and the inverse of the
+// factor has a zero block between the parts.  Parts are padded to whole
+// 32 x 32 tiles in front, the separator behind, with identity rows.
+// Factored at 13 x 7 x 7 nodes (1911 DOFs): 840 us as one band, 500 us split; at
+// 12 x 8 x 10 (2880 DOFs, band 269): 2200 us by tile-parallel launches, 1340 us.
+//
+// coarse_dof: the DOF of entry c of that order (-1: padding).  part_dof: of
+// row r of part q followed by the separator.
 // ---------------------------------------------------------------------------
 constexpr int NB = 32;
 
-__global__ __launch_bounds__(256) void k_assemble(Grid g, const double *__restrict__ A, double *__restrict__ AQ, int N,
-                                                 int back)
+__device__ __forceinline__ int coarse_dof(const CoarseMap &m, int c)
 {
-    const int r = blockIdx.x;
+    if (m.ps == 0) return c < m.n ? c : -1;  // one part
+    if (c < m.o2) return c >= m.pad1 ? c - m.pad1 : -1;
+    if (c < m.os) {
+        c -= m.o2 + m.pad2;
+        if (c < 0) return -1;
+        const int q = c / m.p;
+        return (m.nplanes - 1 - q) * m.p + (c - q * m.p);
+    }
+    c -= m.os;
+    return c < m.p ? m.a * m.p + c : -1;
+}
+
+__device__ __forceinline__ int part_dof(const CoarseMap &m, int q, int r)
+{
+    const int len = q == 0 ? m.o2 : m.os - m.o2;
+    return coarse_dof(m, r < len ? (q == 0 ? r : m.o2 + r) : m.os + r - len);
+}
+
+// Dense coarsest assembly (assembAc, mgcg1.cu:1747-1806) of each part with the
+// separator.  One block per row writes its columns from `back` tiles before
+// its own tile to the end of that (zeros included: nothing beyond is read),
+// each thread one column: the entry sums the elements that hold both nodes, up
+// to 8.  The separator's own block goes to part 1 (part 2: zeros).  mask (may
+// be null): the rows and columns of fixed DOFs are decoupled, 1e10 on their
+// diagonal (CorrCsAQc, Homogenization/QNC/mgcg9.cu:1005-1028).  (One thread
+// per row that added its 192 element entries to zeroed memory one by one took
+// 29-60 us after a fill of the whole matrix; 5-8 us now, and no fill.)
+__global__ __launch_bounds__(256) void k_assemble(Grid g, CoarseMap m, const double *__restrict__ A,
+                                                 const uint8_t *__restrict__ mask, CoarseParts P, int back)
+{
+    int q = 0, r = blockIdx.x;
+    if (P.np > 1 && r >= P.n[0]) {
+        q = 1;
+        r -= P.n[0];
+    }
     const int c0 = max(0, r / NB - back) * NB, c1 = (r / NB + 1) * NB;
-    const int nr = r / 3, cr = r - 3 * nr;
+    const int len = q == 0 ? m.o2 : m.os - m.o2;
+    const int dr = part_dof(m, q, r);
+    const int nr = dr / 3, cr = dr - 3 * nr;
     const int j = nr % g.nny, k = (nr / g.nny) % g.nnz, i = nr / (g.nny * g.nnz);
+    const bool rfix = mask && dr >= 0 && ((mask[nr] >> cr) & 1u);
     for (int c = c0 + (int)threadIdx.x; c < c1; c += 256) {
         double v = 0.0;
-        if (r >= g.ndof || c >= g.ndof) {
-            v = r == c ? 1.0 : 0.0;
-        } else {
-            const int nc = c / 3, cc = c - 3 * nc;
+        const int dc = part_dof(m, q, c);
+        const bool second = q == 1 && r >= len && c >= len;  // the separator's block of part 2
+        if (dr < 0 || dc < 0) {
+            v = r == c && !second ? 1.0 : 0.0;
+        } else if (!second) {
+            const int nc = dc / 3, cc = dc - 3 * nc;
             const int dj = nc % g.nny - j, dk = (nc / g.nny) % g.nnz - k, di = nc / (g.nny * g.nnz) - i;
-            if (abs(di) <= 1 && abs(dk) <= 1 && abs(dj) <= 1) {
+            if (mask && (rfix || ((mask[nc] >> cc) & 1u))) {
+                v = dr == dc ? 1e10 : 0.0;
+            } else if (abs(di) <= 1 && abs(dk) <= 1 && abs(dj) <= 1) {
                 for (int ei = 0; ei < 2; ++ei)
                     for (int ek = 0; ek < 2; ++ek)
                         for (int ej = 0; ej < 2; ++ej) {
@@ -492,22 +538,21 @@ __global__ __launch_bounds__(256) void k_assemble(Grid g, const double *__restri
                             if (ex < 0 || ex >= g.nx || ey < 0 || ey >= g.ny || ez < 0 || ez >= g.nz) continue;
                             if (bx < 0 || bx > 1 || by < 0 || by > 1 || bz < 0 || bz > 1) continue;
                             const long e = (long)g.ny * g.nz * ex + (long)g.ny * ez + ey;
-                            const int m = 3 * lidx2(1 - ei, 1 - ej, 1 - ek) + cr, n = 3 * lidx2(bx, by, bz) + cc;
-                            v += A[(long)pidx2(m, n) * g.nel + e];
+                            const int mm = 3 * lidx2(1 - ei, 1 - ej, 1 - ek) + cr, nn = 3 * lidx2(bx, by, bz) + cc;
+                            v += A[(long)pidx2(mm, nn) * g.nel + e];
                         }
             }
         }
-        AQ[(long)r * N + c] = v;
+        P.A[q][(long)r * P.n[q] + c] = v;
     }
 }
 
-// `bw`: the matrix's lower bandwidth.  The factorisation reads up to nbt =
-// (bw + 2 NB - 2) / NB tiles before a row's own, the corners of the inverse's
-// products up to 2 nbt - 1.
-void launch_assemble(hipStream_t s, const Grid &g, const double *A, double *AQ, int bw)
+// The factorisation reads up to nbt = (bw + 2 NB - 2) / NB tiles before a
+// row's own, the corners of the inverse's products up to 2 nbt - 1.
+void launch_assemble(hipStream_t s, const Grid &g, const double *A, const uint8_t *mask, const Coarse &C)
 {
-    const int N = (int)((g.ndof + NB - 1) / NB * NB);
-    k_assemble<<<N, 256, 0, s>>>(g, A, AQ, N, 2 * ((bw + 2 * NB - 2) / NB));
+    const CoarseParts P = coarse_parts(C);
+    k_assemble<<<P.n[0] + (P.np > 1 ? P.n[1] : 0), 256, 0, s>>>(g, C.map, A, mask, P, 2 * ((C.bw + 2 * NB - 2) / NB));
 }
 
 // ---------------------------------------------------------------------------
@@ -688,14 +733,20 @@ __global__ __launch_bounds__(256) void k_syrk_update(double *A, int N, int k0)
     }
 }
 
-// Inverse of each 32x32 diagonal factor tile, written into Linv.
-__global__ __launch_bounds__(64) void k_trtri_diag(const double *A, double *Linv, int N)
+// Inverse of each 32x32 diagonal factor tile, written into Linv (one block
+// per tile of the whole order).
+__global__ __launch_bounds__(64) void k_trtri_diag(CoarseBlocks B, double *Linv, int N)
 {
     __shared__ double L[NB][NB + 1];
     const int k0 = blockIdx.x * NB;
-    for (int q = threadIdx.x; q < NB * NB; q += 64) {
-        const int r = q / NB, c = q % NB;
-        L[r][c] = c <= r ? A[(long)(k0 + r) * N + k0 + c] : 0.0;
+    int q = 0;
+    while (q + 1 < B.nblk && k0 >= B.off[q + 1]) ++q;
+    const double *A = B.L[q];
+    const long ld = B.ld[q];
+    const int l0 = k0 - B.off[q];
+    for (int t = threadIdx.x; t < NB * NB; t += 64) {
+        const int r = t / NB, c = t % NB;
+        L[r][c] = c <= r ? A[(l0 + r) * ld + l0 + c] : 0.0;
     }
     __syncthreads();
     const int col = threadIdx.x;
@@ -703,10 +754,10 @@ __global__ __launch_bounds__(64) void k_trtri_diag(const double *A, double *Linv
     double x[NB];
 #pragma unroll
     for (int r = 0; r < NB; ++r) {
-        double s = (r == col) ? 1.0 : 0.0;
+        double t = (r == col) ? 1.0 : 0.0;
 #pragma unroll
-        for (int m = 0; m < r; ++m) s -= L[r][m] * x[m];
-        x[r] = (r < col) ? 0.0 : s / L[r][r];
+        for (int m = 0; m < r; ++m) t -= L[r][m] * x[m];
+        x[r] = (r < col) ? 0.0 : t / L[r][r];
     }
 #pragma unroll
     for (int r = 0; r < NB; ++r) Linv[(long)(k0 + r) * N + k0 + col] = x[r];
@@ -743,7 +794,10 @@ __global__ void k_transpose(const double *__restrict__ In, double *__restrict__ 
 // and are skipped: panel row x of a step (counted from the row below its
 // tile) is zero for x >= bw.
 // ---------------------------------------------------------------------------
-constexpr int kBandRowsMax = 256;
+// The separator split (coarse_dof) runs it on both parts at once, stopping
+// after the parts' own columns: what is pending is then applied to the
+// separator's block, which a second launch adds up and factors.
+constexpr int kBandRowsMax = 272;  // LDS: two buffers of 304 x 33 doubles
 constexpr int kCholThreads = 512;  // 2 waves per SIMD: 256 VGPRs for a panel row
 constexpr int kCholWaves = kCholThreads / 64;
 constexpr int kCholRows = NB + kBandRowsMax;  // rows of a block column in LDS
@@ -911,23 +965,36 @@ __device__ __forceinline__ void column_blocks(double (*D)[NB + 1], const double 
     }
 }
 
-__global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, int band_rows, int bw, int *flag)
+// block b factors the first `steps` block columns of a.A[b] (order n, row
+// stride ld)
+struct CholArgs {
+    double *A[2];
+    long ld[2];
+    int n[2], steps[2];
+    int band_rows, bw;
+    int *flag;
+};
+
+__global__ __launch_bounds__(kCholThreads) void k_chol_band(CholArgs a)
 {
     __shared__ double buf[2][kCholRows][NB + 1];
     __shared__ double rdg[NB];  // 1/L[jj][jj] of the current tile
+    double *A = a.A[blockIdx.x];
+    const long ld = a.ld[blockIdx.x];
+    const int N = a.n[blockIdx.x], nb = N / NB, steps = a.steps[blockIdx.x];
+    const int band_rows = a.band_rows, bw = a.bw;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int nb = N / NB;
     bool bad = false;
-    load_column(buf[0], A, N, min(N, NB + band_rows), tid, kCholThreads);  // block column 0 as assembled
+    load_column(buf[0], A, ld, min(N, NB + band_rows), tid, kCholThreads);  // block column 0 as assembled
     __syncthreads();
-    for (int k = 0; k < nb; ++k) {
+    for (int k = 0; k < steps; ++k) {
         double(*Cur)[NB + 1] = buf[k & 1];
         double(*Oth)[NB + 1] = buf[(k + 1) & 1];  // panel k-1 in phase A, block column k+1 from phase B on
         const long k0 = (long)k * NB;
         const int rows = min(N - (int)k0 - NB, band_rows);   // panel rows of step k
         const int prows = k > 0 ? min(N - (int)k0, band_rows) : 0;  // panel rows of step k-1 (from row k0)
-        const int rc = prows > NB ? min(2 * (prows / NB - 1), max(0, (bw - NB + 15) / 16)) : 0;  // rest block rows
+        const int rc = prows > NB ? min((prows - NB) / 16, max(0, (bw - NB + 15) / 16)) : 0;  // rest block rows
         // A. factor the tile | step k-1's update of the trailing band in
         // global memory and of column k's panel rows in LDS (slots from 4:
         // below the diagonal tile), by the waves off the factoring wave's
@@ -937,8 +1004,8 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
             if (lane < NB) rdg[lane] = 1.0 / Cur[lane][lane];
         } else if (wave != 4 && k > 0) {
             const int aw = wave - 1 - (wave > 4);  // 0..5
-            if (rc > 0) rest_blocks<0>(A, N, k0, Oth, lane, 2 * rc - 1, aw, kCholWaves - 2);
-            if (rc > 2) rest_blocks<1>(A, N, k0, Oth, lane, (rc - 2) * (rc - 1) / 2, aw, kCholWaves - 2);
+            if (rc > 0) rest_blocks<0>(A, ld, k0, Oth, lane, 2 * rc - 1, aw, kCholWaves - 2);
+            if (rc > 2) rest_blocks<1>(A, ld, k0, Oth, lane, (rc - 2) * (rc - 1) / 2, aw, kCholWaves - 2);
             column_blocks(Cur, Oth, lane, 4 + aw, 2 * (min(prows, bw + 15) / 16), kCholWaves - 2);
         }
         __syncthreads();
@@ -957,7 +1024,7 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
 #pragma unroll
             for (int c = 0; c < NB; ++c) Lr[c] = Cur[lr][c];
 #pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = Cur[NB + tid][c];  // rows past the panel: stale, not stored
+            for (int c = 0; c < 16; ++c) x[c] = Cur[min(NB + tid, kCholRows - 1)][c];  // rows past the panel: stale, not stored
             trsm_cols<0, 16>(x, Lr, rdg);
             if (tid < rows) {
 #pragma unroll
@@ -966,15 +1033,15 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
         } else {
             const int t0 = tid - tw, nt = kCholThreads - tw;
             const int n = k + 1 < nb ? min(N - (int)k0 - NB, NB + band_rows) * NB : 0;
-            const double *G = A + (k0 + NB) * N + k0 + NB;
+            const double *G = A + (k0 + NB) * ld + k0 + NB;
 #pragma unroll
             for (int u = 0; u < NB; ++u) {
                 const int q = t0 + u * nt;
-                x[u] = q < n ? G[(long)(q / NB) * N + q % NB] : 0.0;
+                x[u] = q < n ? G[(long)(q / NB) * ld + q % NB] : 0.0;
             }
             for (int q = t0; q < NB * NB; q += nt) {
                 const int r = q / NB, c = q % NB;
-                if (c <= r) A[(k0 + r) * N + k0 + c] = Cur[r][c];
+                if (c <= r) A[(k0 + r) * ld + k0 + c] = Cur[r][c];
             }
         }
         __syncthreads();
@@ -990,7 +1057,7 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
         __syncthreads();
         if (tid < tw) {
 #pragma unroll
-            for (int c = 16; c < NB; ++c) x[c] = Cur[NB + tid][c];
+            for (int c = 16; c < NB; ++c) x[c] = Cur[min(NB + tid, kCholRows - 1)][c];
             trsm_cols<16, NB>(x, Lr, rdg);
             if (tid < rows) {
 #pragma unroll
@@ -1004,12 +1071,12 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
                 const int q = t0 + u * nt;
                 if (q < n) Oth[q / NB][q % NB] = x[u];
             }
-            load_column(Oth, A + (k0 + NB) * N + k0 + NB, N, n / NB, t0 + NB * nt, nt);  // the rest, if any
+            load_column(Oth, A + (k0 + NB) * ld + k0 + NB, ld, n / NB, t0 + NB * nt, nt);  // the rest, if any
         }
         __syncthreads();
         // C. store panel k; the diagonal tile of column k+1 -= panel k's
         // first tile x its transpose (slots 0, 2, 3)
-        for (int q = tid; q < rows * NB; q += kCholThreads) A[(k0 + NB + q / NB) * N + k0 + q % NB] = Cur[NB + q / NB][q % NB];
+        for (int q = tid; q < rows * NB; q += kCholThreads) A[(k0 + NB + q / NB) * ld + k0 + q % NB] = Cur[NB + q / NB][q % NB];
         if (k + 1 < nb && wave < 3) {
             const int sl = wave == 0 ? 0 : wave + 1;
             const int ra = (sl >> 1) * 16, rb = (sl & 1) * 16;
@@ -1019,7 +1086,32 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
         }
         __syncthreads();
     }
-    if (bad && tid == 0) flag[0] = 1;
+    if (steps < nb) {
+        // what the last step leaves pending: the trailing band and the panel
+        // rows of block column `steps` (in LDS, its diagonal tile is current)
+        double(*P)[NB + 1] = buf[(steps - 1) & 1];
+        double(*D)[NB + 1] = buf[steps & 1];
+        const long k0 = (long)steps * NB;
+        const int prows = min(N - (int)k0, band_rows);
+        const int rc = prows > NB ? min((prows - NB) / 16, max(0, (bw - NB + 15) / 16)) : 0;
+        if (rc > 0) rest_blocks<0>(A, ld, k0, P, lane, 2 * rc - 1, wave, kCholWaves);
+        if (rc > 2) rest_blocks<1>(A, ld, k0, P, lane, (rc - 2) * (rc - 1) / 2, wave, kCholWaves);
+        column_blocks(D, P, lane, 4 + wave, 2 * (min(prows, bw + 15) / 16), kCholWaves);
+        __syncthreads();
+        const int rows = min(N - (int)k0, NB + band_rows);
+        for (int q = tid; q < rows * NB; q += kCholThreads)
+            A[(k0 + q / NB) * ld + k0 + q % NB] = D[q / NB][q % NB];
+    }
+    if (bad && tid == 0) a.flag[0] = 1;
+}
+
+// row blockIdx.x of the lower triangle: A += B (the two parts' updates of the
+// separator's block)
+__global__ __launch_bounds__(256) void k_add_lower(int n, const double *__restrict__ B, long ldb,
+                                                  double *__restrict__ A, long lda)
+{
+    const long r = blockIdx.x;
+    for (int c = threadIdx.x; c <= r && c < n; c += 256) A[r * lda + c] += B[r * ldb + c];
 }
 
 // ---------------------------------------------------------------------------
@@ -1037,7 +1129,8 @@ __global__ __launch_bounds__(kCholThreads) void k_chol_band(double *A, int N, in
 // 2 ceil(log2 nb) launches instead of a march down nb dependent block rows.
 // ---------------------------------------------------------------------------
 struct LinvLevel {
-    int g, nb, nbt;  // group size in tiles, tiles of the matrix, band in tiles
+    int g, nbt;      // group size in tiles, band in tiles
+    int groups;      // groups per diagonal block
     long wstride;    // doubles of W per group
 };
 
@@ -1104,39 +1197,110 @@ __device__ __forceinline__ void dgemm_tile64(const double *__restrict__ A, long 
                 C[(long)(qi + a * 16 + 4 * v + (lane >> 4)) * ldc + qj + b * 16 + (lane & 15)] = alpha * d[a][b][v];
 }
 
+// blockIdx.z: diagonal block x group
 template <int STEP>
-__global__ __launch_bounds__(256) void k_linv_level(const double *__restrict__ L, double *X, double *W, int N,
-                                                   LinvLevel lv)
+__global__ __launch_bounds__(256) void k_linv_level(CoarseBlocks B, double *Li, double *W, int N, LinvLevel lv)
 {
-    const int z = blockIdx.z, n1 = lv.g / 2, s = z * lv.g, h = s + n1;
-    if (h >= lv.nb) return;
-    const int n2 = min(lv.g, lv.nb - s) - n1;
+    const int q = blockIdx.z / lv.groups, z = blockIdx.z - q * lv.groups;
+    const int nb = (B.off[q + 1] - B.off[q]) / NB, n1 = lv.g / 2, s = z * lv.g, h = s + n1;
+    if (h >= nb) return;
+    const int n2 = min(lv.g, nb - s) - n1;
     const int r = min(lv.nbt, n2), c = min(lv.nbt, n1);
-    double *Wz = W + z * lv.wstride;
+    const double *L = B.L[q];
+    const long ldl = B.ld[q];
+    double *X = Li + (long)B.off[q] * N + B.off[q];
+    double *Wz = W + blockIdx.z * lv.wstride;
     const long ldw = (long)n1 * NB;
     if (STEP == 0)  // W = L21[0:r, n1-c:n1] X11[n1-c:n1, 0:n1]
-        dgemm_tile64(L + (long)h * NB * N + (long)(h - c) * NB, N, X + (long)(h - c) * NB * N + (long)s * NB, N, Wz,
+        dgemm_tile64(L + (long)h * NB * ldl + (long)(h - c) * NB, ldl, X + (long)(h - c) * NB * N + (long)s * NB, N, Wz,
                      ldw, r * NB, n1 * NB, c * NB, 1.0);
     else  // X21 = -X22[0:n2, 0:r] W
         dgemm_tile64(X + (long)h * NB * N + (long)h * NB, N, Wz, ldw, X + (long)h * NB * N + (long)s * NB, N, n2 * NB,
                      n1 * NB, r * NB, -1.0);
 }
 
-// Levels 2, 4, ... of the halving; X holds the diagonal tile inverses and
-// zeros above them, W has room for wcap doubles.
-static void launch_linv_levels(hipStream_t s, const double *L, double *X, double *W, long wcap, int N, int nbt)
+// The separator's rows of the inverse, blockIdx.z = part q: W = X_q L_qq^-1
+// with X_q the separator's rows of the part's factor (nonzero in the last nbt
+// tiles), then -L_ss^-1 W.
+template <int STEP>
+__global__ __launch_bounds__(256) void k_linv_sep(CoarseBlocks B, double *Li, double *W, int N, int nbt)
 {
-    const int nb = N / NB;
+    const int q = blockIdx.z, o = B.off[q], nq = B.off[q + 1] - o, os = B.off[2], ps = B.off[3] - os;
+    const int c = min(nbt, nq / NB) * NB;
+    double *Wz = W + (long)q * ps * N;
+    if (STEP == 0)
+        dgemm_tile64(B.L[q] + (long)nq * B.ld[q] + nq - c, B.ld[q], Li + (long)(o + nq - c) * N + o, N, Wz, nq, ps, nq, c,
+                     1.0);
+    else
+        dgemm_tile64(Li + (long)os * N + os, N, Wz, nq, Li + (long)os * N + o, N, ps, nq, ps, -1.0);
+}
+
+// Levels 2, 4, ... of the halving on every diagonal block at once; Li holds
+// the diagonal tile inverses and zeros above them, W has room for wcap doubles.
+static void launch_linv_levels(hipStream_t s, const CoarseBlocks &B, double *Li, double *W, long wcap, int N, int nbt)
+{
+    int nb = 0;
+    for (int q = 0; q < B.nblk; ++q) nb = std::max(nb, (B.off[q + 1] - B.off[q]) / NB);
     for (int g = 2; g / 2 < nb; g *= 2) {
         const int n1 = g / 2;
         const int groups = (nb - n1 + g - 1) / g;
         const int rmax = std::min(nbt, n1);
-        const LinvLevel lv{g, nb, nbt, (long)rmax * NB * n1 * NB};
-        if (lv.wstride * groups > wcap) throw std::runtime_error("coarsest inverse: work buffer too small");
-        const unsigned tn = (unsigned)((n1 * NB + 63) / 64);
-        k_linv_level<0><<<dim3(tn, (unsigned)((rmax * NB + 63) / 64), (unsigned)groups), 256, 0, s>>>(L, X, W, N, lv);
-        k_linv_level<1><<<dim3(tn, tn, (unsigned)groups), 256, 0, s>>>(L, X, W, N, lv);
+        const LinvLevel lv{g, nbt, groups, (long)rmax * NB * n1 * NB};
+        if (lv.wstride * groups * B.nblk > wcap) throw std::runtime_error("coarsest inverse: work buffer too small");
+        const unsigned tn = (unsigned)((n1 * NB + 63) / 64), tz = (unsigned)(groups * B.nblk);
+        k_linv_level<0><<<dim3(tn, (unsigned)((rmax * NB + 63) / 64), tz), 256, 0, s>>>(B, Li, W, N, lv);
+        k_linv_level<1><<<dim3(tn, tn, tz), 256, 0, s>>>(B, Li, W, N, lv);
     }
+    if (B.nblk == 3) {
+        const int ps = B.off[3] - B.off[2], nq = std::max(B.off[1], B.off[2] - B.off[1]);
+        if (2L * ps * N > wcap) throw std::runtime_error("coarsest inverse: work buffer too small");
+        const dim3 grid((unsigned)((nq + 63) / 64), (unsigned)((ps + 63) / 64), 2);
+        k_linv_sep<0><<<grid, 256, 0, s>>>(B, Li, W, N, nbt);
+        k_linv_sep<1><<<grid, 256, 0, s>>>(B, Li, W, N, nbt);
+    }
+}
+
+// The split pays from about ten tile steps on (each saved step is 10-14 us,
+// the separator's launches cost about 20 us) and needs two planes per part.
+void coarse_layout(Coarse &C, const Grid &g, bool periodic)
+{
+    CoarseMap &m = C.map;
+    m = CoarseMap();
+    m.n = C.n;
+    m.p = 3 * g.nny * g.nnz;
+    m.nplanes = g.nnx;
+    auto up = [](int v) { return (v + NB - 1) / NB * NB; };
+    const int N1 = up(C.n);
+    m.o2 = m.os = m.N = N1;
+    if (periodic || C.bw > kBandRowsMax || g.nnx < 5 || N1 / NB < 10) return;
+    m.a = g.nnx / 2;
+    const int p1 = m.a * m.p, p2 = (g.nnx - 1 - m.a) * m.p;
+    m.o2 = up(p1);
+    m.pad1 = m.o2 - p1;
+    m.os = m.o2 + up(p2);
+    m.pad2 = up(p2) - p2;
+    m.ps = up(m.p);
+    m.N = m.os + m.ps;
+}
+
+CoarseParts coarse_parts(const Coarse &C)
+{
+    const CoarseMap &m = C.map;
+    CoarseParts P{};
+    P.np = m.ps ? 2 : 1;
+    P.A[0] = C.AQ;
+    P.n[0] = m.o2 + m.ps;
+    if (m.ps) {
+        P.A[1] = C.AQ + (long)P.n[0] * P.n[0];
+        P.n[1] = m.os - m.o2 + m.ps;
+    }
+    return P;
+}
+
+long coarse_matrix_len(const Coarse &C)
+{
+    const CoarseParts P = coarse_parts(C);
+    return (long)P.n[0] * P.n[0] + (long)P.n[1] * P.n[1];
 }
 
 void coarse_factor(hipStream_t s0, Coarse &C, bool lag)
@@ -1145,19 +1309,38 @@ void coarse_factor(hipStream_t s0, Coarse &C, bool lag)
     C.solve_waits = C.target == C.cur;
     C.Linv = C.Lbuf[C.cur];
     C.LinvT = C.LTbuf[C.cur];
-    const int N = (C.n + NB - 1) / NB * NB;
-    const int nb = N / NB;
+    const int N = C.map.N, nb = N / NB, ps = C.map.ps;
     // the factor of a banded matrix keeps its band: panel rows and trailing
     // tiles beyond it are exact zeros and are skipped
     const int bw = std::max(1, std::min(C.bw, N));
-    const int band_rows = (bw + NB - 1) / NB * NB;
     hipStream_t s = C.side;
     HIPCHK(hipEventRecord(C.ev_in, s0));
     HIPCHK(hipStreamWaitEvent(s, C.ev_in, 0));
     HIPCHK(hipMemsetAsync(C.flag, 0, sizeof(int), s));
-    if (band_rows <= kBandRowsMax) {
-        k_chol_band<<<1, kCholThreads, 0, s>>>(C.AQ, N, band_rows, bw, C.flag);
+    if (bw <= kBandRowsMax) {
+        const CoarseParts P = coarse_parts(C);
+        CholArgs a{};
+        a.band_rows = (bw + 15) / 16 * 16;
+        a.bw = bw;
+        a.flag = C.flag;
+        for (int q = 0; q < P.np; ++q) {
+            a.A[q] = P.A[q];
+            a.ld[q] = a.n[q] = P.n[q];
+            a.steps[q] = (P.n[q] - ps) / NB;
+        }
+        k_chol_band<<<P.np, kCholThreads, 0, s>>>(a);
+        if (ps) {
+            const int l0 = P.n[0] - ps, l1 = P.n[1] - ps;
+            a.A[0] = P.A[0] + (long)l0 * P.n[0] + l0;
+            a.n[0] = ps;
+            a.steps[0] = ps / NB;
+            k_add_lower<<<ps, 256, 0, s>>>(ps, P.A[1] + (long)l1 * P.n[1] + l1, P.n[1], a.A[0], P.n[0]);
+            a.band_rows = std::max(ps - NB, 16);  // dense
+            a.bw = ps;
+            k_chol_band<<<1, kCholThreads, 0, s>>>(a);
+        }
     } else {
+        const int band_rows = (bw + NB - 1) / NB * NB;
         for (int kb = 0; kb < nb; ++kb) {
             const int k0 = kb * NB;
             k_potrf_diag<<<1, 64, 0, s>>>(C.AQ, N, k0, C.flag);
@@ -1181,16 +1364,30 @@ void coarse_finish(const Coarse &C)
 {
     if (!C.inv_pending) return;
     C.inv_pending = false;
-    const int N = (C.n + NB - 1) / NB * NB;
-    const int nb = N / NB;
+    const CoarseMap &m = C.map;
+    const int N = m.N, nb = N / NB;
     const int bw = std::max(1, std::min(C.bw, N));
     double *Li = C.Lbuf[C.target], *LiT = C.LTbuf[C.target];
     hipStream_t s = C.side;
+    const CoarseParts P = coarse_parts(C);
+    CoarseBlocks B{};
+    B.nblk = m.ps ? 3 : 1;
+    B.off[0] = 0;
+    B.L[0] = P.A[0];
+    B.ld[0] = P.n[0];
+    B.off[1] = m.ps ? m.o2 : N;
+    if (m.ps) {
+        B.L[1] = P.A[1];
+        B.ld[1] = P.n[1];
+        B.off[2] = m.os;
+        B.L[2] = P.A[0] + (long)m.o2 * P.n[0] + m.o2;
+        B.ld[2] = P.n[0];
+        B.off[3] = N;
+    }
     launch_fill(s, Li, (long)N * N, 0.0);
-    k_trtri_diag<<<nb, 64, 0, s>>>(C.AQ, Li, N);
-    const int nbt = std::min((bw + 2 * NB - 2) / NB, nb);
+    k_trtri_diag<<<nb, 64, 0, s>>>(B, Li, N);
     // the transpose's buffer is free until the last step: it holds W
-    launch_linv_levels(s, C.AQ, Li, LiT, (long)N * N, N, nbt);
+    launch_linv_levels(s, B, Li, LiT, (long)N * N, N, (bw + 2 * NB - 2) / NB);
     k_transpose<<<dim3(nb, nb), 256, 0, s>>>(Li, LiT, N);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(C.ev_done, s));
@@ -1255,34 +1452,61 @@ void coarse_switch(Coarse &C, hipStream_t s)
 // (mgcg1.c:431-432).  Each thread issues kTrmvLoads row entries (and as
 // many of b) before its first product, so a row of up to 2048 entries is
 // one memory round trip; the skip flag is read while they are in flight.
+// Rows and columns are in the factor's order (coarse_dof), the right-hand side
+// and the solution in the level's; a row of one part skips the other's columns
+// (zeros), which with the split halves the bytes read.
 // ---------------------------------------------------------------------------
 constexpr int kTrmvThreads = 256, kTrmvLoads = 8;
 
 template <bool UPPER, class Ti, class To>
-__global__ __launch_bounds__(kTrmvThreads) void k_trmv(const double *__restrict__ M, const Ti *__restrict__ b,
-                                                      To *__restrict__ x, int N, int n,
+__global__ __launch_bounds__(kTrmvThreads) void k_trmv(CoarseMap m, const double *__restrict__ M,
+                                                      const Ti *__restrict__ b, To *__restrict__ x,
                                                       const uint8_t *__restrict__ mask, const int *ctl)
 {
     __shared__ double red[kTrmvThreads / 64];
     ctl = batch_ctl(ctl);
     // lower: b has n entries, x has N (the padded y); upper: the reverse
-    b = batch_ptr(b, UPPER ? (long)N : (long)n);
-    x = batch_ptr(x, UPPER ? (long)n : (long)N);
-    const int row = blockIdx.x;  // < n: the grid has n blocks
-    const int lo = UPPER ? row : 0, hi = UPPER ? n - 1 : row;
-    const double *__restrict__ Mr = M + (long)row * N;
+    b = batch_ptr(b, UPPER ? (long)m.N : (long)m.n);
+    x = batch_ptr(x, UPPER ? (long)m.n : (long)m.N);
+    const int row = blockIdx.x;  // < N
+    // columns lo .. lo + cnt - 1, those from `cut` on shifted by `skip` (the
+    // separator's columns of a row of part 1)
+    const bool split = m.ps > 0;
+    int lo, cnt, cut, skip = 0;
+    if (!UPPER) {
+        lo = split && row >= m.o2 && row < m.os ? m.o2 : 0;
+        cnt = row + 1 - lo;
+        cut = m.N;
+    } else {
+        lo = row;
+        cnt = m.N - row;
+        cut = m.N;
+        if (split && row < m.o2) {
+            cut = m.o2;
+            skip = m.os - m.o2;
+            cnt -= skip;
+        }
+    }
+    const double *__restrict__ Mr = M + (long)row * m.N;
     double s = 0.0;
-    for (int c0 = lo + (int)threadIdx.x; c0 <= hi; c0 += kTrmvThreads * kTrmvLoads) {
+    for (int t0 = (int)threadIdx.x; t0 < cnt; t0 += kTrmvThreads * kTrmvLoads) {
         double mv[kTrmvLoads], bv[kTrmvLoads];
 #pragma unroll
         for (int u = 0; u < kTrmvLoads; ++u) {
-            const int c = c0 + kTrmvThreads * u;
-            const int cc = c <= hi ? c : c0;  // in the row's band (c0 <= hi)
-            const double m = Mr[cc];
-            mv[u] = c <= hi ? m : 0.0;  // entries past the triangle are never used
-            bv[u] = (double)b[cc];
+            const int t = t0 + kTrmvThreads * u;
+            int c = lo + (t < cnt ? t : t0);  // in the row
+            c += c >= cut ? skip : 0;
+            const double a = Mr[c];
+            if (UPPER) {
+                bv[u] = (double)b[c];
+                mv[u] = t < cnt ? a : 0.0;
+            } else {
+                const int d = coarse_dof(m, c);
+                bv[u] = (double)b[d < 0 ? 0 : d];
+                mv[u] = t < cnt && d >= 0 ? a : 0.0;
+            }
         }
-        if (c0 == lo + (int)threadIdx.x && ctl && ctl[0]) return;
+        if (t0 == (int)threadIdx.x && ctl && ctl[0]) return;
 #pragma unroll
         for (int u = 0; u < kTrmvLoads; ++u) s += mv[u] * bv[u];
     }
@@ -1293,8 +1517,14 @@ __global__ __launch_bounds__(kTrmvThreads) void k_trmv(const double *__restrict_
     __syncthreads();
     if (threadIdx.x == 0) {
         s = (red[0] + red[1]) + (red[2] + red[3]);
-        if (UPPER && mask && ((mask[row / 3] >> (row % 3)) & 1u)) s = 0.0;
-        x[row] = (To)s;
+        if (UPPER) {
+            const int d = coarse_dof(m, row);
+            if (d < 0) return;
+            if (mask && ((mask[d / 3] >> (d % 3)) & 1u)) s = 0.0;
+            x[d] = (To)s;
+        } else {
+            x[row] = (To)s;  // padding rows: 0
+        }
     }
 }
 
@@ -1303,16 +1533,15 @@ __global__ __launch_bounds__(kTrmvThreads) void k_trmv(const double *__restrict_
 template <class T>
 void launch_coarse_solve(hipStream_t s, const Coarse &C, const T *b, T *x, const uint8_t *mask, const int *ctl, int nb)
 {
-    const int N = (C.n + NB - 1) / NB * NB;
     coarse_finish(C);  // also a lagged factorisation's, which runs meanwhile
     if (C.solve_waits && !C.waited) {  // the factorisation of this hierarchy, once per stream order
         HIPCHK(hipStreamWaitEvent(s, C.ev_done, 0));
         C.waited = true;
     }
     // C.y has room for kMaxBatch right-hand sides
-    k_trmv<false, T, double>
-        <<<dim3(C.n, 1, batch_dim(nb)), kTrmvThreads, 0, s>>>(C.Linv, b, C.y, N, C.n, nullptr, ctl);
-    k_trmv<true, double, T><<<dim3(C.n, 1, batch_dim(nb)), kTrmvThreads, 0, s>>>(C.LinvT, C.y, x, N, C.n, mask, ctl);
+    const dim3 grid(C.map.N, 1, batch_dim(nb));
+    k_trmv<false, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.Linv, b, C.y, nullptr, ctl);
+    k_trmv<true, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.LinvT, C.y, x, mask, ctl);
 }
 template void launch_coarse_solve<double>(hipStream_t, const Coarse &, const double *, double *, const uint8_t *,
                                           const int *, int);

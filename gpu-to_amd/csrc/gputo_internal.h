@@ -170,11 +170,33 @@ struct Level {
     std::vector<int> fixed;       // fixed list (0-based DOF), reference order
 };
 
+// Order of the factored coarsest matrix (coarse_dof in coarse.hip): N entries;
+// ps = 0: the DOFs in order (o2 = os = N), else two parts that end at o2 and os
+// and the separator plane a.
+struct CoarseMap {
+    int n = 0, N = 0;
+    int o2 = 0, os = 0, ps = 0, pad1 = 0, pad2 = 0;
+    int p = 0, nplanes = 0, a = 0;  // DOFs of a plane, planes
+};
+// the matrices that are factored (each part followed by the separator, row
+// stride = order), and the diagonal blocks of the whole factor
+struct CoarseParts {
+    int np;
+    double *A[2];
+    int n[2];
+};
+struct CoarseBlocks {
+    int nblk, off[4];
+    const double *L[3];
+    long ld[3];
+};
+
 struct Coarse {
     int n = 0;
+    CoarseMap map;
     bool direct = true;      // factored (else smoothed: mgcg9 above 20000 DOFs)
     int bw = 0;              // lower bandwidth of the assembled matrix (node-major DOFs)
-    double *AQ = nullptr;       // dense matrix, then its Cholesky factor (lower)
+    double *AQ = nullptr;       // dense matrix (matrices of the parts), then the Cholesky factor (lower)
     double *Linv = nullptr;     // inverse of the factor used by the solves (lower, row-major)
     double *LinvT = nullptr;    // its transpose (row-major)
     double *Lbuf[2] = {}, *LTbuf[2] = {};  // two inverse buffers (lagged factorisation)
@@ -323,7 +345,11 @@ void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, d
 void launch_coarse_cx(hipStream_t s, const Grid &gc, const double *CXf, double *CXc);
 void launch_ke_elements(hipStream_t s, const Grid &g, const double *CX, const double *Ke, double *A);
 void launch_zero_rowcol(hipStream_t s, int N, const int *fixed_d, int nfd, double *AQ);
-void launch_assemble(hipStream_t s, const Grid &g, const double *A, double *AQ, int bw);
+// mask: decouple the fixed DOFs (mgcg9), or null
+void launch_assemble(hipStream_t s, const Grid &g, const double *A, const uint8_t *mask, const Coarse &C);
+void coarse_layout(Coarse &C, const Grid &g, bool periodic);  // C.map from C.n, C.bw
+CoarseParts coarse_parts(const Coarse &C);
+long coarse_matrix_len(const Coarse &C);  // doubles of C.AQ
 // Factor C.AQ on C.side after the work on s.  lag: when an earlier factor
 // exists, write the new one into the other buffer and let the solves keep
 // the earlier one (coarse_adopt switches at the next setup).

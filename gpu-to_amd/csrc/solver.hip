@@ -389,11 +389,12 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         if (h->C.direct) {
             if (!vc.A) vc.A = dalloc<double>(h, 300 * vc.g.nel);  // nl = 2
             launch_ke_elements(s, vc.g, vc.CXl, h->Ke, vc.A);
-            if (per)
+            if (per) {
                 launch_assemble_per(s, vc.g, vc.A, h->C.AQ);
-            else
-                launch_assemble(s, vc.g, vc.A, h->C.AQ, h->C.bw);
-            launch_zero_rowcol(s, (h->C.n + 31) / 32 * 32, vc.fixed_d, (int)vc.fixed.size(), h->C.AQ);
+                launch_zero_rowcol(s, h->C.map.N, vc.fixed_d, (int)vc.fixed.size(), h->C.AQ);
+            } else {
+                launch_assemble(s, vc.g, vc.A, vc.mask, h->C);
+            }
             HIPCHK(hipGetLastError());
             coarse_factor(s, h->C, coarse_lagged(h->prm));
         }
@@ -433,10 +434,10 @@ int setup_hierarchy(gputo_handle *h, const std::vector<int> &fixed0)
         if (per) {
             // the wrapped matrix with the fixed rows and columns decoupled
             launch_assemble_per(s, v.g, v.A, h->C.AQ);
-            launch_zero_rowcol(s, (h->C.n + 31) / 32 * 32, v.fixed_d, (int)v.fixed.size(), h->C.AQ);
+            launch_zero_rowcol(s, h->C.map.N, v.fixed_d, (int)v.fixed.size(), h->C.AQ);
         } else {
             launch_corrcsa(s, v.g, v.fixed_d, (int)v.fixed.size(), v.A, p.corr_mirrored);
-            launch_assemble(s, v.g, v.A, h->C.AQ, h->C.bw);
+            launch_assemble(s, v.g, v.A, nullptr, h->C);
         }
     }
     HIPCHK(hipGetLastError());
@@ -978,9 +979,10 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
             C.bw = 3 * (gc.nny * gc.nnz + gc.nny + 1) + 2;
             if (h->prm.periodic) C.bw = C.n;  // wrapped couplings: no band
         }
-        const long N = (C.n + 31) / 32 * 32;
+        coarse_layout(C, h->L[nl - 1].g, h->prm.periodic != 0);
+        const long N = C.map.N;
         if (dense_ok) {
-            C.AQ = dalloc<double>(h, N * N);
+            C.AQ = dalloc<double>(h, coarse_matrix_len(C));
             for (int b = 0; b < 2; ++b) {
                 C.Lbuf[b] = dalloc<double>(h, N * N);
                 C.LTbuf[b] = dalloc<double>(h, N * N);

@@ -1,0 +1,62 @@
+"""The coarsest solve where the factorisation is split at the middle plane
+(band of at most 272 rows, at least ten 32-row tiles, five planes), against
+numpy's dense solve of the assembled matrix.
+
+Coarsest grids (nodes): 7x7x3 (parts of 189 DOFs in 192 rows), 8x5x5
+(parts of four and three planes), 5x5x5 (two
+planes to a part), 17x4x5 (many steps), 9x9x9 (band 275: not split) and, with
+the decoupled fixed DOFs of the mgcg9 engine, 12x8x10 (band 269, the widest
+that is split).  Tolerance as for the unsplit solve: the conditioning of the
+penalised matrix (1e-9)."""
+import numpy as np
+import pytest
+
+from conftest import cantilever_case
+
+pytestmark = pytest.mark.gpu
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / max(np.abs(b).max(), 1e-300)
+
+
+@pytest.mark.parametrize("coarse", [(6, 6, 2), (7, 4, 4), (4, 4, 4), (16, 3, 4), (8, 8, 8)])
+def test_split_coarse_solve(gputo, oracle, coarse):
+    cx, cy, cz = coarse
+    nelx, nely, nelz = 2 * cx, 2 * cy, 2 * cz
+    print("case", coarse, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=8)
+    s = gputo.Solver(nelx, nely, nelz, 2)
+    try:
+        s.setup(Ke, CX, fixed)
+        A, _, fd = s.level_matrices(1)
+        AQ = oracle.assemble(A, cx, cy, cz)
+        rng = np.random.default_rng(9)
+        for _ in range(2):
+            b = rng.uniform(-1, 1, AQ.shape[0])
+            b[(fd - 1).astype(int)] = 0.0
+            x = s.coarse_solve(b)
+            xr = np.linalg.solve(AQ, b)
+            xr[(fd - 1).astype(int)] = 0.0
+            assert rel(x, xr) < 1e-9
+    finally:
+        s.close()
+
+
+@pytest.mark.parametrize("mesh,nl", [((44, 28, 36), 3), ((28, 16, 16), 3)])
+def test_split_decoupled_fixed_dofs(gputo, oracle, mesh, nl):
+    """One V-cycle of the mgcg9 engine, whose fixed rows and columns are
+    decoupled while the matrix is assembled."""
+    nelx, nely, nelz = mesh
+    print("case", mesh, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=10)
+    r = np.random.default_rng(11).uniform(-1, 1, F.size)
+    r[(fixed - 1).astype(int)] = 0.0
+    s = gputo.Solver(nelx, nely, nelz, nl, preset=2)
+    try:
+        z = s.vcycle(Ke, CX, fixed, r)
+    finally:
+        s.close()
+    oracle.lib().or_set_nswp(2)
+    zo = oracle.vcycle_once(Ke, CX, fixed, nelx, nely, nelz, nl, r, preset=2)
+    assert rel(z, zo) < 1e-9
