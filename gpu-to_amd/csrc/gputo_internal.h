@@ -237,6 +237,8 @@ struct BatchState {
     float *r32 = nullptr, *z32 = nullptr;  // the FP32 V-cycle's right-hand side and result
 };
 
+struct HostStage;
+
 }  // namespace gputo
 
 struct gputo_handle {
@@ -267,6 +269,8 @@ struct gputo_handle {
     bool masks_ready = false;     // level fixed lists and masks match L[0].fixed
     std::vector<void *> allocs;
     struct ToState *to = nullptr;
+    struct ToState *to_kept = nullptr;  // an ended design loop's buffers, for the next one
+    gputo::HostStage *stage = nullptr;  // pinned slots of the host copies (hostio.hip)
     gputo::MixedState *mx = nullptr;
     gputo::LearnState *ln = nullptr;  // learned level-2 correction (params.learned)
     // per-fine-element Galerkin tables of levels 1..gt_max (device, packed
@@ -425,7 +429,23 @@ __device__ __forceinline__ double block_sum(double v)
 }
 
 
-void to_release(gputo_handle *h);  // frees the design-loop state (driver.hip)
+void to_release(gputo_handle *h);  // ends the design loop, its buffers stay with the handle (driver.hip)
+void to_destroy(gputo_handle *h);
+// ---- host arrays (hostio.hip) ------------------------------------------
+// dev null: the host array is only checked.  check: FP64 values, all finite.
+struct HostJob {
+    void *dev;
+    void *host;
+    size_t bytes;
+    bool check;
+};
+// In stream order on h->stream; the host arrays may be reused on return.
+// False: a checked array holds a NaN or an infinity (what is on the device is
+// then undefined).
+bool host_upload(gputo_handle *h, const HostJob *jobs, int njobs);
+void host_download(gputo_handle *h, const HostJob *jobs, int njobs);
+void stage_destroy(gputo_handle *h);  // after the stream's work
+void launch_flip_y(hipStream_t s, double *u, long nnod);
 
 // ---- periodic unit cell (periodic.hip) --------------------------------
 // A periodic vector lives on the full node grid; the nodes with i = nx,

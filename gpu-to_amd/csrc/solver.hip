@@ -1013,10 +1013,11 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
 int gputo_destroy(gputo_handle *h)
 {
     if (!h) return 0;
-    to_release(h);
+    to_destroy(h);
     learn_destroy(h);
     mixed_destroy(h);
     if (h->stream) hipStreamSynchronize(h->stream);
+    stage_destroy(h);
     if (h->C.side) hipStreamSynchronize(h->C.side);
     for (void *p : h->allocs) hipFree(p);
     if (h->sc_host) hipHostFree(h->sc_host);
@@ -1054,16 +1055,22 @@ int gputo_set_params(gputo_handle *h, const gputo_params *params)
     return 0;
 }
 
-static int upload_problem(gputo_handle *h, const double *Ke0, const double *CX, const double *fixed, int nfd,
-                          std::vector<int> &fx)
+// F (may be null) goes to h->Fv.  Nothing that an earlier call left on the
+// device changes before every array is known to be finite.
+static int upload_problem(gputo_handle *h, const double *Ke0, const double *F, const double *CX, const double *fixed,
+                          int nfd, std::vector<int> &fx)
 {
     const Grid &g0 = h->L[0].g;
     if (!Ke0 || !CX || (nfd > 0 && !fixed) || nfd < 0 || nfd > g0.ndof) return GPUTO_ERR_ARGUMENT;
-    if (!all_finite(Ke0, 576) || !all_finite(CX, g0.nel)) return GPUTO_ERR_NONFINITE;
+    if (!all_finite(Ke0, 576)) return GPUTO_ERR_NONFINITE;
+    const size_t cb = g0.nel * sizeof(double);
+    const HostJob in[2] = {{nullptr, (void *)CX, cb, true}, {h->Fv, (void *)F, g0.ndof * sizeof(double), true}};
+    if (!host_upload(h, in, F ? 2 : 1)) return GPUTO_ERR_NONFINITE;
     fx.resize(nfd);
     for (int n = 0; n < nfd; ++n) fx[n] = (int)fixed[n] - 1;  // (int)FDofs[n]-1, mgcg1.c:663
     set_ke(h, Ke0);
-    HIPCHK(hipMemcpyAsync(h->CX, CX, g0.nel * sizeof(double), hipMemcpyHostToDevice, h->stream));
+    const HostJob cx = {h->CX, (void *)CX, cb, false};
+    host_upload(h, &cx, 1);
     return 0;
 }
 
@@ -1072,7 +1079,7 @@ int gputo_setup(gputo_handle *h, const double *Ke0, const double *CX, const doub
     if (!h) return GPUTO_ERR_ARGUMENT;
     try {
         std::vector<int> fx;
-        if (int rc = upload_problem(h, Ke0, CX, fixed, nfd, fx)) return rc;
+        if (int rc = upload_problem(h, Ke0, nullptr, CX, fixed, nfd, fx)) return rc;
         if (int rc = setup_hierarchy(h, fx)) return rc;
         if (int rc = coarse_check(h->C)) {
             h->hier_ready = false;
@@ -1094,13 +1101,11 @@ int gputo_mgcg1(gputo_handle *h, const double *Ke0, const double *F, double *U, 
     try {
         const Grid &g0 = h->L[0].g;
         std::vector<int> fx;
-        int rc = upload_problem(h, Ke0, CX, fixed, nfd, fx);
-        if (rc == 0 && !all_finite(F, g0.ndof)) rc = GPUTO_ERR_NONFINITE;
+        int rc = upload_problem(h, Ke0, F, CX, fixed, nfd, fx);
         if (rc) {
             *nit = rc;
             return rc;
         }
-        HIPCHK(hipMemcpyAsync(h->Fv, F, g0.ndof * sizeof(double), hipMemcpyHostToDevice, h->stream));
         rc = setup_hierarchy(h, fx);
         if (rc == 0) {
             rc = run_pcg(h, h->Fv, h->Uv, tol, maxit, relres, nit);
@@ -1109,9 +1114,9 @@ int gputo_mgcg1(gputo_handle *h, const double *Ke0, const double *F, double *U, 
             *nit = rc;
             return rc;
         }
-        HIPCHK(hipMemcpyAsync(U, h->Uv, g0.ndof * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(hipStreamSynchronize(h->stream));
-        for (long n = 1; n < g0.ndof; n += 3) U[n] = -U[n];  // MATLAB frame (mgcg1.cu:282-283)
+        launch_flip_y(h->stream, h->Uv, g0.nnod);
+        const HostJob out = {h->Uv, U, g0.ndof * sizeof(double), false};
+        host_download(h, &out, 1);
         return 0;
     } catch (...) {
         int rc = map_exception();
@@ -1153,7 +1158,7 @@ static int host_op(gputo_handle *h, int mode, const double *Ke0, const double *C
     try {
         const Grid &g0 = h->L[0].g;
         std::vector<int> fx;
-        if (int rc = upload_problem(h, Ke0, CX, fixed, nfd, fx)) return rc;
+        if (int rc = upload_problem(h, Ke0, nullptr, CX, fixed, nfd, fx)) return rc;
         if (int rc = validate_fixed(fx, g0.ndof)) return rc;
         std::vector<uint8_t> m = node_mask(fx, g0);
         hipStream_t s = h->stream;
@@ -1196,7 +1201,7 @@ int gputo_matvec_mixed(gputo_handle *h, int kernel, const double *Ke0, const dou
     try {
         const Grid &g0 = h->L[0].g;
         std::vector<int> fx;
-        if (int rc = upload_problem(h, Ke0, CX, fixed, nfd, fx)) return rc;
+        if (int rc = upload_problem(h, Ke0, nullptr, CX, fixed, nfd, fx)) return rc;
         if (int rc = validate_fixed(fx, g0.ndof)) return rc;
         std::vector<uint8_t> m = node_mask(fx, g0);
         hipStream_t s = h->stream;

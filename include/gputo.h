@@ -306,7 +306,8 @@ typedef struct gputo_to_stats {
 
 /* Start a design loop on this handle: x0 (nel doubles, design variables),
  * F (ndof doubles, C frame), fixed (1-based doubles).  Device-resident
- * state persists until gputo_to_end. */
+ * state persists until gputo_to_end; its device memory stays with the handle
+ * for the next design loop and is freed by gputo_destroy. */
 int gputo_to_begin(gputo_handle *h, const double *Ke0, const double *x0, const double *F, const double *fixed,
                    int nfd, const gputo_to_config *cfg);
 /* One design iteration: filter, projection, CX, MGCG solve, sensitivity,
