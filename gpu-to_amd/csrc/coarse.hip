@@ -482,7 +482,7 @@ __device__ __forceinline__ int coarse_dof(const CoarseMap &m, int c)
     if (c < m.os) {
         c -= m.o2 + m.pad2;
         if (c < 0) return -1;
-        const int q = c / m.p;
+        const int q = (int)(((float)c + 0.5f) * m.rp);  // c / p: exact below 2^20
         return (m.nplanes - 1 - q) * m.p + (c - q * m.p);
     }
     c -= m.os;
@@ -1280,6 +1280,7 @@ void coarse_layout(Coarse &C, const Grid &g, bool periodic)
     m.os = m.o2 + up(p2);
     m.pad2 = up(p2) - p2;
     m.ps = up(m.p);
+    m.rp = 1.0f / (float)m.p;
     m.N = m.os + m.ps;
 }
 

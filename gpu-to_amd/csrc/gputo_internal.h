@@ -79,7 +79,7 @@ struct OpArgsT {
     const T *Ke;           // 24x24 row-major (level 0)
     const T *CX;           // element scale (level 0)
     const T *A;            // packed 300 x nel entry-major element matrices (levels >= 1)
-    const T *S;            // assembled node stencils [27][3][3][nnod] of the same operator, or null
+    const T *S;            // assembled node stencils [14][3][3][stencil_ld] of the same operator, or null
     const T *U;            // input vector
     const T *F;            // right-hand side (defect / Jacobi)
     const T *AD;           // diagonal (Jacobi)
@@ -177,6 +177,7 @@ struct CoarseMap {
     int n = 0, N = 0;
     int o2 = 0, os = 0, ps = 0, pad1 = 0, pad2 = 0;
     int p = 0, nplanes = 0, a = 0;  // DOFs of a plane, planes
+    float rp = 0.0f;                // 1/p
 };
 // the matrices that are factored (each part followed by the separator, row
 // stride = order), and the diagonal blocks of the whole factor
@@ -310,6 +311,8 @@ void launch_recip(hipStream_t s, const double *AD, double *RD, long n, int strid
 // S = the operator of the packed element matrices A as node stencils
 void launch_stencil_build(hipStream_t s, const Grid &g, const double *A, double *S);
 constexpr int kStencilEntries = 126;  // the own and 13 forward 3 x 3 blocks per node (the rest by symmetry)
+constexpr int kStencilNodes = 16;     // nodes of a workgroup; rows of S are whole workgroups long
+__host__ __device__ inline long stencil_ld(long nnod) { return (nnod + kStencilNodes - 1) / kStencilNodes * kStencilNodes; }
 template <class T>
 void launch_restrict(hipStream_t s, const Grid &gc, const T *Rf, T *Fc, const uint8_t *maskc, const int *ctl,
                      int nb = 1);

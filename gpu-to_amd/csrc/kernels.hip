@@ -440,7 +440,7 @@ __global__ __launch_bounds__(kBlock) void k_stored(OpArgsT<T> a)
 // element position), and the element matrices are symmetric, so block
 // 26 - b of node p + d is exactly the transpose of block b of node p: only
 // the node's own block and the 13 forward blocks (b >= 13) are stored,
-// S[(9 (b - 13) + 3 r + c) nnod + node], and a backward block is read
+// S[(9 (b - 13) + 3 r + c) ld + node], and a backward block is read
 // transposed at the neighbour.  Zero blocks stand for neighbours outside
 // the grid.  Built once per setup from the element matrices, applied by
 // k_stencil with 81 coalesced matrix loads and 27 neighbour loads per node,
@@ -477,7 +477,7 @@ __global__ void k_stencil_build(Grid g, const double *__restrict__ A, double *__
                     for (int c = 0; c < 3; ++c) sb[3 * r + c] += A[(long)pidx(3 * la + r, 3 * lb + c) * g.nel + e];
             }
 #pragma unroll
-    for (int q = 0; q < 9; ++q) S[(long)(9 * (b - 13) + q) * nnod + nod] = sb[q];
+    for (int q = 0; q < 9; ++q) S[(long)(9 * (b - 13) + q) * stencil_ld(nnod) + nod] = sb[q];
 }
 
 void launch_stencil_build(hipStream_t s, const Grid &g, const double *A, double *S)
@@ -485,132 +485,93 @@ void launch_stencil_build(hipStream_t s, const Grid &g, const double *A, double 
     k_stencil_build<<<dim3((unsigned)((g.nnod + 255) / 256), 14), 256, 0, s>>>(g, A, S);
 }
 
-// Three waves per 64 consecutive nodes: wave w sums the 9 blocks of the
-// neighbour plane di = w - 1 (FP32: all 108 loads in flight together; FP64:
-// one dk row of 36 at a time), the three plane sums meet in LDS and wave 1
-// (the node's own plane) adds them in plane order and finishes as k_stored
-// does.  On the small levels a launch is a few memory round trips long, so
-// every load is issued in the first one: wave 1 fetches its epilogue
-// operands (mask, F, AD, own u) with the stencil, and the skip flag is read
-// alongside and tested once they are in flight.
-// Stencil products of neighbour plane di = W - 1 for one node (lane): the
-// blocks b = 9W + 3 (dk+1) + (dj+1), read at the node when b >= 13 and
-// transposed at the neighbour (its block 26 - b) when b < 13.  Returns false
-// when the solve has converged (the flag is read once the first loads are
-// in flight).
-template <int W, class T, int MODE>
-__device__ __forceinline__ bool stencil_plane(const OpArgsT<T> &a, long p, long pc, int j, int k, long pw, T &y0,
-                                              T &y1, T &y2)
-{
-    const long nnod = a.g.nnod;
-    constexpr int NR = sizeof(T) == 8 ? 1 : 3;  // dk rows per batch
-#pragma unroll
-    for (int r0 = 0; r0 < 3; r0 += NR) {
-        T sv[NR][3][9], uu[NR][3][3];
-#pragma unroll
-        for (int rr = 0; rr < NR; ++rr) {
-            const int dk = r0 + rr - 1;
-#pragma unroll
-            for (int c3 = 0; c3 < 3; ++c3) {
-                const int dj = c3 - 1;
-                const int kk = k + dk, jj = j + dj;
-                const bool ok = kk >= 0 && kk < a.g.nnz && jj >= 0 && jj < a.g.nny;
-                // outside the grid the block is zero: read any valid node
-                const long nb = ok ? pw + (dk * a.g.nny + dj) : pc;
-                const int b = 9 * W + 3 * (r0 + rr) + c3;
-                if (b >= 13) {
-                    const T *__restrict__ Sb = a.S + (long)(9 * (b - 13)) * nnod + p;
-#pragma unroll
-                    for (int q = 0; q < 9; ++q) sv[rr][c3][q] = Sb[(long)q * nnod];
-                } else {
-                    const T *__restrict__ Sb = a.S + (long)(9 * (13 - b)) * nnod + nb;
-#pragma unroll
-                    for (int r = 0; r < 3; ++r)
-#pragma unroll
-                        for (int c = 0; c < 3; ++c) {
-                            const T v = Sb[(long)(3 * c + r) * nnod];
-                            sv[rr][c3][3 * r + c] = ok ? v : T(0);
-                        }
-                }
-#pragma unroll
-                for (int c = 0; c < 3; ++c) uu[rr][c3][c] = stored_u<T, MODE>(a, 3 * nb + c);
-            }
-        }
-        if (r0 == 0 && a.ctl && a.ctl[0]) return false;  // converged: nothing is written
-#pragma unroll
-        for (int rr = 0; rr < NR; ++rr)
-#pragma unroll
-            for (int c3 = 0; c3 < 3; ++c3) {
-                const T *m = sv[rr][c3];
-                const T *u = uu[rr][c3];
-                y0 += m[0] * u[0] + m[1] * u[1] + m[2] * u[2];
-                y1 += m[3] * u[0] + m[4] * u[1] + m[5] * u[2];
-                y2 += m[6] * u[0] + m[7] * u[1] + m[8] * u[2];
-            }
-    }
-    return true;
-}
+// Sixteen consecutive nodes per workgroup and one thread per node and block b:
+// 9 matrix loads and 3 of u, all in flight together, read at the node when
+// b >= 13 and transposed at the neighbour (its block 26 - b) when b < 13.  The
+// products meet in LDS, and one thread per DOF adds them plane by plane and
+// finishes as k_stored does.  A small level is a launch and a memory round
+// trip long, so its few nodes are spread over many CUs and every load is
+// issued in the first trip: the finishing threads fetch their operands (mask,
+// F, AD, own u) with the stencil, and the skip flag is read alongside and
+// tested once they are in flight.  A large one is bound by the bytes of S: each
+// XCD takes one contiguous range of nodes, so the transposed blocks, which the
+// neighbours' owners read too, come from its L2, and sixteen FP64 entries are
+// one cache line (rows of S are padded to it).  (64 nodes per workgroup, one
+// wave per plane, dealt over the XCDs: a sweep took 5.4 us at 637 nodes in
+// FP64, 3.7 now; 4.75 at 4225 nodes in FP32, 3.75 now; the FP64 sweeps of
+// 30625 and 4225 nodes 8.5 us on average, 7.15 now.)
+constexpr int kStThreads = kStencilNodes * 28;  // 27 blocks, and a full last wave
 
 template <class T, int MODE>
-__global__ __launch_bounds__(192) void k_stencil(OpArgsT<T> a)
+__global__ __launch_bounds__(kStThreads) void k_stencil(OpArgsT<T> a)
 {
     batch_shift(a);
-    __shared__ T red[2][3][64];
+    __shared__ T red[27][kStencilNodes][3];
     const Grid g = a.g;
-    const long nnod = g.nnod;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const long p = (long)blockIdx.x * 64 + lane;
-    const bool live = p < nnod;
-    const long pc = live ? p : 0;
+    const unsigned nblk = (unsigned)((g.nnod + kStencilNodes - 1) / kStencilNodes);
+    const unsigned tb = (unsigned)xcd_tile(blockIdx.x, nblk);
+    if (tb >= nblk) return;  // padding block of the XCD order
+    const int b = min((int)threadIdx.x / kStencilNodes, 26);
+    const long p0 = (long)tb * kStencilNodes;
+    const long pc = min(p0 + (threadIdx.x & (kStencilNodes - 1)), (long)g.nnod - 1);
     // 32-bit decomposition (a level has far fewer than 2^32 nodes)
     const unsigned pu = (unsigned)pc, q1 = pu / (unsigned)g.nny;
     const int j = (int)(pu - q1 * (unsigned)g.nny), k = (int)(q1 % (unsigned)g.nnz), i = (int)(q1 / (unsigned)g.nnz);
-    const int ii = i + w - 1;
-    const long pw = pc + (long)(w - 1) * ((long)g.nny * g.nnz);  // the node's image in plane ii
-    // epilogue operands of wave 1 (in bounds for every lane: node pc)
-    const long dof = 3 * pc;
-    unsigned msk = 0;
-    T fe[3] = {T(0), T(0), T(0)}, ade[3] = {T(1), T(1), T(1)}, ue[3] = {T(0), T(0), T(0)};
-    if (w == 1) {
-        msk = a.mask[pc];
+    const int ii = i + b / 9 - 1, kk = k + (b / 3) % 3 - 1, jj = j + b % 3 - 1;
+    // outside the grid the block is zero: any valid node is read
+    const bool ok = ii >= 0 && ii < g.nnx && kk >= 0 && kk < g.nnz && jj >= 0 && jj < g.nny;
+    const long nb = ok ? ((long)ii * g.nnz + kk) * g.nny + jj : pc;
+    const bool fwd = b >= 13;
+    const long ld = stencil_ld(g.nnod);
+    const T *__restrict__ Sb = a.S + 9 * ld * (fwd ? b - 13 : 13 - b) + (fwd ? pc : nb);
+    const long sr = fwd ? 3 * ld : ld, sc = fwd ? ld : 3 * ld;
+    T m[3][3], u[3];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            if (MODE != OP_MATVEC) fe[c] = a.F[dof + c];
-            if (MODE != OP_MATVEC && MODE != OP_DEFECT) ade[c] = a.AD[dof + c];
-            if (MODE == OP_JACOBI) ue[c] = a.U[dof + c];
-        }
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) m[r][c] = Sb[r * sr + c * sc];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) u[c] = stored_u<T, MODE>(a, 3 * nb + c);
+    // the finishing threads' operands (in bounds for every thread)
+    const int nd = threadIdx.x / 3, fc = threadIdx.x - 3 * nd;
+    const bool fin = nd < kStencilNodes && p0 + nd < g.nnod;
+    const long dof = fin ? 3 * p0 + threadIdx.x : 0;
+    unsigned msk = 0;
+    T fe = T(0), ade = T(1), ue = T(0);
+    if (threadIdx.x < 64) {
+        msk = a.mask[fin ? p0 + nd : 0] >> fc;
+        if (MODE != OP_MATVEC) fe = a.F[dof];
+        if (MODE != OP_MATVEC && MODE != OP_DEFECT) ade = a.AD[dof];
+        if (MODE == OP_JACOBI) ue = a.U[dof];
     }
-    T y0 = T(0), y1 = T(0), y2 = T(0);
-    if (live && ii >= 0 && ii < g.nnx) {
-        const bool go = w == 0   ? stencil_plane<0, T, MODE>(a, p, pc, j, k, pw, y0, y1, y2)
-                        : w == 1 ? stencil_plane<1, T, MODE>(a, p, pc, j, k, pw, y0, y1, y2)
-                                 : stencil_plane<2, T, MODE>(a, p, pc, j, k, pw, y0, y1, y2);
-        if (!go) return;
-    }
-    if (a.ctl && a.ctl[0]) return;
-    if (w != 1) {
-        red[w >> 1][0][lane] = y0;
-        red[w >> 1][1][lane] = y1;
-        red[w >> 1][2][lane] = y2;
+    if (a.ctl && a.ctl[0]) return;  // converged: nothing is written
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const T y = m[r][0] * u[0] + m[r][1] * u[1] + m[r][2] * u[2];
+        red[b][threadIdx.x & (kStencilNodes - 1)][r] = ok ? y : T(0);  // the spare threads repeat block 26
     }
     __syncthreads();
-    if (w != 1 || !live) return;
-    const T om = T(a.omega), one = T(1);
-    const T yv[3] = {y0, y1, y2};
+    if (!fin) return;
+    const T *rd = &red[0][0][0] + threadIdx.x;
+    T yp[3];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        const T yc = red[0][c][lane] + yv[c] + red[1][c][lane];
-        const bool fixed = (msk >> c) & 1u;
-        const T u = (MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT) ? T(a.prerelax) * fe[c] / ade[c] : ue[c];
-        if (MODE == OP_MATVEC) {
-            a.out[dof + c] = fixed ? T(0) : yc;
-        } else if (MODE == OP_DEFECT || MODE == OP_PRE_DEFECT) {
-            a.out[dof + c] = fixed ? T(0) : fe[c] - yc;
-            if (MODE == OP_PRE_DEFECT) a.out2[dof + c] = u;
-        } else {
-            const T rv = fixed ? T(0) : fe[c] - yc;
-            a.out[dof + c] = (one - om) * u + om * (rv + ade[c] * u) / ade[c];
-        }
+    for (int w = 0; w < 3; ++w) {
+        yp[w] = rd[27 * kStencilNodes * w];
+#pragma unroll
+        for (int q = 1; q < 9; ++q) yp[w] += rd[3 * kStencilNodes * (9 * w + q)];
+    }
+    const T yc = yp[0] + yp[1] + yp[2];
+    const T om = T(a.omega), one = T(1);
+    const bool fixed = msk & 1u;
+    const T uv = (MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT) ? T(a.prerelax) * fe / ade : ue;
+    if (MODE == OP_MATVEC) {
+        a.out[dof] = fixed ? T(0) : yc;
+    } else if (MODE == OP_DEFECT || MODE == OP_PRE_DEFECT) {
+        a.out[dof] = fixed ? T(0) : fe - yc;
+        if (MODE == OP_PRE_DEFECT) a.out2[dof] = uv;
+    } else {
+        const T rv = fixed ? T(0) : fe - yc;
+        a.out[dof] = (one - om) * uv + om * (rv + ade * uv) / ade;
     }
 }
 
@@ -619,7 +580,8 @@ void launch_opA(hipStream_t s, int mode, const OpArgsT<T> &a)
 {
     if (a.S && !a.partials) {
         // the stencil form (its launches carry no fused dot)
-        const dim3 sg((unsigned)((a.g.nnod + 63) / 64), 1, batch_dim(a.nb)), sb(192);
+        const long nblk = (a.g.nnod + kStencilNodes - 1) / kStencilNodes;
+        const dim3 sg((unsigned)xcd_launch(nblk), 1, batch_dim(a.nb)), sb(kStThreads);
         switch (mode) {
         case OP_MATVEC: k_stencil<T, OP_MATVEC><<<sg, sb, 0, s>>>(a); return;
         case OP_DEFECT: k_stencil<T, OP_DEFECT><<<sg, sb, 0, s>>>(a); return;
@@ -716,61 +678,74 @@ void launch_recip(hipStream_t s, const double *AD, double *RD, long n, int strid
 
 // ---------------------------------------------------------------------------
 // Restriction F_c = P^T R_f, F_c[fixed] = 0 (rstrFc + ZeroBCc,
-// mgcg1.cu:792-831): one thread per coarse node gathers the 27 fine nodes
-// around (2I,2J,2K) with weight 2^-(|di|+|dj|+|dk|).
+// mgcg1.cu:792-831): each coarse node gathers the 27 fine nodes around
+// (2I,2J,2K) with weight 2^-(|di|+|dj|+|dk|), one wave per 64 coarse nodes and
+// fine plane di; the three plane sums meet in LDS and are added in plane
+// order, and an XCD takes a contiguous range, whose fine planes are read twice.
+// (All 27 nodes in one thread: 81 scattered loads of up to 24 cache lines each
+// kept the few blocks of a small level busy: 4.2 us at 48x24x24 on average
+// over the levels, 3.0 now; 7.6 and 7.0 us at 192x96x96 in FP64.)
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ __launch_bounds__(kBlock) void k_restrict(Grid gc, const T *__restrict__ Rf, T *__restrict__ Fc,
-                                                    const uint8_t *__restrict__ maskc, const int *ctl)
+__global__ __launch_bounds__(192) void k_restrict(Grid gc, const T *__restrict__ Rf, T *__restrict__ Fc,
+                                                 const uint8_t *__restrict__ maskc, const int *ctl)
 {
     ctl = batch_ctl(ctl);
-    const long nod = (long)blockIdx.x * kBlock + threadIdx.x;
-    if (nod >= gc.nnod) return;
+    __shared__ T red[3][64][3];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned nblk = (unsigned)((gc.nnod + 63) / 64);
+    const long p0 = xcd_tile(blockIdx.x, nblk) * 64, p = p0 + lane, nod = p < gc.nnod ? p : 0;
+    if (p0 >= gc.nnod) return;  // padding block of the XCD order
     const unsigned nu = (unsigned)nod, q1 = nu / (unsigned)gc.nny;  // 32-bit: far fewer than 2^32 nodes
     const int J = (int)(nu - q1 * (unsigned)gc.nny);
     const int K = (int)(q1 % (unsigned)gc.nnz);
     const int I = (int)(q1 / (unsigned)gc.nnz);
     const int fny = 2 * gc.ny + 1, fnz = 2 * gc.nz + 1, fnx = 2 * gc.nx + 1;
-    const long fc = (long)fny * fnz * (2 * I) + (long)fny * (2 * K) + 2 * J;  // the fine node at (2I,2K,2J)
+    const int di = w - 1;
+    const bool plane = 2 * I + di >= 0 && 2 * I + di < fnx;
+    const long fc = (long)fny * fnz * (2 * I + di) + (long)fny * (2 * K) + 2 * J;  // the fine node (2I + di, 2K, 2J)
     Rf = batch_ptr(Rf, 3L * fnx * fny * fnz);
     Fc = batch_ptr(Fc, gc.ndof);
-    // all 27 fine nodes' loads are issued before the first product; nodes
+    // all 9 fine nodes' loads are issued before the first product; nodes
     // outside the mesh read node 0 with weight 0 (no branches around loads)
-    T v[27][3], w[27];
+    T v[9][3], wt[9];
 #pragma unroll
-    for (int di = -1; di <= 1; ++di)
+    for (int dk = -1; dk <= 1; ++dk)
 #pragma unroll
-        for (int dk = -1; dk <= 1; ++dk)
-#pragma unroll
-            for (int dj = -1; dj <= 1; ++dj) {
-                const int q = 9 * (di + 1) + 3 * (dk + 1) + (dj + 1);
-                const int iP = 2 * I + di, kP = 2 * K + dk, jP = 2 * J + dj;
-                const bool ok = iP >= 0 && iP < fnx && kP >= 0 && kP < fnz && jP >= 0 && jP < fny;
-                const long f = ok ? 3 * (fc + ((long)di * fny * fnz + dk * fny + dj)) : 0;
-                w[q] = ok ? T(1) / (T)(1 << (abs(di) + abs(dj) + abs(dk))) : T(0);
-                v[q][0] = Rf[f];
-                v[q][1] = Rf[f + 1];
-                v[q][2] = Rf[f + 2];
-            }
-    const unsigned m = maskc[nod];
+        for (int dj = -1; dj <= 1; ++dj) {
+            const int q = 3 * (dk + 1) + (dj + 1);
+            const int kP = 2 * K + dk, jP = 2 * J + dj;
+            const bool ok = plane && kP >= 0 && kP < fnz && jP >= 0 && jP < fny;
+            const long f = ok ? 3 * (fc + (dk * fny + dj)) : 0;
+            wt[q] = ok ? T(1) / (T)(1 << (abs(dj) + abs(dk))) : T(0);
+            v[q][0] = Rf[f];
+            v[q][1] = Rf[f + 1];
+            v[q][2] = Rf[f + 2];
+        }
+    // one thread per DOF finishes
+    const int nd = threadIdx.x / 3;
+    const bool fin = p0 + nd < gc.nnod;
+    const unsigned m = maskc[fin ? p0 + nd : 0] >> (threadIdx.x - 3 * nd);
     if (ctl && ctl[0]) return;  // read while the loads above are in flight
-    T s0 = T(0), s1 = T(0), s2 = T(0);
+    const T wi = w == 1 ? T(1) : T(0.5);
 #pragma unroll
-    for (int q = 0; q < 27; ++q) {
-        s0 += w[q] * v[q][0];
-        s1 += w[q] * v[q][1];
-        s2 += w[q] * v[q][2];
+    for (int c = 0; c < 3; ++c) {
+        T s = T(0);
+#pragma unroll
+        for (int q = 0; q < 9; ++q) s += wt[q] * v[q][c];
+        red[w][lane][c] = wi * s;
     }
-    Fc[3 * nod + 0] = (m & 1u) ? T(0) : s0;
-    Fc[3 * nod + 1] = (m & 2u) ? T(0) : s1;
-    Fc[3 * nod + 2] = (m & 4u) ? T(0) : s2;
+    __syncthreads();
+    if (!fin) return;
+    const T *rd = &red[0][0][0] + threadIdx.x;
+    const T s = rd[0] + rd[192] + rd[384];
+    Fc[3 * p0 + threadIdx.x] = (m & 1u) ? T(0) : s;
 }
 
 template <class T>
 void launch_restrict(hipStream_t s, const Grid &gc, const T *Rf, T *Fc, const uint8_t *maskc, const int *ctl, int nb)
 {
-    k_restrict<T><<<dim3((unsigned)((gc.nnod + kBlock - 1) / kBlock), 1, batch_dim(nb)), kBlock, 0, s>>>(gc, Rf, Fc,
-                                                                                                       maskc, ctl);
+    k_restrict<T><<<dim3((unsigned)xcd_launch((gc.nnod + 63) / 64), 1, batch_dim(nb)), 192, 0, s>>>(gc, Rf, Fc, maskc, ctl);
 }
 template void launch_restrict<double>(hipStream_t, const Grid &, const double *, double *, const uint8_t *, const int *,
                                       int);

@@ -43,7 +43,7 @@ void mixed_create(gputo_handle *h)
         v.RD = v.AD + g.ndof;
         v.Tmp = malloc_dev<float>(m, g.ndof);
         if (l > 0) {
-            if (h->L[l].S) v.S = m->S32[l] = malloc_dev<float>(m, (long)kStencilEntries * g.nnod);
+            if (h->L[l].S) v.S = m->S32[l] = malloc_dev<float>(m, (long)kStencilEntries * stencil_ld(g.nnod));
             v.CX = m->CXl32[l] = malloc_dev<float>(m, g.nel);
         }
     }
@@ -151,7 +151,7 @@ static void mixed_prepare(gputo_handle *h)
             // its FP64 factor), level 1 from its element matrices when the
             // handle was created without a stencil for it
             if (m->S32[l]) {
-                c.add(v.S, m->S32[l], (long)kStencilEntries * v.g.nnod);
+                c.add(v.S, m->S32[l], (long)kStencilEntries * stencil_ld(v.g.nnod));
             } else {
                 if (!m->A32) m->A32 = malloc_dev<float>(m, 300 * v.g.nel);
                 m->H.L[1].A = m->A32;

@@ -950,7 +950,7 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
                 v.CXl = dalloc<double>(h, v.g.nel);
                 // node stencils of the stored levels the V-cycle smooths
                 if (l < nl - 1 && !(l == 1 && use_l1_mf(h->prm, nl, v.mw64)))
-                    v.S = dalloc<double>(h, (long)kStencilEntries * v.g.nnod);
+                    v.S = dalloc<double>(h, (long)kStencilEntries * stencil_ld(v.g.nnod));
             }
         }
         const Grid &g0 = h->L[0].g;
