@@ -60,6 +60,7 @@ __device__ __forceinline__ long xcd_tile(long b, long ntiles)
 // offsets.
 constexpr int kMdMaxWaves = 8;
 struct ModalWork {
+    int flat = 0;  // one group of NW waves per element layer instead of a march
     int NW = 0, W = 0, R = 0, M = 0, TI = 0;
     int ns = 0, nch = 0, nib = 0;
     __host__ __device__ long blocks() const { return (long)ns * nch * nib; }

@@ -609,30 +609,209 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     }
 }
 
+// The level-1 operator on small meshes: one group of NW waves per element
+// layer, TI + 1 of them, where a march of TI + 1 layers takes as many layer
+// times (about 0.9 us each, the Gauss points of one element in one lane).
+// Group q owns element layer i0 - 1 + q and, from the second on, finishes the
+// node layer below it: its own share of row k stays in registers, its share of
+// row k + 1 and both of the group below's come through LDS, one barrier in all.
+// It holds one layer's modes (160-172 registers in FP64, 78-86 in FP32).
+// A sweep in the solve at 225 nodes FP64 4.9 -> 4.4 us, 4225 nodes 5.3 -> 4.6,
+// 15625 nodes of six right-hand sides (periodic) 15.5 -> 13.1, 30625 nodes FP32
+// 5.2 -> 4.7 us.  Level 0's layer is a third of that: no gain at any size.
+constexpr int kMdFlatWaves = 8;
+
+template <class T, int MODE, bool PER>
+__global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
+{
+    constexpr bool PRE = MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT;
+    constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI;
+    constexpr bool MV = MODE == OP_MATVEC;
+    constexpr int S = (int)sizeof(T);
+    batch_shift(a);
+    extern __shared__ double md_lds[];
+    const int ne = 63 * w.NW + 1;
+    const Grid &g = a.g;
+    const unsigned nb = (unsigned)w.blocks();
+    const unsigned tb = (unsigned)xcd_tile(blockIdx.x, nb);
+    if (tb >= nb) return;  // padding block of the XCD order
+    const int ch = (int)(tb % (unsigned)w.nch);
+    const unsigned r1 = tb / (unsigned)w.nch;
+    const int s = (int)(r1 % (unsigned)w.ns), i0 = (int)(r1 / (unsigned)w.ns) * w.TI;
+    const int i1 = min(i0 + w.TI, PER ? g.nx : g.nnx);  // owned node layers (PER: masters only)
+    if (PER && i0 >= i1) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = wave / w.NW, t = (wave - q * w.NW) * 63 + lane;
+    // [group][9][ne]: own share of row k + 1, of the layer above rows k, k + 1
+    T *ex = reinterpret_cast<T *>(md_lds) + 9 * q * ne + t;
+    // entry, element and own node as in k_modal
+    const unsigned qs = (unsigned)(ch * w.M + t + w.R - 1);
+    const int kq = (int)(qs / (unsigned)w.R), c = (int)(qs - (unsigned)(kq * w.R));
+    const int k = kq - 2, j = s * w.W - 1 + c;
+    const int ke = PER && k == -1 ? g.nz - 1 : k, je = PER && j == -1 ? g.ny - 1 : j;
+    const bool el_ok = ke >= 0 && ke < g.nz && je >= 0 && je < g.ny;
+    const bool own = lane > 0 && t > w.R && t <= w.R + w.M && c > 0 && k >= 0 && k < (PER ? g.nz : g.nnz) &&
+                     j < (PER ? g.ny : g.nny);
+    const int plane = g.nny * g.nnz, nod0 = k * g.nny + j, enod = ke * g.nny + je;
+    const int lo = el_ok ? 3 * S * enod : kMdOut, hi = el_ok ? 3 * S * (enod + g.nny) : kMdOut;
+    const int eo = el_ok ? S * (4 * ke * g.ny + 2 * je) : kMdOut, oo = own ? 3 * S * nod0 : kMdOut;
+    const long vb = (long)S * g.ndof;
+    const MdBuf BU = md_buf(PRE ? a.F : a.U, vb), BF = md_buf(a.F, MV ? 0 : vb);
+    const MdBuf BD = md_buf(a.RD, JAC || PRE ? vb : 0), BE = md_buf(CX, 8L * S * g.nel);
+    const MdBuf BM = md_buf(a.mask, a.mask ? g.nnod : 0);  // no mask: reads 0
+    const int fp = 3 * S * plane, ep = 4 * S * g.ny * g.nz;  // bytes of a node layer, of a layer of scales
+    const T pr = T(a.prerelax), om = T(a.omega);
+
+    const int il = i0 - 1 + q;  // the group's element layer, and the node layer below it
+    const int ie = PER && il < 0 ? g.nx - 1 : il;
+    const bool el = ie >= 0 && ie < g.nx && il < i1, emit = q > 0 && il < i1;
+    T u[4][6], d[4][6], e[8], f[3], de[3], ue[3];  // node rows: lower layer k, k + 1, upper layer k, k + 1
+    unsigned m8 = 0;
+    if (el) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int so = (p < 2 ? ie : il + 1) * fp;
+            md_ld6(BU, p & 1 ? hi : lo, so, u[p]);
+            if (PRE) md_ld6(BD, p & 1 ? hi : lo, so, d[p]);
+        }
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {  // children (is, iz): the pair along j
+            T v[2];
+            md_ld2(BE, eo + (p & 1) * 2 * S * g.ny, (2 * ie + (p >> 1)) * ep, v);
+            e[2 * p] = v[0];
+            e[2 * p + 1] = v[1];
+        }
+    }
+    if (emit) {
+        m8 = __builtin_amdgcn_raw_buffer_load_b8(BM, own ? nod0 : kMdOut, il * plane, 0);
+        if (!MV) md_ld3(BF, oo, il * fp, f);
+        if (JAC || PRE) md_ld3(BD, oo, il * fp, de);
+        if (!PRE && MODE != OP_DEFECT) md_ld3(BU, oo, il * fp, ue);
+    }
+    if (a.ctl && a.ctl[0]) return;  // converged: read with the loads above
+    T y[3] = {T(0), T(0), T(0)};
+    if (el) {
+        if (PRE) {
+#pragma unroll
+            for (int p = 0; p < 4; ++p)
+#pragma unroll
+                for (int x = 0; x < 6; ++x) u[p][x] = pr * (u[p][x] * d[p][x]);
+        }
+        Jk<T> pa, pb;
+        md_jk(u[0], u[1], pa);
+        md_jk(u[2], u[3], pb);
+        T m[3][2][2][2];
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    m[cc][0][b][x] = pa.v[cc][b][x] + pb.v[cc][b][x];
+                    m[cc][1][b][x] = pb.v[cc][b][x] - pa.v[cc][b][x];
+                }
+        const T cx[2][2][2] = {{{e[0], e[2]}, {e[1], e[3]}}, {{e[4], e[6]}, {e[5], e[7]}}};
+        md_element_gp(m, a.mc, cx);
+        // forces of one layer to its rows: v for row k, vh for row k + 1
+        auto rows = [&](const T (&s4)[2][2], T &v, T &vh) {
+            const T l0 = s4[0][0] - s4[0][1], l1 = s4[1][0] - s4[1][1];
+            const T h0 = s4[0][0] + s4[0][1], h1 = s4[1][0] + s4[1][1];
+            v = (l0 - l1) + md_below(l0 + l1);
+            vh = (h0 - h1) + md_below(h0 + h1);
+        };
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) {
+            T below[2][2], above[2][2], yh, z, zh;
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int x = 0; x < 2; ++x) {
+                    const T r1v = m[cc][1][b][x], r0v = b == 0 && x == 0 ? T(0) : m[cc][0][b][x];  // no force from a translation
+                    below[b][x] = r0v - r1v;
+                    above[b][x] = r0v + r1v;
+                }
+            rows(below, y[cc], yh);
+            rows(above, z, zh);
+            if (lane > 0) {
+                ex[cc * ne] = yh;
+                ex[(3 + cc) * ne] = z;
+                ex[(6 + cc) * ne] = zh;
+            }
+        }
+    }
+    __syncthreads();
+    if (!emit || !own) return;
+    const T *ey = ex - 9 * ne;  // the group below
+    const long dof = 3 * ((long)il * plane + nod0);
+#pragma unroll
+    for (int cc = 0; cc < 3; ++cc) {
+        T yc = y[cc];
+        if (el) yc += ex[cc * ne - w.R];
+        if (PER || il > 0) yc += ey[(3 + cc) * ne] + ey[(6 + cc) * ne - w.R];
+        const bool fixed = (m8 >> cc) & 1u;
+        T v;
+        if (MV) {
+            v = fixed ? T(0) : yc;
+        } else if (!JAC) {
+            v = fixed ? T(0) : f[cc] - yc;
+            if (PRE) a.out2[dof + cc] = pr * (f[cc] * de[cc]);
+        } else {
+            const T uo = PRE ? pr * (f[cc] * de[cc]) : ue[cc];
+            v = fma(om * de[cc], fixed ? T(0) : f[cc] - yc, uo);
+        }
+        a.out[dof + cc] = v;
+        if (PER) {
+            // the images: an iterate's value, 0 for a residual
+            const bool bi = il == 0, bk = k == 0, bj = j == 0;
+            if (bi || bk || bj) {
+                const T im = JAC ? v : T(0);
+                const long di = 3L * plane * g.nx, dk = 3L * g.nny * g.nz, dj = 3L * g.ny;
+#pragma unroll
+                for (int p = 1; p < 8; ++p)
+                    if ((!(p & 4) || bi) && (!(p & 2) || bk) && (!(p & 1) || bj))
+                        a.out[dof + cc + (p & 4 ? di : 0) + (p & 2 ? dk : 0) + (p & 1 ? dj : 0)] = im;
+            }
+        }
+    }
+}
+
+template <class T, class TU, int MODE, int EL, bool PER>
+void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX)
+{
+    const ModalWork &w = a.mw;
+    const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb));
+    const unsigned ne = 63u * w.NW + 1u;
+    if constexpr (EL == 1) {
+        if (w.flat && !a.partials) {
+            k_modal_flat<T, MODE, PER>
+                <<<grid, 64 * w.NW * (w.TI + 1), 9u * (w.TI + 1) * ne * sizeof(T), s>>>(a, w, CX);
+            return;
+        }
+    }
+    k_modal<T, TU, MODE, EL, PER><<<grid, 64 * w.NW, 6u * ne * sizeof(T), s>>>(a, w, CX);
+}
+
 template <class T, int EL>
 void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
 {
-    const ModalWork &w = a.mw;
-    const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb)), block(64 * w.NW);
-    const unsigned lds = 6u * (63u * w.NW + 1u) * sizeof(T);
     if (a.per) {
         switch (mode) {
-        case OP_MATVEC: k_modal<T, T, OP_MATVEC, EL, true><<<grid, block, lds, s>>>(a, w, CX); break;
-        case OP_DEFECT: k_modal<T, T, OP_DEFECT, EL, true><<<grid, block, lds, s>>>(a, w, CX); break;
-        case OP_JACOBI: k_modal<T, T, OP_JACOBI, EL, true><<<grid, block, lds, s>>>(a, w, CX); break;
+        case OP_MATVEC: launch_mode<T, T, OP_MATVEC, EL, true>(s, a, CX); break;
+        case OP_DEFECT: launch_mode<T, T, OP_DEFECT, EL, true>(s, a, CX); break;
+        case OP_JACOBI: launch_mode<T, T, OP_JACOBI, EL, true>(s, a, CX); break;
         default: throw std::runtime_error("periodic operator: mode");  // the prerelaxed modes read F on images
         }
         return;
     }
     switch (mode) {
-    case OP_MATVEC: k_modal<T, T, OP_MATVEC, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_DEFECT: k_modal<T, T, OP_DEFECT, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_JACOBI: k_modal<T, T, OP_JACOBI, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_PRE_JACOBI: k_modal<T, T, OP_PRE_JACOBI, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
-    case OP_PRE_DEFECT: k_modal<T, T, OP_PRE_DEFECT, EL, false><<<grid, block, lds, s>>>(a, w, CX); break;
+    case OP_MATVEC: launch_mode<T, T, OP_MATVEC, EL, false>(s, a, CX); break;
+    case OP_DEFECT: launch_mode<T, T, OP_DEFECT, EL, false>(s, a, CX); break;
+    case OP_JACOBI: launch_mode<T, T, OP_JACOBI, EL, false>(s, a, CX); break;
+    case OP_PRE_JACOBI: launch_mode<T, T, OP_PRE_JACOBI, EL, false>(s, a, CX); break;
+    case OP_PRE_DEFECT: launch_mode<T, T, OP_PRE_DEFECT, EL, false>(s, a, CX); break;
     case OP_MATVEC_UF:
         if constexpr (EL == 0 && std::is_same<T, double>::value)
-            k_modal<double, float, OP_MATVEC_UF, 0, false><<<grid, block, lds, s>>>(a, w, CX);
+            launch_mode<double, float, OP_MATVEC_UF, 0, false>(s, a, CX);
         break;
     default: break;
     }
@@ -752,6 +931,24 @@ ModalWork modal_work(const Grid &g, int bytes, int el, int children)
     ModalWork best;
     // 32-bit byte offsets
     if ((long)bytes * g.ndof >= kMdOut || (long)bytes * children * g.nel >= kMdOut) return best;
+    if (el) {
+        // k_modal_flat where one block per CU covers the mesh, with one wave
+        // per SIMD in FP64 (TI <= 3; two share its double rate: 7.2 against
+        // 7.2 us at 64x32x32 elements) and two in FP32 (4.8 against 5.4 us;
+        // beyond, with two blocks per CU, 9.5 against 8.7 us at 96x48x48), the
+        // fewest layers first: a block of two layers starts and ends sooner
+        for (int TI = 1; TI <= (bytes == 8 ? 3 : 7); ++TI)
+            for (int ns = 1; ns <= 8; ++ns) {
+                const int W = (g.nny + ns - 1) / ns, R = W + 1, M = std::min(63 - R, R * g.nnz);
+                if (M < 16 || (ns > 1 && W < 4)) continue;
+                const int nsr = (g.nny + W - 1) / W, nch = (R * g.nnz + M - 1) / M, nib = (g.nnx + TI - 1) / TI;
+                if ((long)nsr * nch * nib > 256) continue;
+                best.flat = 1;
+                best.NW = 1, best.W = W, best.R = R, best.M = M;
+                best.ns = nsr, best.nch = nch, best.TI = TI, best.nib = nib;
+                return best;
+            }
+    }
     const int waves = bytes == 8 ? (el ? 1 : 2) : (el ? 3 : 4);  // resident per SIMD (md_min_waves)
     const double per_wave = el ? 0.9 : 0.38;                     // a wave's layer with its SIMD alone, in us
     const double latency = 1.2;

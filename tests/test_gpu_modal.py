@@ -42,15 +42,14 @@ def references(Ku, u, f, ad, fx):
     return out
 
 
-@pytest.mark.parametrize("mesh", MESHES)
-def test_modal_operators_vs_oracle(gputo, oracle, mesh):
+def check_levels(gputo, oracle, mesh, levels):
     nelx, nely, nelz, nl = mesh
     print("case", mesh, flush=True)
     Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=61, kind="smooth")
     s = gputo.Solver(nelx, nely, nelz, nl, precision=1)
     s.setup(Ke, CX, fixed)
     rng = np.random.default_rng(62)
-    for level in range(1 if nl < 3 else 2):
+    for level in levels:
         if level == 0:
             ad, fx = oracle.prepad0(Ke, CX, nelx, nely, nelz), (fixed - 1).astype(np.int64)
 
@@ -70,6 +69,18 @@ def test_modal_operators_vs_oracle(gputo, oracle, mesh):
                 assert rel(y, ref[mode]) < tol, (level, mode, fp32, rel(y, ref[mode]))
                 assert np.array_equal(y, s.level_apply(level, 1 + level, mode, u, f, fp32=fp32))
     s.close()
+
+
+@pytest.mark.parametrize("mesh", MESHES)
+def test_modal_operators_vs_oracle(gputo, oracle, mesh):
+    check_levels(gputo, oracle, mesh, range(1 if mesh[3] < 3 else 2))
+
+
+@pytest.mark.parametrize("mesh", [(16, 8, 8, 3), (48, 48, 48, 4), (88, 40, 56, 4), (120, 56, 56, 4)])
+def test_level1_with_a_wave_group_per_layer(gputo, oracle, mesh):
+    """Level-1 grids whose blocks own one, two, three (a last block of fewer) and,
+    FP32 only, six node layers with a wave per element layer."""
+    check_levels(gputo, oracle, mesh, [1])
 
 
 @pytest.mark.parametrize("mesh", [(4, 6, 8, 2), (20, 68, 44, 3)])
