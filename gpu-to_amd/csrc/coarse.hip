@@ -458,17 +458,17 @@ void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, d
 }
 
 // ---------------------------------------------------------------------------
-// Order of the factored coarsest matrix.  A band matrix eliminated from one
-// end has no parallelism beyond one column block: its steps are a chain.  The
-// node planes i = const are therefore split at the middle plane a: part 1
+// Order of the factored coarsest matrix.  The steps of a band matrix eliminated
+// from one end are a chain.  The node planes i = const are therefore split at the middle plane a: part 1
 // holds planes 0 .. a-1 in order, part 2 planes nnx-1 .. a+1 in reverse, and
 // the separator, plane a, comes last.  Each part followed by the separator is
-// a band matrix of its own (the parts do not couple), so two workgroups
-// eliminate them at once, the chain is half as long, and the inverse of the
-// factor has a zero block between the parts.  Parts are padded to whole
+// a band matrix of its own (the parts do not couple), so both are eliminated at
+// once, the chain is half as long, and the inverse of the factor has a zero
+// block between the parts.  Parts are padded to whole
 // 32 x 32 tiles in front, the separator behind, with identity rows.
-// Factored at 13 x 7 x 7 nodes (1911 DOFs): 840 us as one band, 500 us split; at
-// 12 x 8 x 10 (2880 DOFs, band 269): 2200 us by tile-parallel launches, 1340 us.
+// The factorisation takes 295 us at 13 x 7 x 7 nodes (1911 DOFs; 840 in one
+// workgroup as one band) and 470 at 12 x 8 x 10 (2880; 2200 as one band by three
+// launches per block column).
 //
 // coarse_dof: the DOF of entry c of that order (-1: padding).  part_dof: of
 // row r of part q followed by the separator.
@@ -556,9 +556,9 @@ void launch_assemble(hipStream_t s, const Grid &g, const double *A, const uint8_
 }
 
 // ---------------------------------------------------------------------------
-// Blocked right-looking Cholesky A = L L^T on the N x N row-major matrix
-// (lower triangle used), NB = 32: factor the diagonal tile in LDS, solve
-// the panel below it, update the trailing lower triangle.
+// Blocked right-looking Cholesky A = L L^T on a row-major matrix (lower triangle
+// used), NB = 32: factor the diagonal tile, solve the panel below it, update the
+// trailing lower triangle.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ double readlane_f64(double v, int lane)
 {
@@ -569,7 +569,7 @@ __device__ __forceinline__ double readlane_f64(double v, int lane)
 }
 
 // Columns J0..J1-1 of the tile factorisation in one wave, lane r < NB
-// holding row r in L: at step jj the pivot comes from lane jj and each
+// holding row r in L (r >= NB: a row below the tile): at step jj the pivot comes from lane jj and each
 // multiplier L[c][jj] from lane c by v_readlane (scalar operands of the
 // updates), so no memory round trip is on the chain of pivots.  Only
 // columns below J1 are updated.  Entries right of the diagonal (c > r) take
@@ -606,91 +606,6 @@ __device__ __forceinline__ void wave_lds_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// One full wave factors the 32x32 diagonal tile at T in LDS (row stride
-// ld, lower triangle) in two halves of 16 columns.  The first half's
-// contribution to the second, T11 -= L10 L10^T (16x16, K = 16), runs as
-// four v_mfma_f64_16x16x4f64 with L10 staged in LDS (operand layout at
-// dgemm_tile64); the product is passed back through the tile's unused
-// upper-right block.  Returns true on a non-positive pivot.
-__device__ __forceinline__ bool potrf_tile(double *T, int ld)
-{
-    const int lane = threadIdx.x & 63;
-    const int r = lane < NB ? lane : NB - 1;  // lanes >= NB shadow row NB-1, results dropped
-    double L[NB];
-#pragma unroll
-    for (int c = 0; c < NB; ++c) L[c] = c <= r ? T[r * ld + c] : 0.0;
-    bool bad = false;
-    potrf_cols<0, 16>(L, r, bad);
-    if (lane < NB) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) T[r * ld + c] = L[c];
-    }
-    wave_lds_sync();
-    f64x4 d = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int kk = 0; kk < 16; kk += 4) {
-        const double a = T[(16 + (lane & 15)) * ld + kk + (lane >> 4)];  // A = B = L10
-        d = __builtin_amdgcn_mfma_f64_16x16x4f64(a, a, d, 0, 0, 0);
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) T[(4 * v + (lane >> 4)) * ld + 16 + (lane & 15)] = d[v];
-    wave_lds_sync();
-    if (r >= 16) {
-#pragma unroll
-        for (int c = 16; c < NB; ++c) L[c] -= T[(r - 16) * ld + c];
-    }
-    potrf_cols<16, NB>(L, r, bad);
-    wave_lds_sync();  // every lane has read the product before the tile is overwritten
-    if (lane < NB) {
-#pragma unroll
-        for (int c = 0; c < NB; ++c)
-            if (c <= r) T[r * ld + c] = L[c];
-    }
-    return bad;
-}
-
-__global__ __launch_bounds__(64) void k_potrf_diag(double *A, int N, int k0, int *flag)
-{
-    __shared__ double T[NB][NB + 1];
-    for (int q = threadIdx.x; q < NB * NB; q += 64) T[q / NB][q % NB] = A[(long)(k0 + q / NB) * N + k0 + q % NB];
-    __syncthreads();
-    const bool bad = potrf_tile(&T[0][0], NB + 1);
-    __syncthreads();
-    for (int q = threadIdx.x; q < NB * NB; q += 64)
-        if (q % NB <= q / NB) A[(long)(k0 + q / NB) * N + k0 + q % NB] = T[q / NB][q % NB];
-    if (bad && threadIdx.x == 0) flag[0] = 1;
-}
-
-
-// Panel rows solve x L^T = p: x[jj] = (p[jj] - sum_{m<jj} x[m] L[jj][m]) rd[jj]
-// with rd[jj] = 1/L[jj][jj] computed once per tile.
-__global__ __launch_bounds__(256) void k_trsm_panel(double *A, int N, int k0, int rows)
-{
-    __shared__ double L[NB][NB + 1];
-    __shared__ double rd[NB];
-    for (int q = threadIdx.x; q < NB * NB; q += 256) {
-        const int r = q / NB, c = q % NB;
-        L[r][c] = c <= r ? A[(long)(k0 + r) * N + k0 + c] : 0.0;
-    }
-    __syncthreads();
-    if (threadIdx.x < NB) rd[threadIdx.x] = 1.0 / L[threadIdx.x][threadIdx.x];
-    __syncthreads();
-    const long row = (long)k0 + NB + (long)blockIdx.x * 256 + threadIdx.x;
-    if (row >= (long)k0 + NB + rows) return;
-    double x[NB];
-#pragma unroll
-    for (int c = 0; c < NB; ++c) x[c] = A[row * N + k0 + c];
-#pragma unroll
-    for (int jj = 0; jj < NB; ++jj) {
-        double s = x[jj];
-#pragma unroll
-        for (int m = 0; m < jj; ++m) s -= x[m] * L[jj][m];
-        x[jj] = s * rd[jj];
-    }
-#pragma unroll
-    for (int c = 0; c < NB; ++c) A[row * N + k0 + c] = x[c];
-}
-
 __device__ __forceinline__ void tri_index(int b, int &ti, int &tj)
 {
     // b-th tile of a lower-triangular tile set: (ti, tj) with tj <= ti
@@ -699,38 +614,6 @@ __device__ __forceinline__ void tri_index(int b, int &ti, int &tj)
     while (t * (t + 1) / 2 > b) --t;
     ti = t;
     tj = b - t * (t + 1) / 2;
-}
-
-// the same for the few tiles of a band step, by integer steps (the index is
-// wave-uniform, so this runs on the scalar unit)
-__device__ __forceinline__ void tri_index_small(int b, int &ti, int &tj)
-{
-    int t = 0;
-    while ((t + 1) * (t + 2) / 2 <= b) ++t;
-    ti = t;
-    tj = b - t * (t + 1) / 2;
-}
-
-__global__ __launch_bounds__(256) void k_syrk_update(double *A, int N, int k0)
-{
-    __shared__ double Pi[NB][NB + 1], Pj[NB][NB + 1];
-    int ti, tj;
-    tri_index(blockIdx.x, ti, tj);
-    const int base = k0 + NB;
-    const int r0 = base + ti * NB, c0 = base + tj * NB;
-    for (int q = threadIdx.x; q < NB * NB; q += 256) {
-        const int r = q / NB, c = q % NB;
-        Pi[r][c] = A[(long)(r0 + r) * N + k0 + c];
-        Pj[r][c] = A[(long)(c0 + r) * N + k0 + c];
-    }
-    __syncthreads();
-    for (int q = threadIdx.x; q < NB * NB; q += 256) {
-        const int r = q / NB, c = q % NB;
-        double s = 0.0;
-#pragma unroll
-        for (int m = 0; m < NB; ++m) s += Pi[r][m] * Pj[c][m];
-        A[(long)(r0 + r) * N + c0 + c] -= s;
-    }
 }
 
 // Inverse of each 32x32 diagonal factor tile, written into Linv (one block
@@ -772,36 +655,6 @@ __global__ void k_transpose(const double *__restrict__ In, double *__restrict__ 
     for (int q = threadIdx.x; q < NB * NB; q += blockDim.x) Out[(long)(bj + q / NB) * N + bi + q % NB] = T[q % NB][q / NB];
 }
 
-// ---------------------------------------------------------------------------
-// The same factorisation in one workgroup when the band spans at most
-// kBandRowsMax rows below the diagonal tile (the coarsest grids of the
-// usual hierarchies), with a look-ahead.  At step k block column k (the
-// diagonal tile and the panel below it) sits in LDS, its tile already
-// updated by the earlier steps:
-//   A. wave 0 factors the tile while waves off its SIMD apply step k-1's
-//      update to the trailing band (in global memory) and to the panel rows
-//      of column k (in LDS);
-//   B. one thread per panel row solves the panel in two halves of 16
-//      columns while the other waves load block column k+1 and store the
-//      factored tile;
-//   C. panel k is stored, and the diagonal tile of column k+1 receives step
-//      k's update, so it is ready for step k+1's factorisation.
-// Every entry receives the updates of the steps in increasing order, as in
-// the tile-parallel kernels.  The trailing products run on
-// v_mfma_f64_16x16x4f64 in 16x16 blocks (operand layout at dgemm_tile64).
-// Blocks above the diagonal of a diagonal tile are never read and are not
-// updated, and blocks whose panel rows lie past the band are exact zeros
-// and are skipped: panel row x of a step (counted from the row below its
-// tile) is zero for x >= bw.
-// ---------------------------------------------------------------------------
-// The separator split (coarse_dof) runs it on both parts at once, stopping
-// after the parts' own columns: what is pending is then applied to the
-// separator's block, which a second launch adds up and factors.
-constexpr int kBandRowsMax = 272;  // LDS: two buffers of 304 x 33 doubles
-constexpr int kCholThreads = 512;  // 2 waves per SIMD: 256 VGPRs for a panel row
-constexpr int kCholWaves = kCholThreads / 64;
-constexpr int kCholRows = NB + kBandRowsMax;  // rows of a block column in LDS
-
 // sum_m P[ra + i][m] P[rb + j][m] for a 16x16 block, D layout of the MFMA;
 // every operand is read from LDS before the chain starts, so the matrix
 // core does not wait on each pair of reads
@@ -820,289 +673,116 @@ __device__ __forceinline__ f64x4 panel_product(const double (*P)[NB + 1], int ra
     return d;
 }
 
-// two blocks at once: independent accumulation chains overlap on the
-// matrix core
-__device__ __forceinline__ void panel_product2(const double (*P)[NB + 1], int ra0, int rb0, int ra1, int rb1, int lane,
-                                               f64x4 &d0, f64x4 &d1)
-{
-    const int i = lane & 15, k = lane >> 4;
-    double fa0[NB / 4], fb0[NB / 4], fa1[NB / 4], fb1[NB / 4];
-#pragma unroll
-    for (int s = 0; s < NB / 4; ++s) {
-        fa0[s] = P[ra0 + i][4 * s + k];
-        fb0[s] = P[rb0 + i][4 * s + k];
-        fa1[s] = P[ra1 + i][4 * s + k];
-        fb1[s] = P[rb1 + i][4 * s + k];
-    }
-    d0 = f64x4{0.0, 0.0, 0.0, 0.0};
-    d1 = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int s = 0; s < NB / 4; ++s) {
-        d0 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa0[s], fb0[s], d0, 0, 0, 0);
-        d1 = __builtin_amdgcn_mfma_f64_16x16x4f64(fa1[s], fb1[s], d1, 0, 0, 0);
-    }
-}
-
-// Columns J0..J1-1 of one panel row's substitution x L^T = p (x[m] receives
-// its updates in the same order as in k_trsm_panel), updating columns below
-// J1 only; Lr: row c of the factored tile in lane c.
-template <int J0, int J1>
-__device__ __forceinline__ void trsm_cols(double (&x)[NB], const double (&Lr)[NB], const double *rdg)
-{
-#pragma unroll
-    for (int jj = J0; jj < J1; ++jj) {
-        x[jj] *= rdg[jj];
-        // column jj of the tile is read out once x[jj] is final: otherwise
-        // the compiler hoists every readlane and spills them
-        double lcol = Lr[jj];
-        asm volatile("" : "+v"(lcol) : "v"(x[jj]));
-#pragma unroll
-        for (int m = jj + 1; m < J1; ++m) x[m] -= x[jj] * readlane_f64(lcol, m);
-    }
-}
-
-// rows x NB entries of the matrix at G (row stride N) into LDS, kLoads
-// loads in flight per thread; thread t0 of nt
-constexpr int kLoads = 24;
-__device__ __forceinline__ void load_column(double (*D)[NB + 1], const double *G, long N, int rows, int t0, int nt)
-{
-    const int n = rows * NB;
-    for (int q0 = t0; q0 < n; q0 += kLoads * nt) {
-        double v[kLoads];
-#pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const int q = q0 + u * nt;
-            v[u] = q < n ? G[(long)(q / NB) * N + q % NB] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kLoads; ++u) {
-            const int q = q0 + u * nt;
-            if (q < n) D[q / NB][q % NB] = v[u];
-        }
-    }
-}
-
-// Step k-1's update of global 16x16 blocks (R, C) of the trailing band, R
-// and C counted in 16-row blocks from row k0 + NB: A -= P_R P_C^T with P
-// the panel of step k-1 in LDS (row NB + 16 R for block row R).  Items
-// i0, i0 + stride, ... < items, mapped to blocks by MAP: 0 the blocks of
-// tile column k+1 (C < 2), 1 those right of it (2 <= C <= R).  All loads
-// of a batch are issued before its first store (the memory counter also
-// waits for earlier stores).
-template <int MAP>
-__device__ __forceinline__ void rest_blocks(double *A, long N, long k0, const double (*P)[NB + 1], int lane, int items,
-                                            int i0, int stride)
-{
-    constexpr int kBatch = 6;
-    const long lo = (long)(lane >> 4) * N + (lane & 15);  // the lane's entry of a block
-    for (int w0 = i0; w0 < items; w0 += kBatch * stride) {
-        double old[kBatch][4];
-        long go[kBatch];  // uniform: the block's first entry
-        int ra[kBatch], rb[kBatch];
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-            const int w = w0 + b * stride;
-            if (w < items) {
-                int R, C;
-                if (MAP == 0) {  // slot 2R + C, slot 1 (above the diagonal) skipped
-                    const int sl = w + (w >= 1);
-                    R = sl >> 1;
-                    C = sl & 1;
-                } else {
-                    tri_index_small(w, R, C);
-                    R += 2;
-                    C += 2;
-                }
-                ra[b] = NB + 16 * R;
-                rb[b] = NB + 16 * C;
-                go[b] = (k0 + ra[b]) * N + k0 + rb[b];
-#pragma unroll
-                for (int v = 0; v < 4; ++v) old[b][v] = A[go[b] + lo + 4L * v * N];
-            }
-        }
-        // every product of the batch first, then the stores: a store before
-        // a product would make the next operand waits wait for it too
-        f64x4 d[kBatch];
-#pragma unroll
-        for (int b = 0; b < kBatch; b += 2) {
-            if (w0 + (b + 1) * stride < items)
-                panel_product2(P, NB + ra[b], NB + rb[b], NB + ra[b + 1], NB + rb[b + 1], lane, d[b], d[b + 1]);
-            else if (w0 + b * stride < items)
-                d[b] = panel_product(P, NB + ra[b], NB + rb[b], lane);
-        }
-#pragma unroll
-        for (int b = 0; b < kBatch; ++b) {
-            if (w0 + b * stride < items) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v) A[go[b] + lo + 4L * v * N] = old[b][v] - d[b][v];
-            }
-        }
-    }
-}
-
-// Step k's update of the column buffer D (the next block column, row q of D
-// = panel row q of P's step): the 16x16 blocks in slots sl = 2R + C, C < 2,
-// sl = s0, s0 + stride, ... < s1, slot 1 (above the diagonal) excluded
-__device__ __forceinline__ void column_blocks(double (*D)[NB + 1], const double (*P)[NB + 1], int lane, int s0, int s1,
-                                              int stride)
-{
-    for (int sl = s0; sl < s1; sl += 2 * stride) {
-        const int t0 = sl, t1 = sl + stride;
-        const int ra0 = (t0 >> 1) * 16, rb0 = (t0 & 1) * 16, ra1 = (t1 >> 1) * 16, rb1 = (t1 & 1) * 16;
-        if (t1 < s1) {
-            f64x4 d0, d1;
-            panel_product2(P, NB + ra0, NB + rb0, NB + ra1, NB + rb1, lane, d0, d1);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                D[ra0 + 4 * v + (lane >> 4)][rb0 + (lane & 15)] -= d0[v];
-                D[ra1 + 4 * v + (lane >> 4)][rb1 + (lane & 15)] -= d1[v];
-            }
-        } else {
-            const f64x4 d = panel_product(P, NB + ra0, NB + rb0, lane);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) D[ra0 + 4 * v + (lane >> 4)][rb0 + (lane & 15)] -= d[v];
-        }
-    }
-}
-
-// block b factors the first `steps` block columns of a.A[b] (order n, row
-// stride ld)
-struct CholArgs {
-    double *A[2];
+// ---------------------------------------------------------------------------
+// Cholesky A = L L^T of the lower band, one launch per block column of 32 (a
+// step).  Every workgroup owns one 32x32 tile (ti, tj) of the trailing band and
+// does all it needs for it: it factors the step's diagonal tile, solves the two
+// panel tiles of its rows and columns and subtracts their product.  The
+// repeated work costs nothing (the CUs would idle), and nothing waits for
+// another workgroup.  The factor goes to its own matrix, since other workgroups
+// of the launch still read the panel as it was.  A step takes 8.8 us, of which
+// the launch 2.7, the loads 1 and the chain of 32 pivots 2, whatever the band:
+// in one workgroup with a look-ahead (the FP64 rate of one CU, barriers) it
+// took 7 us at a band of 65 rows, 13 at 173 and 25 at 269, with three launches
+// per step (tile, panel, update) 25 us.
+// ---------------------------------------------------------------------------
+struct CholStep {
+    double *A[2], *L[2];
     long ld[2];
     int n[2], steps[2];
-    int band_rows, bw;
+    int nt;  // tiles of the band below the diagonal tile
     int *flag;
 };
 
-__global__ __launch_bounds__(kCholThreads) void k_chol_band(CholArgs a)
+__global__ __launch_bounds__(256) void k_chol_step(CholStep a, int k)
 {
-    __shared__ double buf[2][kCholRows][NB + 1];
-    __shared__ double rdg[NB];  // 1/L[jj][jj] of the current tile
-    double *A = a.A[blockIdx.x];
-    const long ld = a.ld[blockIdx.x];
-    const int N = a.n[blockIdx.x], nb = N / NB, steps = a.steps[blockIdx.x];
-    const int band_rows = a.band_rows, bw = a.bw;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    bool bad = false;
-    load_column(buf[0], A, ld, min(N, NB + band_rows), tid, kCholThreads);  // block column 0 as assembled
+    __shared__ double W[4 * NB][NB + 1];  // the diagonal tile and a panel tile, for wave 0 and for wave 1
+    const int q = blockIdx.y;
+    if (k >= a.steps[q]) return;
+    const long ld = a.ld[q], k0 = (long)k * NB;
+    const int nt = min(a.nt, a.n[q] / NB - k - 1);
+    int ti, tj;
+    tri_index(blockIdx.x, ti, tj);
+    const bool tile = ti < nt;
+    if (!tile && blockIdx.x > 0) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const double *Ak = a.A[q] + k0 * ld + k0;
+    const long ri = (long)(ti + 1) * NB, rj = (long)(tj + 1) * NB;
+    // this wave's quadrant of the tile, in the MFMA's result layout
+    double *Tq = a.A[q] + (k0 + ri + 16 * (wave >> 1) + (lane >> 4)) * ld + k0 + rj + 16 * (wave & 1) + (lane & 15);
+    double d[4], pi[4] = {}, pj[4] = {}, old[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        d[u] = Ak[r * ld + c];
+        if (tile) {
+            pi[u] = Ak[(ri + r) * ld + c];
+            pj[u] = Ak[(rj + r) * ld + c];
+            old[u] = Tq[4 * u * ld];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        W[r][c] = d[u];
+        W[NB + r][c] = pi[u];
+        W[2 * NB + r][c] = d[u];
+        W[3 * NB + r][c] = pj[u];
+    }
     __syncthreads();
-    for (int k = 0; k < steps; ++k) {
-        double(*Cur)[NB + 1] = buf[k & 1];
-        double(*Oth)[NB + 1] = buf[(k + 1) & 1];  // panel k-1 in phase A, block column k+1 from phase B on
-        const long k0 = (long)k * NB;
-        const int rows = min(N - (int)k0 - NB, band_rows);   // panel rows of step k
-        const int prows = k > 0 ? min(N - (int)k0, band_rows) : 0;  // panel rows of step k-1 (from row k0)
-        const int rc = prows > NB ? min((prows - NB) / 16, max(0, (bw - NB + 15) / 16)) : 0;  // rest block rows
-        // A. factor the tile | step k-1's update of the trailing band in
-        // global memory and of column k's panel rows in LDS (slots from 4:
-        // below the diagonal tile), by the waves off the factoring wave's
-        // SIMD (waves w and w + 4 share a SIMD)
-        if (wave == 0) {
-            bad |= potrf_tile(&Cur[0][0], NB + 1);
-            if (lane < NB) rdg[lane] = 1.0 / Cur[lane][lane];
-        } else if (wave != 4 && k > 0) {
-            const int aw = wave - 1 - (wave > 4);  // 0..5
-            if (rc > 0) rest_blocks<0>(A, ld, k0, Oth, lane, 2 * rc - 1, aw, kCholWaves - 2);
-            if (rc > 2) rest_blocks<1>(A, ld, k0, Oth, lane, (rc - 2) * (rc - 1) / 2, aw, kCholWaves - 2);
-            column_blocks(Cur, Oth, lane, 4 + aw, 2 * (min(prows, bw + 15) / 16), kCholWaves - 2);
-        }
-        __syncthreads();
-        // B. panel solve, one row per thread, in two halves of 16 columns
-        // (column-oriented substitution; lane c of each wave holds row c of
-        // the factored tile, whose entries reach the other lanes by
-        // v_readlane) | the other waves load block column k+1 into x (it
-        // reaches LDS after the second half, so the loads stay in flight
-        // meanwhile) and store the tile (after the loads, which would
-        // otherwise wait for the stores).  Between the halves, P[:, 16:32]
-        // -= P[:, 0:16] L[16:32, 0:16]^T on the matrix cores.
-        const int tw = (rows + 63) & ~63;  // threads of the waves with panel rows
-        double Lr[NB], x[NB];
-        if (tid < tw) {
-            const int lr = lane < NB ? lane : NB - 1;
+    if (wave < 2) {
+        // lane r < NB holds row r of the diagonal tile, the others a row of the
+        // panel tile: the column operations that factor the one solve the other
+        // (x L^T = p).  In two halves of 16 columns, the second updated by the
+        // first on the matrix cores.
+        double(*V)[NB + 1] = W + 2 * NB * wave;
+        double L[NB];
+        bool bad = false;
+        const int r = lane < NB ? lane : 2 * NB;  // below every column
 #pragma unroll
-            for (int c = 0; c < NB; ++c) Lr[c] = Cur[lr][c];
+        for (int c = 0; c < NB; ++c) L[c] = c <= r ? V[lane][c] : 0.0;
+        potrf_cols<0, 16>(L, r, bad);
+        wave_lds_sync();  // every lane has read its row
 #pragma unroll
-            for (int c = 0; c < 16; ++c) x[c] = Cur[min(NB + tid, kCholRows - 1)][c];  // rows past the panel: stale, not stored
-            trsm_cols<0, 16>(x, Lr, rdg);
-            if (tid < rows) {
+        for (int c = 0; c < 16; ++c) V[lane][c] = L[c];
+        wave_lds_sync();
+        f64x4 v[3];
 #pragma unroll
-                for (int c = 0; c < 16; ++c) Cur[NB + tid][c] = x[c];
-            }
-        } else {
-            const int t0 = tid - tw, nt = kCholThreads - tw;
-            const int n = k + 1 < nb ? min(N - (int)k0 - NB, NB + band_rows) * NB : 0;
-            const double *G = A + (k0 + NB) * ld + k0 + NB;
-#pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                const int q = t0 + u * nt;
-                x[u] = q < n ? G[(long)(q / NB) * ld + q % NB] : 0.0;
-            }
-            for (int q = t0; q < NB * NB; q += nt) {
-                const int r = q / NB, c = q % NB;
-                if (c <= r) A[(k0 + r) * ld + k0 + c] = Cur[r][c];
-            }
-        }
-        __syncthreads();
-        for (int w = wave; w < min(rows, bw + 15) / 16; w += kCholWaves) {  // panel rows past the band are zero
-            f64x4 d = {0.0, 0.0, 0.0, 0.0};
+        for (int rb = 0; rb < 3; ++rb) {
+            v[rb] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int kk = 0; kk < 16; kk += 4)
-                d = __builtin_amdgcn_mfma_f64_16x16x4f64(Cur[NB + 16 * w + (lane & 15)][kk + (lane >> 4)],
-                                                         Cur[16 + (lane & 15)][kk + (lane >> 4)], d, 0, 0, 0);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) Cur[NB + 16 * w + 4 * v + (lane >> 4)][16 + (lane & 15)] -= d[v];
+                v[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(V[16 * (rb + 1) + (lane & 15)][kk + (lane >> 4)],
+                                                             V[16 + (lane & 15)][kk + (lane >> 4)], v[rb], 0, 0, 0);
         }
-        __syncthreads();
-        if (tid < tw) {
 #pragma unroll
-            for (int c = 16; c < NB; ++c) x[c] = Cur[min(NB + tid, kCholRows - 1)][c];
-            trsm_cols<16, NB>(x, Lr, rdg);
-            if (tid < rows) {
+        for (int rb = 0; rb < 3; ++rb)
 #pragma unroll
-                for (int c = 16; c < NB; ++c) Cur[NB + tid][c] = x[c];
-            }
-        } else {
-            const int t0 = tid - tw, nt = kCholThreads - tw;
-            const int n = k + 1 < nb ? min(N - (int)k0 - NB, NB + band_rows) * NB : 0;
+            for (int u = 0; u < 4; ++u) V[16 * (rb + 1) + 4 * u + (lane >> 4)][16 + (lane & 15)] = v[rb][u];
+        wave_lds_sync();
+        if (lane >= 16) {
 #pragma unroll
-            for (int u = 0; u < NB; ++u) {
-                const int q = t0 + u * nt;
-                if (q < n) Oth[q / NB][q % NB] = x[u];
-            }
-            load_column(Oth, A + (k0 + NB) * ld + k0 + NB, ld, n / NB, t0 + NB * nt, nt);  // the rest, if any
+            for (int c = 16; c < NB; ++c) L[c] -= V[lane][c];
         }
-        __syncthreads();
-        // C. store panel k; the diagonal tile of column k+1 -= panel k's
-        // first tile x its transpose (slots 0, 2, 3)
-        for (int q = tid; q < rows * NB; q += kCholThreads) A[(k0 + NB + q / NB) * ld + k0 + q % NB] = Cur[NB + q / NB][q % NB];
-        if (k + 1 < nb && wave < 3) {
-            const int sl = wave == 0 ? 0 : wave + 1;
-            const int ra = (sl >> 1) * 16, rb = (sl & 1) * 16;
-            const f64x4 d = panel_product(Cur, NB + ra, NB + rb, lane);
+        potrf_cols<16, NB>(L, r, bad);
+        wave_lds_sync();
 #pragma unroll
-            for (int v = 0; v < 4; ++v) Oth[ra + 4 * v + (lane >> 4)][rb + (lane & 15)] -= d[v];
-        }
-        __syncthreads();
+        for (int c = 16; c < NB; ++c) V[lane][c] = L[c];
+        if (bad && blockIdx.x == 0 && tid == 0) a.flag[0] = 1;
     }
-    if (steps < nb) {
-        // what the last step leaves pending: the trailing band and the panel
-        // rows of block column `steps` (in LDS, its diagonal tile is current)
-        double(*P)[NB + 1] = buf[(steps - 1) & 1];
-        double(*D)[NB + 1] = buf[steps & 1];
-        const long k0 = (long)steps * NB;
-        const int prows = min(N - (int)k0, band_rows);
-        const int rc = prows > NB ? min((prows - NB) / 16, max(0, (bw - NB + 15) / 16)) : 0;
-        if (rc > 0) rest_blocks<0>(A, ld, k0, P, lane, 2 * rc - 1, wave, kCholWaves);
-        if (rc > 2) rest_blocks<1>(A, ld, k0, P, lane, (rc - 2) * (rc - 1) / 2, wave, kCholWaves);
-        column_blocks(D, P, lane, 4 + wave, 2 * (min(prows, bw + 15) / 16), kCholWaves);
-        __syncthreads();
-        const int rows = min(N - (int)k0, NB + band_rows);
-        for (int q = tid; q < rows * NB; q += kCholThreads)
-            A[(k0 + q / NB) * ld + k0 + q % NB] = D[q / NB][q % NB];
+    __syncthreads();
+    if (tile) {
+        const f64x4 v = panel_product(W, NB + 16 * (wave >> 1), 3 * NB + 16 * (wave & 1), lane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) Tq[4 * u * ld] = old[u] - v[u];
     }
-    if (bad && tid == 0) a.flag[0] = 1;
+    if (tj > 0) return;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        if (blockIdx.x == 0 && c <= r) a.L[q][(k0 + r) * ld + k0 + c] = W[r][c];
+        if (tile) a.L[q][(k0 + ri + r) * ld + k0 + c] = W[NB + r][c];
+    }
 }
 
 // row blockIdx.x of the lower triangle: A += B (the two parts' updates of the
@@ -1260,8 +940,8 @@ static void launch_linv_levels(hipStream_t s, const CoarseBlocks &B, double *Li,
     }
 }
 
-// The split pays from about ten tile steps on (each saved step is 10-14 us,
-// the separator's launches cost about 20 us) and needs two planes per part.
+// The split saves 2 of 5 steps of 8.8 us at 5x3x3 nodes already (the sum of the
+// updates costs 4.7); it needs two planes per part.
 void coarse_layout(Coarse &C, const Grid &g, bool periodic)
 {
     CoarseMap &m = C.map;
@@ -1272,7 +952,7 @@ void coarse_layout(Coarse &C, const Grid &g, bool periodic)
     auto up = [](int v) { return (v + NB - 1) / NB * NB; };
     const int N1 = up(C.n);
     m.o2 = m.os = m.N = N1;
-    if (periodic || C.bw > kBandRowsMax || g.nnx < 5 || N1 / NB < 10) return;
+    if (periodic || g.nnx < 5 || N1 / NB < 4) return;
     m.a = g.nnx / 2;
     const int p1 = m.a * m.p, p2 = (g.nnx - 1 - m.a) * m.p;
     m.o2 = up(p1);
@@ -1295,13 +975,27 @@ CoarseParts coarse_parts(const Coarse &C)
         P.A[1] = C.AQ + (long)P.n[0] * P.n[0];
         P.n[1] = m.os - m.o2 + m.ps;
     }
+    // the factor goes to matrices of its own behind these
+    const long half = (long)P.n[0] * P.n[0] + (long)P.n[1] * P.n[1];
+    for (int q = 0; q < P.np; ++q) P.L[q] = P.A[q] + half;
     return P;
 }
 
 long coarse_matrix_len(const Coarse &C)
 {
     const CoarseParts P = coarse_parts(C);
-    return (long)P.n[0] * P.n[0] + (long)P.n[1] * P.n[1];
+    return 2 * ((long)P.n[0] * P.n[0] + (long)P.n[1] * P.n[1]);
+}
+
+static void launch_chol_steps(hipStream_t s, const CholStep &a, int np)
+{
+    const int steps = std::max(a.steps[0], np > 1 ? a.steps[1] : 0);
+    for (int k = 0; k < steps; ++k) {
+        int nt = 0;
+        for (int q = 0; q < np; ++q)
+            if (k < a.steps[q]) nt = std::max(nt, std::min(a.nt, a.n[q] / NB - k - 1));
+        k_chol_step<<<dim3((unsigned)std::max(1, nt * (nt + 1) / 2), (unsigned)np), 256, 0, s>>>(a, k);
+    }
 }
 
 void coarse_factor(hipStream_t s0, Coarse &C, bool lag)
@@ -1310,7 +1004,7 @@ void coarse_factor(hipStream_t s0, Coarse &C, bool lag)
     C.solve_waits = C.target == C.cur;
     C.Linv = C.Lbuf[C.cur];
     C.LinvT = C.LTbuf[C.cur];
-    const int N = C.map.N, nb = N / NB, ps = C.map.ps;
+    const int N = C.map.N, ps = C.map.ps;
     // the factor of a banded matrix keeps its band: panel rows and trailing
     // tiles beyond it are exact zeros and are skipped
     const int bw = std::max(1, std::min(C.bw, N));
@@ -1318,40 +1012,26 @@ void coarse_factor(hipStream_t s0, Coarse &C, bool lag)
     HIPCHK(hipEventRecord(C.ev_in, s0));
     HIPCHK(hipStreamWaitEvent(s, C.ev_in, 0));
     HIPCHK(hipMemsetAsync(C.flag, 0, sizeof(int), s));
-    if (bw <= kBandRowsMax) {
-        const CoarseParts P = coarse_parts(C);
-        CholArgs a{};
-        a.band_rows = (bw + 15) / 16 * 16;
-        a.bw = bw;
-        a.flag = C.flag;
-        for (int q = 0; q < P.np; ++q) {
-            a.A[q] = P.A[q];
-            a.ld[q] = a.n[q] = P.n[q];
-            a.steps[q] = (P.n[q] - ps) / NB;
-        }
-        k_chol_band<<<P.np, kCholThreads, 0, s>>>(a);
-        if (ps) {
-            const int l0 = P.n[0] - ps, l1 = P.n[1] - ps;
-            a.A[0] = P.A[0] + (long)l0 * P.n[0] + l0;
-            a.n[0] = ps;
-            a.steps[0] = ps / NB;
-            k_add_lower<<<ps, 256, 0, s>>>(ps, P.A[1] + (long)l1 * P.n[1] + l1, P.n[1], a.A[0], P.n[0]);
-            a.band_rows = std::max(ps - NB, 16);  // dense
-            a.bw = ps;
-            k_chol_band<<<1, kCholThreads, 0, s>>>(a);
-        }
-    } else {
-        const int band_rows = (bw + NB - 1) / NB * NB;
-        for (int kb = 0; kb < nb; ++kb) {
-            const int k0 = kb * NB;
-            k_potrf_diag<<<1, 64, 0, s>>>(C.AQ, N, k0, C.flag);
-            const int rows = std::min(N - k0 - NB, band_rows);
-            if (rows > 0) {
-                k_trsm_panel<<<(rows + 255) / 256, 256, 0, s>>>(C.AQ, N, k0, rows);
-                const int nt = rows / NB;
-                k_syrk_update<<<nt * (nt + 1) / 2, 256, 0, s>>>(C.AQ, N, k0);
-            }
-        }
+    const CoarseParts P = coarse_parts(C);
+    CholStep a{};
+    a.flag = C.flag;
+    for (int q = 0; q < P.np; ++q) {
+        a.A[q] = P.A[q];
+        a.L[q] = P.L[q];
+        a.ld[q] = a.n[q] = P.n[q];
+        a.steps[q] = (P.n[q] - ps) / NB;
+    }
+    a.nt = (bw + NB - 1) / NB;
+    launch_chol_steps(s, a, P.np);
+    if (ps) {
+        const long l0 = P.n[0] - ps, l1 = P.n[1] - ps;
+        a.A[0] += l0 * (P.n[0] + 1);
+        a.L[0] += l0 * (P.n[0] + 1);
+        k_add_lower<<<ps, 256, 0, s>>>(ps, P.A[1] + l1 * (P.n[1] + 1), P.n[1], a.A[0], P.n[0]);
+        a.n[0] = ps;
+        a.steps[0] = ps / NB;
+        a.nt = ps / NB;  // dense
+        launch_chol_steps(s, a, 1);
     }
     HIPCHK(hipGetLastError());
     // the inverse's launches are enqueued by coarse_finish, when the host
@@ -1374,14 +1054,14 @@ void coarse_finish(const Coarse &C)
     CoarseBlocks B{};
     B.nblk = m.ps ? 3 : 1;
     B.off[0] = 0;
-    B.L[0] = P.A[0];
+    B.L[0] = P.L[0];
     B.ld[0] = P.n[0];
     B.off[1] = m.ps ? m.o2 : N;
     if (m.ps) {
-        B.L[1] = P.A[1];
+        B.L[1] = P.L[1];
         B.ld[1] = P.n[1];
         B.off[2] = m.os;
-        B.L[2] = P.A[0] + (long)m.o2 * P.n[0] + m.o2;
+        B.L[2] = P.L[0] + (long)m.o2 * P.n[0] + m.o2;
         B.ld[2] = P.n[0];
         B.off[3] = N;
     }

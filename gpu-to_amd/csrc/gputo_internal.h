@@ -184,7 +184,7 @@ struct CoarseMap {
 // stride = order), and the diagonal blocks of the whole factor
 struct CoarseParts {
     int np;
-    double *A[2];
+    double *A[2], *L[2];  // L: where the factor is
     int n[2];
 };
 struct CoarseBlocks {
@@ -198,7 +198,7 @@ struct Coarse {
     CoarseMap map;
     bool direct = true;      // factored (else smoothed: mgcg9 above 20000 DOFs)
     int bw = 0;              // lower bandwidth of the assembled matrix (node-major DOFs)
-    double *AQ = nullptr;       // dense matrix (matrices of the parts), then the Cholesky factor (lower)
+    double *AQ = nullptr;       // dense matrix (matrices of the parts, updated by the factorisation), then their factors
     double *Linv = nullptr;     // inverse of the factor used by the solves (lower, row-major)
     double *LinvT = nullptr;    // its transpose (row-major)
     double *Lbuf[2] = {}, *LTbuf[2] = {};  // two inverse buffers (lagged factorisation)

@@ -983,6 +983,8 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
         const long N = C.map.N;
         if (dense_ok) {
             C.AQ = dalloc<double>(h, coarse_matrix_len(C));
+            // entries outside the band are never written and stay 0 in the factor
+            launch_fill<double>(h->stream, C.AQ, coarse_matrix_len(C), 0.0);
             for (int b = 0; b < 2; ++b) {
                 C.Lbuf[b] = dalloc<double>(h, N * N);
                 C.LTbuf[b] = dalloc<double>(h, N * N);

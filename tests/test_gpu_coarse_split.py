@@ -1,13 +1,13 @@
-"""The coarsest solve where the factorisation is split at the middle plane
-(band of at most 272 rows, at least ten 32-row tiles, five planes), against
-numpy's dense solve of the assembled matrix.
+"""The coarsest solve, whose factorisation is split at the middle plane from five
+planes and four 32-row tiles on, against numpy's dense solve of the assembled
+matrix.
 
-Coarsest grids (nodes): 7x7x3 (parts of 189 DOFs in 192 rows), 8x5x5
-(parts of four and three planes), 5x5x5 (two
-planes to a part), 17x4x5 (many steps), 9x9x9 (band 275: not split) and, with
-the decoupled fixed DOFs of the mgcg9 engine, 12x8x10 (band 269, the widest
-that is split).  Tolerance as for the unsplit solve: the conditioning of the
-penalised matrix (1e-9)."""
+Coarsest grids (nodes): 7x7x3 (parts of 189 DOFs in 192 rows), 8x5x5 (parts of
+four and three planes), 5x5x5 (two planes to a part), 17x4x5 (many steps),
+9x9x9 (band 275), 5x3x3 (five tiles), 5x2x2 and 3x3x3 (too few rows to split),
+4x9x9 (too few planes, wide band) and, with the decoupled fixed DOFs of the
+mgcg9 engine, 12x8x10 and 8x5x5.  Tolerance as for the other coarsest solves:
+the conditioning of the penalised matrix (1e-9)."""
 import numpy as np
 import pytest
 
@@ -20,7 +20,8 @@ def rel(a, b):
     return np.abs(a - b).max() / max(np.abs(b).max(), 1e-300)
 
 
-@pytest.mark.parametrize("coarse", [(6, 6, 2), (7, 4, 4), (4, 4, 4), (16, 3, 4), (8, 8, 8)])
+@pytest.mark.parametrize("coarse", [(6, 6, 2), (7, 4, 4), (4, 4, 4), (16, 3, 4), (8, 8, 8), (4, 2, 2), (4, 1, 1),
+                                    (2, 2, 2), (3, 8, 8)])
 def test_split_coarse_solve(gputo, oracle, coarse):
     cx, cy, cz = coarse
     nelx, nely, nelz = 2 * cx, 2 * cy, 2 * cz
