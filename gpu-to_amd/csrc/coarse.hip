@@ -203,7 +203,7 @@ void launch_coarse_galerkin(hipStream_t s, const Grid &gc, const double *Af, dou
 // as the child-by-child product, summed in a different order.
 // ---------------------------------------------------------------------------
 // The product on the matrix cores: D[p][e] = sum_f T[f][p] CX0[fine(e, f)]
-// as v_mfma_f64_16x16x4f64 tiles (operand layout at dgemm_tile64), p (the
+// as v_mfma_f64_16x16x4f64 tiles (operand layout at dgemm_tile32), p (the
 // packed entry) along the rows and e along the columns, so the stores of a
 // tile row are contiguous in A (p-major).  One wave per 32 x 32 tile of
 // (p, e), four waves per workgroup; the operands come straight from L2 (the
@@ -616,39 +616,74 @@ __device__ __forceinline__ void tri_index(int b, int &ti, int &tj)
     tj = b - t * (t + 1) / 2;
 }
 
-// Inverse of each 32x32 diagonal factor tile, written into Linv (one block
-// per tile of the whole order).
+// Inverse of each 32x32 diagonal factor tile, written into Linv (one wave per
+// tile of the whole order): lane c < 32 solves column c of the inverse of its
+// 16x16 half, then X10 = -X11 L10 X00 on the matrix cores.  (32 rows in turn
+// with a division each: 14 us; 7 us.)
 __global__ __launch_bounds__(64) void k_trtri_diag(CoarseBlocks B, double *Linv, int N)
 {
-    __shared__ double L[NB][NB + 1];
-    const int k0 = blockIdx.x * NB;
+    __shared__ double L[NB][NB + 1], X[NB][NB + 1], P[16][17], rd[NB];
+    const int k0 = blockIdx.x * NB, lane = threadIdx.x;
     int q = 0;
     while (q + 1 < B.nblk && k0 >= B.off[q + 1]) ++q;
     const double *A = B.L[q];
     const long ld = B.ld[q];
     const int l0 = k0 - B.off[q];
-    for (int t = threadIdx.x; t < NB * NB; t += 64) {
-        const int r = t / NB, c = t % NB;
-        L[r][c] = c <= r ? A[(l0 + r) * ld + l0 + c] : 0.0;
+    double v[NB * NB / 64];
+#pragma unroll
+    for (int u = 0; u < NB * NB / 64; ++u) {
+        const int r = (lane + 64 * u) / NB, c = lane % NB;
+        v[u] = c <= r ? A[(l0 + r) * ld + l0 + c] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < NB * NB / 64; ++u) {
+        const int r = (lane + 64 * u) / NB, c = lane % NB;
+        L[r][c] = v[u];
+        X[r][c] = 0.0;
+        if (r == c) rd[r] = 1.0 / v[u];
     }
     __syncthreads();
-    const int col = threadIdx.x;
-    if (col >= NB) return;
-    double x[NB];
+    if (lane < NB) {
+        const int h = lane & 16, col = lane & 15;
+        double x[16];
 #pragma unroll
-    for (int r = 0; r < NB; ++r) {
-        double t = (r == col) ? 1.0 : 0.0;
+        for (int r = 0; r < 16; ++r) {
+            double t = r == col ? 1.0 : 0.0;
 #pragma unroll
-        for (int m = 0; m < r; ++m) t -= L[r][m] * x[m];
-        x[r] = (r < col) ? 0.0 : t / L[r][r];
+            for (int m = 0; m < r; ++m) t -= L[h + r][h + m] * x[m];
+            x[r] = r < col ? 0.0 : t * rd[h + r];
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) X[h + r][lane] = x[r];
     }
+    __syncthreads();
+    const int i = lane & 15, kq = lane >> 4;
+    f64x4 d = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int r = 0; r < NB; ++r) Linv[(long)(k0 + r) * N + k0 + col] = x[r];
+    for (int kk = 0; kk < 16; kk += 4)  // L10 X00
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(L[16 + i][kk + kq], X[kk + kq][i], d, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) P[4 * u + kq][i] = d[u];
+    __syncthreads();
+    d = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int kk = 0; kk < 16; kk += 4)
+        d = __builtin_amdgcn_mfma_f64_16x16x4f64(X[16 + i][16 + kk + kq], P[kk + kq][i], d, 0, 0, 0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) X[16 + 4 * u + kq][i] = -d[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NB * NB / 64; ++u) {
+        const int r = (lane + 64 * u) / NB, c = lane % NB;
+        Linv[(long)(k0 + r) * N + k0 + c] = X[r][c];
+    }
 }
 
+// of the tiles on and below the diagonal: the others are neither written nor read
 __global__ void k_transpose(const double *__restrict__ In, double *__restrict__ Out, int N)
 {
     __shared__ double T[NB][NB + 1];
+    if (blockIdx.x > blockIdx.y) return;
     const int bi = blockIdx.y * NB, bj = blockIdx.x * NB;
     for (int q = threadIdx.x; q < NB * NB; q += blockDim.x) T[q / NB][q % NB] = In[(long)(bi + q / NB) * N + bj + q % NB];
     __syncthreads();
@@ -814,70 +849,79 @@ struct LinvLevel {
     long wstride;    // doubles of W per group
 };
 
-// One 64x64 tile of C = alpha A B, with A (M x K), B (K x Nc) and C
-// row-major (leading dimensions lda, ldb, ldc), M, Nc and K multiples of 32.
-// Four waves, each a 32x32 quadrant as 2 x 2 v_mfma_f64_16x16x4f64 tiles;
-// the operand layout of that instruction: A[i][k] in lane i + 16k, B[k][j]
-// in lane j + 16k, D[4v + q][j] in element v of lane j + 16q.
-__device__ __forceinline__ void dgemm_tile64(const double *__restrict__ A, long lda, const double *__restrict__ B,
-                                             long ldb, double *__restrict__ C, long ldc, int M, int Nc, int K,
+// A 32x32 tile of C = alpha A B over K columns of A (a multiple of 32), all
+// row-major, 16-byte aligned rows: i0, j0 its first row and column.  The four
+// waves take a quarter of K each, as 2 x 2 v_mfma_f64_16x16x4f64 tiles, and meet
+// in LDS.  Operands go straight from memory into registers, one batch of eight
+// columns ahead: a lane of group g = lane / 16 holds columns 2g and 2g + 1 of
+// the eight (one 16-byte load of A; the order of a sum's terms is free as long
+// as both operands use the same).  Operand layout of that instruction: A[i][k]
+// in lane i + 16k, B[k][j] in lane j + 16k, D[4v + q][j] in element v of lane
+// j + 16q.  (64x64 tiles staged through LDS 32 columns at a time had few
+// workgroups, two barriers and a round trip per 32 columns: a launch took 12 us
+// at 1911 DOFs, 5.1 now; 15 to 30 with the whole of K in one wave.)
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void dgemm_tile32(const double *__restrict__ A, long lda, const double *__restrict__ B,
+                                             long ldb, double *__restrict__ C, long ldc, int i0, int j0, int K,
                                              double alpha)
 {
-    __shared__ double As[64][33];
-    __shared__ double Bs[32][65];
-    const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64;
-    if (i0 >= M || j0 >= Nc) return;  // whole workgroup
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int wr = w >> 1, wc = w & 1;
-    f64x4 d[2][2];
+    __shared__ double red[4][NB][NB + 1];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = lane & 15;
+    const int steps = K / 32;  // of 8 columns, per wave
+    const int k0 = w * (K / 4) + 2 * (lane >> 4);
+    const double *a0 = A + (long)(i0 + i) * lda + k0, *a1 = a0 + 16 * lda;
+    const double *b0 = B + (long)k0 * ldb + j0 + i;
+    f64x4 d[2][2] = {};
+    struct Ops {
+        f64x2 a[2];
+        double b[2][2];
+    } x, y;
+    auto load = [&](int s, Ops &o) {
+        o.a[0] = *reinterpret_cast<const f64x2 *>(a0 + 8 * s);
+        o.a[1] = *reinterpret_cast<const f64x2 *>(a1 + 8 * s);
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) d[a][b] = f64x4{0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        // rows past M (A) and columns past Nc (B) read as zeros
-        double av[8], bv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int r = (tid >> 5) + 8 * u, c = tid & 31;
-            av[u] = i0 + r < M ? A[(long)(i0 + r) * lda + k0 + c] : 0.0;
+        for (int e = 0; e < 2; ++e) {
+            o.b[e][0] = b0[(8 * s + e) * ldb];
+            o.b[e][1] = b0[(8 * s + e) * ldb + 16];
         }
+    };
+    auto multiply = [&](const Ops &o) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int r = (tid >> 6) + 4 * u, c = tid & 63;
-            bv[u] = j0 + c < Nc ? B[(long)(k0 + r) * ldb + j0 + c] : 0.0;
-        }
-        __syncthreads();  // the previous step's readers are done
+        for (int e = 0; e < 2; ++e)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) As[(tid >> 5) + 8 * u][tid & 31] = av[u];
+            for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) Bs[(tid >> 6) + 4 * u][tid & 63] = bv[u];
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 32; kk += 4) {
-            double fa[2], fb[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) fa[a] = As[wr * 32 + a * 16 + (lane & 15)][kk + (lane >> 4)];
-#pragma unroll
-            for (int b = 0; b < 2; ++b) fb[b] = Bs[kk + (lane >> 4)][wc * 32 + b * 16 + (lane & 15)];
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) d[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[a], fb[b], d[a][b], 0, 0, 0);
-        }
+                for (int q = 0; q < 2; ++q)
+                    d[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[p][e], o.b[e][q], d[p][q], 0, 0, 0);
+    };
+    load(0, x);
+    int s = 0;
+    for (; s + 2 < steps; s += 2) {
+        load(s + 1, y);
+        multiply(x);
+        load(s + 2, x);
+        multiply(y);
     }
-    const int qi = i0 + wr * 32, qj = j0 + wc * 32;
-    if (qi >= M || qj >= Nc) return;
+    if (s + 1 < steps) load(s + 1, y);
+    multiply(x);
+    if (s + 1 < steps) multiply(y);
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int p = 0; p < 2; ++p)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
-            for (int v = 0; v < 4; ++v)
-                C[(long)(qi + a * 16 + 4 * v + (lane >> 4)) * ldc + qj + b * 16 + (lane & 15)] = alpha * d[a][b][v];
+            for (int v = 0; v < 4; ++v) red[w][16 * p + 4 * v + (lane >> 4)][16 * q + i] = d[p][q][v];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        C[(long)(i0 + r) * ldc + j0 + c] = alpha * ((red[0][r][c] + red[1][r][c]) + (red[2][r][c] + red[3][r][c]));
+    }
 }
 
-// blockIdx.z: diagonal block x group
+// blockIdx.z: diagonal block x group.  Tiles above the diagonal of X are
+// neither read nor written.
 template <int STEP>
 __global__ __launch_bounds__(256) void k_linv_level(CoarseBlocks B, double *Li, double *W, int N, LinvLevel lv)
 {
@@ -886,17 +930,21 @@ __global__ __launch_bounds__(256) void k_linv_level(CoarseBlocks B, double *Li, 
     if (h >= nb) return;
     const int n2 = min(lv.g, nb - s) - n1;
     const int r = min(lv.nbt, n2), c = min(lv.nbt, n1);
+    const int ti = blockIdx.y, tj = blockIdx.x;
+    if (ti >= (STEP == 0 ? r : n2)) return;
     const double *L = B.L[q];
     const long ldl = B.ld[q];
     double *X = Li + (long)B.off[q] * N + B.off[q];
     double *Wz = W + blockIdx.z * lv.wstride;
     const long ldw = (long)n1 * NB;
-    if (STEP == 0)  // W = L21[0:r, n1-c:n1] X11[n1-c:n1, 0:n1]
-        dgemm_tile64(L + (long)h * NB * ldl + (long)(h - c) * NB, ldl, X + (long)(h - c) * NB * N + (long)s * NB, N, Wz,
-                     ldw, r * NB, n1 * NB, c * NB, 1.0);
-    else  // X21 = -X22[0:n2, 0:r] W
-        dgemm_tile64(X + (long)h * NB * N + (long)h * NB, N, Wz, ldw, X + (long)h * NB * N + (long)s * NB, N, n2 * NB,
-                     n1 * NB, r * NB, -1.0);
+    if (STEP == 0) {  // W = L21[0:r, n1-c:n1] X11[n1-c:n1, 0:n1], rows of X11 from tile tj on
+        const int k = max(n1 - c, tj);
+        dgemm_tile32(L + (long)h * NB * ldl + (long)(s + k) * NB, ldl, X + (long)(s + k) * NB * N + (long)s * NB,
+                             N, Wz, ldw, ti * NB, tj * NB, (n1 - k) * NB, 1.0);
+    } else {  // X21 = -X22[0:n2, 0:r] W, columns of X22 up to tile ti
+        dgemm_tile32(X + (long)h * NB * N + (long)h * NB, N, Wz, ldw, X + (long)h * NB * N + (long)s * NB, N,
+                             ti * NB, tj * NB, min(r, ti + 1) * NB, -1.0);
+    }
 }
 
 // The separator's rows of the inverse, blockIdx.z = part q: W = X_q L_qq^-1
@@ -906,17 +954,21 @@ template <int STEP>
 __global__ __launch_bounds__(256) void k_linv_sep(CoarseBlocks B, double *Li, double *W, int N, int nbt)
 {
     const int q = blockIdx.z, o = B.off[q], nq = B.off[q + 1] - o, os = B.off[2], ps = B.off[3] - os;
-    const int c = min(nbt, nq / NB) * NB;
+    const int ti = blockIdx.y, tj = blockIdx.x;
+    if (tj * NB >= nq) return;
     double *Wz = W + (long)q * ps * N;
-    if (STEP == 0)
-        dgemm_tile64(B.L[q] + (long)nq * B.ld[q] + nq - c, B.ld[q], Li + (long)(o + nq - c) * N + o, N, Wz, nq, ps, nq, c,
-                     1.0);
-    else
-        dgemm_tile64(Li + (long)os * N + os, N, Wz, nq, Li + (long)os * N + o, N, ps, nq, ps, -1.0);
+    if (STEP == 0) {
+        const int k = max(nq / NB - nbt, tj) * NB;
+        dgemm_tile32(B.L[q] + (long)nq * B.ld[q] + k, B.ld[q], Li + (long)(o + k) * N + o, N, Wz, nq, ti * NB,
+                             tj * NB, nq - k, 1.0);
+    } else {
+        dgemm_tile32(Li + (long)os * N + os, N, Wz, nq, Li + (long)os * N + o, N, ti * NB, tj * NB,
+                             (ti + 1) * NB, -1.0);
+    }
 }
 
 // Levels 2, 4, ... of the halving on every diagonal block at once; Li holds
-// the diagonal tile inverses and zeros above them, W has room for wcap doubles.
+// the diagonal tile inverses, W has room for wcap doubles.
 static void launch_linv_levels(hipStream_t s, const CoarseBlocks &B, double *Li, double *W, long wcap, int N, int nbt)
 {
     int nb = 0;
@@ -927,14 +979,14 @@ static void launch_linv_levels(hipStream_t s, const CoarseBlocks &B, double *Li,
         const int rmax = std::min(nbt, n1);
         const LinvLevel lv{g, nbt, groups, (long)rmax * NB * n1 * NB};
         if (lv.wstride * groups * B.nblk > wcap) throw std::runtime_error("coarsest inverse: work buffer too small");
-        const unsigned tn = (unsigned)((n1 * NB + 63) / 64), tz = (unsigned)(groups * B.nblk);
-        k_linv_level<0><<<dim3(tn, (unsigned)((rmax * NB + 63) / 64), tz), 256, 0, s>>>(B, Li, W, N, lv);
+        const unsigned tn = (unsigned)n1, tz = (unsigned)(groups * B.nblk);
+        k_linv_level<0><<<dim3(tn, (unsigned)rmax, tz), 256, 0, s>>>(B, Li, W, N, lv);
         k_linv_level<1><<<dim3(tn, tn, tz), 256, 0, s>>>(B, Li, W, N, lv);
     }
     if (B.nblk == 3) {
         const int ps = B.off[3] - B.off[2], nq = std::max(B.off[1], B.off[2] - B.off[1]);
         if (2L * ps * N > wcap) throw std::runtime_error("coarsest inverse: work buffer too small");
-        const dim3 grid((unsigned)((nq + 63) / 64), (unsigned)((ps + 63) / 64), 2);
+        const dim3 grid((unsigned)(nq / NB), (unsigned)(ps / NB), 2);
         k_linv_sep<0><<<grid, 256, 0, s>>>(B, Li, W, N, nbt);
         k_linv_sep<1><<<grid, 256, 0, s>>>(B, Li, W, N, nbt);
     }
@@ -1065,7 +1117,6 @@ void coarse_finish(const Coarse &C)
         B.ld[2] = P.n[0];
         B.off[3] = N;
     }
-    launch_fill(s, Li, (long)N * N, 0.0);
     k_trtri_diag<<<nb, 64, 0, s>>>(B, Li, N);
     // the transpose's buffer is free until the last step: it holds W
     launch_linv_levels(s, B, Li, LiT, (long)N * N, N, (bw + 2 * NB - 2) / NB);
