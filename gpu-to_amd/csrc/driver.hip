@@ -15,17 +15,21 @@
 
 using namespace gputo;
 
+namespace {
+struct OcState;
+}
+
 // The device buffers of a design loop.  The loop's state is new with each
 // gputo_to_begin; its buffers stay with the handle from one loop to the next
 // (their sizes are the mesh's) and are freed with it: freeing and allocating
 // 270 MB took 4.5 ms per restart at 192x96x96.
 struct ToBuffers {
     double *x = nullptr, *xPhys = nullptr, *xOld = nullptr, *Hs = nullptr, *dHs = nullptr, *dsK = nullptr;
-    double *dc = nullptr, *dv = nullptr, *tmp = nullptr, *ocP = nullptr, *CX = nullptr, *F = nullptr, *U = nullptr;
+    double *dc = nullptr, *dv = nullptr, *tmp = nullptr, *ocP = nullptr, *F = nullptr, *U = nullptr;
     double *w = nullptr;     // filter weights
     double *part = nullptr;  // reduction partials [32][kRedBlocks]
-    double *red = nullptr;   // finalised sums [32]
-    double *red_host = nullptr;
+    OcState *oc = nullptr;  // the bisection's state
+    double *red_host = nullptr;    // pinned: sums and the bisection's result (kSum...)
     int *fixed_d = nullptr;
     size_t nfixed = 0;       // room in fixed_d
     std::vector<void *> allocs;
@@ -45,6 +49,8 @@ namespace {
 
 constexpr int kMaxFilterWeights = 15 * 15 * 15;  // rmin <= 8: half width at most 7
 constexpr int kCand = 31;  // OC candidates per pass: a depth-5 bisection tree
+// words of red_host: eta sums; change and volume; compliance; the bisection's done and lmid
+enum { kSumEta = 0, kSumPhys = 2, kSumComp = 4, kSumOc = 5, kSumCount = 8 };
 
 template <class T>
 T *talloc(ToBuffers *t, size_t n)
@@ -74,28 +80,82 @@ __device__ __forceinline__ double wsum256(double v)
 }
 
 // imfilter(in, h, 'symmetric') on the (nely, nelz, nelx) array = element
-// order (top3D125mod.m:96,108,140-141); optional pre-division by `div`.
-__global__ __launch_bounds__(256) void k_filter(Grid g, const double *__restrict__ in, const double *__restrict__ div,
-                                               const double *__restrict__ w, int fw, double *__restrict__ out)
+// order (top3D125mod.m:96,108,140-141), divided by `div` where given.  FW > 0:
+// the half width, and the loads of a plane dx (FW = 1: of all three) are in
+// flight together; with a loop over the neighbours each waited for its weight
+// and its value: 38 us at 192x96x96 and FW = 1, 26 now (9.4 and 4.2 us at
+// 48x24x24).  FW = 0: any half width fw.  Field 0 or 1 by blockIdx.y.
+struct FilterField {
+    const double *in, *div;
+    double *out;
+};
+
+template <int FW>
+__global__ __launch_bounds__(256) void k_filter(Grid g, FilterField f0, FilterField f1, const double *__restrict__ w,
+                                               int fw)
 {
     const long e = (long)blockIdx.x * 256 + threadIdx.x;
     if (e >= g.nel) return;
-    const int j = (int)(e % g.ny), k = (int)((e / g.ny) % g.nz), i = (int)(e / ((long)g.ny * g.nz));
+    const FilterField f = blockIdx.y ? f1 : f0;
+    const double *__restrict__ in = f.in;
+    const unsigned eu = (unsigned)e, q1 = eu / (unsigned)g.ny;  // far fewer than 2^32 elements
+    const int j = (int)(eu - q1 * (unsigned)g.ny), k = (int)(q1 % (unsigned)g.nz), i = (int)(q1 / (unsigned)g.nz);
     double acc = 0.0;
-    int q = 0;
-    for (int dx = -fw; dx <= fw; ++dx) {
-        const int ii = mirror_idx(i + dx, g.nx);
-        for (int dz = -fw; dz <= fw; ++dz) {
-            const int kk = mirror_idx(k + dz, g.nz);
-            for (int dy = -fw; dy <= fw; ++dy, ++q) {
-                const double wq = w[q];
-                if (wq == 0.0) continue;
-                const long f = (long)g.ny * g.nz * ii + (long)g.ny * kk + mirror_idx(j + dy, g.ny);
-                acc += wq * (div ? in[f] / div[f] : in[f]);
+    if constexpr (FW > 0) {
+        constexpr int D = 2 * FW + 1, P = FW == 1 ? 3 : 1;  // planes loaded together
+        int jj[D];
+#pragma unroll
+        for (int y = 0; y < D; ++y) jj[y] = mirror_idx(j + y - FW, g.ny);
+        for (int x0 = 0; x0 < D; x0 += P) {
+            double v[P][D][D];
+#pragma unroll
+            for (int x = 0; x < P; ++x) {
+                const long pi = (long)g.ny * g.nz * mirror_idx(i + x0 + x - FW, g.nx);
+#pragma unroll
+                for (int z = 0; z < D; ++z) {
+                    const long pk = pi + (long)g.ny * mirror_idx(k + z - FW, g.nz);
+#pragma unroll
+                    for (int y = 0; y < D; ++y) v[x][z][y] = in[pk + jj[y]];
+                }
+            }
+#pragma unroll
+            for (int x = 0; x < P; ++x)
+#pragma unroll
+                for (int z = 0; z < D; ++z)
+#pragma unroll
+                    for (int y = 0; y < D; ++y) {
+                        const double wq = w[((x0 + x) * D + z) * D + y];
+                        if (wq != 0.0) acc += wq * v[x][z][y];
+                    }
+        }
+    } else {
+        int q = 0;
+        for (int dx = -fw; dx <= fw; ++dx) {
+            const int ii = mirror_idx(i + dx, g.nx);
+            for (int dz = -fw; dz <= fw; ++dz) {
+                const int kk = mirror_idx(k + dz, g.nz);
+                for (int dy = -fw; dy <= fw; ++dy, ++q) {
+                    const double wq = w[q];
+                    if (wq == 0.0) continue;
+                    acc += wq * in[(long)g.ny * g.nz * ii + (long)g.ny * kk + mirror_idx(j + dy, g.ny)];
+                }
             }
         }
     }
-    out[e] = acc;
+    f.out[e] = f.div ? acc / f.div[e] : acc;
+}
+
+// nf = 1 or 2 fields
+void launch_filter(hipStream_t s, const Grid &g, int nf, const FilterField &f0, const FilterField &f1, const double *w,
+                   int fw)
+{
+    const dim3 grid((unsigned)((g.nel + 255) / 256), (unsigned)nf);
+    switch (fw) {
+    case 1: k_filter<1><<<grid, 256, 0, s>>>(g, f0, f1, w, fw); break;
+    case 2: k_filter<2><<<grid, 256, 0, s>>>(g, f0, f1, w, fw); break;
+    case 3: k_filter<3><<<grid, 256, 0, s>>>(g, f0, f1, w, fw); break;
+    default: k_filter<0><<<grid, 256, 0, s>>>(g, f0, f1, w, fw); break;
+    }
 }
 
 __device__ __forceinline__ double prj_d(double v, double eta, double beta)
@@ -111,13 +171,6 @@ __device__ __forceinline__ double dprj_d(double v, double eta, double beta)
 {
     const double t = tanh(beta * (v - eta));
     return beta * (1 - t * t) / (tanh(beta * eta) + tanh(beta * (1 - eta)));
-}
-
-// xTilde = filtered / Hs (top3D125mod.m:108-109)
-__global__ void k_div(double *__restrict__ x, const double *__restrict__ d, long n)
-{
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    if (e < n) x[e] /= d[e];
 }
 
 // partial sums of prj and deta for the eta Newton step (top3D125mod.m:110-116)
@@ -242,35 +295,153 @@ __device__ __forceinline__ double oc_x(double ocp, double xt, double lmid, doubl
     return v;
 }
 
-// Volume for kCand candidate multipliers at once (the nodes of the next
-// five bisection levels), read x once.
-struct Cands {
+// The OC bisection on the device (top3D125mod.m:143-151): a pass sums the
+// volumes of kCand candidate multipliers at once (the midpoints of the next
+// five bisection levels in heap order: node q has children 2q+1, "volume >
+// volfrac", and 2q+2), reading x once, and walks the tree.  Three passes are
+// enough as a rule, so nothing but the last state returns to the host: with
+// the walk on the host each pass was a copy and a round trip of 25 us.
+struct OcState {
+    double l1, l2, lmid;
     double l[kCand];
+    int done;
 };
 
-__global__ __launch_bounds__(256) void k_oc_volumes(const double *__restrict__ ocP, const double *__restrict__ x, long n,
-                                                   Cands c, int nc, double move, double *part)
+// l1, l2 -> the candidates, one thread each: the bits of q + 1 below its
+// highest are the way from the root
+__device__ __forceinline__ void oc_next(OcState *s)
 {
-    double s[kCand];
-#pragma unroll
-    for (int q = 0; q < kCand; ++q) s[q] = 0.0;
-    for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < n; e += (long)kRedBlocks * 256) {
-        const double o = ocP[e], xt = x[e];
-#pragma unroll
-        for (int q = 0; q < kCand; ++q)
-            if (q < nc) s[q] += oc_x(o, xt, c.l[q], move);
+    const int q = threadIdx.x;
+    if (s->done || q >= kCand) return;
+    double lo = s->l1, hi = s->l2;
+    for (int b = 30 - __builtin_clz(q + 1); b >= 0; --b) {
+        const double mid = 0.5 * (lo + hi);
+        if ((q + 1) >> b & 1)
+            hi = mid;  // volume <= volfrac: l2 = lmid
+        else
+            lo = mid;
     }
-#pragma unroll
-    for (int q = 0; q < kCand; ++q) {
-        const double t = wsum256(s[q]);
-        if (threadIdx.x == 0 && q < nc) part[(long)q * kRedBlocks + blockIdx.x] = t;
-    }
+    s->l[q] = 0.5 * (lo + hi);
 }
 
-__global__ void k_oc_apply(const double *__restrict__ ocP, double *__restrict__ x, long n, double lmid, double move)
+__device__ __forceinline__ bool oc_open(double l1, double l2) { return (l2 - l1) / (l2 + l1) > 1e-4; }
+
+// the bracket from the sum of ocP
+__global__ __launch_bounds__(256) void k_oc_begin(const double *part, double ne, double volfrac, OcState *st)
+{
+    double v = 0.0;
+    for (int i = threadIdx.x; i < kRedBlocks; i += 256) v += part[i];
+    v = wsum256(v);
+    if (threadIdx.x == 0) {
+        st->l1 = 0.0;
+        st->l2 = v / ne / volfrac;
+        st->lmid = 0.0;
+        st->done = !oc_open(0.0, st->l2);
+    }
+    __syncthreads();
+    oc_next(st);
+}
+
+// Partial volumes of eight candidates (blockIdx.y); a candidate is a division
+// and five comparisons per element, 31 of them in one thread took 23 us at
+// 48x24x24 and 49 at 192x96x96, 7.9 and 40 now.
+constexpr int kCandGroup = 8;
+
+__global__ __launch_bounds__(256) void k_oc_volumes(const double *__restrict__ ocP, const double *__restrict__ x, long n,
+                                                   const OcState *__restrict__ st, double move, double *part)
+{
+    __shared__ double ws[4][kCandGroup];
+    if (st->done) return;
+    const int c0 = blockIdx.y * kCandGroup, tid = threadIdx.x;
+    double s[kCandGroup];
+#pragma unroll
+    for (int q = 0; q < kCandGroup; ++q) s[q] = 0.0;
+    if ((long)blockIdx.x * 256 < n) {
+        double l[kCandGroup];
+#pragma unroll
+        for (int q = 0; q < kCandGroup; ++q) l[q] = st->l[min(c0 + q, kCand - 1)];
+        for (long e = (long)blockIdx.x * 256 + tid; e < n; e += (long)kRedBlocks * 256) {
+            const double o = ocP[e], xt = x[e];
+#pragma unroll
+            for (int q = 0; q < kCandGroup; ++q) s[q] += oc_x(o, xt, l[q], move);
+        }
+#pragma unroll
+        for (int q = 0; q < kCandGroup; ++q)
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) s[q] += __shfl_xor(s[q], off, 64);
+    }
+    if ((tid & 63) == 0) {
+#pragma unroll
+        for (int q = 0; q < kCandGroup; ++q) ws[tid >> 6][q] = s[q];
+    }
+    __syncthreads();
+    if (tid < kCandGroup && c0 + tid < kCand)
+        part[(long)(c0 + tid) * kRedBlocks + blockIdx.x] = ws[0][tid] + ws[1][tid] + ws[2][tid] + ws[3][tid];
+}
+
+// One block: the sums of the pass (in k_finalise's order; 256 threads to a sum,
+// eight sums to a thread, every load in flight together), the walk, the next
+// candidates.
+__global__ __launch_bounds__(1024) void k_oc_walk(const double *part, double ne, double volfrac, OcState *st)
+{
+    constexpr int kPer = (kCand + 3) / 4, kLoads = kRedBlocks / 256;
+    __shared__ double ws[kPer][16], sum[4 * kPer];
+    const int tid = threadIdx.x, t = tid & 255;
+    double v[kPer][kLoads];
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+        const int q = min(4 * r + (tid >> 8), kCand - 1);
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) v[r][i] = part[(long)q * kRedBlocks + t + 256 * i];
+    }
+    if (st->done) return;
+#pragma unroll
+    for (int r = 0; r < kPer; ++r) {
+        double x = 0.0;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) x += v[r][i];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off, 64);
+        if ((tid & 63) == 0) ws[r][tid >> 6] = x;
+    }
+    __syncthreads();
+    if (tid < 4 * kPer) {
+        const double *w = ws[tid >> 2] + 4 * (tid & 3);
+        sum[tid] = w[0] + w[1] + w[2] + w[3];
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double l1 = st->l1, l2 = st->l2, lmid;
+        for (int q = 0;;) {
+            lmid = st->l[q];
+            const bool more = sum[q] / ne > volfrac;
+            if (more)
+                l1 = lmid;
+            else
+                l2 = lmid;
+            q = more ? 2 * q + 1 : 2 * q + 2;
+            if (!oc_open(l1, l2) || q >= kCand) break;
+        }
+        st->l1 = l1;
+        st->l2 = l2;
+        st->lmid = lmid;
+        st->done = !oc_open(l1, l2);
+    }
+    __syncthreads();
+    oc_next(st);
+}
+
+// x of the final multiplier, and the state for the host
+__global__ void k_oc_apply(const double *__restrict__ ocP, double *__restrict__ x, long n, const OcState *st,
+                           double move, double *host)
 {
     const long e = (long)blockIdx.x * 256 + threadIdx.x;
-    if (e < n) x[e] = oc_x(ocP[e], x[e], lmid, move);
+    const bool done = st->done;
+    if (e == 0) {
+        host[0] = done ? 1.0 : 0.0;
+        host[1] = st->lmid;
+    }
+    if (done && e < n) x[e] = oc_x(ocP[e], x[e], st->lmid, move);
 }
 
 __global__ void k_edofmat(Grid g, int *cmat)
@@ -308,13 +479,16 @@ std::vector<double> filter_weights(double rmin, int *fw)
     return h;
 }
 
-double reduce_host(ToState *t, hipStream_t s, int nsums, double *out)
+// the partial sums to the pinned words from `slot` on, without a copy
+void launch_finalise(ToState *t, hipStream_t s, int nsums, int slot)
 {
-    k_finalise<<<nsums, 256, 0, s>>>(t->part, nsums, t->red);
-    check_hip(hipMemcpyAsync(t->red_host, t->red, nsums * sizeof(double), hipMemcpyDeviceToHost, s), "copy");
+    k_finalise<<<nsums, 256, 0, s>>>(t->part, nsums, t->red_host + slot);
+}
+
+void reduce_host(ToState *t, hipStream_t s, int nsums, int slot)
+{
+    launch_finalise(t, s, nsums, slot);
     check_hip(hipStreamSynchronize(s), "sync");
-    for (int q = 0; q < nsums; ++q) out[q] = t->red_host[q];
-    return out[0];
 }
 
 int map_exc()
@@ -355,14 +529,14 @@ void gputo::to_destroy(gputo_handle *h)
 static void make_buffers(ToState *t, size_t ne, size_t ndof, size_t nfd)
 {
     if (!t->x) {
-        double **el[] = {&t->x, &t->xPhys, &t->xOld, &t->Hs, &t->dHs, &t->dsK, &t->dc, &t->dv, &t->tmp, &t->ocP, &t->CX};
+        double **el[] = {&t->x, &t->xPhys, &t->xOld, &t->Hs, &t->dHs, &t->dsK, &t->dc, &t->dv, &t->tmp, &t->ocP};
         for (double **p : el) *p = talloc<double>(t, ne);
         t->F = talloc<double>(t, ndof);
         t->U = talloc<double>(t, ndof);
         t->part = talloc<double>(t, (size_t)kCand * kRedBlocks);
-        t->red = talloc<double>(t, kCand);
+        t->oc = talloc<OcState>(t, 1);
         t->w = talloc<double>(t, kMaxFilterWeights);
-        check_hip(hipHostMalloc((void **)&t->red_host, kCand * sizeof(double), hipHostMallocDefault), "hostmalloc");
+        check_hip(hipHostMalloc((void **)&t->red_host, kSumCount * sizeof(double), hipHostMallocDefault), "hostmalloc");
     }
     if (t->nfixed < nfd || !t->fixed_d) {
         if (t->fixed_d) {
@@ -410,7 +584,7 @@ int gputo_filter_f64(gputo_handle *h, const double *in, double rmin, double *out
         hipStream_t s = h->stream;
         hipMemcpyAsync(dw, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, s);
         hipMemcpyAsync(din, in, g.nel * sizeof(double), hipMemcpyHostToDevice, s);
-        k_filter<<<nb256(g.nel), 256, 0, s>>>(g, din, nullptr, dw, fw, dout);
+        launch_filter(s, g, 1, {din, nullptr, dout}, {}, dw, fw);
         hipMemcpyAsync(out, dout, g.nel * sizeof(double), hipMemcpyDeviceToHost, s);
         hipError_t e = hipStreamSynchronize(s);
         hipFree(dw);
@@ -488,7 +662,7 @@ int gputo_to_begin(gputo_handle *h, const double *Ke0, const double *x0, const d
         launch_fill(s, t->xOld, ne, 1.0);  // xOld = 1 (top3D125mod.m:102)
         launch_fill(s, t->U, g.ndof, 0.0);
         launch_fill(s, t->tmp, ne, 1.0);
-        k_filter<<<nb256(ne), 256, 0, s>>>(g, t->tmp, nullptr, t->w, t->fw, t->Hs);  // Hs = imfilter(ones)
+        launch_filter(s, g, 1, {t->tmp, nullptr, t->Hs}, {}, t->w, t->fw);  // Hs = imfilter(ones)
         check_hip(hipGetLastError(), "launch");
         check_hip(hipStreamSynchronize(s), "sync");
         t->loop = 0;
@@ -513,27 +687,24 @@ int gputo_to_iterate(gputo_handle *h, gputo_to_stats *st)
         const auto t0 = std::chrono::steady_clock::now();
         t->loop += 1;
         // RL 1: filtered field and projection (top3D125mod.m:108-121)
-        k_filter<<<nb256(ne), 256, 0, s>>>(g, t->x, nullptr, t->w, t->fw, t->xPhys);
-        k_div<<<nb256(ne), 256, 0, s>>>(t->xPhys, t->Hs, ne);
-        double sums[kCand];
+        launch_filter(s, g, 1, {t->x, t->Hs, t->xPhys}, {}, t->w, t->fw);
+        const double *sums = t->red_host;
         if (c.ft == 3) {
             k_eta_sums<<<kRedBlocks, 256, 0, s>>>(t->xPhys, ne, t->eta, t->beta, t->part);
-            reduce_host(t, s, 2, sums);
-            double f = sums[0] / ne - c.volfrac;
+            reduce_host(t, s, 2, kSumEta);
+            double f = sums[kSumEta] / ne - c.volfrac;
             int it = 0;
             while (std::fabs(f) > 1e-6 && it < 100) {
-                t->eta = t->eta - f / (sums[1] / ne);
+                t->eta = t->eta - f / (sums[kSumEta + 1] / ne);
                 k_eta_sums<<<kRedBlocks, 256, 0, s>>>(t->xPhys, ne, t->eta, t->beta, t->part);
-                reduce_host(t, s, 2, sums);
-                f = sums[0] / ne - c.volfrac;
+                reduce_host(t, s, 2, kSumEta);
+                f = sums[kSumEta] / ne - c.volfrac;
                 ++it;
             }
         }
-        k_physics<<<kRedBlocks, 256, 0, s>>>(t->xPhys, t->xOld, t->Hs, t->dHs, t->CX, t->dsK, ne, c.ft == 3 ? 1 : 0,
+        k_physics<<<kRedBlocks, 256, 0, s>>>(t->xPhys, t->xOld, t->Hs, t->dHs, h->CX, t->dsK, ne, c.ft == 3 ? 1 : 0,
                                              t->eta, t->beta, t->penal, c.Emin, c.E0, t->part);
-        reduce_host(t, s, 2, sums);
-        st->change = std::sqrt(sums[0]) / ne;
-        st->volume = sums[1] / ne;
+        launch_finalise(t, s, 2, kSumPhys);
         // RL 2: solve (top3D125mod.m:130-134)
         hipEvent_t e0, e1;
         hipEventCreate(&e0);
@@ -542,7 +713,6 @@ int gputo_to_iterate(gputo_handle *h, gputo_to_stats *st)
         double relres = 0.0;
         int nit = 0;
         set_ke(h, t->Ke.data());
-        check_hip(hipMemcpyAsync(h->CX, t->CX, ne * sizeof(double), hipMemcpyDeviceToDevice, s), "copy");
         int rc = setup_hierarchy(h, t->fixed);
         if (rc == 0) {
             rc = run_pcg(h, t->F, t->U, c.cg_tol, c.cg_maxit, &relres, &nit);
@@ -554,6 +724,8 @@ int gputo_to_iterate(gputo_handle *h, gputo_to_stats *st)
         hipEventDestroy(e0);
         hipEventDestroy(e1);
         st->seconds_solve = ms * 1e-3;
+        st->change = std::sqrt(sums[kSumPhys]) / ne;  // written before the solve
+        st->volume = sums[kSumPhys + 1] / ne;
         st->relres = relres;
         st->cg_iters = nit;
         if (rc) {
@@ -563,52 +735,34 @@ int gputo_to_iterate(gputo_handle *h, gputo_to_stats *st)
         // RL 3: sensitivities (top3D125mod.m:139-141)
         k_sens<<<nb256(ne), 256, 0, s>>>(g, h->Ke, t->U, t->dsK, t->dHs, 1.0 / ne / c.volfrac, t->tmp, t->ocP,
                                           nullptr);
-        k_filter<<<nb256(ne), 256, 0, s>>>(g, t->tmp, nullptr, t->w, t->fw, t->dc);
-        k_filter<<<nb256(ne), 256, 0, s>>>(g, t->ocP, nullptr, t->w, t->fw, t->dv);
+        launch_filter(s, g, 2, {t->tmp, nullptr, t->dc}, {t->ocP, nullptr, t->dv}, t->w, t->fw);
         // RL 4: OC bisection (top3D125mod.m:143-151)
         k_ocp<<<kRedBlocks, 256, 0, s>>>(t->x, t->dc, t->dv, t->ocP, ne, t->part);
-        reduce_host(t, s, 1, sums);
-        double l1 = 0.0, l2 = sums[0] / ne / c.volfrac, lmid = 0.0;
-        while ((l2 - l1) / (l2 + l1) > 1e-4) {
-            // candidates: the midpoints of the next 5 bisection levels, in
-            // heap order (node q has children 2q+1 = "volume > volfrac")
-            Cands cd;
-            double lo[kCand], hi[kCand];
-            lo[0] = l1;
-            hi[0] = l2;
-            for (int q = 0; q < kCand; ++q) {
-                cd.l[q] = 0.5 * (lo[q] + hi[q]);
-                if (2 * q + 2 < kCand) {
-                    lo[2 * q + 1] = cd.l[q];  // volume > volfrac: l1 = lmid
-                    hi[2 * q + 1] = hi[q];
-                    lo[2 * q + 2] = lo[q];    // else: l2 = lmid
-                    hi[2 * q + 2] = cd.l[q];
-                }
+        k_oc_begin<<<1, 256, 0, s>>>(t->part, (double)ne, c.volfrac, t->oc);
+        const dim3 vols(kRedBlocks, (kCand + kCandGroup - 1) / kCandGroup);
+        auto oc_passes = [&](int np) {
+            for (int p = 0; p < np; ++p) {
+                k_oc_volumes<<<vols, 256, 0, s>>>(t->ocP, t->x, ne, t->oc, c.move, t->part);
+                k_oc_walk<<<1, 1024, 0, s>>>(t->part, (double)ne, c.volfrac, t->oc);
             }
-            k_oc_volumes<<<kRedBlocks, 256, 0, s>>>(t->ocP, t->x, ne, cd, kCand, c.move, t->part);
-            reduce_host(t, s, kCand, sums);
-            int q = 0;
-            for (;;) {
-                lmid = cd.l[q];
-                if (sums[q] / ne > c.volfrac)
-                    l1 = lmid;
-                else
-                    l2 = lmid;
-                const int nxt = (sums[q] / ne > c.volfrac) ? 2 * q + 1 : 2 * q + 2;
-                if (!((l2 - l1) / (l2 + l1) > 1e-4) || nxt >= kCand) break;
-                q = nxt;
-            }
+            k_oc_apply<<<nb256(ne), 256, 0, s>>>(t->ocP, t->x, ne, t->oc, c.move, t->red_host + kSumOc);
+        };
+        oc_passes(3);
+        // RL 5: compliance F'U (top3D125mod.m:155)
+        launch_dot_partial(s, t->F, t->U, g.ndof, t->part, nullptr);
+        reduce_host(t, s, 1, kSumComp);
+        check_hip(hipGetLastError(), "launch");
+        while (sums[kSumOc] == 0.0) {  // the bracket is not narrow enough yet
+            oc_passes(2);
+            check_hip(hipGetLastError(), "launch");
+            check_hip(hipStreamSynchronize(s), "sync");
         }
-        k_oc_apply<<<nb256(ne), 256, 0, s>>>(t->ocP, t->x, ne, lmid, c.move);
+        const double lmid = sums[kSumOc + 1];
         // continuation (top3D125mod.m:32-33,152): cnt(v,{1,1,25,d},loop)
         const int L = t->loop;
         if (L >= 1 && t->penal < 1 && L % 25 == 0) t->penal += 0.25;
         if (L >= 1 && t->beta < 1 && L % 25 == 0) t->beta += 2;
-        // RL 5: compliance F'U (top3D125mod.m:155)
-        launch_dot_partial(s, t->F, t->U, g.ndof, t->part, nullptr);
-        reduce_host(t, s, 1, sums);
-        check_hip(hipGetLastError(), "launch");
-        st->compliance = sums[0];
+        st->compliance = sums[kSumComp];
         st->eta = t->eta;
         st->lmid = lmid;
         st->status = 0;
