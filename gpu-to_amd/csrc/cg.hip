@@ -7,7 +7,8 @@
 //   r -= alpha q (u += alpha p)  alpha = rho / p.q, per-block sums of r.r
 //   check                        one block: residual test, progress word
 //   z = M r                      V-cycle
-//   dots                         per-block sums of r.z (and q.z)
+//   dots                         per-block sums of r.z (and q.z); in FP64 the
+//                                V-cycle's last sweep leaves them
 //   p = z + beta p               beta from rho
 // alpha and beta are formed inside the update that uses them: every block
 // adds the per-block sums in the same order (at most kCgFuse of them, read
@@ -317,6 +318,15 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_dots(const double *__restrict
     }
 }
 
+// sum of p[0..n) to out, for one value per right-hand side
+__global__ __launch_bounds__(kCgThreads) void k_cg_sum(const double *p, int n, double *out, const int *ctl)
+{
+    ctl = batch_ctl(ctl);
+    if (ctl[0]) return;
+    const double s = cg_partials<kCgThreads>(p + (long)blockIdx.z * n, n);
+    if (threadIdx.x == 0) out[blockIdx.z] = s;
+}
+
 // Pout = Z + beta Pin formed in FP64 and rounded once (Pout may be Pin).
 // beta = <r,z>/rho_old, or for a preconditioner that varies between
 // iterations the flexible (Polak-Ribiere) <z, r - r_old>/rho_old with r -
@@ -445,12 +455,19 @@ void launch_cg_check(hipStream_t s, CgScalars *sc, const double *rr, long n, dou
 
 template <class TP, class TZ>
 void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const double *q, TP *Pout, const TP *Pin, long n,
-                         CgScalars *sc, double *dots, bool flex, int maxit, int nb)
+                         CgScalars *sc, double *dots, bool flex, int maxit, int nb, const double *zr, int nzr)
 {
     const int nblk = cg_blocks(n);
     const dim3 gd(nblk, 1, batch_dim(nb));
     const dim3 gp((unsigned)std::min<long>((n + 2 * kBlock - 1) / (2 * kBlock), kCgUpdBlocks), 1, batch_dim(nb));
-    if (flex) {
+    if (zr && !flex) {  // the V-cycle's last sweep left the sums
+        if (nzr > kCgFuse) {
+            k_cg_sum<<<dim3(1, 1, batch_dim(nb)), kCgThreads, 0, s>>>(zr, nzr, dots, &sc->done);
+            zr = dots;
+            nzr = 1;
+        }
+        k_cg_update_p<TP, TZ, false><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, zr, nzr, maxit);
+    } else if (flex) {
         k_cg_dots<TZ, true><<<gd, kCgThreads, 0, s>>>(r, z, q, n, dots, &sc->done);
         k_cg_update_p<TP, TZ, true><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, dots, nblk, maxit);
     } else {
@@ -459,9 +476,11 @@ void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const doub
     }
 }
 template void launch_cg_direction<double, double>(hipStream_t, const double *, const double *, const double *, double *,
-                                                  const double *, long, CgScalars *, double *, bool, int, int);
+                                                  const double *, long, CgScalars *, double *, bool, int, int,
+                                                  const double *, int);
 template void launch_cg_direction<float, float>(hipStream_t, const double *, const float *, const double *, float *,
-                                                const float *, long, CgScalars *, double *, bool, int, int);
+                                                const float *, long, CgScalars *, double *, bool, int, int,
+                                                const double *, int);
 
 void launch_cg_flush_u(hipStream_t s, double *U, const float *P, long n, const double *alog, int m)
 {

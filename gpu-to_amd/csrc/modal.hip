@@ -347,6 +347,8 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     constexpr bool PRE = MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT;
     constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI;
     constexpr bool MV = MODE == OP_MATVEC || MODE == OP_MATVEC_UF;
+    // fused dots: of a matvec u.(K u), of a sweep F.(its result)
+    constexpr bool DOT = MV || (MODE == OP_JACOBI && EL == 0 && sizeof(T) == 8);
     // the next layer's operands are loaded a layer ahead where the registers
     // allow it
     constexpr bool AHEAD = sizeof(T) == 4 ? !PRE : (EL == 0 && !PRE);
@@ -494,6 +496,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
                 const T u = PRE ? pr * (e.f[cc] * e.d[cc]) : T(e.u[cc]);
                 const T rv = fixed ? T(0) : e.f[cc] - yc;
                 v = fma(om * e.d[cc], rv, u);
+                if (DOT) part += (double)e.f[cc] * (double)v;
             }
             a.out[dof + cc] = v;
             if (PER) {
@@ -594,7 +597,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
         load_epi(g.nnx - 1, epi);
         finish(g.nnx - 1, pend, epi);
     }
-    if (MV && a.partials) {
+    if (DOT && a.partials) {
         // fixed butterfly per wave, then the waves in order
         __shared__ double ws[kMdMaxWaves];
 #pragma unroll

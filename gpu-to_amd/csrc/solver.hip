@@ -256,7 +256,12 @@ HierView<double> f64_view(const gputo_handle *h)
 
 OpArgs op_args(const gputo_handle *h, int l) { return view_args(h, f64_view(h), l, &h->sc->done); }
 
-void vcycle(gputo_handle *h, const double *F0, double *U0) { vcycle_t(h, f64_view(h), F0, U0, &h->sc->done); }
+void vcycle(gputo_handle *h, const double *F0, double *U0, double *zr = nullptr)
+{
+    HierView<double> H = f64_view(h);
+    H.zr = zr;
+    vcycle_t(h, H, F0, U0, &h->sc->done);
+}
 
 int validate_fixed(const std::vector<int> &f, long ndof)
 {
@@ -490,10 +495,11 @@ static bool custom_schedule(const gputo_params &p)
 
 // Device-resident PCG (mgcg1.cu:235-280); U, F on the device.
 // z = M r: the FP64 V-cycle, or the FP32 V-cycle of the mixed precisions
-static void precond(gputo_handle *h, const double *r, double *z, bool r32_ready = false, bool pre0_ready = false)
+static void precond(gputo_handle *h, const double *r, double *z, bool r32_ready = false, bool pre0_ready = false,
+                    double *zr = nullptr)
 {
     if (h->prm.precision == GPUTO_PREC_F64)
-        vcycle(h, r, z);
+        vcycle(h, r, z, zr);
     else
         mixed_vcycle(h, r, z, &h->sc->done, r32_ready, pre0_ready);
 }
@@ -551,6 +557,9 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
     const float *ad32 = nullptr;
     double prx = 0.0;
     float *x0 = z32 ? mixed_prerelax_target(h, &ad32, &prx) : nullptr;
+    // FP64: the V-cycle's last sweep leaves the sums of r.z where the matvec left
+    // those of p.q (read by then)
+    double *zr = h->prm.precision == GPUTO_PREC_F64 && !flex && vcycle_dots(h, f64_view(h)) ? h->partials : nullptr;
     auto precond_n = [&](const double *r, double *z, bool r32_ready) {
         if (h->prm.coarse_lag >= 2 && vcycles == h->prm.coarse_lag) {
             coarse_switch(h->C, s);
@@ -562,7 +571,7 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
         if (graphs && vcycles > 0 && r32_ready && !z)
             mixed_vcycle_graph(h, &h->sc->done, pre0);
         else
-            precond(h, r, z, r32_ready, pre0);
+            precond(h, r, z, r32_ready, pre0, zr);
         ++vcycles;
     };
     // ... and then keeps the search direction in FP32: p = z + beta p formed
@@ -657,7 +666,8 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
                                               dots, flex, maxit, 1);
         } else {
             precond_n(h->R, h->Z, r32 != nullptr);
-            launch_cg_direction<double, double>(s, h->R, h->Z, h->Q, h->P, h->P, n, h->sc, dots, flex, maxit, 1);
+            launch_cg_direction<double, double>(s, h->R, h->Z, h->Q, h->P, h->P, n, h->sc, dots, flex, maxit, 1, zr,
+                                                nmv);
         }
     }
     if (p32) launch_cg_flush_u(s, U, p32, n, alog, enq - folded);  // since the last pass (converged: alpha 0)
@@ -786,6 +796,7 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
         batch_view<float>(H32, b.v32, h->nl, nb);
     } else {
         batch_view<double>(H64, b.v64, h->nl, nb);
+        if (!flex && vcycle_dots(h, H64)) H64.zr = b.partials;
     }
     float *r32 = mixed ? b.r32 : nullptr;
     auto precond = [&](const double *r, double *z, bool r32_ready) {
@@ -824,7 +835,8 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
         HIPCHK(hipGetLastError());
         if (enq > 1 && cg_wait(s, h->prog, nb, enq - 1, nullptr)) break;
         precond(b.R, b.Z, r32 != nullptr);
-        launch_cg_direction<double, double>(s, b.R, b.Z, b.Q, b.P, b.P, n, b.sc, dots, flex, maxit, nb);
+        launch_cg_direction<double, double>(s, b.R, b.Z, b.Q, b.P, b.P, n, b.sc, dots, flex, maxit, nb, H64.zr,
+                                            nmv);
     }
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(b.sc_host, b.sc, nb * sizeof(CgScalars), hipMemcpyDeviceToHost, s));
