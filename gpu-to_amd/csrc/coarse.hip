@@ -475,7 +475,7 @@ void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, d
 // ---------------------------------------------------------------------------
 constexpr int NB = 32;
 
-__device__ __forceinline__ int coarse_dof(const CoarseMap &m, int c)
+__host__ __device__ inline int coarse_dof(const CoarseMap &m, int c)
 {
     if (m.ps == 0) return c < m.n ? c : -1;  // one part
     if (c < m.o2) return c >= m.pad1 ? c - m.pad1 : -1;
@@ -1001,6 +1001,7 @@ void coarse_layout(Coarse &C, const Grid &g, bool periodic)
     m.n = C.n;
     m.p = 3 * g.nny * g.nnz;
     m.nplanes = g.nnx;
+    m.rp = 1.0f / (float)m.p;
     auto up = [](int v) { return (v + NB - 1) / NB * NB; };
     const int N1 = up(C.n);
     m.o2 = m.os = m.N = N1;
@@ -1012,8 +1013,14 @@ void coarse_layout(Coarse &C, const Grid &g, bool periodic)
     m.os = m.o2 + up(p2);
     m.pad2 = up(p2) - p2;
     m.ps = up(m.p);
-    m.rp = 1.0f / (float)m.p;
     m.N = m.os + m.ps;
+}
+
+std::vector<int> coarse_dofs(const Coarse &C)
+{
+    std::vector<int> d(C.map.N);
+    for (int c = 0; c < C.map.N; ++c) d[c] = coarse_dof(C.map, c);
+    return d;
 }
 
 CoarseParts coarse_parts(const Coarse &C)
@@ -1179,84 +1186,97 @@ void coarse_switch(Coarse &C, hipStream_t s)
 }
 
 // ---------------------------------------------------------------------------
-// Coarsest solve x = L^-T L^-1 b as two row-parallel triangular products
-// (one 256-thread block per row, fixed reduction order), then x[fixed] = 0
-// (mgcg1.c:431-432).  Each thread issues kTrmvLoads row entries (and as
-// many of b) before its first product, so a row of up to 2048 entries is
-// one memory round trip; the skip flag is read while they are in flight.
-// Rows and columns are in the factor's order (coarse_dof), the right-hand side
-// and the solution in the level's; a row of one part skips the other's columns
-// (zeros), which with the split halves the bytes read.
+// Coarsest solve x = L^-T L^-1 b as two row-parallel triangular products, then
+// x[fixed] = 0 (mgcg1.c:431-432).  One wave per row and, for a batch, all its
+// right-hand sides: a row is read once, two entries per load, kTrmvLoads of
+// them (and of b) in flight before the first product; the longest rows come
+// first.  Rows start and end at whole tiles (the diagonal tiles are stored with
+// their zeros).  Rows and columns are in the factor's order (coarse_dof, from a
+// table: the arithmetic for every column of a row took 2 to 3 us), the
+// right-hand side and the solution in the level's; a row of one part skips the
+// other's columns, which halves the bytes.  (A workgroup per row with single
+// loads and a sum through LDS: 7.1 + 6.3 us at 1911 DOFs and 10.6 + 8.2 at
+// 2880, 5.6 + 5.0 and 8.1 + 6.4 now; six right-hand sides at 1029 DOFs, each with
+// its own pass over the matrix: 14 + 13, 13 + 8.7 now.)
 // ---------------------------------------------------------------------------
 constexpr int kTrmvThreads = 256, kTrmvLoads = 8;
 
-template <bool UPPER, class Ti, class To>
-__global__ __launch_bounds__(kTrmvThreads) void k_trmv(CoarseMap m, const double *__restrict__ M,
+template <bool UPPER, int MAXB, class Ti, class To>
+__global__ __launch_bounds__(kTrmvThreads) void k_trmv(CoarseMap m, const int *__restrict__ dof,
+                                                      const double *__restrict__ M,
                                                       const Ti *__restrict__ b, To *__restrict__ x,
-                                                      const uint8_t *__restrict__ mask, const int *ctl)
+                                                      const uint8_t *__restrict__ mask, const int *ctl, int nb)
 {
-    __shared__ double red[kTrmvThreads / 64];
-    ctl = batch_ctl(ctl);
     // lower: b has n entries, x has N (the padded y); upper: the reverse
-    b = batch_ptr(b, UPPER ? (long)m.N : (long)m.n);
-    x = batch_ptr(x, UPPER ? (long)m.n : (long)m.N);
-    const int row = blockIdx.x;  // < N
+    const long sb = UPPER ? m.N : m.n, sx = UPPER ? m.n : m.N;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int idx = blockIdx.x * (kTrmvThreads / 64) + wave;  // < N
+    const int row = UPPER ? idx : m.N - 1 - idx;
     // columns lo .. lo + cnt - 1, those from `cut` on shifted by `skip` (the
     // separator's columns of a row of part 1)
-    const bool split = m.ps > 0;
-    int lo, cnt, cut, skip = 0;
+    const int tile = row / NB * NB;
+    int lo, cnt, cut = m.N, skip = 0;
     if (!UPPER) {
-        lo = split && row >= m.o2 && row < m.os ? m.o2 : 0;
-        cnt = row + 1 - lo;
-        cut = m.N;
+        lo = m.ps > 0 && row >= m.o2 && row < m.os ? m.o2 : 0;
+        cnt = tile + NB - lo;
     } else {
-        lo = row;
-        cnt = m.N - row;
-        cut = m.N;
-        if (split && row < m.o2) {
+        lo = tile;
+        cnt = m.N - tile;
+        if (m.ps > 0 && row < m.o2) {
             cut = m.o2;
             skip = m.os - m.o2;
             cnt -= skip;
         }
     }
     const double *__restrict__ Mr = M + (long)row * m.N;
-    double s = 0.0;
-    for (int t0 = (int)threadIdx.x; t0 < cnt; t0 += kTrmvThreads * kTrmvLoads) {
-        double mv[kTrmvLoads], bv[kTrmvLoads];
+    double s[MAXB];
+#pragma unroll
+    for (int q = 0; q < MAXB; ++q) s[q] = 0.0;
+    for (int t0 = 2 * lane; t0 < cnt; t0 += 128 * kTrmvLoads) {
+        f64x2 mv[kTrmvLoads];
+        int d0[kTrmvLoads], d1[kTrmvLoads];
 #pragma unroll
         for (int u = 0; u < kTrmvLoads; ++u) {
-            const int t = t0 + kTrmvThreads * u;
+            const int t = t0 + 128 * u;
             int c = lo + (t < cnt ? t : t0);  // in the row
             c += c >= cut ? skip : 0;
-            const double a = Mr[c];
+            mv[u] = *reinterpret_cast<const f64x2 *>(Mr + c);
+            if (t >= cnt) mv[u] = f64x2{0.0, 0.0};
             if (UPPER) {
-                bv[u] = (double)b[c];
-                mv[u] = t < cnt ? a : 0.0;
-            } else {
-                const int d = coarse_dof(m, c);
-                bv[u] = (double)b[d < 0 ? 0 : d];
-                mv[u] = t < cnt && d >= 0 ? a : 0.0;
+                d0[u] = c;
+                d1[u] = c + 1;
+            } else {  // padding: an identity row's entry, times nothing
+                const int2 d = *reinterpret_cast<const int2 *>(dof + c);
+                d0[u] = d.x;
+                d1[u] = d.y;
+                if (d0[u] < 0) d0[u] = 0, mv[u][0] = 0.0;
+                if (d1[u] < 0) d1[u] = 0, mv[u][1] = 0.0;
             }
         }
-        if (t0 == (int)threadIdx.x && ctl && ctl[0]) return;
+        if (MAXB == 1 && ctl && ctl[0]) return;  // converged: read with the loads above
 #pragma unroll
-        for (int u = 0; u < kTrmvLoads; ++u) s += mv[u] * bv[u];
-    }
-    if (ctl && ctl[0]) return;  // the threads with no entries
+        for (int q = 0; q < MAXB; ++q) {
+            if (MAXB > 1 && q >= nb) break;
+            double bv[kTrmvLoads][2];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        s = (red[0] + red[1]) + (red[2] + red[3]);
-        if (UPPER) {
-            const int d = coarse_dof(m, row);
-            if (d < 0) return;
-            if (mask && ((mask[d / 3] >> (d % 3)) & 1u)) s = 0.0;
-            x[d] = (To)s;
-        } else {
-            x[row] = (To)s;  // padding rows: 0
+            for (int u = 0; u < kTrmvLoads; ++u) {
+                bv[u][0] = (double)b[q * sb + d0[u]];
+                bv[u][1] = (double)b[q * sb + d1[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < kTrmvLoads; ++u) s[q] = fma(mv[u][1], bv[u][1], fma(mv[u][0], bv[u][0], s[q]));
         }
+    }
+    const int d = UPPER ? dof[row] : row;
+    const bool fixed = UPPER && mask && d >= 0 && ((mask[d / 3] >> (d % 3)) & 1u);
+#pragma unroll
+    for (int q = 0; q < MAXB; ++q) {
+        if (MAXB > 1 && q >= nb) break;
+        double v = s[q];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        const bool done = ctl && ctl[q * kCtlStride];
+        if (lane == 0 && d >= 0 && !done) x[q * sx + d] = (To)(fixed ? 0.0 : v);  // lower, padding rows: 0
     }
 }
 
@@ -1270,10 +1290,15 @@ void launch_coarse_solve(hipStream_t s, const Coarse &C, const T *b, T *x, const
         HIPCHK(hipStreamWaitEvent(s, C.ev_done, 0));
         C.waited = true;
     }
-    // C.y has room for kMaxBatch right-hand sides
-    const dim3 grid(C.map.N, 1, batch_dim(nb));
-    k_trmv<false, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.Linv, b, C.y, nullptr, ctl);
-    k_trmv<true, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.LinvT, C.y, x, mask, ctl);
+    // C.y has room for kMaxBatch right-hand sides; N is a multiple of the rows of a workgroup
+    const unsigned grid = (unsigned)(C.map.N / (kTrmvThreads / 64));
+    if (nb > 1) {
+        k_trmv<false, kMaxBatch, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.Linv, b, C.y, nullptr, ctl, nb);
+        k_trmv<true, kMaxBatch, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.LinvT, C.y, x, mask, ctl, nb);
+    } else {
+        k_trmv<false, 1, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.Linv, b, C.y, nullptr, ctl, 1);
+        k_trmv<true, 1, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.LinvT, C.y, x, mask, ctl, 1);
+    }
 }
 template void launch_coarse_solve<double>(hipStream_t, const Coarse &, const double *, double *, const uint8_t *,
                                           const int *, int);

@@ -196,6 +196,7 @@ struct CoarseBlocks {
 struct Coarse {
     int n = 0;
     CoarseMap map;
+    int *dof = nullptr;      // coarse_dof of every entry
     bool direct = true;      // factored (else smoothed: mgcg9 above 20000 DOFs)
     int bw = 0;              // lower bandwidth of the assembled matrix (node-major DOFs)
     double *AQ = nullptr;       // dense matrix (matrices of the parts, updated by the factorisation), then their factors
@@ -356,6 +357,7 @@ void launch_zero_rowcol(hipStream_t s, int N, const int *fixed_d, int nfd, doubl
 // mask: decouple the fixed DOFs (mgcg9), or null
 void launch_assemble(hipStream_t s, const Grid &g, const double *A, const uint8_t *mask, const Coarse &C);
 void coarse_layout(Coarse &C, const Grid &g, bool periodic);  // C.map from C.n, C.bw
+std::vector<int> coarse_dofs(const Coarse &C);                // coarse_dof of every entry
 CoarseParts coarse_parts(const Coarse &C);
 long coarse_matrix_len(const Coarse &C);  // doubles of C.AQ
 // Factor C.AQ on C.side after the work on s.  lag: when an earlier factor

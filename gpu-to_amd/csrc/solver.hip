@@ -995,6 +995,9 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
         const long N = C.map.N;
         if (dense_ok) {
             C.AQ = dalloc<double>(h, coarse_matrix_len(C));
+            const std::vector<int> dofs = coarse_dofs(C);
+            C.dof = dalloc<int>(h, N);
+            HIPCHK(hipMemcpy(C.dof, dofs.data(), N * sizeof(int), hipMemcpyHostToDevice));
             // entries outside the band are never written and stay 0 in the factor
             launch_fill<double>(h->stream, C.AQ, coarse_matrix_len(C), 0.0);
             for (int b = 0; b < 2; ++b) {
