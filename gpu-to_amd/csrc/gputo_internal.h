@@ -83,6 +83,7 @@ struct OpArgsT {
     const T *S;            // assembled node stencils [14][3][3][stencil_ld] of the same operator, or null
     const T *U;            // input vector
     const T *F;            // right-hand side (defect / Jacobi)
+    const T *Uc;           // OP_INTERP_JACOBI: the coarse level's correction
     const T *AD;           // diagonal (Jacobi)
     const T *RD;           // 1/AD for the modal kernels (null: no Jacobi or prerelaxed mode): one value per
                            // node where Ke0 has one diagonal value, per DOF for the level-1 operator
@@ -110,7 +111,8 @@ enum OpMode {
     OP_JACOBI = 2,      // out = (1-w) U + w (r + AD U)/AD with r = F - K U masked; partials = sum F.out
     OP_PRE_JACOBI = 3,  // as OP_JACOBI with U = prerelax*F/AD formed on the fly
     OP_PRE_DEFECT = 4,  // U = prerelax*F/AD written to out2, out = F - K U masked
-    OP_MATVEC_UF = 5    // as OP_MATVEC with the input Uf in FP32 (level-0 node-gather, FP64)
+    OP_MATVEC_UF = 5,   // as OP_MATVEC with the input Uf in FP32 (level-0 node-gather, FP64)
+    OP_INTERP_JACOBI = 6  // as OP_JACOBI with U + P Uc, 0 at fixed DOFs, in U's place (k_modal_flat, k_stencil)
 };
 
 // Scalars of one device-resident PCG (all on the device, one struct).
@@ -140,12 +142,18 @@ __device__ __forceinline__ P *batch_ptr(P *p, long stride)
     return p ? p + (long)blockIdx.z * stride : p;
 }
 __device__ __forceinline__ const int *batch_ctl(const int *ctl) { return batch_ptr(ctl, kCtlStride); }
+// DOFs of the level below a level of even element counts
+__host__ __device__ inline long coarse_ndof(const Grid &g)
+{
+    return 3L * (g.nx / 2 + 1) * (g.ny / 2 + 1) * (g.nz / 2 + 1);
+}
 template <class T>
 __device__ __forceinline__ void batch_shift(OpArgsT<T> &a)
 {
     const long st = a.g.ndof;
     a.U = batch_ptr(a.U, st);
     a.F = batch_ptr(a.F, st);
+    a.Uc = batch_ptr(a.Uc, coarse_ndof(a.g));
     a.out = batch_ptr(a.out, st);
     a.out2 = batch_ptr(a.out2, st);
     a.partials = batch_ptr(a.partials, (long)gridDim.x);

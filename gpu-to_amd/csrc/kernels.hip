@@ -317,6 +317,47 @@ void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a)
     }
 }
 
+// P Uc at one fine node (i, k, j) (interpc, mgcg1.cu:1587-1641): the mean of
+// the 1, 2, 4 or 8 coarse nodes around it according to its parity.  All 8
+// corners (ia|ib, ja|jb, ka|kb) are loaded together; for an even index a == b
+// and the second corner counts 0, so each coarse node enters once.
+template <class T>
+struct Prolong {
+    T v[8][3], on[8], w;
+    __device__ __forceinline__ void load(const Grid &gf, const T *__restrict__ Uc, int i, int k, int j)
+    {
+        const int cny = gf.ny / 2 + 1, cnz = gf.nz / 2 + 1;
+        const int ia = i >> 1, ib = (i + 1) >> 1, ja = j >> 1, jb = (j + 1) >> 1, ka = k >> 1, kb = (k + 1) >> 1;
+        w = T(1) / (T)(1 << ((i & 1) + (j & 1) + (k & 1)));
+#pragma unroll
+        for (int ci = 0; ci < 2; ++ci)
+#pragma unroll
+            for (int ck = 0; ck < 2; ++ck)
+#pragma unroll
+                for (int cj = 0; cj < 2; ++cj) {
+                    const int q = 4 * ci + 2 * ck + cj;
+                    const int I = ci ? ib : ia, K = ck ? kb : ka, J = cj ? jb : ja;
+                    const bool dup = (ci && ib == ia) || (ck && kb == ka) || (cj && jb == ja);
+                    const long c = 3 * ((long)cny * cnz * I + (long)cny * K + J);
+                    on[q] = dup ? T(0) : T(1);
+                    v[q][0] = Uc[c];
+                    v[q][1] = Uc[c + 1];
+                    v[q][2] = Uc[c + 2];
+                }
+    }
+    // u += P Uc
+    __device__ __forceinline__ void add(T *u) const
+    {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            T s = T(0);
+#pragma unroll
+            for (int q = 0; q < 8; ++q) s += on[q] * v[q][c];
+            u[c] = u[c] + w * s;
+        }
+    }
+};
+
 // ---------------------------------------------------------------------------
 // Operator of a level with stored element matrices (levels >= 1; the
 // element-matrix products of defectc / multAV, Cantilever/TOP3D125MGCGCUDA/
@@ -507,6 +548,7 @@ __global__ __launch_bounds__(kStThreads) void k_stencil(OpArgsT<T> a)
 {
     batch_shift(a);
     __shared__ T red[27][kStencilNodes][3];
+    __shared__ T own[MODE == OP_INTERP_JACOBI ? kStencilNodes : 1][3];
     const Grid g = a.g;
     const unsigned nblk = (unsigned)((g.nnod + kStencilNodes - 1) / kStencilNodes);
     const unsigned tb = (unsigned)xcd_tile(blockIdx.x, nblk);
@@ -532,6 +574,12 @@ __global__ __launch_bounds__(kStThreads) void k_stencil(OpArgsT<T> a)
         for (int c = 0; c < 3; ++c) m[r][c] = Sb[r * sr + c * sc];
 #pragma unroll
     for (int c = 0; c < 3; ++c) u[c] = stored_u<T, MODE>(a, 3 * nb + c);
+    Prolong<T> co;
+    unsigned mu = 0;
+    if (MODE == OP_INTERP_JACOBI) {
+        co.load(g, a.Uc, ok ? ii : i, ok ? kk : k, ok ? jj : j);
+        mu = a.mask[nb];
+    }
     // the finishing threads' operands (in bounds for every thread)
     const int nd = threadIdx.x / 3, fc = threadIdx.x - 3 * nd;
     const bool fin = nd < kStencilNodes && p0 + nd < g.nnod;
@@ -545,6 +593,14 @@ __global__ __launch_bounds__(kStThreads) void k_stencil(OpArgsT<T> a)
         if (MODE == OP_JACOBI) ue = a.U[dof];
     }
     if (a.ctl && a.ctl[0]) return;  // converged: nothing is written
+    if (MODE == OP_INTERP_JACOBI) {
+        co.add(u);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            if ((mu >> c) & 1u) u[c] = T(0);
+            if (b == 13) own[threadIdx.x & (kStencilNodes - 1)][c] = u[c];
+        }
+    }
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
         const T y = m[r][0] * u[0] + m[r][1] * u[1] + m[r][2] * u[2];
@@ -552,6 +608,7 @@ __global__ __launch_bounds__(kStThreads) void k_stencil(OpArgsT<T> a)
     }
     __syncthreads();
     if (!fin) return;
+    if (MODE == OP_INTERP_JACOBI) ue = own[nd][fc];
     const T *rd = &red[0][0][0] + threadIdx.x;
     T yp[3];
 #pragma unroll
@@ -588,6 +645,7 @@ void launch_opA(hipStream_t s, int mode, const OpArgsT<T> &a)
         case OP_JACOBI: k_stencil<T, OP_JACOBI><<<sg, sb, 0, s>>>(a); return;
         case OP_PRE_JACOBI: k_stencil<T, OP_PRE_JACOBI><<<sg, sb, 0, s>>>(a); return;
         case OP_PRE_DEFECT: k_stencil<T, OP_PRE_DEFECT><<<sg, sb, 0, s>>>(a); return;
+        case OP_INTERP_JACOBI: k_stencil<T, OP_INTERP_JACOBI><<<sg, sb, 0, s>>>(a); return;
         default: return;
         }
     }
@@ -770,45 +828,19 @@ __global__ __launch_bounds__(kBlock) void k_interp(Grid gf, const T *__restrict_
     const int j = (int)(nu - q1 * (unsigned)gf.nny);
     const int k = (int)(q1 % (unsigned)gf.nnz);
     const int i = (int)(q1 / (unsigned)gf.nnz);
-    const int cny = gf.ny / 2 + 1, cnz = gf.nz / 2 + 1;
-    Uc = batch_ptr(Uc, 3L * (gf.nx / 2 + 1) * cny * cnz);
+    Uc = batch_ptr(Uc, coarse_ndof(gf));
     Uin = batch_ptr(Uin, gf.ndof);
     Uout = batch_ptr(Uout, gf.ndof);
-    const int ia = i >> 1, ib = (i + 1) >> 1, ja = j >> 1, jb = (j + 1) >> 1, ka = k >> 1, kb = (k + 1) >> 1;
-    const T w = T(1) / (T)(1 << ((i & 1) + (j & 1) + (k & 1)));
-    // corners (ia|ib, ja|jb, ka|kb), all 8 loaded together; for an even
-    // index a == b and the second corner counts 0, so each coarse node
-    // enters once
-    T v[8][3], on[8];
-#pragma unroll
-    for (int ci = 0; ci < 2; ++ci)
-#pragma unroll
-        for (int ck = 0; ck < 2; ++ck)
-#pragma unroll
-            for (int cj = 0; cj < 2; ++cj) {
-                const int q = 4 * ci + 2 * ck + cj;
-                const int I = ci ? ib : ia, K = ck ? kb : ka, J = cj ? jb : ja;
-                const bool dup = (ci && ib == ia) || (ck && kb == ka) || (cj && jb == ja);
-                const long c = 3 * ((long)cny * cnz * I + (long)cny * K + J);
-                on[q] = dup ? T(0) : T(1);
-                v[q][0] = Uc[c];
-                v[q][1] = Uc[c + 1];
-                v[q][2] = Uc[c + 2];
-            }
+    Prolong<T> c;
+    c.load(gf, Uc, i, k, j);
     const long d = 3 * nod;
     const T u0 = Uin[d + 0], u1 = Uin[d + 1], u2 = Uin[d + 2];
     const unsigned m = zero_fixed ? maskf[nod] : 0u;
     if (ctl && ctl[0]) return;  // read while the loads above are in flight
-    T s0 = T(0), s1 = T(0), s2 = T(0);
+    T v[3] = {u0, u1, u2};
+    c.add(v);
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-        s0 += on[q] * v[q][0];
-        s1 += on[q] * v[q][1];
-        s2 += on[q] * v[q][2];
-    }
-    Uout[d + 0] = (m & 1u) ? T(0) : u0 + w * s0;
-    Uout[d + 1] = (m & 2u) ? T(0) : u1 + w * s1;
-    Uout[d + 2] = (m & 4u) ? T(0) : u2 + w * s2;
+    for (int x = 0; x < 3; ++x) Uout[d + x] = (m >> x) & 1u ? T(0) : v[x];
 }
 
 template <class T>

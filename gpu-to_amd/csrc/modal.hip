@@ -320,6 +320,30 @@ __device__ __forceinline__ void md_element_gp(T (&m)[3][2][2][2], const T *C, co
     }
 }
 
+// P Uc at the 4 nodes (k, j), (k, j + 1), (k + 1, j), (k + 1, j + 1) of a node
+// layer, added to the node rows lo and hi; fixed DOFs become 0.  The nodes of a
+// fine element lie in one coarse element: c holds its node pairs along j, rows
+// K and K + 1 (K = k / 2), already averaged over the coarse layers; ko, jo: k,
+// j odd; m: the nodes' fixed bits.
+template <class T>
+__device__ __forceinline__ void md_prolong(const T (&c)[2][6], bool ko, bool jo, const unsigned (&m)[4], T (&lo)[6],
+                                          T (&hi)[6])
+{
+    const T h = T(0.5);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+        // rows k and k + 1 at the coarse columns
+        const T m0 = h * (c[0][x] + c[1][x]), m1 = h * (c[0][3 + x] + c[1][3 + x]);
+        const T l0 = ko ? m0 : c[0][x], l1 = ko ? m1 : c[0][3 + x];
+        const T h0 = ko ? c[1][x] : m0, h1 = ko ? c[1][3 + x] : m1;
+        const T lm = h * (l0 + l1), hm = h * (h0 + h1);
+        lo[x] = (m[0] >> x) & 1u ? T(0) : lo[x] + (jo ? lm : l0);
+        lo[3 + x] = (m[1] >> x) & 1u ? T(0) : lo[3 + x] + (jo ? l1 : lm);
+        hi[x] = (m[2] >> x) & 1u ? T(0) : hi[x] + (jo ? hm : h0);
+        hi[3 + x] = (m[3] >> x) & 1u ? T(0) : hi[3 + x] + (jo ? h1 : hm);
+    }
+}
+
 // Element scales of one element layer at a column: one (level 0) or one per
 // child (level 1).
 template <class T, int EL>
@@ -622,13 +646,19 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
 // A sweep in the solve at 225 nodes FP64 4.9 -> 4.4 us, 4225 nodes 5.3 -> 4.6,
 // 15625 nodes of six right-hand sides (periodic) 15.5 -> 13.1, 30625 nodes FP32
 // 5.2 -> 4.7 us.  Level 0's layer is a third of that: no gain at any size.
+// OP_INTERP_JACOBI: a group reads its coarse element with the rest and adds the
+// correction to its 8 nodes, 5.8-6.0 us where the interpolation (3.1) and the
+// sweep took 7.7 (225 to 4225 nodes FP64).  A march would wait for the coarse
+// nodes in every layer: its level-0 sweep went from 35 to 64 us at 192x96x96 and
+// from 4.8 to 8.4 at 48x24x24, more than the interpolation.
 constexpr int kMdFlatWaves = 8;
 
 template <class T, int MODE, bool PER>
 __global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
 {
     constexpr bool PRE = MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT;
-    constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI;
+    constexpr bool INT = MODE == OP_INTERP_JACOBI;
+    constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI || INT;
     constexpr bool MV = MODE == OP_MATVEC;
     constexpr int S = (int)sizeof(T);
     batch_shift(a);
@@ -655,8 +685,13 @@ __global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, 
     const bool el_ok = ke >= 0 && ke < g.nz && je >= 0 && je < g.ny;
     const bool own = lane > 0 && t > w.R && t <= w.R + w.M && c > 0 && k >= 0 && k < (PER ? g.nz : g.nnz) &&
                      j < (PER ? g.ny : g.nny);
-    const int plane = g.nny * g.nnz, nod0 = k * g.nny + j, enod = ke * g.nny + je;
-    const int lo = el_ok ? 3 * S * enod : kMdOut, hi = el_ok ? 3 * S * (enod + g.nny) : kMdOut;
+    // INT: the pair of row k holds the own node, also where no element follows it
+    // along j (then as its second) or k
+    const bool nod_ok = INT ? ke >= 0 && ke < g.nnz && je >= 0 && je < g.nny : el_ok;
+    const bool jlast = INT && je == g.ny;
+    const int jp = jlast ? je - 1 : je;
+    const int plane = g.nny * g.nnz, nod0 = k * g.nny + j, enod = ke * g.nny + jp;
+    const int lo = nod_ok ? 3 * S * enod : kMdOut, hi = el_ok ? 3 * S * (enod + g.nny) : kMdOut;
     const int eo = el_ok ? S * (4 * ke * g.ny + 2 * je) : kMdOut, oo = own ? 3 * S * nod0 : kMdOut;
     const long vb = (long)S * g.ndof;
     const MdBuf BU = md_buf(PRE ? a.F : a.U, vb), BF = md_buf(a.F, MV ? 0 : vb);
@@ -670,6 +705,36 @@ __global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, 
     const bool el = ie >= 0 && ie < g.nx && il < i1, emit = q > 0 && il < i1;
     T u[4][6], d[4][6], e[8], f[3], de[3], ue[3];  // node rows: lower layer k, k + 1, upper layer k, k + 1
     unsigned m8 = 0;
+    T cv[INT ? 4 : 1][6];  // INT: the coarse element's node pairs, rows K, K + 1 of its two layers
+    unsigned mk[2][4];
+    if constexpr (INT) {
+        const int cny = g.ny / 2 + 1, cp = 3 * S * cny * (g.nz / 2 + 1);
+        const MdBuf BC = md_buf(a.Uc, (long)S * coarse_ndof(g));
+        const int clo = nod_ok ? 3 * S * ((ke >> 1) * cny + (jp >> 1)) : kMdOut;
+        const int chi = nod_ok && ke < g.nz ? clo + 3 * S * cny : kMdOut;
+        const int mlo = nod_ok ? enod : kMdOut, mhi = el_ok ? enod + g.nny : kMdOut;
+        if (el || emit) {
+            md_ld6(BC, clo, (il >> 1) * cp, cv[0]);
+            md_ld6(BC, chi, (il >> 1) * cp, cv[1]);
+            if (el) {
+                md_ld6(BC, clo, ((il >> 1) + 1) * cp, cv[2]);
+                md_ld6(BC, chi, ((il >> 1) + 1) * cp, cv[3]);
+            }
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                if (p == 0 || el) {
+                    const int so = (il + p) * plane;
+                    mk[p][0] = __builtin_amdgcn_raw_buffer_load_b8(BM, mlo, so, 0);
+                    mk[p][1] = __builtin_amdgcn_raw_buffer_load_b8(BM, mlo + 1, so, 0);
+                    mk[p][2] = __builtin_amdgcn_raw_buffer_load_b8(BM, mhi, so, 0);
+                    mk[p][3] = __builtin_amdgcn_raw_buffer_load_b8(BM, mhi + 1, so, 0);
+                }
+            if (!el) {  // the mesh's last node layer: its own node alone
+                md_ld6(BU, lo, il * fp, u[0]);
+                md_ld6(BU, hi, il * fp, u[1]);
+            }
+        }
+    }
     if (el) {
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -689,10 +754,28 @@ __global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, 
         m8 = __builtin_amdgcn_raw_buffer_load_b8(BM, own ? nod0 : kMdOut, il * plane, 0);
         if (!MV) md_ld3(BF, oo, il * fp, f);
         if (JAC || PRE) md_ld3(BD, oo, il * fp, de);
-        if (!PRE && MODE != OP_DEFECT) md_ld3(BU, oo, il * fp, ue);
+        if (!PRE && !INT && MODE != OP_DEFECT) md_ld3(BU, oo, il * fp, ue);
     }
     if (a.ctl && a.ctl[0]) return;  // converged: read with the loads above
     T y[3] = {T(0), T(0), T(0)};
+    if constexpr (INT) {
+        if (el || emit) {
+            T cc[2][2][6];  // the lower and the upper layer
+            const bool odd = il & 1;
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int x = 0; x < 6; ++x) {
+                    const T mean = el ? T(0.5) * (cv[r][x] + cv[2 + r][x]) : T(0);
+                    cc[0][r][x] = odd ? mean : cv[r][x];
+                    cc[1][r][x] = odd ? cv[2 + r][x] : mean;
+                }
+            md_prolong(cc[0], ke & 1, jp & 1, mk[0], u[0], u[1]);
+            if (el) md_prolong(cc[1], ke & 1, jp & 1, mk[1], u[2], u[3]);
+#pragma unroll
+            for (int x = 0; x < 3; ++x) ue[x] = jlast ? u[0][3 + x] : u[0][x];
+        }
+    }
     if (el) {
         if (PRE) {
 #pragma unroll
@@ -778,6 +861,15 @@ __global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, 
     }
 }
 
+template <class T, int MODE, bool PER>
+void launch_flat(hipStream_t s, const OpArgsT<T> &a, const T *CX)
+{
+    const ModalWork &w = a.mw;
+    const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb));
+    const unsigned ne = 63u * w.NW + 1u;
+    k_modal_flat<T, MODE, PER><<<grid, 64 * w.NW * (w.TI + 1), 9u * (w.TI + 1) * ne * sizeof(T), s>>>(a, w, CX);
+}
+
 template <class T, class TU, int MODE, int EL, bool PER>
 void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX)
 {
@@ -786,8 +878,7 @@ void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX)
     const unsigned ne = 63u * w.NW + 1u;
     if constexpr (EL == 1) {
         if (w.flat && !a.partials) {
-            k_modal_flat<T, MODE, PER>
-                <<<grid, 64 * w.NW * (w.TI + 1), 9u * (w.TI + 1) * ne * sizeof(T), s>>>(a, w, CX);
+            launch_flat<T, MODE, PER>(s, a, CX);
             return;
         }
     }
@@ -812,6 +903,11 @@ void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
     case OP_JACOBI: launch_mode<T, T, OP_JACOBI, EL, false>(s, a, CX); break;
     case OP_PRE_JACOBI: launch_mode<T, T, OP_PRE_JACOBI, EL, false>(s, a, CX); break;
     case OP_PRE_DEFECT: launch_mode<T, T, OP_PRE_DEFECT, EL, false>(s, a, CX); break;
+    case OP_INTERP_JACOBI:
+        // interp_fused (vcycle.h) asks for it only here
+        if (EL != 1 || !a.mw.flat || a.partials) throw std::runtime_error("fused interpolation: tiling");
+        launch_flat<T, OP_INTERP_JACOBI, false>(s, a, CX);
+        break;
     case OP_MATVEC_UF:
         if constexpr (EL == 0 && std::is_same<T, double>::value)
             launch_mode<double, float, OP_MATVEC_UF, 0, false>(s, a, CX);

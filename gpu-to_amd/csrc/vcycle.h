@@ -195,13 +195,41 @@ void sweeps_per(const gputo_handle *h, const HierView<T> &H, int l, const T *F, 
 template <class T>
 bool vcycle_dots(const gputo_handle *h, const HierView<T> &H);
 
-// n damped-Jacobi sweeps on level l ending in U; `pre` forms the first
-// sweep's input as prerelax*F/AD (preRelc, mgcg1.cu:1190-1197); `in_tmp`:
-// the input iterate is in the level's Tmp (an odd n then needs no copy); zr: the
-// last sweep's sums of U.F (vcycle_dots).
 template <class T>
-void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T *U, int n, bool pre, const int *ctl,
-              bool in_tmp = false, double *zr = nullptr)
+int sweeps_of(const gputo_handle *h, int l, bool post);
+
+// Whether the first sweep after level l's coarse correction adds the
+// correction itself (OP_INTERP_JACOBI), which saves a small level a launch
+// (3.1 us) for 1.0-1.4 us: the level-1 operator with a wave group per layer, and
+// node stencils of up to two workgroups per CU (3.8 + 3.2 -> 4.7 us at 637 nodes
+// in FP64, 3.7 + 3.2 -> 4.9 at 4225 in FP32).  A larger one is bound by its
+// bytes and reads each coarse node 27 times: levels of 30625 and 4225 nodes in
+// FP64 went from 7.0 to 13.1 us on average, for interpolations of 3 to 5.
+template <class T>
+bool interp_fused(const gputo_handle *h, const HierView<T> &H, int l)
+{
+    if (l == 0 || H.per || H.mg9 || !preset_of(h->prm).zero_after_interp || sweeps_of<T>(h, l, true) < 1) return false;
+    if (l == 1 && H.l1_mf) return std::is_same<T, double>::value ? h->L[1].mw64.flat : h->L[1].mw32.flat;
+    return H.L[l].S != nullptr && h->L[l].g.nnod <= 2L * 256 * kStencilNodes;
+}
+
+// Where level l's pre-smoothing leaves its iterate: an odd number of post-sweeps
+// whose first one adds the correction starts from Tmp, so the last one writes U
+// without a copy.
+template <class T>
+bool pre_in_tmp(const gputo_handle *h, const HierView<T> &H, int l)
+{
+    return l < h->nl - 1 && interp_fused(h, H, l) && sweeps_of<T>(h, l, true) % 2 == 1;
+}
+
+// n damped-Jacobi sweeps on level l ending in U, alternating with Tmp; `pre`
+// forms the first sweep's input as prerelax*F/AD (preRelc, mgcg1.cu:1190-1197);
+// `in_tmp`: the input iterate is in Tmp (an odd n then needs no copy); zr: the
+// last sweep's sums of U.F (vcycle_dots); Uc: the first sweep's input is the
+// iterate plus P Uc (interp_fused).
+template <class T>
+void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T *U, T *Tmp, int n, bool pre,
+              const int *ctl, bool in_tmp = false, double *zr = nullptr, const T *Uc = nullptr)
 {
     const bool fused = per_fused(h, H, l);
     if (H.per && !fused) return sweeps_per(h, H, l, F, U, n, pre, ctl);
@@ -211,7 +239,7 @@ void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T 
         // pass, where the sweeps from it end in U
         const Preset p = preset_of(h->prm);
         in_tmp = n % 2 == 1;
-        launch_per_jacobi<T>(h->stream, h->L[l].g, in_tmp ? v.Tmp : U, v.R, F, v.AD, h->L[l].mask, p.omega, p.prerelax,
+        launch_per_jacobi<T>(h->stream, h->L[l].g, in_tmp ? Tmp : U, v.R, F, v.AD, h->L[l].mask, p.omega, p.prerelax,
                              1, ctl, H.nb);
         pre = false;
     }
@@ -223,24 +251,25 @@ void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T 
         // 87 us against 22 + 70 us).  It goes where the sweeps end in U.
         in_tmp = n % 2 == 1;
         if (!H.pre0_ready)
-            launch_prerelax<T>(h->stream, F, v.AD, in_tmp ? v.Tmp : U, h->L[l].g.ndof, preset_of(h->prm).prerelax,
+            launch_prerelax<T>(h->stream, F, v.AD, in_tmp ? Tmp : U, h->L[l].g.ndof, preset_of(h->prm).prerelax,
                                ctl, H.nb);
         pre = false;
     }
-    const T *src = in_tmp ? v.Tmp : U;
+    const T *src = in_tmp ? Tmp : U;
     for (int s = 0; s < n; ++s) {
-        T *dst = ((n - 1 - s) % 2 == 0) ? U : v.Tmp;
+        T *dst = ((n - 1 - s) % 2 == 0) ? U : Tmp;
         if (!(pre && s == 0) && dst == src) {
-            launch_copy<T, T>(h->stream, U, v.Tmp, h->L[l].g.ndof, ctl, H.nb);
-            src = v.Tmp;
+            launch_copy<T, T>(h->stream, U, Tmp, h->L[l].g.ndof, ctl, H.nb);
+            src = Tmp;
         }
         OpArgsT<T> a = view_args(h, H, l, ctl);
         a.U = src;
         a.F = F;
         a.out = dst;
         a.per = fused;
+        a.Uc = Uc;
         if (s == n - 1) a.partials = zr;
-        level_op(h, H, l, (pre && s == 0) ? OP_PRE_JACOBI : OP_JACOBI, a);
+        level_op(h, H, l, s > 0 ? OP_JACOBI : (pre ? OP_PRE_JACOBI : (Uc ? OP_INTERP_JACOBI : OP_JACOBI)), a);
         src = dst;
     }
 }
@@ -290,7 +319,9 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
         const LevelView<T> &v = H.L[l];
         const Level &lv = h->L[l];
         const T *F = l == 0 ? F0 : v.F;
-        T *U = l == 0 ? U0 : v.U;
+        T *const Ul = l == 0 ? U0 : v.U;
+        const bool tmp = pre_in_tmp(h, H, l);
+        T *U = tmp ? v.Tmp : Ul, *O = tmp ? Ul : v.Tmp;
         if (l > 0) {
             launch_restrict<T>(h->stream, lv.g, H.L[l - 1].R, v.F, lv.mask, ctl, H.nb);
             if (H.per) launch_per_fold<T>(h->stream, lv.g, v.F, 0, ctl, H.nb);
@@ -307,7 +338,7 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
                 if (npre == 0)
                     launch_per_jacobi<T>(h->stream, lv.g, U, v.R, F, v.AD, lv.mask, p.omega, p.prerelax, 1, ctl, H.nb);
                 else
-                    sweeps_t(h, H, l, F, U, npre, true, ctl);
+                    sweeps_t(h, H, l, F, U, O, npre, true, ctl);
                 OpArgsT<T> a = view_args(h, H, l, ctl);
                 a.U = U;
                 a.F = F;
@@ -319,7 +350,7 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
         } else if (!h->C.direct) {
             // coarsest level too large to factor: 10*npre sweeps from the
             // level's previous iterate (mgcg9.cu:553-563)
-            sweeps_t(h, H, l, F, U, 10 * p.npre, false, ctl);
+            sweeps_t(h, H, l, F, U, O, 10 * p.npre, false, ctl);
         } else {
             launch_coarse_solve<T>(h->stream, h->C, F, U, lv.mask, ctl, H.nb);
             if (H.per) launch_per_bcast<T>(h->stream, lv.g, U, ctl, H.nb);
@@ -333,9 +364,12 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
         // writes U without a copy
         const int npost = sweeps_of<T>(h, l, true);
         const bool to_tmp = (!H.per || per_fused(h, H, l)) && npost % 2 == 1;
-        launch_interp_to<T>(h->stream, h->L[l].g, H.L[l + 1].U, U, to_tmp ? H.L[l].Tmp : U, h->L[l].mask,
-                            p.zero_after_interp, ctl, H.nb);
-        sweeps_t(h, H, l, F, U, npost, false, ctl, to_tmp, l == 0 ? H.zr : nullptr);
+        const bool fused = interp_fused(h, H, l);
+        if (!fused)
+            launch_interp_to<T>(h->stream, h->L[l].g, H.L[l + 1].U, U, to_tmp ? v.Tmp : U, h->L[l].mask,
+                                p.zero_after_interp, ctl, H.nb);
+        sweeps_t(h, H, l, F, U, v.Tmp, npost, false, ctl, to_tmp, l == 0 ? H.zr : nullptr,
+                 fused ? H.L[l + 1].U : nullptr);
         if constexpr (std::is_same<T, float>::value) {
             if (H.learn && l == kLearnLevel) learn_stage(const_cast<gputo_handle *>(h), H, l, F, U, ctl);
         }

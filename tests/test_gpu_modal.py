@@ -137,3 +137,44 @@ def test_periodic_form_is_translation_invariant(gputo, cell):
     assert np.array_equal(u[:, :, 0], u[:, :, -1])
     assert np.array_equal(u[:, :, :, 0], u[:, :, :, -1])
     s.close()
+
+
+@pytest.mark.parametrize("preset", [0, 1])
+@pytest.mark.parametrize("mesh", [(16, 8, 8, 3), (4, 124, 4, 3), (4, 4, 260, 3), (260, 4, 8, 3), (12, 36, 20, 3),
+                                  (16, 16, 16, 4), (72, 56, 40, 4), (112, 96, 48, 5)])
+def test_correction_added_by_the_first_post_sweep(gputo, oracle, mesh, preset):
+    """A V-cycle whose first sweep after a coarse correction adds it (the level-1
+    operator with a wave group per layer, preset 0, and the node stencils), on
+    grids at the edges of the kernels' tiles, with fixed DOFs inside the mesh and
+    at its last node: the oracle's interpolation and sweeps, 1e-9 as the other
+    V-cycle tests."""
+    nelx, nely, nelz, nl = mesh
+    print("case", mesh, preset, flush=True)
+    Ke, F, CX, face = cantilever_case(nelx, nely, nelz, seed=65)
+    last = F.size
+    fixed = np.unique(np.concatenate([face, [last - 1, last, 3 * (last // 3 // 2) + 2]])).astype(np.float64)
+    s = gputo.Solver(nelx, nely, nelz, nl, preset=preset)
+    r = np.random.default_rng(66).uniform(-1, 1, s.ndof)
+    r[(fixed - 1).astype(int)] = 0.0
+    z = s.vcycle(Ke, CX, fixed, r)
+    assert rel(z, oracle.vcycle_once(Ke, CX, fixed, nelx, nely, nelz, nl, r, preset=preset)) < 1e-9
+    s.close()
+
+
+@pytest.mark.parametrize("mesh", [(16, 8, 8, 3), (12, 36, 20, 3), (16, 16, 16, 4), (72, 56, 40, 4)])
+def test_correction_added_by_the_first_post_sweep_fp32(gputo, mesh):
+    """The same in FP32: the mixed solve ends at the FP64 solve's solution within
+    a tenth more iterations (one at least) -- a correction that misses nodes
+    costs several times as many."""
+    nelx, nely, nelz, nl = mesh
+    print("case", mesh, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=65)
+    out = []
+    for precision in (0, 1):
+        s = gputo.Solver(nelx, nely, nelz, nl, precision=precision)
+        U, _, nit, rc = s.solve(Ke, F, CX, fixed, 1e-10, 500)
+        s.close()
+        assert rc == 0
+        out.append((U, nit))
+    assert out[1][1] <= out[0][1] + max(1, out[0][1] // 10)
+    assert rel(out[1][0], out[0][0]) < 1e-8
