@@ -16,7 +16,9 @@
 // scalars.  That takes two one-block launches of 2.8-4.5 us out of an
 // iteration.  No block reads a field that its own kernel writes: rho (read
 // for alpha) is written with beta, rho_p (read for beta) with alpha.  The
-// check stays a launch of its own: the V-cycle's kernels all need its answer.
+// check is a block of the V-cycle's first level-0 launch where that is a modal
+// kernel in a prerelaxed mode (as a launch: 2.7 us).  Its other blocks may or may not see a flag that
+// is set meanwhile; what they write at convergence is not read any more.
 //
 // Sums are two-stage with fixed grids and fixed orders, so results do not
 // depend on timing; products and sums are FP64 for both vector types.  The
@@ -256,39 +258,13 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_update_r(double *__restrict__
     if (threadIdx.x == 0) rr[blockIdx.x] = s;
 }
 
-// The residual test.  prog (pinned host memory, one word per right-hand side)
-// tells the host how far the iteration is: iterations tested << 1 | converged
-// in the low half, the relative residual in FP32 in the high half; one 64-bit
-// store, so the host never sees them apart.
-__global__ __launch_bounds__(kBlock) void k_cg_check(CgScalars *sc, const double *p, int n, double tol,
-                                                    unsigned long long *prog)
+// the residual test of a launch of its own (batches, level-0 kernels without it)
+__global__ __launch_bounds__(64) void k_cg_check(CgTest t)
 {
-    sc += blockIdx.z;
-    p += (long)blockIdx.z * n;
-    const double res0 = sc->res0;
-    int done = sc->done;
-    const int it = sc->it;
-    const double rr = cg_partials<kBlock>(p, n);
-    if (threadIdx.x) return;
-    double rel = sc->relres;
-    if (!done) {
-        rel = sqrt(rr) / res0;
-        sc->rr = rr;
-        sc->relres = rel;
-        if (!(rel < INFINITY)) {
-            sc->bad = 1;
-            done = 1;
-        } else if (rel < tol) {
-            done = 1;
-        }
-        if (done) {
-            sc->done = 1;
-            sc->nit = it;
-        }
-    }
-    const unsigned long long w =
-        ((unsigned long long)__builtin_bit_cast(unsigned, (float)rel) << 32) | ((unsigned)(it + 1) << 1) | (unsigned)done;
-    __hip_atomic_store(&prog[blockIdx.z], w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    t.sc += blockIdx.z;
+    t.rr += (long)blockIdx.z * t.n;
+    t.prog += blockIdx.z;
+    cg_test(t);
 }
 
 // sums of r.z at dots[0..blocks) and, FLEX, of q.z after them
@@ -448,10 +424,18 @@ void launch_cg_update_r(hipStream_t s, double *R, const double *Q, long n, CgSca
                                                                  0.0f);
 }
 
-void launch_cg_check(hipStream_t s, CgScalars *sc, const double *rr, long n, double tol, unsigned long long *prog, int nb)
+CgTest cg_test_of(CgScalars *sc, const double *rr, long n, double tol, unsigned long long *prog)
 {
-    k_cg_check<<<dim3(1, 1, batch_dim(nb)), kBlock, 0, s>>>(sc, rr, cg_blocks(n), tol, prog);
+    CgTest t;
+    t.sc = sc;
+    t.rr = rr;
+    t.n = cg_blocks(n);
+    t.tol = tol;
+    t.prog = prog;
+    return t;
 }
+
+void launch_cg_check(hipStream_t s, const CgTest &t, int nb) { k_cg_check<<<dim3(1, 1, batch_dim(nb)), 64, 0, s>>>(t); }
 
 template <class TP, class TZ>
 void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const double *q, TP *Pout, const TP *Pin, long n,

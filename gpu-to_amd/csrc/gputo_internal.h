@@ -72,35 +72,55 @@ bool modal_constants(const double *Ke0, double *C);      // C[8]; false: Ke0 has
 Tile choose_tile(const Grid &g);   // level-0 node-gather bricks
 Tile stored_tile(const Grid &g);   // stored-matrix operator (at most kStNodes nodes)
 
-// Arguments of the node-gather operator kernels (T = double or float).
+struct CgScalars;
+// The residual test of a PCG iteration: the sums of r.r (n <= 256 of them) and
+// the pinned progress word it is reported in.
+struct CgTest {
+    CgScalars *sc = nullptr;  // null: no test
+    const double *rr = nullptr;
+    int n = 0;
+    double tol = 0.0;
+    unsigned long long *prog = nullptr;
+};
+
+// Arguments of the operator kernels (T = double or float).  A kernel takes the
+// smallest part that it reads: a small level's launch is short enough for the
+// lines of its argument buffer to show (48 bytes more: 7.12 -> 7.26 us per FP32
+// level-0 sweep at 96x48x48, 4.73 -> 4.86 per level-1 sweep).
 template <class T>
-struct OpArgsT {
+struct OpStencil {  // k_stencil
     Grid g;
+    const T *U;            // input vector
+    const T *F;            // right-hand side (defect / Jacobi)
+    T *out;                // result vector
+    const T *S;            // assembled node stencils [14][3][3][stencil_ld] of the same operator, or null
+    const T *AD;           // diagonal (Jacobi)
+    const uint8_t *mask;   // per node: bit d set when DOF 3n+d is fixed
+    const int *ctl;        // ctl[0] != 0: skip (converged)
+    const T *Uc;           // OP_INTERP_JACOBI: the coarse level's correction
+    T *out2;               // second result (prerelax+defect writes U and R)
+    double omega, prerelax;
+};
+template <class T>
+struct OpModal : OpStencil<T> {  // k_modal, k_modal_flat
+    const T *RD;           // 1/AD for the modal kernels (null: no Jacobi or prerelaxed mode): one value per
+                           // node where Ke0 has one diagonal value, per DOF for the level-1 operator
+    double *partials;      // per-block partial sums (fused dot), may be null
+    ModalWork mw;          // the level's tiling
+    T mc[8];               // modal constants of Ke0
+    double cx_floor;       // > 0: element scales below it count as 0 (mgcg9 smoother defect)
+    const float *Uf;       // OP_MATVEC_UF: the input vector in FP32
+};
+template <class T>
+struct OpArgsT : OpModal<T> {
     Tile t;
     const T *Ke;           // 24x24 row-major (level 0)
     const T *CX;           // element scale (level 0)
     const T *A;            // packed 300 x nel entry-major element matrices (levels >= 1)
-    const T *S;            // assembled node stencils [14][3][3][stencil_ld] of the same operator, or null
-    const T *U;            // input vector
-    const T *F;            // right-hand side (defect / Jacobi)
-    const T *Uc;           // OP_INTERP_JACOBI: the coarse level's correction
-    const T *AD;           // diagonal (Jacobi)
-    const T *RD;           // 1/AD for the modal kernels (null: no Jacobi or prerelaxed mode): one value per
-                           // node where Ke0 has one diagonal value, per DOF for the level-1 operator
-    const uint8_t *mask;   // per node: bit d set when DOF 3n+d is fixed
-    T *out;                // result vector
-    T *out2;               // second result (prerelax+defect writes U and R)
-    double *partials;      // per-block partial sums (fused dot), may be null
-    const float *Uf;       // OP_MATVEC_UF: the input vector in FP32
-    const int *ctl;        // ctl[0] != 0: skip (converged)
     int nb;                // right-hand sides of a batched launch (0 or 1: one)
-    double omega, prerelax;
-    double cx_floor;       // > 0: element scales below it count as 0 (mgcg9 smoother defect)
     int kc;                // Ke0 has the unit-H8 class structure: use kv
     T kv[kKeMaxClasses];   // value of each Ke0 entry class (kKeClass)
     int modal;             // Ke0 has the isotropic modal form: use mc and mw
-    T mc[8];               // its modal constants
-    ModalWork mw;          // the level's tiling
     int per;               // modal kernels: periodic cell, the result complete on masters and images
 };
 using OpArgs = OpArgsT<double>;
@@ -125,6 +145,51 @@ struct CgScalars {
     int nru;         // replacements done
 };
 
+// The residual test, by one wave.  prog (pinned host memory) tells the host how
+// far the iteration is: iterations tested << 1 | converged in the low half, the
+// relative residual in FP32 in the high half; one 64-bit store, so the host never
+// sees them apart.
+constexpr int kCgBlocks = 256;  // blocks (= partial sums) of the PCG's reductions at most
+__device__ __forceinline__ void cg_test(const CgTest &t)
+{
+    CgScalars *sc = t.sc;
+    const double res0 = sc->res0;
+    int done = sc->done;
+    const int it = sc->it;
+    double v[kCgBlocks / 64], rr = 0.0;
+#pragma unroll
+    for (int q = 0; q < kCgBlocks / 64; ++q) {
+        const int i = 64 * q + (int)(threadIdx.x & 63);
+        v[q] = i < t.n ? t.rr[i] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < kCgBlocks / 64; ++q) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) v[q] += __shfl_xor(v[q], off, 64);
+        rr += v[q];
+    }
+    if (threadIdx.x) return;
+    double rel = sc->relres;
+    if (!done) {
+        rel = sqrt(rr) / res0;
+        sc->rr = rr;
+        sc->relres = rel;
+        if (!(rel < INFINITY)) {
+            sc->bad = 1;
+            done = 1;
+        } else if (rel < t.tol) {
+            done = 1;
+        }
+        if (done) {
+            sc->done = 1;
+            sc->nit = it;
+        }
+    }
+    const unsigned long long w =
+        ((unsigned long long)__builtin_bit_cast(unsigned, (float)rel) << 32) | ((unsigned)(it + 1) << 1) | (unsigned)done;
+    __hip_atomic_store(t.prog, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Batched launches: several right-hand sides on one hierarchy, one per
 // blockIdx.z.  The vectors of a batch follow each other with the level's DOF
 // count (or the vector length n) as stride, each right-hand side has its own
@@ -148,7 +213,7 @@ __host__ __device__ inline long coarse_ndof(const Grid &g)
     return 3L * (g.nx / 2 + 1) * (g.ny / 2 + 1) * (g.nz / 2 + 1);
 }
 template <class T>
-__device__ __forceinline__ void batch_shift(OpArgsT<T> &a)
+__device__ __forceinline__ void batch_shift(OpStencil<T> &a)
 {
     const long st = a.g.ndof;
     a.U = batch_ptr(a.U, st);
@@ -156,8 +221,13 @@ __device__ __forceinline__ void batch_shift(OpArgsT<T> &a)
     a.Uc = batch_ptr(a.Uc, coarse_ndof(a.g));
     a.out = batch_ptr(a.out, st);
     a.out2 = batch_ptr(a.out2, st);
-    a.partials = batch_ptr(a.partials, (long)gridDim.x);
     a.ctl = batch_ctl(a.ctl);
+}
+template <class T>
+__device__ __forceinline__ void batch_shift(OpModal<T> &a)
+{
+    batch_shift(static_cast<OpStencil<T> &>(a));
+    a.partials = batch_ptr(a.partials, (long)gridDim.x);
 }
 // values of OpArgsT::RD on level l: per node, per DOF on level 1 (which may be
 // the rediscretised one); it follows AD in one allocation
@@ -297,9 +367,10 @@ struct gputo_handle {
 namespace gputo {
 
 // ---- launch helpers (kernels.hip) ------------------------------------
-template <class T> void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a);
+template <class T> void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a, const CgTest *test = nullptr);
 void launch_op0_uf(hipStream_t s, const OpArgs &a);  // OP_MATVEC_UF
-template <class T> void launch_op0_modal(hipStream_t s, int mode, const OpArgsT<T> &a);
+// test: the PCG's residual test, run by a block of its own (the prerelaxed modes)
+template <class T> void launch_op0_modal(hipStream_t s, int mode, const OpArgsT<T> &a, const CgTest *test = nullptr);
 // whether launch_op0 takes the modal kernel for `mode`, and the blocks
 // (= partial sums per right-hand side) of its launch
 template <class T>
@@ -390,7 +461,6 @@ void launch_coarse_solve(hipStream_t s, const Coarse &C, const T *b, T *x, const
 // Steps of the PCG (cg.hip).  pq: npq per-block sums of p.q; rr, dots: room
 // for kCgBlocks (2 kCgBlocks, flexible beta) sums per right-hand side, apart
 // from pq.
-constexpr int kCgBlocks = 256;  // most blocks of a CG reduction
 constexpr int kCgFuse = 2048;   // most sums that every block of an update reads (2.4 % of a solve with 1100, 2 % with 1300)
 // U = 0, R = F (R32, X0 as launch_cg_update_r) and the first residual norm
 void launch_cg_start(hipStream_t s, const double *F, double *U, double *R, long n, CgScalars *sc, double *rr,
@@ -414,8 +484,8 @@ void launch_cg_update_r(hipStream_t s, double *R, const double *Q, long n, CgSca
                         double prerelax = 0.0);
 void launch_cg_flush_u(hipStream_t s, double *U, const float *P, long n, const double *alog, int m);
 // residual test from the sums of an update over n elements
-void launch_cg_check(hipStream_t s, CgScalars *sc, const double *rr, long n, double tol, unsigned long long *prog,
-                     int nb = 1);
+CgTest cg_test_of(CgScalars *sc, const double *rr, long n, double tol, unsigned long long *prog);
+void launch_cg_check(hipStream_t s, const CgTest &t, int nb = 1);
 // dots of z and Pout = z + beta Pin (flex: Polak-Ribiere beta)
 template <class TP, class TZ>
 void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const double *q, TP *Pout, const TP *Pin, long n,

@@ -292,9 +292,9 @@ __global__ __launch_bounds__(kBlock) void k_gather(OpArgsT<T> a)
 }
 
 template <class T>
-void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a)
+void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a, const CgTest *test)
 {
-    if (op0_is_modal(a, mode)) return launch_op0_modal<T>(s, mode, a);
+    if (op0_is_modal(a, mode)) return launch_op0_modal<T>(s, mode, a, test);
     const dim3 grid((unsigned)xcd_launch(a.t.blocks()), 1, batch_dim(a.nb)), block(kBlock);
     if (a.kc) {
         switch (mode) {
@@ -371,7 +371,7 @@ struct Prolong {
 // the small coarse levels, whose cost is load latency, occupied.
 // ---------------------------------------------------------------------------
 template <class T, int MODE>
-__device__ __forceinline__ T stored_u(const OpArgsT<T> &a, long dof)
+__device__ __forceinline__ T stored_u(const OpStencil<T> &a, long dof)
 {
     if (MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT) return T(a.prerelax) * a.F[dof] / a.AD[dof];
     return a.U[dof];
@@ -544,7 +544,7 @@ void launch_stencil_build(hipStream_t s, const Grid &g, const double *A, double 
 constexpr int kStThreads = kStencilNodes * 28;  // 27 blocks, and a full last wave
 
 template <class T, int MODE>
-__global__ __launch_bounds__(kStThreads) void k_stencil(OpArgsT<T> a)
+__global__ __launch_bounds__(kStThreads) void k_stencil(OpStencil<T> a)
 {
     batch_shift(a);
     __shared__ T red[27][kStencilNodes][3];
@@ -659,7 +659,7 @@ void launch_opA(hipStream_t s, int mode, const OpArgsT<T> &a)
     default: break;
     }
 }
-template void launch_op0<double>(hipStream_t, int, const OpArgsT<double> &);
+template void launch_op0<double>(hipStream_t, int, const OpArgsT<double> &, const CgTest *);
 
 void launch_op0_uf(hipStream_t s, const OpArgs &a)
 {
@@ -670,7 +670,7 @@ void launch_op0_uf(hipStream_t s, const OpArgs &a)
     else
         k_gather<double, OP_MATVEC_UF, false><<<grid, block, 0, s>>>(a);
 }
-template void launch_op0<float>(hipStream_t, int, const OpArgsT<float> &);
+template void launch_op0<float>(hipStream_t, int, const OpArgsT<float> &, const CgTest *);
 template void launch_opA<double>(hipStream_t, int, const OpArgsT<double> &);
 template void launch_opA<float>(hipStream_t, int, const OpArgsT<float> &);
 

@@ -42,7 +42,7 @@ void mixed_begin(gputo_handle *h);                                        // FP3
 // pre0_ready: the prerelaxed level-0 iterate is already in
 // mixed_prerelax_target(h) (formed from mixed_r32(h) by the caller)
 void mixed_vcycle(gputo_handle *h, const double *r, double *z, const int *ctl, bool r32_ready = false,
-                  bool pre0_ready = false);
+                  bool pre0_ready = false, const CgTest &test = CgTest());
 // Where the FP32 V-cycle's first level-0 pass writes the prerelaxed iterate
 // prerelax*F/AD (its sweeps then start from it), with that AD and prerelax;
 // null when the V-cycle does not start with that pass.
@@ -54,7 +54,8 @@ float *mixed_prerelax_target(gputo_handle *h, const float **ad, double *prerelax
 // Results equal mixed_vcycle's bit for bit.  The graph holds the
 // hierarchy's pointers and values: it is dropped by mixed_begin, mixed_end
 // and mixed_graph_drop.
-void mixed_vcycle_graph(gputo_handle *h, const int *ctl, bool pre0_ready = false);
+void mixed_vcycle_graph(gputo_handle *h, const int *ctl, bool pre0_ready = false, const CgTest &test = CgTest());
+bool mixed_tests(gputo_handle *h);  // whether its V-cycles run the residual test (vcycle_tests)
 void mixed_graph_drop(gputo_handle *h);
 float *mixed_r32(gputo_handle *h);        // the FP32 right-hand side of the V-cycle
 const float *mixed_z32(gputo_handle *h);  // the FP32 result of the last V-cycle

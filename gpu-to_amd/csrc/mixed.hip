@@ -170,15 +170,18 @@ static void mixed_prepare(gputo_handle *h)
 // z = V(r) with the FP32 V-cycle: r (FP64) is rounded to FP32, the whole
 // cycle runs on the FP32 copies of the hierarchy (FP64 coarsest Cholesky
 // inside), and z is widened back to FP64 for the FP64 Krylov recurrences.
-void mixed_vcycle(gputo_handle *h, const double *r, double *z, const int *ctl, bool r32_ready, bool pre0_ready)
+void mixed_vcycle(gputo_handle *h, const double *r, double *z, const int *ctl, bool r32_ready, bool pre0_ready,
+                  const CgTest &test)
 {
     MixedState *m = h->mx;
     hipStream_t s = h->stream;
     const long n = h->L[0].g.ndof;
     if (!r32_ready) launch_copy<double, float>(s, r, m->R, n, ctl);
     m->H.pre0_ready = pre0_ready;
+    m->H.test = test;
     vcycle_t<float>(h, m->H, m->R, m->Z, ctl);
     m->H.pre0_ready = false;
+    m->H.test = CgTest();
     if (z) launch_copy<float, double>(s, m->Z, z, n, ctl);
 }
 
@@ -203,13 +206,15 @@ void mixed_graph_drop(gputo_handle *h)
     m->vc_exec = nullptr;
 }
 
-void mixed_vcycle_graph(gputo_handle *h, const int *ctl, bool pre0_ready)
+bool mixed_tests(gputo_handle *h) { return vcycle_tests(h, h->mx->H); }
+
+void mixed_vcycle_graph(gputo_handle *h, const int *ctl, bool pre0_ready, const CgTest &test)
 {
     MixedState *m = h->mx;
     hipStream_t s = h->stream;
     const int kind = m->H.learn ? learn_stage_kind(h) : 0;
     if (kind < 0) {
-        mixed_vcycle(h, nullptr, nullptr, ctl, true, pre0_ready);
+        mixed_vcycle(h, nullptr, nullptr, ctl, true, pre0_ready, test);
         return;
     }
     if (!m->vc_exec || kind != m->vc_kind || ctl != m->vc_ctl || pre0_ready != m->vc_pre0) {
@@ -219,9 +224,10 @@ void mixed_vcycle_graph(gputo_handle *h, const int *ctl, bool pre0_ready)
         hipGraph_t g = nullptr;
         check_hip(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "graph capture");
         try {
-            mixed_vcycle(h, nullptr, nullptr, ctl, true, pre0_ready);
+            mixed_vcycle(h, nullptr, nullptr, ctl, true, pre0_ready, test);
         } catch (...) {
             m->H.pre0_ready = false;
+            m->H.test = CgTest();
             (void)hipStreamEndCapture(s, &g);
             if (g) (void)hipGraphDestroy(g);
             throw;
@@ -252,6 +258,7 @@ void mixed_begin(gputo_handle *h)
     mixed_graph_drop(h);
     mixed_prepare(h);
     h->mx->H.pre0_ready = false;
+    h->mx->H.test = CgTest();
 }
 
 void mixed_end(gputo_handle *h, int nit, int converged)

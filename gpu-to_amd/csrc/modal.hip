@@ -364,10 +364,25 @@ constexpr int md_min_waves()
     return sizeof(T) == 8 ? (EL == 0 ? 2 : 1) : (EL == 0 ? 4 : 3);
 }
 
+// Whether a launch may carry the PCG's residual test: the prerelaxed modes, which
+// start a V-cycle.  (The FP32 cycle of a mixed solve starts with a plain sweep;
+// with the test in that kernel too its solves were 1 to 1.5 % slower.)  The
+// test goes first, and seven idle blocks behind it keep the tiles on their XCDs.
+constexpr unsigned kMdTestBlocks = 8;
+template <int MODE, int EL, bool PER>
+constexpr bool md_tests()
+{
+    return EL == 0 && !PER && (MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT);
+}
+struct MdNoTest {};
+template <int MODE, int EL, bool PER>
+using MdTest = std::conditional_t<md_tests<MODE, EL, PER>(), CgTest, MdNoTest>;
+
 template <class T, class TU, int MODE, int EL, bool PER>
 __global__ __launch_bounds__((sizeof(T) == 8 && EL == 1 ? 4 : kMdMaxWaves) * 64) __attribute__((amdgpu_waves_per_eu(md_min_waves<T, EL>())))
-void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
+void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
 {
+    const ModalWork &w = a.mw;
     constexpr bool PRE = MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT;
     constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI;
     constexpr bool MV = MODE == OP_MATVEC || MODE == OP_MATVEC_UF;
@@ -377,6 +392,16 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     // allow it
     constexpr bool AHEAD = sizeof(T) == 4 ? !PRE : (EL == 0 && !PRE);
     constexpr int SU = (int)sizeof(TU), S = (int)sizeof(T);
+    unsigned bx = blockIdx.x;
+    if constexpr (md_tests<MODE, EL, PER>()) {
+        if (test.sc) {
+            if (bx < kMdTestBlocks) {
+                if (bx == 0 && threadIdx.x < 64) cg_test(test);
+                return;
+            }
+            bx -= kMdTestBlocks;
+        }
+    }
     batch_shift(a);
     if (MODE == OP_MATVEC_UF) a.Uf = batch_ptr(a.Uf, a.g.ndof);
     extern __shared__ double md_lds[];
@@ -384,9 +409,9 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     const int ne = 63 * w.NW + 1;
     const Grid &g = a.g;
     const unsigned nb = (unsigned)w.blocks();
-    const unsigned tb = (unsigned)xcd_tile(blockIdx.x, nb);
+    const unsigned tb = (unsigned)xcd_tile(bx, nb);
     if (tb >= nb) {  // padding block of the XCD order
-        if (a.partials && threadIdx.x == 0) a.partials[blockIdx.x] = 0.0;
+        if (a.partials && threadIdx.x == 0) a.partials[bx] = 0.0;
         return;
     }
     const int ch = (int)(tb % (unsigned)w.nch);
@@ -395,7 +420,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
     // owned node layers (PER: masters only)
     const int i0 = ib * w.TI, i1 = min(i0 + w.TI, PER ? g.nx : g.nnx);
     if (PER && i0 >= i1) {
-        if (a.partials && threadIdx.x == 0) a.partials[blockIdx.x] = 0.0;
+        if (a.partials && threadIdx.x == 0) a.partials[bx] = 0.0;
         return;
     }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -631,7 +656,7 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
         if (threadIdx.x == 0) {
             double v = 0.0;
             for (int q = 0; q < w.NW; ++q) v += ws[q];
-            a.partials[blockIdx.x] = v;
+            a.partials[bx] = v;
         }
     }
 }
@@ -654,8 +679,9 @@ void k_modal(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
 constexpr int kMdFlatWaves = 8;
 
 template <class T, int MODE, bool PER>
-__global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpArgsT<T> a, ModalWork w, const T *__restrict__ CX)
+__global__ __launch_bounds__(kMdFlatWaves * 64) void k_modal_flat(OpModal<T> a, const T *__restrict__ CX)
 {
+    const ModalWork &w = a.mw;
     constexpr bool PRE = MODE == OP_PRE_JACOBI || MODE == OP_PRE_DEFECT;
     constexpr bool INT = MODE == OP_INTERP_JACOBI;
     constexpr bool JAC = MODE == OP_JACOBI || MODE == OP_PRE_JACOBI || INT;
@@ -867,14 +893,22 @@ void launch_flat(hipStream_t s, const OpArgsT<T> &a, const T *CX)
     const ModalWork &w = a.mw;
     const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb));
     const unsigned ne = 63u * w.NW + 1u;
-    k_modal_flat<T, MODE, PER><<<grid, 64 * w.NW * (w.TI + 1), 9u * (w.TI + 1) * ne * sizeof(T), s>>>(a, w, CX);
+    k_modal_flat<T, MODE, PER><<<grid, 64 * w.NW * (w.TI + 1), 9u * (w.TI + 1) * ne * sizeof(T), s>>>(a, CX);
 }
 
 template <class T, class TU, int MODE, int EL, bool PER>
-void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX)
+void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX, const CgTest *tst = nullptr)
 {
     const ModalWork &w = a.mw;
-    const dim3 grid((unsigned)xcd_launch(w.blocks()), 1, batch_dim(a.nb));
+    MdTest<MODE, EL, PER> test{};
+    unsigned tests = 0;
+    if constexpr (md_tests<MODE, EL, PER>()) {
+        if (tst && tst->sc) {
+            test = *tst;
+            tests = kMdTestBlocks;
+        }
+    }
+    const dim3 grid((unsigned)xcd_launch(w.blocks()) + tests, 1, batch_dim(a.nb));
     const unsigned ne = 63u * w.NW + 1u;
     if constexpr (EL == 1) {
         if (w.flat && !a.partials) {
@@ -882,11 +916,11 @@ void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX)
             return;
         }
     }
-    k_modal<T, TU, MODE, EL, PER><<<grid, 64 * w.NW, 6u * ne * sizeof(T), s>>>(a, w, CX);
+    k_modal<T, TU, MODE, EL, PER><<<grid, 64 * w.NW, 6u * ne * sizeof(T), s>>>(a, CX, test);
 }
 
 template <class T, int EL>
-void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
+void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX, const CgTest *test = nullptr)
 {
     if (a.per) {
         switch (mode) {
@@ -901,8 +935,8 @@ void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
     case OP_MATVEC: launch_mode<T, T, OP_MATVEC, EL, false>(s, a, CX); break;
     case OP_DEFECT: launch_mode<T, T, OP_DEFECT, EL, false>(s, a, CX); break;
     case OP_JACOBI: launch_mode<T, T, OP_JACOBI, EL, false>(s, a, CX); break;
-    case OP_PRE_JACOBI: launch_mode<T, T, OP_PRE_JACOBI, EL, false>(s, a, CX); break;
-    case OP_PRE_DEFECT: launch_mode<T, T, OP_PRE_DEFECT, EL, false>(s, a, CX); break;
+    case OP_PRE_JACOBI: launch_mode<T, T, OP_PRE_JACOBI, EL, false>(s, a, CX, test); break;
+    case OP_PRE_DEFECT: launch_mode<T, T, OP_PRE_DEFECT, EL, false>(s, a, CX, test); break;
     case OP_INTERP_JACOBI:
         // interp_fused (vcycle.h) asks for it only here
         if (EL != 1 || !a.mw.flat || a.partials) throw std::runtime_error("fused interpolation: tiling");
@@ -919,12 +953,12 @@ void launch(hipStream_t s, int mode, const OpArgsT<T> &a, const T *CX)
 }  // namespace
 
 template <class T>
-void launch_op0_modal(hipStream_t s, int mode, const OpArgsT<T> &a)
+void launch_op0_modal(hipStream_t s, int mode, const OpArgsT<T> &a, const CgTest *test)
 {
-    launch<T, 0>(s, mode, a, a.CX);
+    launch<T, 0>(s, mode, a, a.CX, test);
 }
-template void launch_op0_modal<double>(hipStream_t, int, const OpArgsT<double> &);
-template void launch_op0_modal<float>(hipStream_t, int, const OpArgsT<float> &);
+template void launch_op0_modal<double>(hipStream_t, int, const OpArgsT<double> &, const CgTest *);
+template void launch_op0_modal<float>(hipStream_t, int, const OpArgsT<float> &, const CgTest *);
 
 template <class T>
 void launch_op1_mf(hipStream_t s, int mode, OpArgsT<T> a, const T *CXf, double nu)

@@ -256,10 +256,11 @@ HierView<double> f64_view(const gputo_handle *h)
 
 OpArgs op_args(const gputo_handle *h, int l) { return view_args(h, f64_view(h), l, &h->sc->done); }
 
-void vcycle(gputo_handle *h, const double *F0, double *U0, double *zr = nullptr)
+void vcycle(gputo_handle *h, const double *F0, double *U0, double *zr = nullptr, const CgTest &test = CgTest())
 {
     HierView<double> H = f64_view(h);
     H.zr = zr;
+    H.test = test;
     vcycle_t(h, H, F0, U0, &h->sc->done);
 }
 
@@ -496,12 +497,12 @@ static bool custom_schedule(const gputo_params &p)
 // Device-resident PCG (mgcg1.cu:235-280); U, F on the device.
 // z = M r: the FP64 V-cycle, or the FP32 V-cycle of the mixed precisions
 static void precond(gputo_handle *h, const double *r, double *z, bool r32_ready = false, bool pre0_ready = false,
-                    double *zr = nullptr)
+                    double *zr = nullptr, const CgTest &test = CgTest())
 {
     if (h->prm.precision == GPUTO_PREC_F64)
-        vcycle(h, r, z, zr);
+        vcycle(h, r, z, zr, test);
     else
-        mixed_vcycle(h, r, z, &h->sc->done, r32_ready, pre0_ready);
+        mixed_vcycle(h, r, z, &h->sc->done, r32_ready, pre0_ready, test);
 }
 
 // Wait until every right-hand side's progress word shows `seq` tested
@@ -560,7 +561,11 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
     // FP64: the V-cycle's last sweep leaves the sums of r.z where the matvec left
     // those of p.q (read by then)
     double *zr = h->prm.precision == GPUTO_PREC_F64 && !flex && vcycle_dots(h, f64_view(h)) ? h->partials : nullptr;
+    // the V-cycle's first sweep runs the residual test
+    const bool tests = h->prm.precision == GPUTO_PREC_F64 ? vcycle_tests(h, f64_view(h)) : mixed_tests(h);
+    const CgTest test = cg_test_of(h->sc, h->rr, h->L[0].g.ndof, tol, h->prog);
     auto precond_n = [&](const double *r, double *z, bool r32_ready) {
+        const CgTest tv = tests && vcycles > 0 ? test : CgTest();  // the first one precedes the first update
         if (h->prm.coarse_lag >= 2 && vcycles == h->prm.coarse_lag) {
             coarse_switch(h->C, s);
             if (graphs) mixed_graph_drop(h);  // it holds the previous factor
@@ -569,9 +574,9 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
         // (the first V-cycle, launched from the host, holds the wait for the
         // coarsest factorisation)
         if (graphs && vcycles > 0 && r32_ready && !z)
-            mixed_vcycle_graph(h, &h->sc->done, pre0);
+            mixed_vcycle_graph(h, &h->sc->done, pre0, tv);
         else
-            precond(h, r, z, r32_ready, pre0, zr);
+            precond(h, r, z, r32_ready, pre0, zr, tv);
         ++vcycles;
     };
     // ... and then keeps the search direction in FP32: p = z + beta p formed
@@ -609,9 +614,10 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
         precond_n(h->R, h->P, false);
         launch_cg_rho<double>(s, h->R, h->P, n, h->sc, dots);
     }
-    // Iteration k is enqueued in two halves: the matvec, update and residual
-    // test, then the V-cycle and the new direction.  Before the second half the
-    // host waits for the test of iteration k - 1 (a word in pinned memory; the
+    // Iteration k is enqueued in two halves: the matvec and update, then the
+    // residual test (a launch, or part of the V-cycle's first one), the V-cycle and
+    // the new direction.  Before the second half the host waits for the test of
+    // iteration k - 1 (a word in pinned memory; the
     // device is then at the start of that iteration's V-cycle), so the stream
     // always holds about one iteration of work and never drains, and at
     // convergence one enqueued iteration skips its work.
@@ -646,7 +652,7 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
         } else {
             launch_cg_update_ur(s, U, h->R, h->P, h->Q, n, h->sc, h->partials, nmv, rr, r32);
         }
-        launch_cg_check(s, h->sc, rr, n, tol, h->prog);
+        if (!tests) launch_cg_check(s, test);
         ++enq;
         HIPCHK(hipGetLastError());
         if (enq > 1) {
@@ -830,7 +836,7 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
         launch_op0(s, OP_MATVEC, a);
         if (per && !a.per) launch_per_fold<double>(s, L0.g, b.Q, 0, ctl, nb);
         launch_cg_update_ur(s, U, b.R, b.P, b.Q, n, b.sc, b.partials, nmv, rr, r32, nb);
-        launch_cg_check(s, b.sc, rr, n, tol, h->prog, nb);
+        launch_cg_check(s, cg_test_of(b.sc, rr, n, tol, h->prog), nb);
         ++enq;
         HIPCHK(hipGetLastError());
         if (enq > 1 && cg_wait(s, h->prog, nb, enq - 1, nullptr)) break;

@@ -78,6 +78,7 @@ struct HierView {
     bool pre0_ready = false;       // level 0's prerelaxed iterate is already formed (by the caller)
     int nb = 1;                    // right-hand sides: level vectors hold nb vectors each, one after another
     double *zr = nullptr;          // result.F0 per block of the last sweep (vcycle_dots)
+    CgTest test;                   // residual test that the first level-0 sweep runs (vcycle_tests)
 };
 
 constexpr int kLearnLevel = 2;
@@ -137,10 +138,11 @@ OpArgsT<T> view_args(const gputo_handle *h, const HierView<T> &H, int l, const i
 }
 
 template <class T>
-void level_op(const gputo_handle *h, const HierView<T> &H, int l, int mode, const OpArgsT<T> &a)
+void level_op(const gputo_handle *h, const HierView<T> &H, int l, int mode, const OpArgsT<T> &a,
+              const CgTest *test = nullptr)
 {
     if (H.mg9) {
-        launch_op0<T>(h->stream, mode, a);  // level scales and the CX floor are in a
+        launch_op0<T>(h->stream, mode, a, test);  // level scales and the CX floor are in a
     } else if (l == 1 && H.l1_mf) {
         launch_op1_mf<T>(h->stream, mode, a, H.CX, kL1Nu);
     } else if (l > 0) {
@@ -149,9 +151,9 @@ void level_op(const gputo_handle *h, const HierView<T> &H, int l, int mode, cons
         if (H.l0 >= L0_MFMA_F32 && H.l0 != L0_MODAL)
             launch_op0_mfma(h->stream, mode, a, H.l0_ctx, H.l0 - L0_MFMA_F32);
         else
-            launch_op0<T>(h->stream, mode, a);
+            launch_op0<T>(h->stream, mode, a, test);
     } else {
-        launch_op0<T>(h->stream, mode, a);
+        launch_op0<T>(h->stream, mode, a, test);
     }
 }
 
@@ -198,6 +200,16 @@ bool vcycle_dots(const gputo_handle *h, const HierView<T> &H);
 template <class T>
 int sweeps_of(const gputo_handle *h, int l, bool post);
 
+// Whether the V-cycle's first level-0 operator can run the PCG's residual test
+// (CgTest): a modal kernel that forms the prerelaxed iterate itself (the
+// FP32 cycles but mgcg9's have it formed by the residual update).
+template <class T>
+bool vcycle_tests(const gputo_handle *h, const HierView<T> &H)
+{
+    if (h->nl < 2 || H.per || H.nb > 1 || !op0_is_modal(view_args(h, H, 0, nullptr), OP_JACOBI)) return false;
+    return std::is_same<T, double>::value || H.mg9;
+}
+
 // Whether the first sweep after level l's coarse correction adds the
 // correction itself (OP_INTERP_JACOBI), which saves a small level a launch
 // (3.1 us) for 1.0-1.4 us: the level-1 operator with a wave group per layer, and
@@ -226,10 +238,11 @@ bool pre_in_tmp(const gputo_handle *h, const HierView<T> &H, int l)
 // forms the first sweep's input as prerelax*F/AD (preRelc, mgcg1.cu:1190-1197);
 // `in_tmp`: the input iterate is in Tmp (an odd n then needs no copy); zr: the
 // last sweep's sums of U.F (vcycle_dots); Uc: the first sweep's input is the
-// iterate plus P Uc (interp_fused).
+// iterate plus P Uc (interp_fused); test: run by the first sweep.
 template <class T>
 void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T *U, T *Tmp, int n, bool pre,
-              const int *ctl, bool in_tmp = false, double *zr = nullptr, const T *Uc = nullptr)
+              const int *ctl, bool in_tmp = false, double *zr = nullptr, const T *Uc = nullptr,
+              const CgTest *test = nullptr)
 {
     const bool fused = per_fused(h, H, l);
     if (H.per && !fused) return sweeps_per(h, H, l, F, U, n, pre, ctl);
@@ -269,7 +282,8 @@ void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T 
         a.per = fused;
         a.Uc = Uc;
         if (s == n - 1) a.partials = zr;
-        level_op(h, H, l, s > 0 ? OP_JACOBI : (pre ? OP_PRE_JACOBI : (Uc ? OP_INTERP_JACOBI : OP_JACOBI)), a);
+        level_op(h, H, l, s > 0 ? OP_JACOBI : (pre ? OP_PRE_JACOBI : (Uc ? OP_INTERP_JACOBI : OP_JACOBI)), a,
+                 s == 0 ? test : nullptr);
         src = dst;
     }
 }
@@ -333,12 +347,13 @@ void vcycle_t(const gputo_handle *h, const HierView<T> &H, const T *F0, T *U0, c
                 a.F = F;
                 a.out = v.R;
                 a.out2 = U;
-                level_op(h, H, l, OP_PRE_DEFECT, a);
+                level_op(h, H, l, OP_PRE_DEFECT, a, l == 0 ? &H.test : nullptr);
             } else {
                 if (npre == 0)
                     launch_per_jacobi<T>(h->stream, lv.g, U, v.R, F, v.AD, lv.mask, p.omega, p.prerelax, 1, ctl, H.nb);
                 else
-                    sweeps_t(h, H, l, F, U, O, npre, true, ctl);
+                    sweeps_t(h, H, l, F, U, O, npre, true, ctl, false, nullptr, (const T *)nullptr,
+                             l == 0 ? &H.test : nullptr);
                 OpArgsT<T> a = view_args(h, H, l, ctl);
                 a.U = U;
                 a.F = F;
