@@ -920,6 +920,77 @@ __device__ __forceinline__ void dgemm_tile32(const double *__restrict__ A, long 
     }
 }
 
+// A^-1 = X^T X, X the inverse of the factor, of a small matrix (kCoarseFull), one
+// 32x32 tile per workgroup, in the place of the transpose: a solve is then one
+// product instead of two.  Rows of X before the tile's later column are zero,
+// rows of the other part and what couples the parts are neither stored nor read:
+// the rows of X that count are up to two ranges, one after the other for the four
+// waves, which split them as in dgemm_tile32.  Both triangles are formed, the sums
+// of (i, j) and (j, i) in the same order: A^-1 is symmetric bit for bit.
+__global__ __launch_bounds__(256) void k_inverse_product(CoarseMap m, const double *__restrict__ X,
+                                                         double *__restrict__ Out)
+{
+    __shared__ double red[4][NB][NB + 1];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, i = lane & 15;
+    const int i0 = blockIdx.y * NB, j0 = blockIdx.x * NB, from = max(i0, j0);
+    // rows from .. from + n1 - 1 (none when the columns are of different parts),
+    // then the separator's
+    int n1 = m.N - from, sep = 0;
+    if (m.ps > 0 && from < m.os) {
+        const bool same = (i0 < m.o2) == (j0 < m.o2);
+        n1 = same ? (from < m.o2 ? m.o2 : m.os) - from : 0;
+        sep = m.ps;
+    }
+    const int steps = (n1 + sep) / 32;  // of 8 rows, per wave
+    struct Ops {
+        double a[2][2], b[2][2];
+    } x, y;
+    auto load = [&](int s, Ops &o) {
+        const int r = 8 * (w * steps + s);
+        const double *p = X + (long)((r < n1 ? from + r : m.os + r - n1) + 2 * (lane >> 4)) * m.N + i;
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                o.a[e][h] = p[(long)e * m.N + i0 + 16 * h];
+                o.b[e][h] = p[(long)e * m.N + j0 + 16 * h];
+            }
+    };
+    f64x4 d[2][2] = {};
+    auto multiply = [&](const Ops &o) {
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    d[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(o.a[e][p], o.b[e][q], d[p][q], 0, 0, 0);
+    };
+    load(0, x);
+    int s = 0;
+    for (; s + 2 < steps; s += 2) {
+        load(s + 1, y);
+        multiply(x);
+        load(s + 2, x);
+        multiply(y);
+    }
+    if (s + 1 < steps) load(s + 1, y);
+    multiply(x);
+    if (s + 1 < steps) multiply(y);
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) red[w][16 * p + 4 * v + (lane >> 4)][16 * q + i] = d[p][q][v];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        Out[(long)(i0 + r) * m.N + j0 + c] = (red[0][r][c] + red[1][r][c]) + (red[2][r][c] + red[3][r][c]);
+    }
+}
+
 // blockIdx.z: diagonal block x group.  Tiles above the diagonal of X are
 // neither read nor written.
 template <int STEP>
@@ -1125,9 +1196,12 @@ void coarse_finish(const Coarse &C)
         B.off[3] = N;
     }
     k_trtri_diag<<<nb, 64, 0, s>>>(B, Li, N);
-    // the transpose's buffer is free until the last step: it holds W
+    // the last step's buffer is free until then: it holds W
     launch_linv_levels(s, B, Li, LiT, (long)N * N, N, (bw + 2 * NB - 2) / NB);
-    k_transpose<<<dim3(nb, nb), 256, 0, s>>>(Li, LiT, N);
+    if (N <= kCoarseFull)
+        k_inverse_product<<<dim3(nb, nb), 256, 0, s>>>(m, Li, LiT);
+    else
+        k_transpose<<<dim3(nb, nb), 256, 0, s>>>(Li, LiT, N);
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(C.ev_done, s));
 }
@@ -1186,8 +1260,9 @@ void coarse_switch(Coarse &C, hipStream_t s)
 }
 
 // ---------------------------------------------------------------------------
-// Coarsest solve x = L^-T L^-1 b as two row-parallel triangular products, then
-// x[fixed] = 0 (mgcg1.c:431-432).  One wave per row and, for a batch, all its
+// Coarsest solve x = L^-T L^-1 b as two row-parallel triangular products, or
+// one with the whole inverse (kCoarseFull), then x[fixed] = 0
+// (mgcg1.c:431-432).  One wave per row and, for a batch, all its
 // right-hand sides: a row is read once, two entries per load, kTrmvLoads of
 // them (and of b) in flight before the first product; the longest rows come
 // first.  Rows start and end at whole tiles (the diagonal tiles are stored with
@@ -1201,22 +1276,28 @@ void coarse_switch(Coarse &C, hipStream_t s)
 // ---------------------------------------------------------------------------
 constexpr int kTrmvThreads = 256, kTrmvLoads = 8;
 
-template <bool UPPER, int MAXB, class Ti, class To>
+enum TrmvKind { TRMV_LOWER, TRMV_UPPER, TRMV_FULL };
+
+template <TrmvKind KIND, int MAXB, class Ti, class To>
 __global__ __launch_bounds__(kTrmvThreads) void k_trmv(CoarseMap m, const int *__restrict__ dof,
                                                       const double *__restrict__ M,
                                                       const Ti *__restrict__ b, To *__restrict__ x,
                                                       const uint8_t *__restrict__ mask, const int *ctl, int nb)
 {
-    // lower: b has n entries, x has N (the padded y); upper: the reverse
-    const long sb = UPPER ? m.N : m.n, sx = UPPER ? m.n : m.N;
+    // lower: b has n entries, x has N (the padded y); upper: the reverse; full: both n
+    constexpr bool UPPER = KIND == TRMV_UPPER, FULL = KIND == TRMV_FULL, LOWER = KIND == TRMV_LOWER;
+    const long sb = UPPER ? m.N : m.n, sx = LOWER ? m.N : m.n;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int idx = blockIdx.x * (kTrmvThreads / 64) + wave;  // < N
-    const int row = UPPER ? idx : m.N - 1 - idx;
+    const int row = LOWER ? m.N - 1 - idx : idx;
     // columns lo .. lo + cnt - 1, those from `cut` on shifted by `skip` (the
     // separator's columns of a row of part 1)
     const int tile = row / NB * NB;
     int lo, cnt, cut = m.N, skip = 0;
-    if (!UPPER) {
+    if (FULL) {
+        lo = 0;
+        cnt = m.N;
+    } else if (LOWER) {
         lo = m.ps > 0 && row >= m.o2 && row < m.os ? m.o2 : 0;
         cnt = tile + NB - lo;
     } else {
@@ -1267,8 +1348,8 @@ __global__ __launch_bounds__(kTrmvThreads) void k_trmv(CoarseMap m, const int *_
             for (int u = 0; u < kTrmvLoads; ++u) s[q] = fma(mv[u][1], bv[u][1], fma(mv[u][0], bv[u][0], s[q]));
         }
     }
-    const int d = UPPER ? dof[row] : row;
-    const bool fixed = UPPER && mask && d >= 0 && ((mask[d / 3] >> (d % 3)) & 1u);
+    const int d = LOWER ? row : dof[row];
+    const bool fixed = !LOWER && mask && d >= 0 && ((mask[d / 3] >> (d % 3)) & 1u);
 #pragma unroll
     for (int q = 0; q < MAXB; ++q) {
         if (MAXB > 1 && q >= nb) break;
@@ -1292,13 +1373,19 @@ void launch_coarse_solve(hipStream_t s, const Coarse &C, const T *b, T *x, const
     }
     // C.y has room for kMaxBatch right-hand sides; N is a multiple of the rows of a workgroup
     const unsigned grid = (unsigned)(C.map.N / (kTrmvThreads / 64));
-    if (nb > 1) {
-        k_trmv<false, kMaxBatch, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.Linv, b, C.y, nullptr, ctl, nb);
-        k_trmv<true, kMaxBatch, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.LinvT, C.y, x, mask, ctl, nb);
-    } else {
-        k_trmv<false, 1, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.Linv, b, C.y, nullptr, ctl, 1);
-        k_trmv<true, 1, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.LinvT, C.y, x, mask, ctl, 1);
-    }
+    auto run = [&](auto maxb) {
+        constexpr int MB = decltype(maxb)::value;
+        if (C.map.N <= kCoarseFull) {
+            k_trmv<TRMV_FULL, MB, T, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.LinvT, b, x, mask, ctl, nb);
+            return;
+        }
+        k_trmv<TRMV_LOWER, MB, T, double><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.Linv, b, C.y, nullptr, ctl, nb);
+        k_trmv<TRMV_UPPER, MB, double, T><<<grid, kTrmvThreads, 0, s>>>(C.map, C.dof, C.LinvT, C.y, x, mask, ctl, nb);
+    };
+    if (nb > 1)
+        run(std::integral_constant<int, kMaxBatch>());
+    else
+        run(std::integral_constant<int, 1>());
 }
 template void launch_coarse_solve<double>(hipStream_t, const Coarse &, const double *, double *, const uint8_t *,
                                           const int *, int);

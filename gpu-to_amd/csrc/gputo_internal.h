@@ -271,6 +271,13 @@ struct CoarseBlocks {
     long ld[3];
 };
 
+// Orders up to which the whole inverse is formed and applied: the product replaces
+// a launch in every V-cycle (3.2-3.7 us), at the cost of N^3 operations in place of
+// the transpose in every setup.  A mgcg1 call of 10 iterations: 1343 -> 1300 us at
+// 525 DOFs, 1495 -> 1462 at 1008; the error against a solve in 80 bits is the same to
+// two digits (up to 8e-14 at a condition of 1e15).  From there on the product
+// grows faster (it is dense where the factor's inverse has its zero block).
+constexpr int kCoarseFull = 1024;
 struct Coarse {
     int n = 0;
     CoarseMap map;
@@ -279,7 +286,7 @@ struct Coarse {
     int bw = 0;              // lower bandwidth of the assembled matrix (node-major DOFs)
     double *AQ = nullptr;       // dense matrix (matrices of the parts, updated by the factorisation), then their factors
     double *Linv = nullptr;     // inverse of the factor used by the solves (lower, row-major)
-    double *LinvT = nullptr;    // its transpose (row-major)
+    double *LinvT = nullptr;    // its transpose (row-major); of at most kCoarseFull entries: the whole inverse
     double *Lbuf[2] = {}, *LTbuf[2] = {};  // two inverse buffers (lagged factorisation)
     int cur = 0;                // buffer of Linv/LinvT
     int target = 0;             // buffer the factorisation in flight writes

@@ -61,3 +61,30 @@ def test_split_decoupled_fixed_dofs(gputo, oracle, mesh, nl):
     oracle.lib().or_set_nswp(2)
     zo = oracle.vcycle_once(Ke, CX, fixed, nelx, nely, nelz, nl, r, preset=2)
     assert rel(z, zo) < 1e-9
+
+
+@pytest.mark.parametrize("mesh", [(2, 2, 2, 2), (4, 4, 4, 2), (8, 4, 4, 2), (12, 8, 8, 2), (14, 12, 10, 2), (16, 10, 12, 2)])
+def test_whole_inverse(gputo, oracle, mesh):
+    """Coarsest solves by the whole inverse: one tile, three without the split, two
+    parts of different lengths, 1024 entries (the most), and the two products just
+    above; FP32 vectors through a mixed solve.  Tolerance of the other coarsest
+    solves."""
+    nelx, nely, nelz, nl = mesh
+    print("case", mesh, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=8)
+    s = gputo.Solver(nelx, nely, nelz, nl)
+    s.setup(Ke, CX, fixed)
+    A, _, fd = s.level_matrices(nl - 1)
+    AQ = oracle.assemble(A, nelx // 2, nely // 2, nelz // 2)
+    b = np.random.default_rng(9).uniform(-1, 1, AQ.shape[0])
+    b[(fd - 1).astype(int)] = 0.0
+    x = s.coarse_solve(b)
+    xr = np.linalg.solve(AQ, b)
+    xr[(fd - 1).astype(int)] = 0.0
+    assert np.abs(x - xr).max() < 1e-9 * np.abs(xr).max()
+    U, _, _, rc = s.solve(Ke, F, CX, fixed, 1e-10, 500)
+    s.close()
+    m = gputo.Solver(nelx, nely, nelz, nl, precision=1)
+    Um, _, _, rcm = m.solve(Ke, F, CX, fixed, 1e-10, 500)
+    m.close()
+    assert rc == 0 and rcm == 0 and np.abs(Um - U).max() < 1e-8 * np.abs(U).max()
