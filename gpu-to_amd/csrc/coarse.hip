@@ -690,17 +690,18 @@ __global__ void k_transpose(const double *__restrict__ In, double *__restrict__ 
     for (int q = threadIdx.x; q < NB * NB; q += blockDim.x) Out[(long)(bj + q / NB) * N + bi + q % NB] = T[q % NB][q / NB];
 }
 
-// sum_m P[ra + i][m] P[rb + j][m] for a 16x16 block, D layout of the MFMA;
+// sum_m A[i][m] B[j][m] for a 16x16 block, D layout of the MFMA;
 // every operand is read from LDS before the chain starts, so the matrix
 // core does not wait on each pair of reads
-__device__ __forceinline__ f64x4 panel_product(const double (*P)[NB + 1], int ra, int rb, int lane)
+typedef double CholTile[NB][NB + 1];
+__device__ __forceinline__ f64x4 panel_product(const double (*A)[NB + 1], const double (*B)[NB + 1], int lane)
 {
     const int i = lane & 15, k = lane >> 4;
     double fa[NB / 4], fb[NB / 4];
 #pragma unroll
     for (int s = 0; s < NB / 4; ++s) {
-        fa[s] = P[ra + i][4 * s + k];
-        fb[s] = P[rb + i][4 * s + k];
+        fa[s] = A[i][4 * s + k];
+        fb[s] = B[i][4 * s + k];
     }
     f64x4 d = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
@@ -708,18 +709,64 @@ __device__ __forceinline__ f64x4 panel_product(const double (*P)[NB + 1], int ra
     return d;
 }
 
+// One wave: D = L L^T in place (lower triangle) and P <- P L^-T.  Lane r < NB
+// holds row r of D, the others a row of P: the column operations that factor the
+// one solve the other.  In two halves of 16 columns, the second updated by the
+// first on the matrix cores.
+__device__ __forceinline__ bool factor_solve(CholTile &D, CholTile &P, int lane)
+{
+    double L[NB];
+    bool bad = false;
+    const int r = lane < NB ? lane : 2 * NB;  // below every column
+    double *V = lane < NB ? D[lane] : P[lane - NB];
+#pragma unroll
+    for (int c = 0; c < NB; ++c) L[c] = c <= r ? V[c] : 0.0;
+    potrf_cols<0, 16>(L, r, bad);
+    wave_lds_sync();  // every lane has read its row
+#pragma unroll
+    for (int c = 0; c < 16; ++c) V[c] = L[c];
+    wave_lds_sync();
+    f64x4 v[3];
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+        const double(*R)[NB + 1] = rb == 0 ? D + 16 : P + 16 * (rb - 1);
+        v[rb] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int kk = 0; kk < 16; kk += 4)
+            v[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(R[lane & 15][kk + (lane >> 4)],
+                                                         D[16 + (lane & 15)][kk + (lane >> 4)], v[rb], 0, 0, 0);
+    }
+#pragma unroll
+    for (int rb = 0; rb < 3; ++rb) {
+        double(*R)[NB + 1] = rb == 0 ? D + 16 : P + 16 * (rb - 1);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) R[4 * u + (lane >> 4)][16 + (lane & 15)] = v[rb][u];
+    }
+    wave_lds_sync();
+    if (lane >= 16) {
+#pragma unroll
+        for (int c = 16; c < NB; ++c) L[c] -= V[c];
+    }
+    potrf_cols<16, NB>(L, r, bad);
+    wave_lds_sync();
+#pragma unroll
+    for (int c = 16; c < NB; ++c) V[c] = L[c];
+    return bad;
+}
+
 // ---------------------------------------------------------------------------
-// Cholesky A = L L^T of the lower band, one launch per block column of 32 (a
-// step).  Every workgroup owns one 32x32 tile (ti, tj) of the trailing band and
-// does all it needs for it: it factors the step's diagonal tile, solves the two
-// panel tiles of its rows and columns and subtracts their product.  The
-// repeated work costs nothing (the CUs would idle), and nothing waits for
-// another workgroup.  The factor goes to its own matrix, since other workgroups
-// of the launch still read the panel as it was.  A step takes 8.8 us, of which
-// the launch 2.7, the loads 1 and the chain of 32 pivots 2, whatever the band:
-// in one workgroup with a look-ahead (the FP64 rate of one CU, barriers) it
-// took 7 us at a band of 65 rows, 13 at 173 and 25 at 269, with three launches
-// per step (tile, panel, update) 25 us.
+// Cholesky A = L L^T of the lower band, one launch per two block columns of 32 (a
+// step; a last odd one alone).  Every workgroup owns one 32x32 tile (ti, tj) of
+// the trailing band and does all it needs for it: it factors the step's diagonal
+// tiles, solves the panel tiles of its rows and columns and subtracts their
+// products.  The repeated work costs nothing (the CUs would idle), and nothing
+// waits for another workgroup.  The factor goes to its own matrix, since other
+// workgroups of the launch still read the panel as it was.  A step of one block
+// column takes 8.7 us, of which the launch 2.7, the loads 1 and the chain of 32
+// pivots most of the rest, whatever the band; of two 15.7.  (In one workgroup with
+// a look-ahead, the FP64 rate of one CU and barriers: 7 us per block column at a
+// band of 65 rows, 13 at 173 and 25 at 269; with three launches per block
+// column, tile, panel and update, 25 us.)
 // ---------------------------------------------------------------------------
 struct CholStep {
     double *A[2], *L[2];
@@ -729,11 +776,11 @@ struct CholStep {
     int *flag;
 };
 
-__global__ __launch_bounds__(256) void k_chol_step(CholStep a, int k)
+__global__ __launch_bounds__(256) void k_chol_step(CholStep a)
 {
-    __shared__ double W[4 * NB][NB + 1];  // the diagonal tile and a panel tile, for wave 0 and for wave 1
-    const int q = blockIdx.y;
-    if (k >= a.steps[q]) return;
+    __shared__ CholTile W[4];  // the diagonal tile and a panel tile, for wave 0 and for wave 1
+    const int q = blockIdx.y, k = a.steps[q] - 1;
+    if (!(a.steps[q] & 1)) return;  // the last block column, where their number is odd
     const long ld = a.ld[q], k0 = (long)k * NB;
     const int nt = min(a.nt, a.n[q] / NB - k - 1);
     int ti, tj;
@@ -759,55 +806,16 @@ __global__ __launch_bounds__(256) void k_chol_step(CholStep a, int k)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int r = (tid >> 5) + 8 * u, c = tid & 31;
-        W[r][c] = d[u];
-        W[NB + r][c] = pi[u];
-        W[2 * NB + r][c] = d[u];
-        W[3 * NB + r][c] = pj[u];
+        W[0][r][c] = d[u];
+        W[1][r][c] = pi[u];
+        W[2][r][c] = d[u];
+        W[3][r][c] = pj[u];
     }
     __syncthreads();
-    if (wave < 2) {
-        // lane r < NB holds row r of the diagonal tile, the others a row of the
-        // panel tile: the column operations that factor the one solve the other
-        // (x L^T = p).  In two halves of 16 columns, the second updated by the
-        // first on the matrix cores.
-        double(*V)[NB + 1] = W + 2 * NB * wave;
-        double L[NB];
-        bool bad = false;
-        const int r = lane < NB ? lane : 2 * NB;  // below every column
-#pragma unroll
-        for (int c = 0; c < NB; ++c) L[c] = c <= r ? V[lane][c] : 0.0;
-        potrf_cols<0, 16>(L, r, bad);
-        wave_lds_sync();  // every lane has read its row
-#pragma unroll
-        for (int c = 0; c < 16; ++c) V[lane][c] = L[c];
-        wave_lds_sync();
-        f64x4 v[3];
-#pragma unroll
-        for (int rb = 0; rb < 3; ++rb) {
-            v[rb] = f64x4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int kk = 0; kk < 16; kk += 4)
-                v[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(V[16 * (rb + 1) + (lane & 15)][kk + (lane >> 4)],
-                                                             V[16 + (lane & 15)][kk + (lane >> 4)], v[rb], 0, 0, 0);
-        }
-#pragma unroll
-        for (int rb = 0; rb < 3; ++rb)
-#pragma unroll
-            for (int u = 0; u < 4; ++u) V[16 * (rb + 1) + 4 * u + (lane >> 4)][16 + (lane & 15)] = v[rb][u];
-        wave_lds_sync();
-        if (lane >= 16) {
-#pragma unroll
-            for (int c = 16; c < NB; ++c) L[c] -= V[lane][c];
-        }
-        potrf_cols<16, NB>(L, r, bad);
-        wave_lds_sync();
-#pragma unroll
-        for (int c = 16; c < NB; ++c) V[lane][c] = L[c];
-        if (bad && blockIdx.x == 0 && tid == 0) a.flag[0] = 1;
-    }
+    if (wave < 2 && factor_solve(W[2 * wave], W[2 * wave + 1], lane) && blockIdx.x == 0 && tid == 0) a.flag[0] = 1;
     __syncthreads();
     if (tile) {
-        const f64x4 v = panel_product(W, NB + 16 * (wave >> 1), 3 * NB + 16 * (wave & 1), lane);
+        const f64x4 v = panel_product(W[1] + 16 * (wave >> 1), W[3] + 16 * (wave & 1), lane);
 #pragma unroll
         for (int u = 0; u < 4; ++u) Tq[4 * u * ld] = old[u] - v[u];
     }
@@ -815,8 +823,99 @@ __global__ __launch_bounds__(256) void k_chol_step(CholStep a, int k)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int r = (tid >> 5) + 8 * u, c = tid & 31;
-        if (blockIdx.x == 0 && c <= r) a.L[q][(k0 + r) * ld + k0 + c] = W[r][c];
-        if (tile) a.L[q][(k0 + ri + r) * ld + k0 + c] = W[NB + r][c];
+        if (blockIdx.x == 0 && c <= r) a.L[q][(k0 + r) * ld + k0 + c] = W[0][r][c];
+        if (tile) a.L[q][(k0 + ri + r) * ld + k0 + c] = W[1][r][c];
+    }
+}
+
+// Block columns k and k + 1 of every part that has both.  Wave 0 solves the tile
+// between the two diagonal tiles, waves 1 and 2 the panel tiles of the workgroup's
+// rows and columns, each with its own copy of the first diagonal tile; the second
+// diagonal tile and the second panel tiles are updated on the matrix cores
+// (quadrant w of each by wave w), then waves 1 and 2 go on with those.
+__global__ __launch_bounds__(256) void k_chol_step2(CholStep a, int k)
+{
+    __shared__ CholTile D[3], X, P[2], Q[2];  // diagonal tile (a copy per wave), the tile below it, panel tiles
+    const int q = blockIdx.y;
+    if (k + 1 >= a.steps[q]) return;
+    const long ld = a.ld[q], k0 = (long)k * NB;
+    const int nt = min(a.nt, a.n[q] / NB - k - 2);
+    int ti, tj;
+    tri_index(blockIdx.x, ti, tj);
+    const bool tile = ti < nt;
+    if (!tile && blockIdx.x > 0) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qr = 16 * (wave >> 1), qc = 16 * (wave & 1);  // this wave's quadrant
+    double *Ak = a.A[q] + k0 * ld + k0;
+    const long ri = (long)(ti + 2) * NB, rj = (long)(tj + 2) * NB;
+    // quadrants in the MFMA's result layout
+    const long qo = (qr + (lane >> 4)) * ld + qc + (lane & 15);
+    double *Tq = Ak + ri * ld + rj + qo;
+    const double *Eq = Ak + NB * ld + NB + qo, *Pq = Ak + ri * ld + NB + qo, *Jq = Ak + rj * ld + NB + qo;
+    double d[4], x[4], pi[4] = {}, pj[4] = {}, e[4], oi[4] = {}, oj[4] = {}, old[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        d[u] = Ak[r * ld + c];
+        x[u] = Ak[(NB + r) * ld + c];
+        e[u] = Eq[4 * u * ld];
+        if (tile) {
+            pi[u] = Ak[(ri + r) * ld + c];
+            pj[u] = Ak[(rj + r) * ld + c];
+            oi[u] = Pq[4 * u * ld];
+            oj[u] = Jq[4 * u * ld];
+            old[u] = Tq[4 * u * ld];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        D[0][r][c] = D[1][r][c] = D[2][r][c] = d[u];
+        X[r][c] = x[u];
+        P[0][r][c] = pi[u];
+        P[1][r][c] = pj[u];
+    }
+    __syncthreads();
+    bool bad = false;
+    if (wave == 0) bad = factor_solve(D[0], X, lane);
+    if (wave == 1 || wave == 2) factor_solve(D[wave], P[wave - 1], lane);
+    __syncthreads();
+    {
+        const f64x4 ve = panel_product(X + qr, X + qc, lane), vi = panel_product(P[0] + qr, X + qc, lane),
+                    vj = panel_product(P[1] + qr, X + qc, lane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int r = qr + 4 * u + (lane >> 4), c = qc + (lane & 15);
+            D[1][r][c] = D[2][r][c] = e[u] - ve[u];
+            Q[0][r][c] = oi[u] - vi[u];
+            Q[1][r][c] = oj[u] - vj[u];
+        }
+    }
+    __syncthreads();
+    if (wave == 1 || wave == 2) bad = factor_solve(D[wave], Q[wave - 1], lane);
+    if (bad && blockIdx.x == 0 && lane == 0 && wave < 2) a.flag[0] = 1;
+    __syncthreads();
+    if (tile) {
+        const f64x4 v = panel_product(P[0] + qr, P[1] + qc, lane), w = panel_product(Q[0] + qr, Q[1] + qc, lane);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) Tq[4 * u * ld] = (old[u] - v[u]) - w[u];
+    }
+    if (tj > 0) return;
+    double *Lk = a.L[q] + k0 * ld + k0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int r = (tid >> 5) + 8 * u, c = tid & 31;
+        if (blockIdx.x == 0) {
+            Lk[(NB + r) * ld + c] = X[r][c];
+            if (c <= r) {
+                Lk[r * ld + c] = D[0][r][c];
+                Lk[(NB + r) * ld + NB + c] = D[1][r][c];
+            }
+        }
+        if (tile) {
+            Lk[(ri + r) * ld + c] = P[0][r][c];
+            Lk[(ri + r) * ld + NB + c] = Q[0][r][c];
+        }
     }
 }
 
@@ -1119,13 +1218,18 @@ long coarse_matrix_len(const Coarse &C)
 
 static void launch_chol_steps(hipStream_t s, const CholStep &a, int np)
 {
-    const int steps = std::max(a.steps[0], np > 1 ? a.steps[1] : 0);
-    for (int k = 0; k < steps; ++k) {
-        int nt = 0;
+    auto blocks = [&](int nt) { return dim3((unsigned)std::max(1, nt * (nt + 1) / 2), (unsigned)np); };
+    int last = -1;  // most trailing tiles after an odd last block column
+    for (int q = 0; q < np; ++q)
+        if (a.steps[q] & 1) last = std::max(last, std::min(a.nt, a.n[q] / NB - a.steps[q]));
+    for (int k = 0;; k += 2) {
+        int nt = -1;
         for (int q = 0; q < np; ++q)
-            if (k < a.steps[q]) nt = std::max(nt, std::min(a.nt, a.n[q] / NB - k - 1));
-        k_chol_step<<<dim3((unsigned)std::max(1, nt * (nt + 1) / 2), (unsigned)np), 256, 0, s>>>(a, k);
+            if (k + 1 < a.steps[q]) nt = std::max(nt, std::min(a.nt, a.n[q] / NB - k - 2));
+        if (nt < 0) break;
+        k_chol_step2<<<blocks(nt), 256, 0, s>>>(a, k);
     }
+    if (last >= 0) k_chol_step<<<blocks(last), 256, 0, s>>>(a);
 }
 
 void coarse_factor(hipStream_t s0, Coarse &C, bool lag)

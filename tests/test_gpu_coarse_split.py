@@ -88,3 +88,23 @@ def test_whole_inverse(gputo, oracle, mesh):
     Um, _, _, rcm = m.solve(Ke, F, CX, fixed, 1e-10, 500)
     m.close()
     assert rc == 0 and rcm == 0 and np.abs(Um - U).max() < 1e-8 * np.abs(U).max()
+
+
+@pytest.mark.parametrize("coarse", [(9, 2, 2), (7, 2, 2), (5, 2, 2), (6, 2, 2), (1, 1, 1)])
+def test_block_columns_in_pairs(gputo, oracle, coarse):
+    """Parts of 5 and 4, 4 and 3, 3 and 2, 3 and 3 block columns (pairs, and a last
+    one alone, in one part or both), and a matrix of one."""
+    nelx, nely, nelz = (2 * c for c in coarse)
+    print("case", coarse, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=8)
+    s = gputo.Solver(nelx, nely, nelz, 2)
+    s.setup(Ke, CX, fixed)
+    A, _, fd = s.level_matrices(1)
+    AQ = oracle.assemble(A, *coarse)
+    b = np.random.default_rng(9).uniform(-1, 1, AQ.shape[0])
+    b[(fd - 1).astype(int)] = 0.0
+    x = s.coarse_solve(b)
+    s.close()
+    xr = np.linalg.solve(AQ, b)
+    xr[(fd - 1).astype(int)] = 0.0
+    assert rel(x, xr) < 1e-9
