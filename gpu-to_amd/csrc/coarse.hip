@@ -1,7 +1,8 @@
 // Coarse levels of the MGCG hierarchy: level-1 rediscretisation from child
 // densities, element-Galerkin operators, the coarsest-level penalty,
 // dense assembly, blocked FP64 Cholesky, the explicit inverse of the
-// factor and the two triangular products that apply it in every V-cycle.
+// factor (of the matrix, when small) and the products that apply it in every
+// V-cycle.
 #include <algorithm>
 #include <cmath>
 #include <stdexcept>
@@ -466,8 +467,8 @@ void launch_corrcsa(hipStream_t s, const Grid &g, const int *fixed_d, int nfd, d
 // once, the chain is half as long, and the inverse of the factor has a zero
 // block between the parts.  Parts are padded to whole
 // 32 x 32 tiles in front, the separator behind, with identity rows.
-// The factorisation takes 295 us at 13 x 7 x 7 nodes (1911 DOFs; 840 in one
-// workgroup as one band) and 470 at 12 x 8 x 10 (2880; 2200 as one band by three
+// The factorisation takes 265 us at 13 x 7 x 7 nodes (1911 DOFs; 840 in one
+// workgroup as one band) and 430 at 12 x 8 x 10 (2880; 2200 as one band by three
 // launches per block column).
 //
 // coarse_dof: the DOF of entry c of that order (-1: padding).  part_dof: of
@@ -1162,8 +1163,9 @@ static void launch_linv_levels(hipStream_t s, const CoarseBlocks &B, double *Li,
     }
 }
 
-// The split saves 2 of 5 steps of 8.8 us at 5x3x3 nodes already (the sum of the
-// updates costs 4.7); it needs two planes per part.
+// The split takes one pair of block columns (15.7 us), the sum of the updates (4.7)
+// and a last one (8.7) at 5x3x3 nodes already, for two pairs and a last one
+// without it; it needs two planes per part.
 void coarse_layout(Coarse &C, const Grid &g, bool periodic)
 {
     CoarseMap &m = C.map;
