@@ -31,7 +31,9 @@
 // t + R + 1, so the block works on R + 1 entries before its own, too.  It
 // marches along i, one element layer per step:
 //   * each lane loads the node pairs (k, j..j+1) and (k+1, j..j+1) of the next
-//     layer (48 contiguous bytes each in FP64) while it works on this one;
+//     layer (48 contiguous bytes each in FP64) while it works on this one (as
+//     few loads as possible: an FP32 pair as three 8-byte loads instead of a
+//     16-byte and an 8-byte one made mixed solves 3 % slower);
 //   * sums and differences along j, k and i, the modal products, and back:
 //     the i direction meets in the lane's registers;
 //   * along j the neighbour's share comes by a one-lane shift (consecutive
@@ -436,13 +438,19 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
                      j < (PER ? g.ny : g.nny);
     const int plane = g.nny * g.nnz;
     const int nod0 = k * g.nny + j;    // own node in its plane
-    const int enod = ke * g.nny + je;  // the element's first node
+    // A sweep's and a matvec's own value comes with the operands: the pair of row k
+    // holds the own node, also where no element follows it along k or j (there as
+    // its second node).  Two loads less per layer: the no-allocation matvec at
+    // 192x96x96 40.1 -> 37.4 us, an FP64 solve 1 % and a mixed one 1.7 % faster.
+    constexpr bool OWN = !PRE && MODE != OP_DEFECT;
+    const bool nod_ok = el_ok || (OWN && own), jlast = OWN && own && j == g.ny;
+    const int enod = ke * g.nny + je - (int)jlast;  // the element's first node
     // byte offsets in a plane of the element's two node rows, of its scale(s)
     // and of the own node
-    const int ulo = el_ok ? 3 * SU * enod : kMdOut, uhi = el_ok ? 3 * SU * (enod + g.nny) : kMdOut;
+    const int ulo = nod_ok ? 3 * SU * enod : kMdOut, uhi = el_ok ? 3 * SU * (enod + g.nny) : kMdOut;
     const int flo = el_ok ? 3 * S * enod : kMdOut, fhi = el_ok ? 3 * S * (enod + g.nny) : kMdOut;
     const int eo = el_ok ? (EL == 0 ? S * (ke * g.ny + je) : S * (4 * ke * g.ny + 2 * je)) : kMdOut;
-    const int oo = own ? 3 * S * nod0 : kMdOut, uo = own ? 3 * SU * nod0 : kMdOut;
+    const int oo = own ? 3 * S * nod0 : kMdOut;
     const long vb = (long)S * g.ndof;
     const MdBuf BU = PRE ? md_buf(a.F, vb)
                          : (MODE == OP_MATVEC_UF ? md_buf(a.Uf, (long)SU * g.ndof) : md_buf(a.U, vb));
@@ -487,12 +495,17 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
             }
         }
     };
+    T own_u[3] = {T(0), T(0), T(0)};  // OWN: the own node of the layer last transformed
     auto jk = [&](const Raw &x, Jk<T> &o) {
         T lo[6], hi[6];
 #pragma unroll
         for (int q = 0; q < 6; ++q) {
             lo[q] = PRE ? pr * (T(x.lo[q]) * x.dlo[EL == 0 ? q / 3 : q]) : T(x.lo[q]);
             hi[q] = PRE ? pr * (T(x.hi[q]) * x.dhi[EL == 0 ? q / 3 : q]) : T(x.hi[q]);
+        }
+        if (OWN) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) own_u[q] = jlast ? lo[3 + q] : lo[q];
         }
         md_jk(lo, hi, o);
     };
@@ -501,8 +514,7 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
     // node layer pl is complete in sum: the k and j directions, the
     // neighbours' shares and the epilogue
     struct Epi {
-        T f[3], d[3];
-        TU u[3];
+        T f[3], d[3], u[3];
         unsigned m;
     };
     auto load_epi = [&](int pl, Epi &e) {
@@ -513,7 +525,6 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
         } else {
             if (JAC || PRE) md_ld3(BD, oo, pl * fp, e.d);
         }
-        if (!PRE && MODE != OP_DEFECT) md_ld3(BU, uo, pl * up, e.u);
     };
     auto finish = [&](int pl, const Jk<T> &sum, const Epi &e) {
         T y[3];
@@ -542,7 +553,7 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
                 if (PRE) a.out2[dof + cc] = pr * (e.f[cc] * e.d[cc]);
             } else {
                 // U = (1-w) U + w (R + AD U)/AD = U + w R/AD  (mgcg1.cu:1199-1206)
-                const T u = PRE ? pr * (e.f[cc] * e.d[cc]) : T(e.u[cc]);
+                const T u = PRE ? pr * (e.f[cc] * e.d[cc]) : e.u[cc];
                 const T rv = fixed ? T(0) : e.f[cc] - yc;
                 v = fma(om * e.d[cc], rv, u);
                 if (DOT) part += (double)e.f[cc] * (double)v;
@@ -589,6 +600,7 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
         // operands go before the prefetch
         Epi epi;
         if (emit && AHEAD) load_epi(pl - 1, epi);
+        const T below_u[3] = {own_u[0], own_u[1], own_u[2]};  // of layer pl - 1
         if (AHEAD) {
             if (pl < hi) {
                 load(pl + 1, xn);
@@ -618,6 +630,10 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
             md_element_gp(m, a.mc, cx);
         }
         if (emit && !AHEAD) load_epi(pl - 1, epi);
+        if (OWN) {
+#pragma unroll
+            for (int cc = 0; cc < 3; ++cc) epi.u[cc] = below_u[cc];
+        }
         Jk<T> sum;
 #pragma unroll
         for (int cc = 0; cc < 3; ++cc)
@@ -644,6 +660,8 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
     if (!PER && i1 == g.nnx) {  // the last node layer of the mesh ends with what is pending
         Epi epi;
         load_epi(g.nnx - 1, epi);
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) epi.u[cc] = own_u[cc];
         finish(g.nnx - 1, pend, epi);
     }
     if (DOT && a.partials) {
