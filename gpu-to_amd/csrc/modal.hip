@@ -55,9 +55,9 @@
 //
 // Measured on MI355X at 192x96x96 (matvecs back to back; before: node-gather,
 // split-BF16 MFMA and Gauss point by Gauss point kernels): FP64 level 0
-// 75 -> 29 us (101 MB of operands, 3.5 TB/s; 87 % of the VALU operations are
+// 75 -> 27.4 us (101 MB of operands, 3.7 TB/s; 87 % of the VALU operations are
 // the transforms and products above), FP32 level 0 66 (node-gather) and 23
-// (MFMA) -> 18.6 us, FP64 level 1 34 -> 12.4 us, FP32 level 1 24 -> 8.8 us;
+// (MFMA) -> 17.1 us, FP64 level 1 34 -> 12.4 us, FP32 level 1 24 -> 8.8 us;
 // an FP64 Jacobi sweep in the solve 65 -> 37 us, an FP32 one 34 (MFMA) ->
 // 25 us.  At 16x8x8 a launch takes 3.5 us against 8-10 us: 27 x 24 dependent
 // products per node are gone.  Level 0 is bound by memory and by the two

@@ -47,7 +47,7 @@ enum L0Kind {
 
 // The FP32 modal kernel takes the place of the node-gather and of the split-
 // BF16 MFMA kernels whose accuracy it reaches or passes: a matvec takes
-// 18.6 us at 192x96x96, against 23.2 us for the two-part split, 39 us for the
+// 17.1 us at 192x96x96, against 23.2 us for the two-part split, 39 us for the
 // three-part one and 66 us for the node-gather.  The one-product flavour
 // keeps its own kernel: its rounding is what that choice asks for.
 inline int l0_resolve(const gputo_handle *h, int kind)
