@@ -380,8 +380,15 @@ struct MdNoTest {};
 template <int MODE, int EL, bool PER>
 using MdTest = std::conditional_t<md_tests<MODE, EL, PER>(), CgTest, MdNoTest>;
 
+// waves of a block at most
+template <class T, int EL>
+constexpr int md_max_waves()
+{
+    return sizeof(T) == 8 && EL == 1 ? 4 : kMdMaxWaves;
+}
+
 template <class T, class TU, int MODE, int EL, bool PER>
-__global__ __launch_bounds__((sizeof(T) == 8 && EL == 1 ? 4 : kMdMaxWaves) * 64) __attribute__((amdgpu_waves_per_eu(md_min_waves<T, EL>())))
+__global__ __launch_bounds__((md_max_waves<T, EL>() * 64)) __attribute__((amdgpu_waves_per_eu(md_min_waves<T, EL>())))
 void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
 {
     const ModalWork &w = a.mw;
@@ -934,6 +941,7 @@ void launch_mode(hipStream_t s, const OpArgsT<T> &a, const T *CX, const CgTest *
             return;
         }
     }
+    if (w.NW > md_max_waves<T, EL>()) throw std::runtime_error("modal operator: tiling of another element");
     k_modal<T, TU, MODE, EL, PER><<<grid, 64 * w.NW, 6u * ne * sizeof(T), s>>>(a, CX, test);
 }
 

@@ -876,6 +876,16 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
 // ============================================================================
 // C ABI
 // ============================================================================
+// The modal tilings of level l under the handle's preset: level 1 of a
+// rediscretised hierarchy runs the level-1 element, whose blocks have fewer waves.
+static void modal_tiles(gputo_handle *h, int l)
+{
+    Level &v = h->L[l];
+    const int el = l == 1 && !preset_of(h->prm).l1_galerkin && !preset_of(h->prm).mg9;
+    v.mw64 = modal_work(v.g, 8, el, l ? 8 : 1);
+    v.mw32 = modal_work(v.g, 4, el, l ? 8 : 1);
+}
+
 extern "C" {
 
 void gputo_default_params(gputo_params *p)
@@ -950,10 +960,7 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
             v.tg = choose_tile(v.g);
             maxblocks = std::max<long>(maxblocks, xcd_launch(v.t.blocks()));
             maxblocks = std::max<long>(maxblocks, xcd_launch(v.tg.blocks()));
-            // level 1 of the rediscretised hierarchy takes the level-1 element
-            const int el = l == 1 && !preset_of(h->prm).l1_galerkin && !preset_of(h->prm).mg9;
-            v.mw64 = modal_work(v.g, 8, el, l ? 8 : 1);
-            v.mw32 = modal_work(v.g, 4, el, l ? 8 : 1);
+            modal_tiles(h, l);
             maxblocks = std::max<long>(maxblocks, std::max(xcd_launch(v.mw64.blocks()), xcd_launch(v.mw32.blocks())));
             v.R = dalloc<double>(h, v.g.ndof);
             v.AD = dalloc<double>(h, v.g.ndof + rd_len(v.g, l));
@@ -1069,7 +1076,9 @@ int gputo_set_params(gputo_handle *h, const gputo_params *params)
     if (params->preset != h->prm.preset) h->hier_ready = false;
     coarse_invalidate(h->C);  // the next setup factors exactly
     if (h->ln) learn_policy_reset(h->ln);  // the fallback re-times the stage under the new parameters
+    const bool retile = params->preset != h->prm.preset;
     h->prm = *params;
+    if (retile) modal_tiles(h, 1);  // its launches leave no partial sums, so none need more room
     try {
         if (h->prm.precision != GPUTO_PREC_F64) mixed_create(h);
     } catch (...) {

@@ -178,3 +178,27 @@ def test_correction_added_by_the_first_post_sweep_fp32(gputo, mesh):
         out.append((U, nit))
     assert out[1][1] <= out[0][1] + max(1, out[0][1] // 10)
     assert rel(out[1][0], out[0][0]) < 1e-8
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("presets", [(1, 0), (2, 0), (0, 2), (0, 1)])
+def test_level1_tiling_follows_the_preset(gputo, presets, precision):
+    """A handle whose preset changes runs the level-1 operator of the new preset,
+    with that element's own tiling: on this mesh the other element's has blocks
+    of eight waves, twice what the FP64 level-1 element has room for.  A handle
+    created with the new preset gives the same solution (1e-10, the solves'
+    tolerance: its Galerkin level 1 has a stencil, the other one's element
+    matrices) in as many iterations."""
+    nelx, nely, nelz, nl = 208, 104, 32, 4
+    print("case", presets, precision, flush=True)
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=68, kind="uniform")
+    s = gputo.Solver(nelx, nely, nelz, nl, preset=presets[0], precision=precision)
+    s.set_params(preset=presets[1])
+    U, _, n, rc = s.solve(Ke, F, CX, fixed, 1e-10, 200)
+    s.close()
+    assert rc == 0
+    s = gputo.Solver(nelx, nely, nelz, nl, preset=presets[1], precision=precision)
+    Uf, _, nf, rc = s.solve(Ke, F, CX, fixed, 1e-10, 200)
+    s.close()
+    assert rc == 0 and n == nf < 200
+    assert rel(U, Uf) < 1e-10 if presets == (0, 1) else np.array_equal(U, Uf)
