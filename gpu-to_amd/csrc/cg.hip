@@ -352,8 +352,9 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_p(TP *Pout, const TP *Pin,
 }
 
 // U += alpha_0 P_0 + ... + alpha_{m-1} P_{m-1}, term by term in that order
-// (the same fused multiply-adds as one update per iteration).  Converged
-// iterations logged alpha 0; their directions are finite, so they add 0.
+// (the same fused multiply-adds as one update per iteration).  An iteration
+// enqueued after convergence logged alpha 0 and left its slot as it was: with an
+// earlier solve's direction, which may not be finite, so the term is left out.
 // One element per thread, its m + 1 loads all in flight together.
 __global__ __launch_bounds__(kBlock) void k_cg_flush_u(double *__restrict__ U, const float *__restrict__ P, long n,
                                                       const double *__restrict__ alog, int m)
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_flush_u(double *__restrict__ U, c
     double u = U[i];
 #pragma unroll
     for (int t = 0; t < kCgLog; ++t)
-        if (t < m) u = fma(alog[t], (double)pv[t], u);
+        if (t < m && alog[t] != 0.0) u = fma(alog[t], (double)pv[t], u);
     U[i] = u;
 }
 

@@ -59,7 +59,6 @@ void mixed_create(gputo_handle *h)
     m->Q = malloc_dev<float>(m, g0.ndof);
     m->Z = malloc_dev<float>(m, g0.ndof);
     m->Pcg = malloc_dev<float>(m, (long)kCgLog * g0.ndof);
-    launch_fill<float>(h->stream, m->Pcg, (long)kCgLog * g0.ndof, 0.0);  // finite: unused slots add 0 * p
     m->alog = malloc_dev<double>(m, kCgLog);
     m->sc = malloc_dev<CgScalars>(m, 1);
     m->norm = malloc_dev<double>(m, 2);

@@ -170,3 +170,26 @@ def test_lagged_factor_dropped_after_parameter_change(gputo):
     assert n1 == n2 and rel(U1, U2) < 1e-12
     s.close()
     fresh.close()
+
+
+def test_solve_after_one_that_overflowed(gputo):
+    """What a solve that ended with a non-finite direction left behind does not
+    reach a later one.  The coarsest factor of the stiff design serves the soft
+    one's first two V-cycles, so its direction overflows FP32 in the second slot;
+    the solve after it converges there.  And a zero load, which never writes the
+    first slot, after an overflow in that one."""
+    nelx, nely, nelz, nl = 16, 8, 8, 3
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=65)
+    for scale, soft in ((1.8e29, 1e-6), (1e38, 1.0)):
+        s = gputo.Solver(nelx, nely, nelz, nl, precision=1, coarse_lag=2)
+        assert s.solve(Ke, F, CX, fixed, 1e-10, 50)[3] == 0
+        assert s.solve(Ke, F * scale, CX * soft, fixed, 1e-10, 50)[3] == gputo._lib.GPUTO_ERR_NONFINITE
+        s.set_params(coarse_lag=0)
+        U, r, n, rc = s.solve(Ke, F * 0.0, CX, fixed, 1e-10, 50)
+        assert rc == 0 and n == 0 and not U.any()
+        U, r, n, rc = s.solve(Ke, F, CX, fixed, 0.98, 50)
+        assert rc == 0 and n == 1 and r < 0.98
+        s.close()
+        fresh = gputo.Solver(nelx, nely, nelz, nl, precision=1)
+        assert np.array_equal(U, fresh.solve(Ke, F, CX, fixed, 0.98, 50)[0])
+        fresh.close()
