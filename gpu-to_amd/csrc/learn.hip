@@ -564,6 +564,7 @@ __global__ __launch_bounds__(256) void k_conv_bwd_w(const float *__restrict__ gz
         }
 #pragma unroll
         for (int c = 0; c < CO; ++c) {
+            if (g[c] == 0.0f) continue;  // adds nothing, also where an input is not finite
 #pragma unroll
             for (int t = 0; t < 27; ++t) acc[28 * c + t] = fmaf(g[c], v[t], acc[28 * c + t]);
             acc[28 * c + 27] += g[c];

@@ -46,11 +46,14 @@ def _up(d, shape):
     return d[:, :, :shape[2], :shape[3], :shape[4]]
 
 
-def forward(params, x, torch):
-    """params: list of (w, b) tensors; x: tensor [1, 4, n0, n1, n2]."""
+def forward(params, x, torch, keep=None):
+    """params: list of (w, b) tensors; x: tensor [1, 4, n0, n1, n2]; keep (may
+    be None): 0 at the positions of e1 that are cut off by their ReLU."""
     F = torch.nn.functional
     (w1, b1), (w2, b2), (w3, b3), (w4, b4), (w5, b5), (w6, b6) = params
     e1 = F.relu(F.conv3d(x, w1, b1, stride=1, padding=1))
+    if keep is not None:
+        e1 = e1 * keep
     e2 = F.relu(F.conv3d(e1, w2, b2, stride=2, padding=1))
     e3 = F.relu(F.conv3d(e2, w3, b3, stride=2, padding=1))
     a2 = F.relu(F.conv3d(e3, w4, b4, stride=1, padding=1))
@@ -61,14 +64,22 @@ def forward(params, x, torch):
 
 
 def run(flat, x, gy=None):
-    """y = N(x) and, with gy, the flat gradient of <gy, y> w.r.t. the params."""
+    """y = N(x) and, with gy, the flat gradient of <gy, y> w.r.t. the params.
+    An input that is NaN cuts off the positions of e1 that read it: the
+    library's ReLU is max(v, 0), which is 0 for a NaN, with gradient 0."""
     import torch
+    nan = np.isnan(x).any(axis=0)
+    keep = None
+    if nan.any():
+        x = np.nan_to_num(x)
+        near = torch.nn.functional.max_pool3d(torch.tensor(nan[None, None].astype(np.float64)), 3, 1, 1)
+        keep = 1.0 - near
     params = unpack(np.asarray(flat, dtype=np.float64), torch)
     for w, b in params:
         w.requires_grad_(True)
         b.requires_grad_(True)
     xt = torch.tensor(np.asarray(x, dtype=np.float64)[None])
-    y = forward(params, xt, torch)
+    y = forward(params, xt, torch, keep)
     if gy is None:
         return y.detach().numpy()[0], None
     (y * torch.tensor(np.asarray(gy, dtype=np.float64)[None])).sum().backward()
