@@ -1087,8 +1087,8 @@ int gputo_set_params(gputo_handle *h, const gputo_params *params)
     return 0;
 }
 
-// F (may be null) goes to h->Fv.  Nothing that an earlier call left on the
-// device changes before every array is known to be finite.
+// F (may be null) goes to h->Fv.  Ke and CX, which the hierarchy of an earlier
+// call stands on, change only once every argument is known to be good.
 static int upload_problem(gputo_handle *h, const double *Ke0, const double *F, const double *CX, const double *fixed,
                           int nfd, std::vector<int> &fx)
 {
@@ -1100,6 +1100,7 @@ static int upload_problem(gputo_handle *h, const double *Ke0, const double *F, c
     if (!host_upload(h, in, F ? 2 : 1)) return GPUTO_ERR_NONFINITE;
     fx.resize(nfd);
     for (int n = 0; n < nfd; ++n) fx[n] = (int)fixed[n] - 1;  // (int)FDofs[n]-1, mgcg1.c:663
+    if (int rc = validate_fixed(fx, g0.ndof)) return rc;
     set_ke(h, Ke0);
     const HostJob cx = {h->CX, (void *)CX, cb, false};
     host_upload(h, &cx, 1);
@@ -1165,10 +1166,13 @@ int gputo_solve_d(gputo_handle *h, const double *Ke0, const double *d_F, double 
         const Grid &g0 = h->L[0].g;
         std::vector<int> fx(nfd);
         if (nfd) HIPCHK(hipMemcpyAsync(fx.data(), d_fixed, nfd * sizeof(int), hipMemcpyDeviceToHost, h->stream));
-        set_ke(h, Ke0);
-        HIPCHK(hipMemcpyAsync(h->CX, d_CX, g0.nel * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
         HIPCHK(hipStreamSynchronize(h->stream));
-        int rc = setup_hierarchy(h, fx);
+        int rc = validate_fixed(fx, g0.ndof);  // before Ke and CX change, as upload_problem
+        if (rc == 0) {
+            set_ke(h, Ke0);
+            HIPCHK(hipMemcpyAsync(h->CX, d_CX, g0.nel * sizeof(double), hipMemcpyDeviceToDevice, h->stream));
+            rc = setup_hierarchy(h, fx);
+        }
         if (rc == 0) {
             rc = run_pcg(h, d_F, d_U, tol, maxit, relres, nit);
         }
@@ -1191,7 +1195,6 @@ static int host_op(gputo_handle *h, int mode, const double *Ke0, const double *C
         const Grid &g0 = h->L[0].g;
         std::vector<int> fx;
         if (int rc = upload_problem(h, Ke0, nullptr, CX, fixed, nfd, fx)) return rc;
-        if (int rc = validate_fixed(fx, g0.ndof)) return rc;
         std::vector<uint8_t> m = node_mask(fx, g0);
         hipStream_t s = h->stream;
         HIPCHK(hipMemcpyAsync(h->L[0].mask, m.data(), m.size(), hipMemcpyHostToDevice, s));
@@ -1234,7 +1237,6 @@ int gputo_matvec_mixed(gputo_handle *h, int kernel, const double *Ke0, const dou
         const Grid &g0 = h->L[0].g;
         std::vector<int> fx;
         if (int rc = upload_problem(h, Ke0, nullptr, CX, fixed, nfd, fx)) return rc;
-        if (int rc = validate_fixed(fx, g0.ndof)) return rc;
         std::vector<uint8_t> m = node_mask(fx, g0);
         hipStream_t s = h->stream;
         HIPCHK(hipMemcpyAsync(h->L[0].mask, m.data(), m.size(), hipMemcpyHostToDevice, s));

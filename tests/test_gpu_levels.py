@@ -206,3 +206,32 @@ def test_level0_fp32_kernel_modes_vs_oracle(gputo, oracle, kernel, tol, mesh):
         assert rel(y, ref) < tol, (mode, rel(y, ref))
         assert np.array_equal(y, s.level_apply(0, 1, mode, u, f, fp32=True))  # deterministic
     s.close()
+
+
+@pytest.mark.parametrize("call", ["setup", "solve", "matvec", "matvec_mixed", "vcycle"])
+def test_refused_call_leaves_the_hierarchy_alone(gputo, call):
+    """A call that is refused (a fixed DOF outside the mesh) with another Ke0 and
+    other densities leaves the hierarchy of the set-up before it: its element
+    matrices and its operators are those of a handle without that call."""
+    nelx, nely, nelz, nl = 16, 8, 8, 3
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=43, kind="smooth")
+    CX2 = cantilever_case(nelx, nely, nelz, seed=44, kind="smooth")[2]
+    bad = np.append(fixed, F.size + 1.0)
+    u = np.random.default_rng(45).uniform(-1, 1, F.size)
+    u1 = u[:3 * 9 * 5 * 5]
+    out = []
+    for refused in (False, True):
+        s = gputo.Solver(nelx, nely, nelz, nl, precision=1)
+        s.setup(Ke, CX, fixed)
+        if refused and call == "solve":
+            assert s.solve(2.0 * Ke, F, CX2, bad, 1e-8, 10)[3] == -5
+        elif refused:
+            args = {"setup": (2.0 * Ke, CX2, bad), "matvec": (2.0 * Ke, CX2, u, bad),
+                    "matvec_mixed": (1, 2.0 * Ke, CX2, u, bad), "vcycle": (2.0 * Ke, CX2, bad, u)}[call]
+            with pytest.raises(gputo.GputoError):
+                getattr(s, call)(*args)
+        out.append([s.level_matrices(1)[0], s.level_apply(0, 1, 0, u), s.level_apply(1, 2, 0, u1),
+                    s.level_apply(1, 1, 0, u1, fp32=True)])
+        s.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
