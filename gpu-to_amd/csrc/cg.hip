@@ -17,8 +17,8 @@
 // iteration.  No block reads a field that its own kernel writes: rho (read
 // for alpha) is written with beta, rho_p (read for beta) with alpha.  The
 // check is a block of the V-cycle's first level-0 launch where that is a modal
-// kernel in a prerelaxed mode (as a launch: 2.7 us).  Its other blocks may or may not see a flag that
-// is set meanwhile; what they write at convergence is not read any more.
+// kernel in a prerelaxed mode (as a launch: 2.7 us).  Its other blocks do not
+// read the flag; what they write at convergence is not read any more.
 //
 // Sums are two-stage with fixed grids and fixed orders, so results do not
 // depend on timing; products and sums are FP64 for both vector types.  The

@@ -370,6 +370,9 @@ constexpr int md_min_waves()
 // start a V-cycle.  (The FP32 cycle of a mixed solve starts with a plain sweep;
 // with the test in that kernel too its solves were 1 to 1.5 % slower.)  The
 // test goes first, and seven idle blocks behind it keep the tiles on their XCDs.
+// The other blocks of such a launch do not look at the flag, which it may set
+// while they run: waves of one block could see different values and part at a
+// barrier.  What they write once it is set is not read any more.
 constexpr unsigned kMdTestBlocks = 8;
 template <int MODE, int EL, bool PER>
 constexpr bool md_tests()
@@ -402,8 +405,10 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
     constexpr bool AHEAD = sizeof(T) == 4 ? !PRE : (EL == 0 && !PRE);
     constexpr int SU = (int)sizeof(TU), S = (int)sizeof(T);
     unsigned bx = blockIdx.x;
+    bool tested = false;  // the launch sets the flag
     if constexpr (md_tests<MODE, EL, PER>()) {
         if (test.sc) {
+            tested = true;
             if (bx < kMdTestBlocks) {
                 if (bx == 0 && threadIdx.x < 64) cg_test(test);
                 return;
@@ -588,7 +593,7 @@ void k_modal(OpModal<T> a, const T *__restrict__ CX, MdTest<MODE, EL, PER> test)
     load(first, xa);
     load(lo + 1, xb);
     load_e(first, ea);
-    if (a.ctl && a.ctl[0]) return;  // converged: read with the loads above
+    if (!tested && a.ctl && a.ctl[0]) return;  // converged: read with the loads above
     Jk<T> pa, pb, pend;
     jk(xa, pa);
 #pragma unroll
