@@ -309,7 +309,7 @@ __global__ __launch_bounds__(kCgThreads) void k_cg_sum(const double *p, int n, d
 // r_old = -alpha q, i.e. -alpha <z,q>/rho_old.
 template <class TP, class TZ, bool FLEX>
 __global__ __launch_bounds__(kBlock) void k_cg_update_p(TP *Pout, const TP *Pin, const TZ *__restrict__ Z, long n,
-                                                       CgScalars *sc, const double *dots, int nd, int maxit)
+                                                       CgScalars *sc, const double *dots, int nd)
 {
     sc += blockIdx.z;
     Pout = batch_ptr(Pout, n);
@@ -330,12 +330,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update_p(TP *Pout, const TP *Pin,
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc->rho = rz;
         sc->beta = be;
-        const int it = sc->it + 1;
-        sc->it = it;
-        if (it >= maxit) {
-            sc->done = 1;
-            sc->nit = maxit;
-        }
+        sc->it += 1;
     }
     for (long i = i0; i < n; i += 2 * stride) {
         const bool two = i + stride < n;
@@ -440,7 +435,7 @@ void launch_cg_check(hipStream_t s, const CgTest &t, int nb) { k_cg_check<<<dim3
 
 template <class TP, class TZ>
 void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const double *q, TP *Pout, const TP *Pin, long n,
-                         CgScalars *sc, double *dots, bool flex, int maxit, int nb, const double *zr, int nzr)
+                         CgScalars *sc, double *dots, bool flex, int nb, const double *zr, int nzr)
 {
     const int nblk = cg_blocks(n);
     const dim3 gd(nblk, 1, batch_dim(nb));
@@ -451,20 +446,20 @@ void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const doub
             zr = dots;
             nzr = 1;
         }
-        k_cg_update_p<TP, TZ, false><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, zr, nzr, maxit);
+        k_cg_update_p<TP, TZ, false><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, zr, nzr);
     } else if (flex) {
         k_cg_dots<TZ, true><<<gd, kCgThreads, 0, s>>>(r, z, q, n, dots, &sc->done);
-        k_cg_update_p<TP, TZ, true><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, dots, nblk, maxit);
+        k_cg_update_p<TP, TZ, true><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, dots, nblk);
     } else {
         k_cg_dots<TZ, false><<<gd, kCgThreads, 0, s>>>(r, z, q, n, dots, &sc->done);
-        k_cg_update_p<TP, TZ, false><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, dots, nblk, maxit);
+        k_cg_update_p<TP, TZ, false><<<gp, kBlock, 0, s>>>(Pout, Pin, z, n, sc, dots, nblk);
     }
 }
 template void launch_cg_direction<double, double>(hipStream_t, const double *, const double *, const double *, double *,
-                                                  const double *, long, CgScalars *, double *, bool, int, int,
+                                                  const double *, long, CgScalars *, double *, bool, int,
                                                   const double *, int);
 template void launch_cg_direction<float, float>(hipStream_t, const double *, const float *, const double *, float *,
-                                                const float *, long, CgScalars *, double *, bool, int, int,
+                                                const float *, long, CgScalars *, double *, bool, int,
                                                 const double *, int);
 
 void launch_cg_flush_u(hipStream_t s, double *U, const float *P, long n, const double *alog, int m)

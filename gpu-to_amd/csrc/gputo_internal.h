@@ -496,7 +496,7 @@ void launch_cg_check(hipStream_t s, const CgTest &t, int nb = 1);
 // dots of z and Pout = z + beta Pin (flex: Polak-Ribiere beta)
 template <class TP, class TZ>
 void launch_cg_direction(hipStream_t s, const double *r, const TZ *z, const double *q, TP *Pout, const TP *Pin, long n,
-                         CgScalars *sc, double *dots, bool flex, int maxit, int nb = 1, const double *zr = nullptr, int nzr = 0);
+                         CgScalars *sc, double *dots, bool flex, int nb = 1, const double *zr = nullptr, int nzr = 0);
 
 void check_hip(hipError_t e, const char *what);  // throws on an error
 #define HIPCHK(x) ::gputo::check_hip((x), #x)

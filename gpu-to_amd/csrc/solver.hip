@@ -669,10 +669,10 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
             // the traffic of an FP64 copy of z)
             precond_n(h->R, nullptr, true);
             launch_cg_direction<float, float>(s, h->R, z32, h->Q, p32 + (long)((sl + 1) % kCgLog) * n, pk, n, h->sc,
-                                              dots, flex, maxit, 1);
+                                              dots, flex);
         } else {
             precond_n(h->R, h->Z, r32 != nullptr);
-            launch_cg_direction<double, double>(s, h->R, h->Z, h->Q, h->P, h->P, n, h->sc, dots, flex, maxit, 1, zr,
+            launch_cg_direction<double, double>(s, h->R, h->Z, h->Q, h->P, h->P, n, h->sc, dots, flex, 1, zr,
                                                 nmv);
         }
     }
@@ -695,7 +695,7 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
         }
         return frc;
     }
-    if (h->prm.precision != GPUTO_PREC_F64) mixed_end(h, *nit, r.done);
+    if (h->prm.precision != GPUTO_PREC_F64) mixed_end(h, *nit, r.done || maxit > 0);
     if (h->ln) {
         int acc = 0, rej = 0;
         learn_end_solve(h, &acc, &rej,
@@ -841,7 +841,7 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
         HIPCHK(hipGetLastError());
         if (enq > 1 && cg_wait(s, h->prog, nb, enq - 1, nullptr)) break;
         precond(b.R, b.Z, r32 != nullptr);
-        launch_cg_direction<double, double>(s, b.R, b.Z, b.Q, b.P, b.P, n, b.sc, dots, flex, maxit, nb, H64.zr,
+        launch_cg_direction<double, double>(s, b.R, b.Z, b.Q, b.P, b.P, n, b.sc, dots, flex, nb, H64.zr,
                                             nmv);
     }
     HIPCHK(hipGetLastError());
@@ -864,7 +864,7 @@ int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double to
             rc = GPUTO_ERR_NONFINITE;
         }
     }
-    if (mixed) mixed_end(h, nit[0], b.sc_host[0].done);
+    if (mixed) mixed_end(h, nit[0], b.sc_host[0].done || maxit > 0);
     if (h->prm.print_level >= 1)
         for (int q = 0; q < nb; ++q)
             std::fprintf(stderr, "gputo: MGCG rhs %d nit=%d relres=%.6g\n", q, nit[q], relres[q]);
