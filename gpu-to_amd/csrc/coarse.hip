@@ -757,17 +757,22 @@ __device__ __forceinline__ bool factor_solve(CholTile &D, CholTile &P, int lane)
 
 // ---------------------------------------------------------------------------
 // Cholesky A = L L^T of the lower band, one launch per two block columns of 32 (a
-// step; a last odd one alone).  Every workgroup owns one 32x32 tile (ti, tj) of
-// the trailing band and does all it needs for it: it factors the step's diagonal
-// tiles, solves the panel tiles of its rows and columns and subtracts their
-// products.  The repeated work costs nothing (the CUs would idle), and nothing
-// waits for another workgroup.  The factor goes to its own matrix, since other
-// workgroups of the launch still read the panel as it was.  A step of one block
-// column takes 8.7 us, of which the launch 2.7, the loads 1 and the chain of 32
-// pivots most of the rest, whatever the band; of two 15.7.  (In one workgroup with
-// a look-ahead, the FP64 rate of one CU and barriers: 7 us per block column at a
-// band of 65 rows, 13 at 173 and 25 at 269; with three launches per block
+// step; a last odd one alone) while the tiles of a step fit the chip.  Every
+// workgroup owns one 32x32 tile (ti, tj) of the trailing band and does all it needs
+// for it: it factors the step's diagonal tiles, solves the panel tiles of its rows
+// and columns and subtracts their products.  The repeated work costs nothing where
+// the CUs would idle, and nothing waits for another workgroup.  The factor goes to
+// its own matrix, since other workgroups of the launch still read the panel as it
+// was.  A step of one block column takes 8.7 us, of which the launch 2.7, the loads
+// 1 and the chain of 32 pivots most of the rest; of two 15.7.  (In one workgroup
+// with a look-ahead, the FP64 rate of one CU and barriers: 7 us per block column at
+// a band of 65 rows, 13 at 173 and 25 at 269; with three launches per block
 // column, tile, panel and update, 25 us.)
+// A step of more than kCholFit tiles would repeat the chain in several rounds: it
+// solves its panel once per row tile, and a second launch updates the trailing
+// band.  The set-up of a periodic cell takes 28.2 ms at 6591 DOFs and 307 at 14739
+// with the first form alone, 8.2 and 82 with both (three launches per block column:
+// 17.3 and 152); a plate of 5x33x33 coarsest nodes (band 3371) 58.4, 23.8 (53.5).
 // ---------------------------------------------------------------------------
 struct CholStep {
     double *A[2], *L[2];
@@ -834,15 +839,19 @@ __global__ __launch_bounds__(256) void k_chol_step(CholStep a)
 // rows and columns, each with its own copy of the first diagonal tile; the second
 // diagonal tile and the second panel tiles are updated on the matrix cores
 // (quadrant w of each by wave w), then waves 1 and 2 go on with those.
+// PANEL: one workgroup per row tile, which leaves the trailing band to
+// k_chol_update.
+template <bool PANEL>
 __global__ __launch_bounds__(256) void k_chol_step2(CholStep a, int k)
 {
-    __shared__ CholTile D[3], X, P[2], Q[2];  // diagonal tile (a copy per wave), the tile below it, panel tiles
+    constexpr int NP = PANEL ? 1 : 2;
+    __shared__ CholTile D[1 + NP], X, P[NP], Q[NP];  // diagonal tile (a copy per wave), the tile below it, panel tiles
     const int q = blockIdx.y;
     if (k + 1 >= a.steps[q]) return;
     const long ld = a.ld[q], k0 = (long)k * NB;
     const int nt = min(a.nt, a.n[q] / NB - k - 2);
-    int ti, tj;
-    tri_index(blockIdx.x, ti, tj);
+    int ti = blockIdx.x, tj = 0;
+    if (!PANEL) tri_index(blockIdx.x, ti, tj);
     const bool tile = ti < nt;
     if (!tile && blockIdx.x > 0) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -862,42 +871,47 @@ __global__ __launch_bounds__(256) void k_chol_step2(CholStep a, int k)
         e[u] = Eq[4 * u * ld];
         if (tile) {
             pi[u] = Ak[(ri + r) * ld + c];
-            pj[u] = Ak[(rj + r) * ld + c];
             oi[u] = Pq[4 * u * ld];
-            oj[u] = Jq[4 * u * ld];
-            old[u] = Tq[4 * u * ld];
+            if (!PANEL) {
+                pj[u] = Ak[(rj + r) * ld + c];
+                oj[u] = Jq[4 * u * ld];
+                old[u] = Tq[4 * u * ld];
+            }
         }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int r = (tid >> 5) + 8 * u, c = tid & 31;
-        D[0][r][c] = D[1][r][c] = D[2][r][c] = d[u];
+#pragma unroll
+        for (int w = 0; w <= NP; ++w) D[w][r][c] = d[u];
         X[r][c] = x[u];
         P[0][r][c] = pi[u];
-        P[1][r][c] = pj[u];
+        if (!PANEL) P[NP - 1][r][c] = pj[u];
     }
     __syncthreads();
     bool bad = false;
     if (wave == 0) bad = factor_solve(D[0], X, lane);
-    if (wave == 1 || wave == 2) factor_solve(D[wave], P[wave - 1], lane);
+    if (wave >= 1 && wave <= NP) factor_solve(D[wave], P[wave - 1], lane);
     __syncthreads();
     {
-        const f64x4 ve = panel_product(X + qr, X + qc, lane), vi = panel_product(P[0] + qr, X + qc, lane),
-                    vj = panel_product(P[1] + qr, X + qc, lane);
+        const f64x4 ve = panel_product(X + qr, X + qc, lane), vi = panel_product(P[0] + qr, X + qc, lane);
+        f64x4 vj = {0.0, 0.0, 0.0, 0.0};
+        if (!PANEL) vj = panel_product(P[NP - 1] + qr, X + qc, lane);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int r = qr + 4 * u + (lane >> 4), c = qc + (lane & 15);
-            D[1][r][c] = D[2][r][c] = e[u] - ve[u];
+#pragma unroll
+            for (int w = 1; w <= NP; ++w) D[w][r][c] = e[u] - ve[u];
             Q[0][r][c] = oi[u] - vi[u];
-            Q[1][r][c] = oj[u] - vj[u];
+            if (!PANEL) Q[NP - 1][r][c] = oj[u] - vj[u];
         }
     }
     __syncthreads();
-    if (wave == 1 || wave == 2) bad = factor_solve(D[wave], Q[wave - 1], lane);
+    if (wave >= 1 && wave <= NP) bad = factor_solve(D[wave], Q[wave - 1], lane);
     if (bad && blockIdx.x == 0 && lane == 0 && wave < 2) a.flag[0] = 1;
     __syncthreads();
-    if (tile) {
-        const f64x4 v = panel_product(P[0] + qr, P[1] + qc, lane), w = panel_product(Q[0] + qr, Q[1] + qc, lane);
+    if (!PANEL && tile) {
+        const f64x4 v = panel_product(P[0] + qr, P[NP - 1] + qc, lane), w = panel_product(Q[0] + qr, Q[NP - 1] + qc, lane);
 #pragma unroll
         for (int u = 0; u < 4; ++u) Tq[4 * u * ld] = (old[u] - v[u]) - w[u];
     }
@@ -918,6 +932,66 @@ __global__ __launch_bounds__(256) void k_chol_step2(CholStep a, int k)
             Lk[(ri + r) * ld + NB + c] = Q[0][r][c];
         }
     }
+}
+
+// The trailing band after k_chol_step2<true>: A -= L L^T over block columns k and
+// k + 1, two by two tiles per workgroup, one per wave.  Both operands are rows of
+// the factor; a lane of group g = lane / 16 holds columns 2g and 2g + 1 of eight (as
+// in dgemm_tile32), and the loads are two batches of eight ahead.
+__global__ __launch_bounds__(256) void k_chol_update(CholStep a, int k)
+{
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    const int q = blockIdx.y;
+    if (k + 1 >= a.steps[q]) return;
+    const int nt = min(a.nt, a.n[q] / NB - k - 2);
+    int ti, tj;
+    tri_index(blockIdx.x, ti, tj);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    ti = 2 * ti + (wave >> 1);
+    tj = 2 * tj + (wave & 1);
+    if (ti >= nt || tj > ti) return;
+    const long ld = a.ld[q], k0 = (long)k * NB, r0 = k0 + 2 * NB;
+    const int i = lane & 15, g = lane >> 4;
+    const double *Li = a.L[q] + (r0 + (long)ti * NB + i) * ld + k0 + 2 * g;
+    const double *Lj = a.L[q] + (r0 + (long)tj * NB + i) * ld + k0 + 2 * g;
+    double *T = a.A[q] + (r0 + (long)ti * NB + g) * ld + r0 + (long)tj * NB + i;
+    constexpr int kBatches = 2 * NB / 8, kAhead = 2;
+    f64x2 fa[kAhead + 1][2], fb[kAhead + 1][2];
+    auto load = [&](int s) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            fa[s % (kAhead + 1)][h] = *reinterpret_cast<const f64x2 *>(Li + 16 * h * ld + 8 * s);
+            fb[s % (kAhead + 1)][h] = *reinterpret_cast<const f64x2 *>(Lj + 16 * h * ld + 8 * s);
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) load(s);
+    double old[2][2][4];
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) old[p][h][v] = T[(16 * p + 4 * v) * ld + 16 * h];
+    f64x4 d[2][2] = {};
+#pragma unroll
+    for (int s = 0; s < kBatches; ++s) {
+        if (s + kAhead < kBatches) load(s + kAhead);
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    d[p][h] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[s % (kAhead + 1)][p][e], fb[s % (kAhead + 1)][h][e],
+                                                                   d[p][h], 0, 0, 0);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) T[(16 * p + 4 * v) * ld + 16 * h] = old[p][h][v] - d[p][h][v];
 }
 
 // row blockIdx.x of the lower triangle: A += B (the two parts' updates of the
@@ -1218,6 +1292,11 @@ long coarse_matrix_len(const Coarse &C)
     return 2 * ((long)P.n[0] * P.n[0] + (long)P.n[1] * P.n[1]);
 }
 
+// Tiles of a step that are resident together: two workgroups per CU (their LDS).
+// Up to there both forms take the same time or the one launch less (4x32x32 at two
+// levels, 406 tiles: 1.30 ms both; 1029 periodic DOFs, up to 496: 0.64 against 0.68).
+constexpr int kCholFit = 512;
+
 static void launch_chol_steps(hipStream_t s, const CholStep &a, int np)
 {
     auto blocks = [&](int nt) { return dim3((unsigned)std::max(1, nt * (nt + 1) / 2), (unsigned)np); };
@@ -1229,7 +1308,13 @@ static void launch_chol_steps(hipStream_t s, const CholStep &a, int np)
         for (int q = 0; q < np; ++q)
             if (k + 1 < a.steps[q]) nt = std::max(nt, std::min(a.nt, a.n[q] / NB - k - 2));
         if (nt < 0) break;
-        k_chol_step2<<<blocks(nt), 256, 0, s>>>(a, k);
+        const int n2 = (nt + 1) / 2;
+        if (nt * (nt + 1) / 2 * np > kCholFit) {
+            k_chol_step2<true><<<dim3((unsigned)nt, (unsigned)np), 256, 0, s>>>(a, k);
+            k_chol_update<<<dim3((unsigned)(n2 * (n2 + 1) / 2), (unsigned)np), 256, 0, s>>>(a, k);
+        } else {
+            k_chol_step2<false><<<blocks(nt), 256, 0, s>>>(a, k);
+        }
     }
     if (last >= 0) k_chol_step<<<blocks(last), 256, 0, s>>>(a);
 }
