@@ -124,6 +124,19 @@ struct OpArgsT : OpModal<T> {
     int per;               // modal kernels: periodic cell, the result complete on masters and images
 };
 using OpArgs = OpArgsT<double>;
+template <class T>
+struct OpTile : OpStencil<T> {  // k_gather, k_stored
+    double *partials, cx_floor;
+    const float *Uf;
+    Tile t;
+    const T *Ke, *CX, *A;
+    T kv[kKeMaxClasses];
+    explicit OpTile(const OpArgsT<T> &a)
+        : OpStencil<T>(a), partials(a.partials), cx_floor(a.cx_floor), Uf(a.Uf), t(a.t), Ke(a.Ke), CX(a.CX), A(a.A)
+    {
+        for (int k = 0; k < kKeMaxClasses; ++k) kv[k] = a.kv[k];
+    }
+};
 
 enum OpMode {
     OP_MATVEC = 0,      // out = K U, masked; partials = sum U.out
@@ -225,6 +238,12 @@ __device__ __forceinline__ void batch_shift(OpStencil<T> &a)
 }
 template <class T>
 __device__ __forceinline__ void batch_shift(OpModal<T> &a)
+{
+    batch_shift(static_cast<OpStencil<T> &>(a));
+    a.partials = batch_ptr(a.partials, (long)gridDim.x);
+}
+template <class T>
+__device__ __forceinline__ void batch_shift(OpTile<T> &a)
 {
     batch_shift(static_cast<OpStencil<T> &>(a));
     a.partials = batch_ptr(a.partials, (long)gridDim.x);

@@ -38,7 +38,7 @@ __host__ __device__ constexpr int pidx(int m, int n) { return n <= m ? m * (m + 
 // No atomics: each output DOF is written by exactly one thread.
 // ---------------------------------------------------------------------------
 template <class T, int MODE, bool KC>
-__global__ __launch_bounds__(kBlock) void k_gather(OpArgsT<T> a)
+__global__ __launch_bounds__(kBlock) void k_gather(OpTile<T> a)
 {
     batch_shift(a);
     if (a.ctl && a.ctl[0]) return;
@@ -296,23 +296,24 @@ void launch_op0(hipStream_t s, int mode, const OpArgsT<T> &a, const CgTest *test
 {
     if (op0_is_modal(a, mode)) return launch_op0_modal<T>(s, mode, a, test);
     const dim3 grid((unsigned)xcd_launch(a.t.blocks()), 1, batch_dim(a.nb)), block(kBlock);
+    const OpTile<T> x(a);
     if (a.kc) {
         switch (mode) {
-        case OP_MATVEC: k_gather<T, OP_MATVEC, true><<<grid, block, 0, s>>>(a); break;
-        case OP_DEFECT: k_gather<T, OP_DEFECT, true><<<grid, block, 0, s>>>(a); break;
-        case OP_JACOBI: k_gather<T, OP_JACOBI, true><<<grid, block, 0, s>>>(a); break;
-        case OP_PRE_JACOBI: k_gather<T, OP_PRE_JACOBI, true><<<grid, block, 0, s>>>(a); break;
-        case OP_PRE_DEFECT: k_gather<T, OP_PRE_DEFECT, true><<<grid, block, 0, s>>>(a); break;
+        case OP_MATVEC: k_gather<T, OP_MATVEC, true><<<grid, block, 0, s>>>(x); break;
+        case OP_DEFECT: k_gather<T, OP_DEFECT, true><<<grid, block, 0, s>>>(x); break;
+        case OP_JACOBI: k_gather<T, OP_JACOBI, true><<<grid, block, 0, s>>>(x); break;
+        case OP_PRE_JACOBI: k_gather<T, OP_PRE_JACOBI, true><<<grid, block, 0, s>>>(x); break;
+        case OP_PRE_DEFECT: k_gather<T, OP_PRE_DEFECT, true><<<grid, block, 0, s>>>(x); break;
         default: break;
         }
         return;
     }
     switch (mode) {
-    case OP_MATVEC: k_gather<T, OP_MATVEC, false><<<grid, block, 0, s>>>(a); break;
-    case OP_DEFECT: k_gather<T, OP_DEFECT, false><<<grid, block, 0, s>>>(a); break;
-    case OP_JACOBI: k_gather<T, OP_JACOBI, false><<<grid, block, 0, s>>>(a); break;
-    case OP_PRE_JACOBI: k_gather<T, OP_PRE_JACOBI, false><<<grid, block, 0, s>>>(a); break;
-    case OP_PRE_DEFECT: k_gather<T, OP_PRE_DEFECT, false><<<grid, block, 0, s>>>(a); break;
+    case OP_MATVEC: k_gather<T, OP_MATVEC, false><<<grid, block, 0, s>>>(x); break;
+    case OP_DEFECT: k_gather<T, OP_DEFECT, false><<<grid, block, 0, s>>>(x); break;
+    case OP_JACOBI: k_gather<T, OP_JACOBI, false><<<grid, block, 0, s>>>(x); break;
+    case OP_PRE_JACOBI: k_gather<T, OP_PRE_JACOBI, false><<<grid, block, 0, s>>>(x); break;
+    case OP_PRE_DEFECT: k_gather<T, OP_PRE_DEFECT, false><<<grid, block, 0, s>>>(x); break;
     default: break;
     }
 }
@@ -378,7 +379,7 @@ __device__ __forceinline__ T stored_u(const OpStencil<T> &a, long dof)
 }
 
 template <class T, int MODE>
-__global__ __launch_bounds__(kBlock) void k_stored(OpArgsT<T> a)
+__global__ __launch_bounds__(kBlock) void k_stored(OpTile<T> a)
 {
     batch_shift(a);
     if (a.ctl && a.ctl[0]) return;
@@ -650,12 +651,13 @@ void launch_opA(hipStream_t s, int mode, const OpArgsT<T> &a)
         }
     }
     const dim3 grid((unsigned)a.t.blocks(), 1, batch_dim(a.nb)), block(kBlock);
+    const OpTile<T> x(a);
     switch (mode) {
-    case OP_MATVEC: k_stored<T, OP_MATVEC><<<grid, block, 0, s>>>(a); break;
-    case OP_DEFECT: k_stored<T, OP_DEFECT><<<grid, block, 0, s>>>(a); break;
-    case OP_JACOBI: k_stored<T, OP_JACOBI><<<grid, block, 0, s>>>(a); break;
-    case OP_PRE_JACOBI: k_stored<T, OP_PRE_JACOBI><<<grid, block, 0, s>>>(a); break;
-    case OP_PRE_DEFECT: k_stored<T, OP_PRE_DEFECT><<<grid, block, 0, s>>>(a); break;
+    case OP_MATVEC: k_stored<T, OP_MATVEC><<<grid, block, 0, s>>>(x); break;
+    case OP_DEFECT: k_stored<T, OP_DEFECT><<<grid, block, 0, s>>>(x); break;
+    case OP_JACOBI: k_stored<T, OP_JACOBI><<<grid, block, 0, s>>>(x); break;
+    case OP_PRE_JACOBI: k_stored<T, OP_PRE_JACOBI><<<grid, block, 0, s>>>(x); break;
+    case OP_PRE_DEFECT: k_stored<T, OP_PRE_DEFECT><<<grid, block, 0, s>>>(x); break;
     default: break;
     }
 }
@@ -665,10 +667,11 @@ void launch_op0_uf(hipStream_t s, const OpArgs &a)
 {
     if (op0_is_modal(a, OP_MATVEC_UF)) return launch_op0_modal<double>(s, OP_MATVEC_UF, a);
     const dim3 grid((unsigned)xcd_launch(a.t.blocks()), 1, batch_dim(a.nb)), block(kBlock);
+    const OpTile<double> x(a);
     if (a.kc)
-        k_gather<double, OP_MATVEC_UF, true><<<grid, block, 0, s>>>(a);
+        k_gather<double, OP_MATVEC_UF, true><<<grid, block, 0, s>>>(x);
     else
-        k_gather<double, OP_MATVEC_UF, false><<<grid, block, 0, s>>>(a);
+        k_gather<double, OP_MATVEC_UF, false><<<grid, block, 0, s>>>(x);
 }
 template void launch_op0<float>(hipStream_t, int, const OpArgsT<float> &, const CgTest *);
 template void launch_opA<double>(hipStream_t, int, const OpArgsT<double> &);
