@@ -158,10 +158,13 @@ struct CgScalars {
     int nru;         // replacements done
 };
 
+constexpr int kMaxBatch = 6;  // the six load cases of a homogenisation
+
 // The residual test, by one wave.  prog (pinned host memory) tells the host how
 // far the iteration is: iterations tested << 1 | converged in the low half, the
 // relative residual in FP32 in the high half; one 64-bit store, so the host never
-// sees them apart.
+// sees them apart.  The residual in FP64 is in the word kMaxBatch further on; the
+// host takes it once its rounding is the one in prog (cg_wait).
 constexpr int kCgBlocks = 256;  // blocks (= partial sums) of the PCG's reductions at most
 __device__ __forceinline__ void cg_test(const CgTest &t)
 {
@@ -200,6 +203,8 @@ __device__ __forceinline__ void cg_test(const CgTest &t)
     }
     const unsigned long long w =
         ((unsigned long long)__builtin_bit_cast(unsigned, (float)rel) << 32) | ((unsigned)(it + 1) << 1) | (unsigned)done;
+    __hip_atomic_store(t.prog + kMaxBatch, __builtin_bit_cast(unsigned long long, rel), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
     __hip_atomic_store(t.prog, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
@@ -212,7 +217,6 @@ __device__ __forceinline__ void cg_test(const CgTest &t)
 // with one right-hand side has blockIdx.z = 0 and is unchanged.
 static_assert(sizeof(CgScalars) % sizeof(int) == 0, "CgScalars stride in ints");
 constexpr int kCtlStride = (int)(sizeof(CgScalars) / sizeof(int));
-constexpr int kMaxBatch = 6;  // the six load cases of a homogenisation
 
 template <class P>
 __device__ __forceinline__ P *batch_ptr(P *p, long stride)

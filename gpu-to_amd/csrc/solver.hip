@@ -508,8 +508,9 @@ static void precond(gputo_handle *h, const double *r, double *z, bool r32_ready 
 // Wait until every right-hand side's progress word shows `seq` tested
 // iterations or convergence; true when all have converged.  rel: the relative
 // residual of the first.  The words come from k_cg_check; a stream that has
-// drained or failed without them ends the wait.
-static bool cg_wait(hipStream_t s, const unsigned long long *prog, int nb, int seq, float *rel)
+// drained or failed without them ends the wait.  The thread spins: a word is seen
+// within a microsecond, where a wait for the stream takes 20.
+static bool cg_wait(hipStream_t s, const unsigned long long *prog, int nb, int seq, double *rel)
 {
     for (long spins = 1;; ++spins) {
         bool all = true, done = true;
@@ -519,7 +520,13 @@ static bool cg_wait(hipStream_t s, const unsigned long long *prog, int nb, int s
             all = all && ((w & 1u) || (int)(w >> 1) >= seq);
         }
         if (all) {
-            if (rel) *rel = __builtin_bit_cast(float, (unsigned)(__atomic_load_n(&prog[0], __ATOMIC_RELAXED) >> 32));
+            if (rel) {
+                const unsigned r32 = (unsigned)(__atomic_load_n(&prog[0], __ATOMIC_RELAXED) >> 32);
+                for (int k = 0; k < 1000; ++k) {  // stored with prog[0], but in no order
+                    *rel = __builtin_bit_cast(double, __atomic_load_n(&prog[kMaxBatch], __ATOMIC_RELAXED));
+                    if (__builtin_bit_cast(unsigned, (float)*rel) == r32) break;
+                }
+            }
             return done;
         }
         if (spins % 65536 == 0) {
@@ -623,7 +630,7 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
     // convergence one enqueued iteration skips its work.
     const OpArgs mv = op_args(h, 0);
     int enq = 0;
-    h->prog[0] = 0;
+    h->prog[0] = h->prog[kMaxBatch] = 0;
     for (;;) {
         const int sl = enq % kCgLog;  // ring slot of this iteration's direction
         float *pk = p32 ? p32 + (long)sl * n : nullptr;
@@ -656,8 +663,8 @@ int run_pcg(gputo_handle *h, const double *F, double *U, double tol, int maxit, 
         ++enq;
         HIPCHK(hipGetLastError());
         if (enq > 1) {
-            float rel = 0.0f;
-            if (cg_wait(s, h->prog, 1, enq - 1, &rel)) break;
+            double rel = 0.0;
+            if (cg_wait(s, h->prog, 1, enq - 1, h->ln ? &rel : nullptr)) break;
             // the learned stage's fallback watches a trial's progress
             if (h->ln && (enq - 1) % 4 == 0)
                 learn_poll(h, enq - 1,
@@ -993,7 +1000,7 @@ int gputo_create(int nelx, int nely, int nelz, int nl, const gputo_params *param
         h->rr = dalloc<double>(h, 3 * kCgBlocks);
         h->sc = dalloc<CgScalars>(h, 1);
         HIPCHK(hipHostMalloc((void **)&h->sc_host, sizeof(CgScalars), hipHostMallocDefault));
-        HIPCHK(hipHostMalloc((void **)&h->prog, kMaxBatch * sizeof(unsigned long long), hipHostMallocDefault));
+        HIPCHK(hipHostMalloc((void **)&h->prog, 2 * kMaxBatch * sizeof(unsigned long long), hipHostMallocDefault));
         std::memset(h->sc_host, 0, sizeof(CgScalars));
         HIPCHK(hipMemcpy(h->sc, h->sc_host, sizeof(CgScalars), hipMemcpyHostToDevice));
         Coarse &C = h->C;
