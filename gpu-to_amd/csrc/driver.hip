@@ -4,7 +4,6 @@
 // MGCG solve, compliance sensitivities, OC bisection), with every
 // element-sized array resident in HBM.  Reductions are two-stage with a
 // fixed summation order.
-#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
@@ -30,8 +29,6 @@ struct ToBuffers {
     double *part = nullptr;  // reduction partials [32][kRedBlocks]
     OcState *oc = nullptr;  // the bisection's state
     double *red_host = nullptr;    // pinned: sums and the bisection's result (kSum...)
-    int *fixed_d = nullptr;
-    size_t nfixed = 0;       // room in fixed_d
     std::vector<void *> allocs;
 };
 
@@ -525,8 +522,8 @@ void gputo::to_destroy(gputo_handle *h)
     h->to = h->to_kept = nullptr;
 }
 
-// the buffers for a mesh of ne elements and ndof DOFs, and nfd fixed DOFs
-static void make_buffers(ToState *t, size_t ne, size_t ndof, size_t nfd)
+// the buffers for a mesh of ne elements and ndof DOFs
+static void make_buffers(ToState *t, size_t ne, size_t ndof)
 {
     if (!t->x) {
         double **el[] = {&t->x, &t->xPhys, &t->xOld, &t->Hs, &t->dHs, &t->dsK, &t->dc, &t->dv, &t->tmp, &t->ocP};
@@ -537,15 +534,6 @@ static void make_buffers(ToState *t, size_t ne, size_t ndof, size_t nfd)
         t->oc = talloc<OcState>(t, 1);
         t->w = talloc<double>(t, kMaxFilterWeights);
         check_hip(hipHostMalloc((void **)&t->red_host, kSumCount * sizeof(double), hipHostMallocDefault), "hostmalloc");
-    }
-    if (t->nfixed < nfd || !t->fixed_d) {
-        if (t->fixed_d) {
-            hipFree(t->fixed_d);
-            t->allocs.erase(std::find(t->allocs.begin(), t->allocs.end(), (void *)t->fixed_d));
-            t->fixed_d = nullptr;
-        }
-        t->fixed_d = talloc<int>(t, nfd);
-        t->nfixed = nfd;
     }
 }
 
@@ -649,7 +637,7 @@ int gputo_to_begin(gputo_handle *h, const double *Ke0, const double *x0, const d
         t->Ke.assign(Ke0, Ke0 + 576);
         t->fixed = std::move(fx);
         const long ne = g.nel;
-        make_buffers(t, ne, g.ndof, nfd);
+        make_buffers(t, ne, g.ndof);
         std::vector<double> w = filter_weights(cfg->rmin, &t->fw);
         hipStream_t s = h->stream;
         check_hip(hipMemcpyAsync(t->w, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, s), "copy");
@@ -657,8 +645,6 @@ int gputo_to_begin(gputo_handle *h, const double *Ke0, const double *x0, const d
                                {t->F, (void *)F, g.ndof * sizeof(double), false}};
         host_upload(h, in, 2);
         check_hip(hipMemcpyAsync(t->xPhys, t->x, ne * sizeof(double), hipMemcpyDeviceToDevice, s), "copy");
-        if (nfd)
-            check_hip(hipMemcpyAsync(t->fixed_d, t->fixed.data(), nfd * sizeof(int), hipMemcpyHostToDevice, s), "copy");
         launch_fill(s, t->xOld, ne, 1.0);  // xOld = 1 (top3D125mod.m:102)
         launch_fill(s, t->U, g.ndof, 0.0);
         launch_fill(s, t->tmp, ne, 1.0);
