@@ -1527,6 +1527,7 @@ int gputo_bench_level(gputo_handle *h, int level, int op, int fp32, int reps, do
 int gputo_coarse_solve_f64(gputo_handle *h, const double *b, double *x)
 {
     if (!h || !h->hier_ready || !b || !x) return GPUTO_ERR_ARGUMENT;
+    if (!h->C.direct) return GPUTO_ERR_ARGUMENT;  // smoothed: there is no factor
     try {
         Level &v = h->L[h->nl - 1];
         hipStream_t s = h->stream;

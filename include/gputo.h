@@ -278,7 +278,9 @@ int gputo_learn_grad(gputo_handle *h, const double *x, const double *gy, double 
 /* `steps` Adam steps (learning rate lr) on the samples of the last solve. */
 int gputo_learn_train(gputo_handle *h, int steps, double lr, double *loss_first, double *loss_last);
 
-/* Coarsest-level solve x = A_c^{-1} b (cholsl1, mgcg1.cu:2175-2232). */
+/* Coarsest-level solve x = A_c^{-1} b (cholsl1, mgcg1.cu:2175-2232);
+ * GPUTO_ERR_ARGUMENT where that level is smoothed instead (GPUTO_PRESET_MGCG9
+ * above 20000 DOFs). */
 int gputo_coarse_solve_f64(gputo_handle *h, const double *b, double *x);
 
 /* ---- index maps (bit-exact parity with the reference) ---------------- */

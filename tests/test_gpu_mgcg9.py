@@ -87,3 +87,14 @@ def test_mgcg9_matlab_interface(gputo, oracle):
     assert abs(cgiters - no) <= 1 and cgres < 1e-9
     assert rel(U, Uo) < 1e-7
     gputo.release_handles()
+
+
+def test_coarse_solve_without_a_factor_is_refused(gputo):
+    """A smoothed coarsest level has no factor to solve with."""
+    nelx, nely, nelz, nl = 64, 32, 32, 2
+    Ke, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=55, kind="smooth")
+    s = gputo.Solver(nelx, nely, nelz, nl, preset=MGCG9)
+    s.setup(Ke, CX, fixed)
+    with pytest.raises(gputo.GputoError):
+        s.coarse_solve(np.zeros(3 * 33 * 17 * 17))
+    s.close()
