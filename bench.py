@@ -19,11 +19,11 @@ sys.path[:0] = [os.path.join(ROOT, "gpu-to_amd"), os.path.join(ROOT, "oracle")]
 
 METRIC = "wall-s/TO iter @1.77M hex, mixed+learned vs FP64 MGCG; matvec HBM GB/s"
 HBM_PEAK_GBS = 8000.0
-FP64_PEAK_TFLOPS = 78.6
-FP32_PEAK_TFLOPS = 157.3
 PMC_SUMMARY = os.path.join(ROOT, "profiles", "level0_operator_cantilever_192x96x96_pmc.md")
 # variant -> (precision, level-0 kernel of the inner solve); kernel ids as
-# gputo_params.l0_kernel (0 = FP64 node-gather for the plain path)
+# gputo_params.l0_kernel (0 = the FP64 operator of the plain path).  The isotropic
+# Ke0 of this benchmark takes the FP64 or FP32 modal kernel for ids 0 to 4; a name
+# keeps the kernel that its id names for other element matrices.
 # name: (precision, level-0 kernel, sweeps before / after the coarse
 # correction on levels 0 and 1 of the FP32 V-cycle (0 = the preset's 3 / 3),
 # coarse_lag: V-cycles that use the previous design's coarsest factor[,
@@ -31,10 +31,10 @@ PMC_SUMMARY = os.path.join(ROOT, "profiles", "level0_operator_cantilever_192x96x
 # of the levels from 2 on[, sweeps of the levels from 3 on]]])
 VARIANTS = {
     "f64": (0, 0, 0, 0, 0),
-    "mixed_gather": (1, 1, 0, 0, 0),  # FP32 inner solve, FP32 node-gather level-0 operator
-    "mixed_mfma9": (2, 2, 0, 0, 0),   # MFMA level-0 operator, three-way BF16 split, all nine products
-    "mixed_mfma": (2, 4, 0, 0, 0),    # MFMA level-0 operator, three-way BF16 split, six products
-    "mixed_mfma3": (2, 3, 0, 0, 0),   # MFMA level-0 operator, two-way BF16 split, three products
+    "mixed_gather": (1, 1, 0, 0, 0),  # FP32 V-cycle with the preset's sweeps
+    "mixed_mfma9": (2, 2, 0, 0, 0),   # the same operators under three other ids
+    "mixed_mfma": (2, 4, 0, 0, 0),
+    "mixed_mfma3": (2, 3, 0, 0, 0),
     "mixed_mfma1": (2, 5, 0, 0, 0),   # MFMA level-0 operator, one BF16 product
     "mixed_mfma3s": (2, 3, 1, 3, 0),  # as mixed_mfma3 with 1 + 3 sweeps on levels 0 and 1
     "mixed_mfma3s3": (2, 3, 1, 3, 3),  # and the previous coarsest factor in the first 3 V-cycles
@@ -448,11 +448,10 @@ def main():
     base = res.get("f64")
 
     # roofline of the dominant kernel (the level-0 operator of the head
-    # variant).  The node-gather kernels (0: FP64, 1: FP32) run their 1152
-    # flop per element on the vector ALUs, an arithmetic intensity above the
-    # ridge of both precisions: priced against the compute peak of their
-    # type.  The MFMA kernels (2-5) have the element products on the matrix
-    # cores at a small fraction of their peak: priced against HBM.
+    # variant), priced against HBM: the modal kernels execute about 190
+    # operations per element and the one-product MFMA kernel (5) has its products
+    # on the matrix cores, both a small fraction of their peaks.  1152 flop per
+    # element is what the plain 24 x 24 product takes.
     kernel = variant_of(head)[1]
     s_bytes = 8 if kernel == 0 else 4
     op_bytes = (2 * ndof + nel) * s_bytes
@@ -460,13 +459,8 @@ def main():
     op_s = r["op_ms"] * 1e-3 if r["op_ms"] else None
     default_size = (args.nelx, args.nely, args.nelz, args.nl) == (192, 96, 96, 5)
     traffic = pmc_traffic(kernel) if default_size else None
-    if kernel <= 1:
-        roof = {"bound": "mfma", "achieved": op_flops / op_s / 1e12 if op_s else None,
-                "peak": FP64_PEAK_TFLOPS if kernel == 0 else FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "traffic": traffic}
-    else:
-        roof = {"bound": "hbm", "achieved": op_bytes / op_s / 1e9 if op_s else None, "peak": HBM_PEAK_GBS,
-                "unit": "GB/s", "traffic": traffic}
+    roof = {"bound": "hbm", "achieved": op_bytes / op_s / 1e9 if op_s else None, "peak": HBM_PEAK_GBS,
+            "unit": "GB/s", "traffic": traffic}
     roof["frac"] = roof["achieved"] / roof["peak"] if roof["achieved"] else None
 
     out = {
@@ -491,7 +485,9 @@ def main():
         },
         "roofline": roof,
         "matvec": {
-            "kernel": "level-0 operator y = K(E) u (%s)" % head,
+            "kernel": "level-0 operator y = K(E) u, %s (%s)"
+                      % ({0: "FP64 modal kernel", 5: "one-product BF16 MFMA kernel"}.get(kernel, "FP32 modal kernel"),
+                         head),
             "ms": r["op_ms"],
             "gelem_per_s": nel / op_s / 1e9 if op_s else None,
             "hbm_gbps_algorithmic": op_bytes / op_s / 1e9 if op_s else None,

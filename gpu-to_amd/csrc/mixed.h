@@ -1,5 +1,5 @@
 // Mixed-precision solve (FP64 iterative refinement around an FP32 inner PCG
-// with an FP32 node-gather or split-BF16 MFMA level-0 operator).
+// with the FP32 modal, node-gather or split-BF16 MFMA level-0 operator).
 #pragma once
 
 #include <vector>

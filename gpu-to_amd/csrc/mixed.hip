@@ -6,8 +6,9 @@
 // what it converges to.  (An FP32 Krylov loop does not reach 1e-8: the FP32
 // operator applied to a smooth field has a relative error of about
 // 6e-8 (L/h)^2, 2e-3 at 192 elements, so its true residual stalls.)  The
-// level-0 FP32 operator is the node-gather kernel or one of the MFMA element
-// kernels (mfma.hip).
+// level-0 FP32 operator is the modal kernel (modal.hip); for a Ke0 without its
+// form, and for the one-product flavour, the node-gather kernel or one of the MFMA
+// element kernels (mfma.hip).
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -90,7 +91,8 @@ void mixed_stats(gputo_handle *h, gputo_to_stats *st)
 }
 
 // Level-0 kernel of the FP32 operators: explicit choice, else the FP32
-// node-gather for MIXED_F32 and the three-way split-BF16 MFMA for MIXED_BF16.
+// node-gather for MIXED_F32 and the three-way split-BF16 MFMA for MIXED_BF16
+// (l0_resolve: the modal kernel in the place of either where Ke0 has its form).
 static int l0_kind(const gputo_params &p, int precision)
 {
     if (p.l0_kernel >= L0_GATHER && p.l0_kernel <= L0_MFMA_BF16X1) return p.l0_kernel;

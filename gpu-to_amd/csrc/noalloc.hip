@@ -6,13 +6,12 @@
 // serving loops.  The caller passes device inputs and outputs.
 //
 // An isotropic Ke0 takes the modal kernel without a mask and then zeroes the
-// fixed DOFs of y: two launches and no memory of its own (three launches,
-// with the mask cleared and set first, took 46.6 us per call at 192x96x96
-// against 39.8 us).  Any other Ke0 with
-// the unit-H8 entry structure takes the node-gather kernel, whose one-byte-
-// per-node fixed-DOF mask lives in `scratch`, a static device array of
-// kScratchBytes per GPU, held until the process ends.  Every such call on a
-// GPU shares that GPU's array, so calls that overlap on one GPU race.
+// fixed DOFs of y: two launches and no memory of its own, 37.4 us per call at
+// 192x96x96 (three launches, with the mask cleared and set first: 7 us more).  Any
+// other Ke0 with the unit-H8 entry structure takes the node-gather kernel (73 us),
+// whose one-byte-per-node fixed-DOF mask lives in `scratch`, a static device array
+// of kScratchBytes per GPU, held until the process ends.  Every such call on a GPU
+// shares that GPU's array, so calls that overlap on one GPU race.
 #include <algorithm>
 #include <cstring>
 #include <mutex>

@@ -785,7 +785,8 @@ static void batch_view(HierView<T> &H, T *const (&v)[kMaxLevels][4], int nl, int
 // smoother, coarsest solve and vector launch applies to all nb vectors, each
 // with its own CG scalars, and a right-hand side that has converged skips
 // the rest (its control word).  The FP32 V-cycle of the mixed path applies
-// level 0 with the FP32 node-gather kernel, whose launches take a batch.
+// level 0 with the FP32 modal kernel, or for a Ke0 without its form with the
+// node-gather: their launches take a batch, the MFMA kernels' do not.
 int run_pcg_batch(gputo_handle *h, const double *F, double *U, int nb, double tol, int maxit, double *relres,
                   int *nit)
 {

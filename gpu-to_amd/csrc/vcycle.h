@@ -257,10 +257,11 @@ void sweeps_t(const gputo_handle *h, const HierView<T> &H, int l, const T *F, T 
         pre = false;
     }
     if (pre && l == 0 && n > 0 && !H.mg9 && H.l0 >= L0_MFMA_F32) {
-        // MFMA level 0: the prerelaxed iterate is written by an elementwise
-        // pass and the first sweep is a plain one (measured at 192x96x96:
-        // 11 + 64 us against 93 us for the fused form, which stages F and AD
-        // for every halo node; the FP64 node-gather keeps its fused form,
+        // FP32 modal and MFMA level 0: the prerelaxed iterate is written by an
+        // elementwise pass (in the CG loop by the residual update, which has r at
+        // hand) and the first sweep is a plain one: an MFMA kernel's 11 + 64 us
+        // against 93 us for the fused form at 192x96x96, which stages F and AD for
+        // every halo node.  The FP32 node-gather keeps its fused form (in FP64
         // 87 us against 22 + 70 us).  It goes where the sweeps end in U.
         in_tmp = n % 2 == 1;
         if (!H.pre0_ready)
