@@ -9,9 +9,13 @@ solves one of 1e-9, which keeps them as well posed as with Ke0 and is far from
 what passes as isotropic (1e-14).
 
 Tolerances as with the isotropic Ke0: relative to max|y|, FP64 1e-13 (summation
-order), FP32 2e-6, the hi+lo split 1e-4; solves to 1e-10 agree to 1e-7, FP64 in
-the oracle's iterations within one, mixed within two more (the hi+lo split: 40);
-homogenised tensors to 1e-8."""
+order), FP32 2e-6, the hi+lo split 1e-4; solves to 1e-10 agree to 1e-7, mixed in
+at most two iterations more than FP64 (the hi+lo split: 40); homogenised tensors
+to 1e-8.  The FP64 solve follows the oracle's: its residual after ten iterations
+agrees to 1e-6 of its value, the rounding of two summation orders times the growth
+of as many iterations.  (The oracle's count is no function of the input: its
+threads' sums are added in any order, and it ends this solve after 29 or 31
+iterations, as 1e-10 falls.)"""
 import ctypes
 import os
 import re
@@ -76,17 +80,23 @@ def test_solve(gputo, oracle, kw, kind):
     _, F, CX, fixed = cantilever_case(nelx, nely, nelz, seed=84, kind="smooth")
     Ke = element(gputo, kind, 1e-9)
     preset = kw.get("preset", 0)
-    Uo, ro, no, rco = oracle.mgcg(Ke, F, CX, fixed, nelx, nely, nelz, nl, 1e-10, 300, preset=preset, nswp=2)
+    Uo, _, no, rco = oracle.mgcg(Ke, F, CX, fixed, nelx, nely, nelz, nl, 1e-10, 300, preset=preset, nswp=2)
     s = gputo.Solver(nelx, nely, nelz, nl, **kw)
     U, r, n, rc = s.solve(Ke, F, CX, fixed, 1e-10, 300)
-    s.close()
-    print("iterations", no, n, flush=True)
     assert rc == 0 and rco == 0 and r < 1e-10 and no < 300
-    if kw.get("precision"):
-        assert n <= no + (40 if kw.get("l0_kernel") == 3 else 2)
-    else:
-        assert abs(n - no) <= 1
     assert rel(U, Uo) < 1e-7
+    if kw.get("precision"):
+        s64 = gputo.Solver(nelx, nely, nelz, nl, preset=preset, nswp=kw.get("nswp", 0))
+        n64 = s64.solve(Ke, F, CX, fixed, 1e-10, 300)[2]
+        s64.close()
+        print("iterations", n64, n, flush=True)
+        assert n <= n64 + (40 if kw.get("l0_kernel") == 3 else 2)
+    else:
+        r10 = s.solve(Ke, F, CX, fixed, 1e-10, 10)[1]
+        ro10 = oracle.mgcg(Ke, F, CX, fixed, nelx, nely, nelz, nl, 1e-10, 10, preset=preset, nswp=2)[1]
+        print("residuals", ro10, r10, flush=True)
+        assert abs(r10 - ro10) <= 1e-6 * ro10
+    s.close()
 
 
 @pytest.mark.parametrize("kind", ["classes", "full"])
