@@ -1151,11 +1151,17 @@ ModalWork modal_work(const Grid &g, int bytes, int el, int children)
     const int waves = bytes == 8 ? (el ? 1 : 2) : (el ? 3 : 4);  // resident per SIMD (md_min_waves)
     const double per_wave = el ? 0.9 : 0.38;                     // a wave's layer with its SIMD alone, in us
     const double latency = 1.2;
+    // Eight strips at most, more where even those are longer than two waves: a block
+    // works on R + 1 entries before its own, and 8 strips of 3801 nodes left 27 of
+    // 504 entries to it (20 mgcg9 iterations at 8x3800x8 9.8 -> 11.4 ms against the
+    // node-gather, 7.4 now), or none.
+    constexpr int kMdLongStrip = 126;
     double cost = 0.0;
     for (int NW = 1; NW <= (bytes == 8 && el ? 4 : kMdMaxWaves); NW *= 2)
-        for (int ns = 1; ns <= 8; ++ns) {
+        for (int ns = 1;; ++ns) {
             const int W = (g.nny + ns - 1) / ns, R = W + 1;
             if (ns > 1 && W < 12) break;
+            if (ns > 8 && W <= kMdLongStrip) break;
             if (63 * NW - R < 16) continue;
             const int M = std::min(63 * NW - R, R * g.nnz);
             const int nsr = (g.nny + W - 1) / W, nch = (R * g.nnz + M - 1) / M;

@@ -202,3 +202,8 @@ def test_level1_tiling_follows_the_preset(gputo, presets, precision):
     s.close()
     assert rc == 0 and n == nf < 200
     assert rel(U, Uf) < 1e-10 if presets == (0, 1) else np.array_equal(U, Uf)
+
+
+def test_long_rows_take_more_than_eight_strips(gputo, oracle):
+    """Rows of 2601 and 1301 nodes, FP64 and FP32, all modes."""
+    check_levels(gputo, oracle, (4, 2600, 4, 3), [0, 1])
