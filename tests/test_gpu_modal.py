@@ -205,5 +205,5 @@ def test_level1_tiling_follows_the_preset(gputo, presets, precision):
 
 
 def test_long_rows_take_more_than_eight_strips(gputo, oracle):
-    """Rows of 2601 and 1301 nodes, FP64 and FP32, all modes."""
-    check_levels(gputo, oracle, (4, 2600, 4, 3), [0, 1])
+    """Rows of 2305 nodes: ten strips in FP64 and fourteen in FP32; level 1 below them."""
+    check_levels(gputo, oracle, (8, 2304, 8, 4), [0, 1])
